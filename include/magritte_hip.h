@@ -367,7 +367,7 @@ int mgr_compute_image(mgr_ctx *ctx, int64_t ray, int precision, double *I_m, dou
 
 /* Launch shape of the radiation-field kernel chosen by its autotuner (no
  * counterpart in the reference): waves of 64 frequency bins per workgroup and
- * traced steps staged per chunk, 0 before the first radiation field of that
+ * points staged per window, 0 before the first radiation field of that
  * precision; with capacity > 0 also the shapes tried by the last tuning and
  * their times on the tuning slice (ms).                                       */
 int mgr_radiation_field_shape(mgr_ctx *ctx, int precision, int *waves_per_group, int *steps_per_chunk,
@@ -381,11 +381,14 @@ int mgr_radiation_field_shape(mgr_ctx *ctx, int precision, int *waves_per_group,
 int mgr_set_radiation_field_shape(mgr_ctx *ctx, int precision, int waves_per_group, int steps_per_chunk);
 
 /* Out-of-window skip of the radiation-field kernels (no counterpart in the
- * reference; on by default): steps at which no bin of a 64-bin wave comes
- * within 10.5 line widths of any line (FP32; the profiles are exactly 0 there)
- * or 11 (1 + 1e-6) widths (FP64; get_eta_and_chi's own window holds no line)
- * are eliminated with eta = 0 and chi at its floor without evaluating the
- * profiles; results are bit-identical either way.  Off evaluates every point. */
+ * reference; on by default): points at which no bin of a 64-bin wave comes
+ * within a window of any line are not evaluated.  FP32: the window is as wide
+ * as the lines' opacity can be felt beside the opacity floor and the radiation
+ * behind it (10.5 widths, where the profiles are exactly 0, at most), and of a
+ * run of such points only the first and the last are evaluated.  FP64: 11
+ * (1 + 1e-6) widths (get_eta_and_chi's own window holds no line), and the
+ * points are eliminated with eta = 0 and chi at its floor.  Results are
+ * bit-identical either way.  Off evaluates every point.                      */
 int mgr_set_window_skip(mgr_ctx *ctx, int enable);
 /* Far-end intensity cache (no counterpart in the reference; on by default):
  * the rescaled boundary intensity entering every (origin, ray) and bin,
@@ -396,7 +399,8 @@ int mgr_set_window_skip(mgr_ctx *ctx, int enable);
  * Results are bit-identical either way; off frees it.                        */
 int mgr_set_far_cache(mgr_ctx *ctx, int enable);
 /* Interpolated points x 64-bin chunks of the cached trace, and how many of
- * them the skip leaves out (chunks beyond the fifth are never skipped).      */
+ * them lie in steps beyond 10.5 widths of every line (chunks beyond the fifth
+ * are never skipped).                                                        */
 int mgr_window_skip_stats(mgr_ctx *ctx, int64_t *point_chunks, int64_t *skipped);
 
 /* Kernel time of the last mgr_compute_radiation_field, measured with HIP

@@ -65,6 +65,13 @@ constexpr double MASK_WINDOW = 10.5;
 // any sub-point whatever the rounding of the shift (~1e-16): eta = 0 and chi
 // at the floor exactly, the values the out-of-window branch uses.
 constexpr double MASK_WINDOW64 = 11.0 * (1.0 + 1e-6);
+// The narrow window of the FP32 kernel's runs: beyond it every line's profile
+// times its opacity is below NEAR_CHI of the opacity floor, all lines together.
+constexpr double NEAR_CHI = 0.5, NEAR_X = 1.0 + NEAR_CHI;
+// The sub-points of a step that can lie in the window of a 64-bin chunk, as
+// 256ths of its n sub-points: sub-point m is out of it for m <= floor(lo n / 256)
+// and for m > ceil((hi + 1) n / 256), with lo | hi << 8.
+constexpr unsigned SPAN_ALL = 0xFF00, SPAN_NONE = 0x00FF;
 constexpr int MAX_INTERPOLATION = 10000; // geometry.tpp:138
 
 // One neighbour entry of the tracer: the neighbour's index and position, so
@@ -175,6 +182,7 @@ struct mgr_ctx {
     std::vector<int64_t> boundary2cell;    // [NB]
     std::vector<int64_t> lam_f_off, lam_f; // CSR: sorted f of each transition k
     std::vector<int64_t> h_cp_num;         // [ncolpar] species of each collision partner
+    std::vector<double>  h_A, h_Bs, h_Ba;  // [L] line data, species after species
 
     // device: static model
     double  *pos = nullptr, *vel = nullptr;        // [N*3]
@@ -298,6 +306,13 @@ struct mgr_ctx {
     // any of the step's sub-points; valid for the current trace and frequencies
     uint8_t *step_mask = nullptr;   // [total segments]
     bool     masks_valid = false;
+    // per 64-bin chunk and step, the sub-points in the window of the FP32 kernel's
+    // runs (set with step_mask, when near_on) and of the FP64 kernel (SPAN_*)
+    uint16_t *span32 = nullptr, *span64 = nullptr;
+    int64_t  span_stride = 0;
+    bool     near_on = false;
+    float   *near_p = nullptr;      // [L + 1] bound on p behind span32, per sorted line and for bins of several
+    int32_t *near_bad = nullptr;    // set when a population exceeds twice its cell's total (until they are set anew)
     uint8_t *step_mask64 = nullptr; // [total segments] the FP64 kernel's bits (MASK_WINDOW64)
     bool     masks64_valid = false;
     float    hdz32_max = 0.0f;      // largest dz' of the cached steps (set with the masks)
@@ -365,6 +380,7 @@ int upload_models(mgr_ctx *ctx, const mgr_model_view *models, int64_t nmodels);
 int free_model(mgr_ctx *ctx);
 int launch_cell_tables(mgr_ctx *ctx);
 int launch_emissivity_opacity(mgr_ctx *ctx);
+int clear_near_bad(mgr_ctx *ctx);   // before the rows of newly set populations (outside graph capture)
 int launch_trace(mgr_ctx *ctx);
 int launch_forward_masks(mgr_ctx *ctx);   // candidate neighbours of every (cell, ray), once
 int launch_radiation_field(mgr_ctx *ctx, int precision);   // kernel + Lambda*

@@ -223,7 +223,8 @@ __global__ void k_emissivity_opacity(int64_t N, const LineTables *__restrict__ t
                                      const int32_t *__restrict__ jrad, const double *__restrict__ pop_all,
                                      const double *__restrict__ IW64, const double *__restrict__ W11,
                                      double *__restrict__ emis, double *__restrict__ opac,
-                                     float4 *__restrict__ row32, double4 *__restrict__ row64)
+                                     float4 *__restrict__ row32, double4 *__restrict__ row64,
+                                     const double *__restrict__ pop_tot, int32_t *__restrict__ near_bad)
 {
     const int L = tb->L;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -245,6 +246,9 @@ __global__ void k_emissivity_opacity(int64_t N, const LineTables *__restrict__ t
     const double ks = o * CHI_SCALE * pref;
     const double iw = IW64[p * L + l];
     row64[p * L + l] = make_double4(W11[p * L + l], iw, es, ks);
+    // the bound behind the FP32 kernel's spans
+    const double most = 2.0 * pop_tot[sp * N + p];
+    if (!(fabs(pop[p * V + i]) <= most && fabs(pop[p * V + j]) <= most)) *near_bad = 1;
     // FP32 row: 1/width scaled by sqrt(log2 e) so that exp(-x^2) = exp2(-x'^2)
     row32[p * L + l] = make_float4((float)(iw * SQRT_LOG2E), (float)es, (float)ks, 0.0f);
 }
@@ -267,8 +271,14 @@ int launch_emissivity_opacity(mgr_ctx *ctx)
     hipLaunchKernelGGL(k_emissivity_opacity, dim3(grid_for(ctx->N * ctx->L, 256)), dim3(256), 0,
                        ctx->stream, ctx->N, ctx->tables, ctx->A, ctx->Bs, ctx->Ba, ctx->irad,
                        ctx->jrad, ctx->pop, ctx->IW64, ctx->W11, ctx->emis, ctx->opac, ctx->row32,
-                       ctx->row64);
+                       ctx->row64, ctx->pop_tot, ctx->near_bad);
     MGR_LAUNCH_CHECK();
+    return MGR_OK;
+}
+
+int clear_near_bad(mgr_ctx *ctx)
+{
+    MGR_HIP(hipMemsetAsync(ctx->near_bad, 0, sizeof(int32_t), ctx->stream));
     return MGR_OK;
 }
 
@@ -675,6 +685,9 @@ int upload_models(mgr_ctx *ctx, const mgr_model_view *models, int64_t nmodels)
     if ((rc = upload(ctx, &ctx->vturb2, m->vturb2, N))) return rc;
     if ((rc = upload(ctx, &ctx->abundance, m->abundance, N * m->nspecs))) return rc;
     if ((rc = upload(ctx, &ctx->tables, &tb, 1))) return rc;
+    ctx->h_A = A_all;
+    ctx->h_Bs = Bs_all;
+    ctx->h_Ba = Ba_all;
     if ((rc = upload(ctx, &ctx->A, A_all.data(), L))) return rc;
     if ((rc = upload(ctx, &ctx->Bs, Bs_all.data(), L))) return rc;
     if ((rc = upload(ctx, &ctx->Ba, Ba_all.data(), L))) return rc;
@@ -725,6 +738,8 @@ int upload_models(mgr_ctx *ctx, const mgr_model_view *models, int64_t nmodels)
     if ((rc = dalloc(ctx, &ctx->Lam, N * F))) return rc;
     if ((rc = dalloc(ctx, &ctx->Ls, N * L))) return rc;
     if ((rc = dalloc(ctx, &ctx->Lpart, N * ((F + WAVE - 1) / WAVE) * L))) return rc;
+    if ((rc = dalloc(ctx, &ctx->near_p, L + 1))) return rc;
+    if ((rc = dalloc(ctx, &ctx->near_bad, 1))) return rc;
     if ((rc = dalloc(ctx, &ctx->Jlin, N * L))) return rc;
     if ((rc = dalloc(ctx, &ctx->Jeff, N * L))) return rc;
     if ((rc = dalloc(ctx, &ctx->Jdif, N * L))) return rc;
@@ -746,6 +761,7 @@ int upload_models(mgr_ctx *ctx, const mgr_model_view *models, int64_t nmodels)
     if ((rc = dalloc(ctx, &ctx->shift_bits, 2))) return rc;
     MGR_HIP(hipHostMalloc((void **)&ctx->h_reduced, 8 * sizeof(double), hipHostMallocDefault));
     MGR_HIP(hipMemset(ctx->err_flag, 0, sizeof(int32_t)));
+    MGR_HIP(hipMemset(ctx->near_bad, 0, sizeof(int32_t)));
     MGR_HIP(hipMemset(ctx->prev1, 0, N * V * sizeof(double)));
     MGR_HIP(hipMemset(ctx->prev2, 0, N * V * sizeof(double)));
     MGR_HIP(hipMemset(ctx->prev3, 0, N * V * sizeof(double)));
@@ -787,7 +803,8 @@ int free_model(mgr_ctx *ctx)
     dfree(ctx->Jeff); dfree(ctx->Jdif); dfree(ctx->err_flag); dfree(ctx->seg_off); dfree(ctx->nseg);
     dfree(ctx->npts); dfree(ctx->seg_cell); dfree(ctx->seg_shift); dfree(ctx->seg_dZ);
     dfree(ctx->seg_f32); dfree(ctx->seg_hdz32); dfree(ctx->far_cell); dfree(ctx->far_shift);
-    dfree(ctx->step_mask); dfree(ctx->step_mask64);
+    dfree(ctx->step_mask); dfree(ctx->step_mask64); dfree(ctx->span32); dfree(ctx->span64);
+    dfree(ctx->near_p); dfree(ctx->near_bad);
     dfree(ctx->far_I32);
     dfree(ctx->far_I64);
     dfree(ctx->shift_bits); dfree(ctx->partials); dfree(ctx->reduced);
@@ -1018,7 +1035,8 @@ int mgr_compute_LTE_level_populations(mgr_ctx *ctx)
                            ctx->pop + ctx->N * ctx->sp_voff[l], ctx->pop_tot + ctx->N * l);
         MGR_LAUNCH_CHECK();
     }
-    int rc = launch_emissivity_opacity(ctx);
+    int rc = clear_near_bad(ctx);
+    if (!rc) rc = launch_emissivity_opacity(ctx);
     if (rc) return rc;
     MGR_HIP(hipStreamSynchronize(ctx->stream));
     ctx->pops_set = true;
@@ -1048,6 +1066,7 @@ int mgr_set_populations(mgr_ctx *ctx, const double *population)
     if (!ctx || !population) return MGR_ERR_ARGUMENT;
     int rc = copy_in(ctx, ctx->pop, population, ctx->N * ctx->V * sizeof(double));
     if (rc) return rc;
+    if ((rc = clear_near_bad(ctx))) return rc;
     if ((rc = launch_emissivity_opacity(ctx))) return rc;
     MGR_HIP(hipStreamSynchronize(ctx->stream));
     ctx->pops_set = true;

@@ -934,6 +934,7 @@ extern "C" int mgr_warm_start(mgr_ctx *ctx, mgr_mlp *mlp)
                            (int)OUT, (int)ctx->L, ctx->irad, ctx->jrad, ctx->Ba, ctx->Bs, dPrev, ctx->pop, dCount);
         if (hipGetLastError() != hipSuccess) rc = ctx->fail(MGR_ERR_DEVICE, "warm-start launch failed");
     }
+    if (!rc) rc = clear_near_bad(ctx);
     if (!rc) rc = launch_emissivity_opacity(ctx);
     unsigned long long nfb = 0;
     if (!rc && (hipMemcpyAsync(&nfb, dCount, sizeof(nfb), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||

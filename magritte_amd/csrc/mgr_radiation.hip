@@ -10,18 +10,24 @@
 // image kernel (Simulation::compute_and_write_image) reuses the same staging
 // and elimination on a rest-frame trace.
 //
-// Work mapping (CDNA4, 64-wide wavefronts): one workgroup per origin cell,
-// one wavefront per chunk of 64 frequency bins (lane = bin).  The workgroup
-// loops over the nrays/2 ray pairs of its origin.  For every ray it stages the
-// cached traced steps, chunk by chunk, into LDS together with the line rows of
-// their cells (11 width, 1/width and the emissivity/opacity prefactors per
-// line), so that the sweep reads uniform LDS broadcasts instead of dependent
-// global gathers.  The interpolation split of every step (set_data,
-// geometry.tpp:100-207) is precomputed at trace time (FP32) or computed once
-// while staging (FP64).  J and the Lambda*
+// Work mapping (CDNA4, 64-wide wavefronts): one wavefront per origin cell and
+// chunk of 64 frequency bins (lane = bin).  The wave loops over the nrays/2 ray
+// pairs of its origin.  For every pair it lays out, from the cached traced
+// steps, the points that can lie in a line window (lane = step, then lane =
+// point; the spans of sub-points in the window are precomputed with the
+// trace), brings their line rows (1/width and the emissivity/opacity
+// prefactors per line) into LDS and walks them (sweep_pair).  J and the Lambda*
 // diagonal accumulate in FP64 registers over rays and are written once per
 // (cell, bin): no atomics.  Workgroups are mapped to XCDs in contiguous origin
 // ranges so that neighbouring origins share an L2.
+//
+// Bound: vector-instruction issue.  On the 64^3 envelope (48 rays, 186 bins) the
+// FP32 kernel issues 2.0e10 vector instructions in 32 ms, 1.0 of one
+// non-transcendental instruction per CU and cycle, of which the points' profiles
+// and recurrences are 19.5 per point and wave, 65 % of all.  Decoding each
+// step in the elimination loop and stepping every point took 49 ms; on the
+// stress envelope (36^3, ~10 points per step) 44 against 19 ms.  FP64: 221
+// against 167 ms and 192 against 105 ms.
 //
 // The tridiagonal Feautrier system of a ray pair is solved two-sided: each ray
 // of the pair is eliminated from its boundary inwards in the Rybicki-Hummer
@@ -84,52 +90,26 @@ template <> struct Prec<float> {
 };
 template <> struct Prec<double> {
     using row_t = double4;  // (11 width, 1/width, E, K)
-    // the hardware reciprocal and two Newton steps (within an ulp or so of
-    // 1/x; the elimination's arguments are normal numbers, chi scaled and
-    // 1 + c x >= 1)
+    // the hardware reciprocal r (measured within 4.6e-8 of 1/x) times
+    // 1/(1 - e) ~ 1 + e + e^2 of its residual e = 1 - x r: within an ulp (1.1e-16
+    // measured), as two Newton steps, one instruction fewer.  The elimination's
+    // arguments are normal numbers (chi scaled and 1 + c x >= 1).
     static __device__ __forceinline__ double rcp(double x)
     {
-        double r = __builtin_amdgcn_rcp(x);
-        double e = __builtin_fma(-x, r, 1.0);
-        r = __builtin_fma(r, e, r);
-        e = __builtin_fma(-x, r, 1.0);
-        return __builtin_fma(r, e, r);
+        const double r = __builtin_amdgcn_rcp(x);
+        const double e = __builtin_fma(-x, r, 1.0);
+        return __builtin_fma(r, __builtin_fma(e, e, e), r);
     }
 };
 
-// One traced step in LDS.  Sub-point m = 1..n of the step lies at
-// shift = s0 + m ds (FP64: s0 = shift of the current point, FP32: s0 and ds
-// are shift - 1 and its increment) with path-length factor dz = dZ HDZ_SCALE and
-// belongs to the current cell for m < half, to `cell` otherwise.
-template <typename real>
+// One traced step in LDS (image kernels).  Sub-point m = 1..n of the step lies
+// at shift s0 + m ds with path-length factor dz = dZ HDZ_SCALE and belongs to
+// the current cell for m < half, to `cell` otherwise.
 struct alignas(32) Step {
-    real    s0, ds, dz;   // first sub-point shift (offset), shift increment, dz'
-    int32_t nh;           // n | half << 14 | out-of-window bits << 27 (STEP_*): one 16-byte read with the above
+    double  s0, ds, dz;
+    int32_t nh;           // n | half << 14 (STEP_*)
     int32_t cell;
 };
-
-// Steps staged for a kernel: the FP32 split of the radiation field, or the
-// FP64 split (FP64 kernels, and the FP32 image, whose shifts stay FP64).
-template <typename real, bool X64> struct StepOf { using type = Step<real>; };
-template <> struct StepOf<float, true> { using type = Step<double>; };
-template <typename real, bool X64> using step_t = typename StepOf<real, X64>::type;
-
-// The sweep's view of staged step e: one 16-byte LDS read for an FP32 record.
-__device__ __forceinline__ void read_step(const Step<float> *st, int e, float &s0, float &ds, float &dz, int &nh)
-{
-    const float4 v = reinterpret_cast<const float4 *>(st + e)[0];
-    s0 = v.x;
-    ds = v.y;
-    dz = v.z;
-    nh = __float_as_int(v.w);
-}
-__device__ __forceinline__ void read_step(const Step<double> *st, int e, double &s0, double &ds, double &dz, int &nh)
-{
-    s0 = st[e].s0;
-    ds = st[e].ds;
-    dz = st[e].dz;
-    nh = st[e].nh;
-}
 
 template <typename real>
 struct RFArgs {
@@ -153,8 +133,11 @@ struct RFArgs {
     uint64_t       L_magic;                   // ceil(2^32 / L): idx / L = (idx * L_magic) >> 32
     const double  *origin_shift;              // FP64 shift of the origin per entry (null: 1, co-moving)
     const uint8_t *step_mask;                 // per step, out-of-window bit per 64-bin chunk (or null)
-    float          noop_lo, noop_hi;          // an out-of-window sub-point after another is an exact no-op on
-                                              // (y, z, p) when noop_lo < y < noop_hi (noop_lo = inf: never)
+    const uint16_t *span;                     // per chunk and step, the sub-points in the window (SPAN_*; or null)
+    int64_t        span_stride;               // steps of a chunk
+    const float   *near_p;                    // FP32: [L + 1] the spans' bound on p per line, and for bins of several lines
+    const int32_t *near_bad;                  // FP32: set when a population exceeds the bounds behind the spans
+    float          noop_lo, noop_hi;          // y in (noop_lo, noop_hi): a run's inner points change nothing
     bool           root_major;                // lane order (lane_bin)
     const int32_t *cell2bdy, *antipod;        // antipod: global ray indices
     const int32_t *cell_model;                // [N] model of each cell
@@ -176,37 +159,65 @@ struct RFArgs {
     int64_t        band_S;                    // band slots per origin
     double        *band_part;                 // [N][nchunk][band_S][L]
     size_t         line_offset;               // FP64: byte offset of the line-frequency copy in LDS
+    int            wave_lds;                  // field kernel: bytes of LDS of each wave
 };
 
 // ---- line profiles ----------------------------------------------------------
 
+// exp(-t) for t >= 0: reduced by multiples of ln 2, whose double is taken in
+// two parts, to |r| <= ln 2 / 2, and there the polynomial of degree 11 that
+// meets exp at the 12 Chebyshev nodes of that interval (relative error below
+// 1.7e-17), scaled by ldexp; 0 from t = 745 on.  18 instructions, without the
+// range and sign handling of the library's exp.
+__device__ __forceinline__ double exp_neg(double t)
+{
+    const double n = __builtin_rint(t * -1.4426950408889634);
+    // ln 2 = 0x1.62e42fee00000p-1 (n times it is exact) + 1.9082149292705877e-10
+    const double r = __builtin_fma(n, -1.9082149292705877e-10, __builtin_fma(n, -0x1.62e42fee00000p-1, -t));
+    double p = 2.511003761756205e-08;
+    p = __builtin_fma(p, r, 2.763263965412376e-07);
+    p = __builtin_fma(p, r, 2.7557240918547625e-06);
+    p = __builtin_fma(p, r, 2.480148548228773e-05);
+    p = __builtin_fma(p, r, 0.00019841269890047143);
+    p = __builtin_fma(p, r, 0.0013888888952314812);
+    p = __builtin_fma(p, r, 0.008333333333319601);
+    p = __builtin_fma(p, r, 0.04166666666648809);
+    p = __builtin_fma(p, r, 0.1666666666666668);
+    p = __builtin_fma(p, r, 0.5000000000000019);
+    p = __builtin_fma(p, r, 1.0);
+    p = __builtin_fma(p, r, 1.0);
+    return __builtin_ldexp(p, (int)n);
+}
+
 // FP64: get_eta_and_chi (simulation.tpp:385-481) for one lane with the exact
 // window: skip while freq_diff > 11 width, include while freq_diff >= -11 width.
-__device__ __forceinline__ void eta_chi64(const RFArgs<double> &a, const double4 *__restrict__ row,
+// row: the first line's row, the others `stride` apart.
+__device__ __forceinline__ void eta_chi64(const RFArgs<double> &a, const double4 *__restrict__ row, int stride,
                                           const double *__restrict__ line, double fs, int lstart, double &eta,
                                           double &chi)
 {
 #pragma clang fp contract(off)
-    const int L = a.L;
-    int l = lstart;
-    double fd = fs - line[l];
-    double4 v = row[l];
-    while (fd > v.x) {
-        if (l >= L - 1) break;
-        l++;
-        fd = fs - line[l];
-        v = row[l];
+    // line[left lines from the last] runs with its row
+    int left = a.L - 1 - lstart;
+    line += lstart;
+    row += lstart * stride;
+    double fd = fs - *line;
+    double4 v = *row;
+    while (fd > v.x && left > 0) {
+        left--;
+        fd = fs - *++line;
+        v = *(row += stride);
     }
     double e_acc = 0.0, c_acc = CHI_FLOOR * CHI_SCALE;
     while (fd >= -v.x) {
         const double x = fd * v.y;
-        const double g = fs * exp(-(x * x));
+        const double g = fs * exp_neg(x * x);
         e_acc += v.z * g;
         c_acc += v.w * g;
-        if (l >= L - 1) break;
-        l++;
-        fd = fs - line[l];
-        v = row[l];
+        if (left <= 0) break;
+        left--;
+        fd = fs - *++line;
+        v = *(row += stride);
     }
     eta = e_acc;
     chi = c_acc;
@@ -220,32 +231,28 @@ __device__ __forceinline__ void eta_chi64(const RFArgs<double> &a, const double4
 struct Lane32 {
     float  nuf;        // nu_f
     float  A0, A1;     // nu_f - nu_l of the first two candidates (or 1e30)
-    int    off0, off1; // byte offsets of their rows
-    int    la, nc;
+    int    la, l1, nc; // the first two (or any line), and how many
     bool   has2, has3; // wave-uniform: some lane has 2 / more than 2 candidates
     double nu_f64;
     double A0d, A1d;   // the same offsets in FP64 (FP32 image variant)
+    const double *line;   // line frequencies (a copy in LDS in the field kernel)
 };
 
-__device__ __forceinline__ float rfl(float x)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
-}
-
-__device__ __forceinline__ void eta_chi32(const RFArgs<float> &a, const float4 *__restrict__ row,
-                                          const Lane32 &ln, float delta, float &eta, float &chi)
+// rows: the first line's row, the others `stride` apart; their w is the shift - 1.
+__device__ __forceinline__ void eta_chi32(const RFArgs<float> &a, const Lane32 &ln, const float4 *__restrict__ rows,
+                                          int stride, float &eta, float &chi)
 {
 #pragma clang fp contract(off)
-    const char *base = reinterpret_cast<const char *>(row);
+    const float4 v0 = rows[ln.la * stride];
+    const float delta = v0.w;
     // nu_f (1 + delta) and (nu_f delta + nu_f - nu_l), each with one rounding
     const float nus = fmaf(delta, ln.nuf, ln.nuf);
-    const float4 v0 = *reinterpret_cast<const float4 *>(base + ln.off0);
     const float x0 = fmaf(delta, ln.nuf, ln.A0) * v0.x;
     const float g0 = nus * __builtin_amdgcn_exp2f(-(x0 * x0));
     float e_acc = v0.y * g0;
     float c_acc = fmaf(v0.z, g0, (float)(CHI_FLOOR * CHI_SCALE));
     if (ln.has2) {
-        const float4 v1 = *reinterpret_cast<const float4 *>(base + ln.off1);
+        const float4 v1 = rows[ln.l1 * stride];
         const float x1 = fmaf(delta, ln.nuf, ln.A1) * v1.x;
         const float g1 = nus * __builtin_amdgcn_exp2f(-(x1 * x1));
         e_acc = fmaf(v1.y, g1, e_acc);
@@ -253,8 +260,8 @@ __device__ __forceinline__ void eta_chi32(const RFArgs<float> &a, const float4 *
         if (ln.has3) {
             for (int c = 2; c < ln.nc; c++) {
                 const int l = ln.la + c;
-                const float4 v = row[l];
-                const float x = fmaf(delta, ln.nuf, (float)(ln.nu_f64 - a.tb->line[l])) * v.x;
+                const float4 v = rows[l * stride];
+                const float x = fmaf(delta, ln.nuf, (float)(ln.nu_f64 - ln.line[l])) * v.x;
                 const float g = nus * __builtin_amdgcn_exp2f(-(x * x));
                 e_acc = fmaf(v.y, g, e_acc);
                 c_acc = fmaf(v.z, g, c_acc);
@@ -273,16 +280,15 @@ __device__ __forceinline__ void eta_chi32(const RFArgs<float> &a, const float4 *
 __device__ __forceinline__ void eta_chi32x(const RFArgs<float> &a, const float4 *__restrict__ row,
                                            const Lane32 &ln, double s, float &eta, float &chi)
 {
-    const char *base = reinterpret_cast<const char *>(row);
     const double t = (s - 1.0) * ln.nu_f64;
     const float nus = (float)(t + ln.nu_f64);
-    const float4 v0 = *reinterpret_cast<const float4 *>(base + ln.off0);
+    const float4 v0 = row[ln.la];
     const float x0 = (float)(t + ln.A0d) * v0.x;
     const float g0 = nus * __builtin_amdgcn_exp2f(-(x0 * x0));
     float e_acc = v0.y * g0;
     float c_acc = fmaf(v0.z, g0, (float)(CHI_FLOOR * CHI_SCALE));
     if (ln.has2) {
-        const float4 v1 = *reinterpret_cast<const float4 *>(base + ln.off1);
+        const float4 v1 = row[ln.l1];
         const float x1 = (float)(t + ln.A1d) * v1.x;
         const float g1 = nus * __builtin_amdgcn_exp2f(-(x1 * x1));
         e_acc = fmaf(v1.y, g1, e_acc);
@@ -397,26 +403,18 @@ struct Sweep {
 
 // Stage the entries e = 0..cnt-1 of chunk [a, b): entry e holds step j = a-1+e
 // (j = -1 is the origin) and the line rows of its cell.
-template <typename real, bool X64 = false>
+template <typename real>
 __device__ __forceinline__ void stage_chunk(const RFArgs<real> &a, int32_t o, int64_t q, int j0,
-                                            int cnt, double dsm, step_t<real, X64> *__restrict__ st,
+                                            int cnt, double dsm, Step *__restrict__ st,
                                             typename Prec<real>::row_t *__restrict__ rw)
 {
     const int64_t s0 = a.seg_off[q];
     const int nthr = blockDim.x;
     for (int e = threadIdx.x; e < cnt; e += nthr) {
         const int j = j0 + e;
-        step_t<real, X64> s;
+        Step s;
         if (j < 0) {
             s.cell = o; s.nh = 0; s.s0 = 0; s.ds = 0; s.dz = 0;
-        } else if constexpr (sizeof(real) == 4 && !X64) {
-            // split at trace time with the same FP64 arithmetic as below
-            const int4 v = a.seg_f32[s0 + j];
-            s.cell = v.x;
-            s.nh = v.y | (a.step_mask ? (int)a.step_mask[s0 + j] << STEP_OUT_SHIFT : 0);
-            s.s0 = __int_as_float(v.z);
-            s.ds = __int_as_float(v.w);
-            s.dz = a.seg_hdz32[s0 + j];
         } else {
             const int32_t c = a.seg_cell[s0 + j];
             const double sn = a.seg_shift[s0 + j];
@@ -424,8 +422,7 @@ __device__ __forceinline__ void stage_chunk(const RFArgs<real> &a, int32_t o, in
             const double sc = (j > 0) ? a.seg_shift[s0 + j - 1] : (a.origin_shift ? a.origin_shift[q] : 1.0);
             const StepSplit sp = split_step(sc, sn, z, dsm);
             s.cell = c;
-            s.nh = sp.n | ((sp.interp ? sp.half : 0) << STEP_HALF_SHIFT) |
-                   (a.step_mask ? (int)a.step_mask[s0 + j] << STEP_OUT_SHIFT : 0);
+            s.nh = sp.n | ((sp.interp ? sp.half : 0) << STEP_HALF_SHIFT);
             s.s0 = sp.interp ? sc : sn;               // absolute FP64 shift
             s.ds = sp.dshift;
             s.dz = sp.dZ * HDZ_SCALE;                 // dz'
@@ -454,6 +451,8 @@ struct LaneCtx<double> {
     double nu_f;
     int    lstart;
     const double *line;   // line frequencies (a copy in LDS in the field kernel)
+    double nu_l;          // frequency of the bin's only candidate line l (-1e30: none)
+    int    l;
 };
 
 template <typename real>
@@ -466,7 +465,8 @@ __device__ __forceinline__ void eval_point<float>(const RFArgs<float> &a, const 
                                                   const float4 *__restrict__ row, float s,
                                                   float &eta, float &chi)
 {
-    eta_chi32(a, row, lc.ln, s, eta, chi);
+    // the rows' w is 0: the shift of the origin
+    eta_chi32(a, lc.ln, row, 1, eta, chi);
 }
 
 template <>
@@ -479,7 +479,7 @@ __device__ __forceinline__ void eval_point<double>(const RFArgs<double> &a, cons
 #pragma clang fp contract(off)
         fs = s * lc.nu_f;
     }
-    eta_chi64(a, row, lc.line, fs, lc.lstart, eta, chi);
+    eta_chi64(a, row, 1, lc.line, fs, lc.lstart, eta, chi);
 }
 
 // The point evaluation of a kernel: eval_point, or the FP32 image variant
@@ -506,8 +506,6 @@ __device__ __forceinline__ float sub_point_shift(float s0, int m, float ds)
 }
 
 __device__ __forceinline__ int rfl_int(int x) { return __builtin_amdgcn_readfirstlane(x); }
-__device__ __forceinline__ float rfl_real(float x) { return rfl(x); }
-__device__ __forceinline__ double rfl_real(double x) { return x; }
 
 // Incoming intensity at the far end of entry q (FP64, unscaled): the
 // boundary intensity of the cell of the last emitted point, rescaled to that
@@ -583,108 +581,52 @@ __global__ __launch_bounds__(256) void k_far_cache(RFArgs<float> a, int Rmax, T 
     }
 }
 
-// One ray of a pair, eliminated from its boundary end (incoming intensity
+// One ray of an image pair, eliminated from its boundary end (incoming intensity
 // I_far, scaled) inwards to the origin, which it leaves pending.
-template <typename real, bool X64 = false>
+template <typename real, bool X64>
 __device__ __forceinline__ Sweep<real> sweep_side(const RFArgs<real> &a, const LaneCtx<real> &lc,
                                                   int32_t o, int64_t q, real I_far, real S_o,
                                                   real chi_o, double dsm,
-                                                  step_t<real, X64> *__restrict__ st,
-                                                  typename Prec<real>::row_t *__restrict__ rw,
-                                                  int chunk = STEP_MASK_CHUNKS)
+                                                  Step *__restrict__ st,
+                                                  typename Prec<real>::row_t *__restrict__ rw)
 {
     using row_t = typename Prec<real>::row_t;
     Sweep<real> sw;
     sw.init(I_far);
-    const real chi_floor = (real)(CHI_FLOOR * CHI_SCALE);
-    // this wave's out-of-window bit in the staged nh word (none past the masked chunks)
-    const unsigned cbit = chunk < STEP_MASK_CHUNKS ? 1u << (STEP_OUT_SHIFT + chunk) : 0u;
     const int ns = a.nseg[q];
     const int L = a.L;
     const int CH = a.ch;
-    // Wave-uniform: the pending point is an out-of-window sub-point and y lies
-    // in (noop_lo, noop_hi) on every lane.  Then each further out-of-window
-    // sub-point closes its row with c <= 2 chi_floor dz'_max, below half an
-    // ulp of y and with c y below 2^-25, so that x = y, q = 1, y stays y and,
-    // with S = 0 pending and p = z, z and p stay as they are: only the pending
-    // point's dz' (and chi dz') moves on.  The result is the same bits as
-    // stepping every sub-point.
-    bool noop = false;
     for (int b_ = ns; b_ > 0; b_ -= CH) {
         const int a_ = b_ > CH ? b_ - CH : 0;
         const int cnt = b_ - a_ + 1;
         __syncthreads();   // the previous chunk is consumed by every wave
-        stage_chunk<real, X64>(a, o, q, a_ - 1, cnt, dsm, st, rw);
-        int e = cnt - 1;
-        while (e >= 1) {
-            decltype(st->s0) s0, ds, dzs;
-            int nhs;
-            read_step(st, e, s0, ds, dzs, nhs);   // s0 and ds stay in VGPRs: one scalar operand per FMA
-            int nh = rfl_int(nhs);                // one readfirstlane: n, half and the chunk bits
-            if (!((unsigned)nh & cbit)) {
-                noop = false;
-                // a run of steps with points inside a line window, in a loop
-                // of its own so that the sweep state keeps its registers
-                for (;;) {
-                    const int n = nh & STEP_N_MASK;
-                    __builtin_assume(n >= 1);   // a traced step emits 1 .. 10000 points (0 fails the trace)
-                    const int half = (nh >> STEP_HALF_SHIFT) & STEP_HALF_MASK;
-                    const real hdz = (real)rfl_real(dzs);
-                    // sub-points m >= half lie in the step's cell (row e), m < half in
-                    // the previous one (row e-1); two loops keep each row's address
-                    // loop-invariant
-                    const row_t *rn = rw + e * L;
-                    const row_t *rc = rw + (e - 1) * L;
-                    const int mlo = half > 1 ? half : 1;
-                    for (int m = n; m >= mlo; --m) {
-                        real eta, chi;
-                        eval_at<real, X64>(a, lc, rn, sub_point_shift(s0, m, ds), eta, chi);
-                        const real S = eta * Prec<real>::rcp(chi);
-                        sw.step(chi);   // on the first point an exact no-op (c = 0, q = 1)
-                        sw.pend(S, chi, hdz);
-                    }
-                    for (int m = (half - 1 < n ? half - 1 : n); m >= 1; --m) {
-                        real eta, chi;
-                        eval_at<real, X64>(a, lc, rc, sub_point_shift(s0, m, ds), eta, chi);
-                        const real S = eta * Prec<real>::rcp(chi);
-                        sw.step(chi);
-                        sw.pend(S, chi, hdz);
-                    }
-                    if (--e < 1) break;
-                    read_step(st, e, s0, ds, dzs, nhs);
-                    nh = rfl_int(nhs);
-                    if ((unsigned)nh & cbit) break;
-                }
-                if (e < 1) break;
-            }
-            // step e: no bin of this wave meets a line window in it, so every
-            // sub-point has eta = 0 and chi at the floor, as evaluated
+        stage_chunk<real>(a, o, q, a_ - 1, cnt, dsm, st, rw);
+        for (int e = cnt - 1; e >= 1; --e) {
+            const int nh = rfl_int(st[e].nh);   // one readfirstlane: n and half are wave-uniform
             const int n = nh & STEP_N_MASK;
-            __builtin_assume(n >= 1);
-            const real hdz = (real)rfl_real(dzs);
-            if (!noop) {
-                // the first closes the row of the last evaluated point
-                sw.step(chi_floor);
-                sw.pend((real)0, chi_floor, hdz);
-                if constexpr (sizeof(real) == 4)
-                    noop = __all(sw.y > a.noop_lo && sw.y < a.noop_hi);
-                if (!noop) {
-                    for (int m = n - 1; m >= 1; --m) {
-                        sw.step(chi_floor);
-                        sw.pend((real)0, chi_floor, hdz);
-                    }
-                    --e;
-                    continue;
-                }
+            const int half = (nh >> STEP_HALF_SHIFT) & STEP_HALF_MASK;
+            const double s0 = st[e].s0, ds = st[e].ds;
+            const real hdz = (real)st[e].dz;
+            // sub-points m >= half lie in the step's cell (row e), m < half in
+            // the previous one (row e-1); two loops keep each row's address
+            // loop-invariant
+            const row_t *rn = rw + e * L;
+            const row_t *rc = rw + (e - 1) * L;
+            const int mlo = half > 1 ? half : 1;
+            for (int m = n; m >= mlo; --m) {
+                real eta, chi;
+                eval_at<real, X64>(a, lc, rn, sub_point_shift(s0, m, ds), eta, chi);
+                const real S = eta * Prec<real>::rcp(chi);
+                sw.step(chi);   // on the first point an exact no-op (c = 0, q = 1)
+                sw.pend(S, chi, hdz);
             }
-            // a no-op stretch: pass over the following out-of-window steps of
-            // the chunk, keeping the dz' of the last one
-            int last = e;
-            while (last > 1 && ((unsigned)rfl_int(st[last - 1].nh) & cbit)) last--;
-            const real hdz_l = last == e ? hdz : (real)rfl_real(st[last].dz);
-            sw.hdz_q = hdz_l;
-            sw.cq = chi_floor * hdz_l;
-            e = last - 1;
+            for (int m = (half - 1 < n ? half - 1 : n); m >= 1; --m) {
+                real eta, chi;
+                eval_at<real, X64>(a, lc, rc, sub_point_shift(s0, m, ds), eta, chi);
+                const real S = eta * Prec<real>::rcp(chi);
+                sw.step(chi);
+                sw.pend(S, chi, hdz);
+            }
         }
     }
     sw.step(chi_o);   // the origin closes the innermost row and is left pending
@@ -700,7 +642,7 @@ __device__ __forceinline__ Sweep<real> sweep_side(const RFArgs<real> &a, const L
 template <typename real, bool X64 = false>
 __device__ __forceinline__ void sweep_outward(const RFArgs<real> &a, const LaneCtx<real> &lc, int32_t o,
                                               int64_t q, double dsm, Sweep<real> &sw,
-                                              step_t<real, X64> *__restrict__ st,
+                                              Step *__restrict__ st,
                                               typename Prec<real>::row_t *__restrict__ rw)
 {
     using row_t = typename Prec<real>::row_t;
@@ -711,14 +653,13 @@ __device__ __forceinline__ void sweep_outward(const RFArgs<real> &a, const LaneC
         const int b_ = a_ + CH < ns ? a_ + CH : ns;
         const int cnt = b_ - a_ + 1;
         __syncthreads();   // the previous chunk is consumed by every wave
-        stage_chunk<real, X64>(a, o, q, a_ - 1, cnt, dsm, st, rw);
+        stage_chunk<real>(a, o, q, a_ - 1, cnt, dsm, st, rw);
         for (int e = 1; e < cnt; ++e) {
             const int nh = rfl_int(st[e].nh);   // one readfirstlane: n and half are wave-uniform
             const int n = nh & STEP_N_MASK;
             const int half = (nh >> STEP_HALF_SHIFT) & STEP_HALF_MASK;
-            const auto s0 = st[e].s0;
-            const auto ds = st[e].ds;
-            const real hdz = (real)rfl_real(st[e].dz);
+            const double s0 = st[e].s0, ds = st[e].ds;
+            const real hdz = (real)st[e].dz;
             const row_t *rn = rw + e * L;
             const row_t *rc = rw + (e - 1) * L;
             const int mhi = half - 1 < n ? half - 1 : n;
@@ -749,6 +690,21 @@ __device__ __forceinline__ real end_u(const Sweep<real> &sw, real I)
     return (sw.p + (real)SQRT2 * I) * Prec<real>::rcp(sw.y + (real)SQRT2);
 }
 
+// FP64 with one candidate line per bin: get_eta_and_chi's window holds at most
+// that line, and a bin further than 11 widths from it gets exp(-x^2) < 3e-53
+// of it instead of nothing, which neither chi's floor nor any sum can feel.
+// v: (anything, 1/width, E, K) of the line.
+__device__ __forceinline__ void eta_chi_one(const LaneCtx<double> &lc, const double4 v, double s, double &eta,
+                                            double &chi)
+{
+#pragma clang fp contract(off)
+    const double fs = s * lc.nu_f;
+    const double x = (fs - lc.nu_l) * v.y;
+    const double g = fs * exp_neg(x * x);
+    eta = v.z * g;
+    chi = __builtin_fma(v.w, g, CHI_FLOOR * CHI_SCALE);
+}
+
 // Per-lane constants of origin o's bin and its own emissivity and opacity at
 // the unshifted frequency nu_f (Simulation::setup takes the origin at
 // nu(o, f), simulation.tpp:209-222).  ONE: no bin has more than one candidate
@@ -776,8 +732,7 @@ __device__ __forceinline__ void origin_point(const RFArgs<real> &a, double nu_f,
         lc.ln.A1 = (nc > 1) ? (float)(nu_f - a.tb->line[l1]) : 1.0e30f;
         lc.ln.A0d = (nc > 0) ? nu_f - a.tb->line[l0] : 1.0e30;
         lc.ln.A1d = (nc > 1) ? nu_f - a.tb->line[l1] : 1.0e30;
-        lc.ln.off0 = l0 * (int)sizeof(float4);
-        lc.ln.off1 = l1 * (int)sizeof(float4);
+        lc.ln.l1 = l1;
         lc.ln.has2 = ONE ? false : __any(nc > 1);
         lc.ln.has3 = ONE ? false : __any(nc > 2);
         if constexpr (X64) eta_chi32x(a, orow, lc.ln, 1.0, eta_o, chi_o);
@@ -787,9 +742,380 @@ __device__ __forceinline__ void origin_point(const RFArgs<real> &a, double nu_f,
         while (ls < a.L - 1 && a.tb->line[ls] * a.lstart_threshold < nu_f) ls++;
         lc.nu_f = nu_f;
         lc.lstart = ls;
-        eval_point<real>(a, lc, orow, (real)1, eta_o, chi_o);
+        if constexpr (ONE) {
+            const bool cand = a.tb->line[ls] * a.cand_lo >= nu_f && a.tb->line[ls] * a.cand_hi <= nu_f;
+            lc.nu_l = cand ? a.tb->line[ls] : -1.0e30;
+            lc.l = ls;
+        }
+        if constexpr (ONE) eta_chi_one(lc, orow[ls], 1.0, eta_o, chi_o);
+        else eval_point<real>(a, lc, orow, (real)1, eta_o, chi_o);
     }
     S_o = eta_o * Prec<real>::rcp(chi_o);
+}
+
+// ---- the radiation field's sweep ---------------------------------------------
+
+// A wave's LDS for one window of up to W = a.ch points (Window, W <= 64):
+//   rows   [L][W + 1] the line rows of each point's cell, with the point's
+//          shift in their spare component: the sweep reads a point's row and
+//          shift in one access at a compile-time distance from the last
+//          point's; the odd stride spreads the lines over the banks;
+//   hdz    [WAVE] path-length factors dz';
+//   stage  [WAVE] the points' shifts and cells;
+//   owner  [WAVE] the points' steps (lanes of the batch).
+template <typename real> struct Stage;
+template <> struct Stage<float> { float s; int32_t cell; };
+template <> struct Stage<double> { double s; int32_t cell, pad; };
+template <typename real>
+struct Window {
+    using row_t = typename Prec<real>::row_t;
+    row_t       *rows;
+    real        *hdz;
+    Stage<real> *stage;
+    int         *owner;
+    static constexpr size_t fixed = WAVE * (sizeof(real) + sizeof(Stage<real>) + sizeof(int));   // bytes beside the rows
+};
+
+constexpr int BATCH = WAVE - 1;   // steps per batch: one lane each, the last lane for the cell before them
+
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ bool lane_of(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+// Inclusive sum and maximum over the lanes up to this one (DPP row shifts and broadcasts).
+__device__ __forceinline__ int scan_add(int x)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+    return x;
+}
+__device__ __forceinline__ int scan_max(int x)   // of values >= 0
+{
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false));
+    return x;
+}
+__device__ __forceinline__ int from_lane(int x, int lane) { return __builtin_amdgcn_ds_bpermute(lane << 2, x); }
+__device__ __forceinline__ float from_lane(float x, int lane)
+{
+    return __int_as_float(from_lane(__float_as_int(x), lane));
+}
+__device__ __forceinline__ double from_lane(double x, int lane)
+{
+    return __hiloint2double(from_lane(__double2hiint(x), lane), from_lane(__double2loint(x), lane));
+}
+
+// The kernel's arguments, read from the kernarg segment where they are used:
+// kept in scalar registers over the whole ray loop they spill into vector
+// lanes, and every restore is a vector instruction.
+template <typename real>
+__device__ __forceinline__ const __attribute__((address_space(4))) RFArgs<real> *kernel_args()
+{
+    auto p = (const __attribute__((address_space(4))) RFArgs<real> *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
+// Emissivity and opacity at point p of a window (W points per line).
+template <typename real, bool ONE>
+__device__ __forceinline__ void eval_window(const RFArgs<real> &a, const LaneCtx<real> &lc, const Window<real> &win,
+                                            int p, int W, real &eta, real &chi)
+{
+    if constexpr (sizeof(real) == 4) {
+        eta_chi32(a, lc.ln, win.rows + p, W + 1, eta, chi);
+    } else if constexpr (ONE) {
+        const double4 v = win.rows[lc.l * (W + 1) + p];
+        eta_chi_one(lc, v, v.x, eta, chi);
+    } else {
+        double fs;
+        {
+#pragma clang fp contract(off)
+            fs = win.stage[p].s * lc.nu_f;
+        }
+        eta_chi64(a, win.rows + p, W + 1, lc.line, fs, lc.lstart, eta, chi);
+    }
+}
+
+// How a wave passes over runs of consecutive points out of the window (FP32).
+// Of such a run only the first point (at the far side) and the last one are
+// evaluated.  The points between them close their rows with
+// c <= 2 X dz'_max, X bounding chi out of the window, and have source
+// functions S <= Smax.  With c below half an ulp of y, c y below 2^-25 and
+// S c below half an ulp of p each of them leaves x = y, q = 1, y as it was and
+// z = p = the value of p after the first point: the same bits as stepping
+// them.  y and p are tested on every lane (noop_lo, noop_hi, p_min); a wave
+// whose state fails the test goes on without skipping what the test needed:
+//   SPAN   sub-points beyond the narrow window (span): the lines add at most
+//          NEAR_CHI of the floor there, X = floor (1 + NEAR_CHI), S as bounded
+//          by near_p;
+//   WIDE   steps beyond MASK_WINDOW widths (step_mask): profiles are 0,
+//          X = floor, S = 0 and any p will do;
+//   NONE   every point is evaluated.
+// The FP64 kernel (SPAN or NONE) steps every point, but evaluates only those
+// within MASK_WINDOW64 widths: beyond, eta = 0 and chi is the floor exactly.
+struct Runs {
+    enum { SPAN = 0, WIDE = 1, NONE = 2 };
+};
+
+// The two rays of a pair, the antipode's (entry qa of ns_a steps) first: each
+// is eliminated from its boundary end inwards to the origin, which closes its
+// innermost row, and adds its y, p and c to y2, p2 and c2 (an empty ray adds
+// none of them); the whole call belongs to one wave.
+//
+// The cached steps of both rays form one list, each ray from its far end
+// inwards, taken up to BATCH steps at a time, one lane each: the rays of most
+// pairs fit one batch, whose set-up is about as much work as a dozen points.
+// The lanes read the steps' in-window spans first and then only what the steps
+// to be evaluated need.  The points of those steps are laid out one per lane
+// (scan of the steps' point counts, owner by a maximum scan), a window at a
+// time, and their rows and shifts go to LDS.  The elimination then walks the
+// window: two LDS reads and the recurrence per point, with no per-step
+// control and no work for the inner points of out-of-window runs.
+template <typename real, bool ONE>
+__device__ __forceinline__ void sweep_pair(const RFArgs<real> &a, const LaneCtx<real> &lc, int32_t o, int64_t qa,
+                                           int ns_a, int64_t qr, int ns_r, real I_a, real I_r, real S_o, real chi_o,
+                                           double dsm, float p_min, int chunk, int mode, const Window<real> &win,
+                                           real &y2, real &p2, real &c2)
+{
+    using row_t = typename Prec<real>::row_t;
+    constexpr bool F32 = sizeof(real) == 4;
+    constexpr bool INROW = F32 || ONE;   // the rows have a component to spare for the shift
+    Sweep<real> sw;
+    sw.init(ns_a > 0 ? I_a : I_r);
+    const real chi_floor = (real)(CHI_FLOOR * CHI_SCALE);
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    const auto *ka = kernel_args<real>();
+    const int L = ka->L, W = ka->ch;
+    // step g of the list lies at far_a - g on the antipode's ray (g < ns_a), at far_r - g on the other
+    const int T = ns_a + ns_r;
+    const int64_t far_a = ka->seg_off[qa] + ns_a - 1, far_r = ka->seg_off[qr] + T - 1;
+    // the origin closes the ray's innermost row
+    auto finish = [&]() {
+        sw.step(chi_o);
+        sw.pend(S_o, chi_o, (real)0);
+        y2 += sw.y;
+        p2 += sw.p;
+        c2 += sw.c;
+    };
+    int g0 = 0, skip = 0;   // next step, and how many of its outermost points are done (FP32, after a failed test)
+    while (g0 < T) {
+        // steps with points in the window and those without (outm)
+        const int nb = T - g0 < BATCH ? T - g0 : BATCH;
+        const int split = ns_a - g0;   // lane of the second ray's first step
+        const int g = g0 + lane;
+        const int64_t at = (g < ns_a ? far_a : far_r) - g;
+        unsigned span = SPAN_ALL;
+        if (lane < nb) {
+            if (mode == Runs::SPAN) span = ka->span[ka->span_stride * chunk + at];
+            else if (F32 && mode == Runs::WIDE) span = (ka->step_mask[at] >> chunk) & 1 ? SPAN_NONE : SPAN_ALL;
+        }
+        const uint64_t valid = (1ull << nb) - 1;   // nb <= 63
+        const uint64_t outm = __ballot(span == SPAN_NONE) & valid;
+        const bool both = split > 0 && split <= nb;   // the first ray ends in this batch
+        const uint64_t second = both && split < WAVE ? 1ull << split : 0;   // lane of the second one's first step
+        // steps to load: those with points in the window, the ends of the runs of
+        // others (runs end with their ray), and the steps before them, whose
+        // cells they also touch (the next lane's)
+        const uint64_t ends = F32 ? outm & ~((outm << 1) & (outm >> 1) & ~second & ~(second >> 1)) : outm;
+        const uint64_t needm = (valid & ~outm) | ends;
+        const uint64_t loadm = needm | (needm << 1);
+        int32_t cell = o;
+        int nh = 0;
+        real st_s0 = 0, st_ds = 0, st_hdz = 0;
+        const bool inner = g == ns_a - 1 || g == T - 1;   // the origin lies before this step
+        if (lane_of(loadm) && g < T) {
+            if constexpr (F32) {
+                const int4 v = ka->seg_f32[at];
+                cell = v.x;
+                nh = v.y;
+                st_s0 = __int_as_float(v.z);
+                st_ds = __int_as_float(v.w);
+                st_hdz = ka->seg_hdz32[at];
+            } else {
+                cell = ka->seg_cell[at];
+                const double sn = ka->seg_shift[at];
+                const double sc = inner ? 1.0 : ka->seg_shift[at - 1];   // co-moving: the origin's shift is 1
+                const StepSplit sp = split_step(sc, sn, ka->seg_dZ[at], dsm);
+                nh = sp.n | ((sp.interp ? sp.half : 0) << STEP_HALF_SHIFT);
+                st_s0 = sp.interp ? sc : sn;
+                st_ds = sp.dshift;
+                st_hdz = sp.dZ * HDZ_SCALE;
+            }
+        }
+        const int32_t next = from_lane(cell, lane + 1);   // on every lane: an idle one would hand out nothing
+        const int32_t before = inner ? o : next;
+        // The sub-points of a step, from its far end inwards: n - hi out of the
+        // window, then `in` inside it, then hi - in outside again (hi = in = 0: a
+        // step of outm).
+        const int n_all = nh & STEP_N_MASK, half = (nh >> STEP_HALF_SHIFT) & STEP_HALF_MASK;
+        const int n = n_all - (lane == 0 ? skip : 0);
+        const bool out = lane_of(outm);
+        int hi = (((int)(span >> 8) + 1) * n_all + 255) >> 8;
+        hi = out ? 0 : hi < n ? hi : n;
+        const int in = out ? 0 : hi - (((int)(span & 255) * n_all) >> 8);
+        // Of a run of out-of-window points only the first and the last are
+        // evaluated (FP32).  A run at a ray's far end needs no first one:
+        // nothing is pending yet, and c = 0 closes nothing.
+        int cf, cn = hi > in ? 1 : 0;   // records before and after the points in the window
+        bool first = false;             // the first record is the run's first point
+        if constexpr (F32) {
+            const uint64_t far_out = __ballot(out || n > hi) & valid, near_out = __ballot(out || hi > in) & valid;
+            const uint64_t fresh = second | ((g0 == 0 || g0 == ns_a) && skip == 0 ? 1 : 0);
+            // a run begins with this step's outer points, or ends with its inner ones
+            const uint64_t begins = far_out & ~((near_out << 1) & ~second);
+            const uint64_t stops = near_out & ~((far_out >> 1) & ~(second >> 1));
+            first = lane_of(begins & ~fresh);
+            const int outer = n - hi;   // points of the outer piece
+            const bool closes = !out || lane_of(stops);   // the outer piece ends its run
+            cf = outer > 0 ? (first ? 1 : 0) + (closes && !(first && outer == 1) ? 1 : 0) : 0;
+            if (hi > in + 1 && lane_of(stops)) cn = 2;
+        } else {
+            cf = n > hi ? 1 : 0;   // one record for all of them
+        }
+        const int cnt = lane < nb ? cf + in + cn : 0;
+        const int incl = scan_add(cnt);
+        const int total = __builtin_amdgcn_readlane(incl, WAVE - 1);
+        const int base = incl - cnt;
+        const int turn = both ? __builtin_amdgcn_readlane(incl, split - 1) : INT32_MAX;   // points of the first ray
+        bool pending = both;
+        const int pack1 = n | hi << 14 | cf << 28 | (first ? 1 << 30 : 0);
+        const int pack2 = in | half << 14;
+        int before_window = 0;   // the last record's step and sub-point, of the window before
+        bool again = false;
+        for (int w0 = 0; w0 < total; w0 += W) {
+            const int cw = total - w0 < W ? total - w0 : W;
+            wave_lds_fence();   // the previous window is consumed
+            if (F32 && w0 > 0) before_window = rfl_int(win.owner[W - 1]);
+            wave_lds_fence();
+            win.owner[lane] = 0;
+            wave_lds_fence();
+            // (base, lane) of the step that begins at a point, or before the window and ends in it
+            if (cnt > 0 && base < w0 + W && base + cnt > w0) win.owner[base > w0 ? base - w0 : 0] = base << 6 | lane;
+            wave_lds_fence();
+            const int bl = scan_max(win.owner[lane]);
+            const int own = bl & (WAVE - 1);
+            const int p1 = from_lane(pack1, own), p2_ = from_lane(pack2, own);
+            const int t = w0 + lane - (bl >> 6), k = t - ((p1 >> 28) & 3);
+            const int o_hi = (p1 >> 14) & STEP_N_MASK, o_in = p2_ & STEP_N_MASK;
+            const bool head = t == 0 && (p1 >> 30) & 1;
+            const bool outer = k < 0, after = k > o_in;
+            bool mark;
+            int m = o_hi - k;
+            if constexpr (F32) {
+                mark = (outer && !head) || after;   // a run's last point
+                if (outer) m = head ? p1 & STEP_N_MASK : o_hi + 1;
+                if (after) m = 1;
+            } else {
+                mark = outer || k >= o_in;
+            }
+            Stage<real> sg;
+            sg.s = sub_point_shift(from_lane(st_s0, own), m, from_lane(st_ds, own));
+            const int32_t c_own = from_lane(cell, own), c_before = from_lane(before, own);
+            sg.cell = m < ((p2_ >> 14) & STEP_HALF_MASK) ? c_before : c_own;
+            if constexpr (!F32) {
+                if (mark) sg.cell = outer ? (p1 & STEP_N_MASK) - o_hi : o_hi - o_in;   // its sub-points
+            }
+            uint64_t marks = __ballot(lane < cw && mark);
+            win.hdz[lane] = from_lane(st_hdz, own);
+            win.stage[lane] = sg;
+            if constexpr (F32) win.owner[lane] = own << 14 | m;
+            wave_lds_fence();
+            {
+                // the rows of WAVE / L points at a time, lane e L + l line l of point e
+                const int per = WAVE / L;
+                const int e0 = (int)(((uint64_t)(uint32_t)lane * ka->L_magic) >> 32), l = lane - e0 * L;
+                const row_t *src = ka->rows + l;
+                row_t *dst = win.rows + l * (W + 1);
+                if (e0 < per)
+                    for (int e = e0; e < cw; e += per) {
+                        if (!F32 && ((marks >> e) & 1)) continue;
+                        const Stage<real> sg_e = win.stage[e];
+                        row_t v = src[(uint32_t)sg_e.cell * (uint32_t)L];   // N L rows < 2^32
+                        if constexpr (F32) v.w = sg_e.s;
+                        else if constexpr (INROW) v.x = sg_e.s;
+                        dst[e] = v;
+                    }
+            }
+            wave_lds_fence();
+            int p = 0;
+            for (;;) {
+                const int e = marks ? (int)__builtin_ctzll(marks) : cw;
+                const bool turns = pending && turn - w0 <= e;
+                const int stop = turns ? turn - w0 : e;
+#pragma unroll 2
+                for (; p < stop; ++p) {
+                    real eta, chi;
+                    eval_window<real, ONE>(a, lc, win, p, W, eta, chi);
+                    const real S = eta * Prec<real>::rcp(chi);
+                    sw.step(chi);   // on a ray's first point an exact no-op (c = 0, q = 1)
+                    sw.pend(S, chi, win.hdz[p]);
+                }
+                if (turns) {
+                    finish();
+                    sw.init(I_r);
+                    pending = false;
+                    continue;
+                }
+                if (e >= cw) break;
+                if constexpr (F32) {
+                    if (__all(sw.y > a.noop_lo && sw.y < a.noop_hi && sw.p > p_min)) {
+                        float eta, chi;
+                        eval_window<real, ONE>(a, lc, win, e, W, eta, chi);
+                        const float h = win.hdz[e];
+                        sw.z = sw.p;
+                        sw.S_q = eta * Prec<real>::rcp(chi);
+                        sw.hdz_q = h;
+                        sw.cq = chi * h;
+                    } else {
+                        // go on in the next mode from the point after the last record, or
+                        // from the ray's first point if this run begins the ray
+                        if (w0 + e == turn) {
+                            g0 = ns_a;
+                            skip = 0;
+                        } else if (w0 + e > 0) {
+                            const int rec = e > 0 ? rfl_int(win.owner[e - 1]) : before_window;
+                            const int m_done = rec & STEP_N_MASK;
+                            g0 += rec >> 14;
+                            skip = rfl_int(ka->seg_f32[(g0 < ns_a ? far_a : far_r) - g0].y & STEP_N_MASK) - (m_done - 1);
+                            if (m_done == 1) {
+                                g0++;
+                                skip = 0;
+                            }
+                        }
+                        mode++;
+                        p_min = -FLT_MAX;
+                        again = true;
+                        break;
+                    }
+                } else {
+                    // out of the window: eta = 0 and chi at the floor at each of its points
+                    const real h = win.hdz[e];
+                    for (int i = rfl_int(win.stage[e].cell); i >= 1; --i) {
+                        sw.step(chi_floor);
+                        sw.pend((real)0, chi_floor, h);
+                    }
+                }
+                marks &= marks - 1;
+                p = e + 1;
+            }
+            if (again) break;
+        }
+        if (!again) {
+            g0 += nb;
+            skip = 0;
+        }
+    }
+    if (ns_r > 0) finish();
 }
 
 // This wave's share of the Lambda* diagonal per transition
@@ -832,15 +1158,21 @@ __device__ __forceinline__ void lambda_partials(const RFArgs<real> &a, int32_t o
 }
 
 // FP32: at least 8 waves per SIMD (at most 64 VGPRs), which hide the LDS
-// latency of the line rows; FP64 is left to the compiler.
-template <typename real, bool ONE = false>
-__global__ __launch_bounds__(WAVE * MAX_WAVES) __attribute__((amdgpu_waves_per_eu(sizeof(real) == 4 ? 8 : 1)))
+// latency of the line rows; 6 where bins have several lines, whose second
+// line's registers spill at 64; FP64: 4.  The waves of a workgroup
+// share nothing but the line table.
+template <typename real, bool ONE>
+__global__ __launch_bounds__(WAVE * MAX_WAVES) __attribute__((amdgpu_waves_per_eu(sizeof(real) == 4 ? (ONE ? 8 : 6) : 4)))
 void k_radiation_field(RFArgs<real> a)
 {
     using row_t = typename Prec<real>::row_t;
     extern __shared__ __align__(16) unsigned char smem[];
-    Step<real> *st = reinterpret_cast<Step<real> *>(smem);
-    row_t *rw = reinterpret_cast<row_t *>(smem + a.row_offset);
+    const int wave = rfl_int((int)(threadIdx.x / WAVE));
+    Window<real> win;
+    win.hdz = reinterpret_cast<real *>(smem + wave * a.wave_lds);
+    win.stage = reinterpret_cast<Stage<real> *>(win.hdz + WAVE);
+    win.owner = reinterpret_cast<int *>(win.stage + WAVE);
+    win.rows = reinterpret_cast<row_t *>(win.owner + WAVE);
 
     // XCD-aware order: consecutive workgroups go to different XCDs, so hand
     // each XCD a contiguous range of origins.
@@ -853,27 +1185,43 @@ void k_radiation_field(RFArgs<real> a)
     const int32_t mdl = a.cell_model[o];
     if (!a.m_active[mdl]) return;         // converged model of a batch: whole workgroup
     const int group = logical - (o - a.o_begin) * a.ngroups;
-    const int wave = threadIdx.x / WAVE;
-    const int chunk = rfl_int(group * a.nwg + wave);   // wave-uniform: scalar skip tests
+    const int chunk = rfl_int(group * a.nwg + wave);   // wave-uniform
+    LaneCtx<real> lc;
+    if constexpr (!ONE) {
+        // the line frequencies that bins of several lines read at every point, in LDS
+        double *lt = reinterpret_cast<double *>(smem + a.line_offset);
+        for (int i = (int)threadIdx.x; i < a.L; i += (int)blockDim.x) lt[i] = a.tb->line[i];
+        __syncthreads();
+        if constexpr (sizeof(real) == 4) lc.ln.line = lt;
+        else lc.line = lt;
+    }
+    if (chunk >= a.nchunk) return;        // a wave without bins: no barrier follows
     const int F = a.F;
     const int slot = chunk * WAVE + (int)(threadIdx.x & (WAVE - 1));
     const bool active = slot < F;
     const int f = lane_bin(active ? slot : F - 1, a.L, F, a.root_major);
     const double nu_f = a.nu[(int64_t)o * F + f];
-    const double dsm = a.dshift_max[o];
+    const double dsm = sizeof(real) == 8 ? a.dshift_max[o] : 0.0;
     const int32_t bo = a.cell2bdy[o];
     const row_t *orow = a.rows + (int64_t)o * a.L;
 
-    LaneCtx<real> lc;
-    if constexpr (sizeof(real) == 8) {
-        // FP64: the line frequencies the profile windows read at every point, in LDS
-        double *lt = reinterpret_cast<double *>(smem + a.line_offset);
-        for (int i = (int)threadIdx.x; i < a.L; i += (int)blockDim.x) lt[i] = a.tb->line[i];
-        __syncthreads();
-        lc.line = lt;
-    }
     real S_o, chi_o;
     origin_point<real, false, ONE>(a, nu_f, orow, lc, S_o, chi_o);
+    // how out-of-window runs are passed over (Runs)
+    int mode = Runs::NONE;
+    float p_near = -FLT_MAX;
+    if (chunk < STEP_MASK_CHUNKS) {
+        if constexpr (sizeof(real) == 4) {
+            if (a.step_mask) mode = Runs::WIDE;
+            if (a.step_mask && a.span && *a.near_bad == 0) {
+                mode = Runs::SPAN;
+                p_near = lc.ln.nc > 1 ? a.near_p[a.L] : a.near_p[lc.ln.la];
+            }
+        } else if (a.span) {
+            mode = Runs::SPAN;
+        }
+    }
+    mode = rfl_int(mode);
 
     int32_t err = 0;
     double J_acc = 0.0, Lam_acc = 0.0;
@@ -886,9 +1234,9 @@ void k_radiation_field(RFArgs<real> a)
         const double w2 = wsc * a.ray_w[rb + r];
         const int64_t qr = qb + r;
         const int64_t qa = qb + (ar - rb);
-        const int n_r = a.npts[qr];
-        const int n_a = a.npts[qa];
-        if (n_r == 0 && n_a == 0) {
+        const int ns_r = rfl_int(a.nseg[qr]);   // a step has at least one point
+        const int ns_a = rfl_int(a.nseg[qa]);
+        if (ns_r == 0 && ns_a == 0) {
             // ndep == 1: u = I_bdy of the origin's boundary entry (sim_radiation.tpp:243-264)
             if (bo < 0) { err |= ERR_EMPTY_SIDE; continue; }
             const double Ib = a.I_bdy[(int64_t)bo * F + f];
@@ -896,26 +1244,25 @@ void k_radiation_field(RFArgs<real> a)
             if (a.u_out && active) a.u_out[((int64_t)r * a.N + o) * F + f] = Ib;
             continue;
         }
-        real u, lam;
-        if (n_r > 0 && n_a > 0) {
-            const real Ia = far_in<real>(a, qa, nu_f, F, f, err);
-            const Sweep<real> A = sweep_side<real>(a, lc, o, qa, Ia, S_o, chi_o, dsm, st, rw, chunk);
-            const real Ir = far_in<real>(a, qr, nu_f, F, f, err);
-            const Sweep<real> B = sweep_side<real>(a, lc, o, qr, Ir, S_o, chi_o, dsm, st, rw, chunk);
-            const real den = Prec<real>::rcp(A.y + B.y);
-            u = (A.p + B.p) * den;
-            lam = (A.c + B.c) * den;
-        } else {
-            const int64_t qs = (n_a > 0) ? qa : qr;
-            const real Is = far_in<real>(a, qs, nu_f, F, f, err);
-            const Sweep<real> A = sweep_side<real>(a, lc, o, qs, Is, S_o, chi_o, dsm, st, rw, chunk);
-            real I_o = 0;
+        // an empty ray (the origin is a boundary cell) is the virtual start with
+        // I_bdy of the origin's boundary entry
+        real y2 = 0, p2 = 0, c2 = 0, z_o = 0;
+        if (ns_a == 0 || ns_r == 0) {
             if (bo < 0) err |= ERR_EMPTY_SIDE;
-            else I_o = (real)(a.I_bdy[(int64_t)bo * F + f] * I_SCALE);
-            const real den = Prec<real>::rcp(A.y + (real)SQRT2);
-            u = (A.p + (real)SQRT2 * I_o) * den;
-            lam = A.c * den;
+            else z_o = (real)SQRT2 * (real)(a.I_bdy[(int64_t)bo * F + f] * I_SCALE);
+            y2 = (real)SQRT2;
         }
+        const real I_a = ns_a > 0 ? far_in<real>(a, qa, nu_f, F, f, err) : (real)0;
+        const real I_r = ns_r > 0 ? far_in<real>(a, qr, nu_f, F, f, err) : (real)0;
+        sweep_pair<real, ONE>(a, lc, o, qa, ns_a, qr, ns_r, I_a, I_r, S_o, chi_o, dsm, p_near, chunk, mode, win, y2,
+                              p2, c2);
+        const real den = Prec<real>::rcp(y2);
+        real u;
+        {
+#pragma clang fp contract(off)
+            u = (p2 + z_o) * den;
+        }
+        const real lam = c2 * den;
         const double u64 = (double)u * (1.0 / I_SCALE);
         J_acc += w2 * u64;
         Lam_acc += w2 * (double)lam;
@@ -945,7 +1292,7 @@ __global__ __launch_bounds__(WAVE * MAX_WAVES) void k_image(RFArgs<real> a, doub
 {
     using row_t = typename Prec<real>::row_t;
     extern __shared__ __align__(16) unsigned char smem[];
-    step_t<real, X64> *st = reinterpret_cast<step_t<real, X64> *>(smem);
+    Step *st = reinterpret_cast<Step *>(smem);
     row_t *rw = reinterpret_cast<row_t *>(smem + a.row_offset);
 
     const int G = gridDim.x;
@@ -1339,7 +1686,7 @@ __global__ void k_band_sum(int64_t N, int64_t SL, int nchunk, const double *__re
 template <typename real, bool X64 = false>
 int max_chunk(const mgr_ctx *ctx)
 {
-    const size_t per_entry = sizeof(step_t<real, X64>) + sizeof(typename Prec<real>::row_t) * ctx->L + 64;
+    const size_t per_entry = sizeof(Step) + sizeof(typename Prec<real>::row_t) * ctx->L + 64;
     const int ch = (int)(LDS_LIMIT / per_entry) - 1;
     return ch < CH_MAX ? ch : CH_MAX;
 }
@@ -1399,9 +1746,23 @@ int make_args(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
     a.grid_real = (int)groups;
     if (ch < 2 || ch > max_chunk<real, X64>(ctx)) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
     a.ch = ch;
-    a.row_offset = ((sizeof(step_t<real, X64>) * (ch + 1) + 63) / 64) * 64;
+    a.row_offset = ((sizeof(Step) * (ch + 1) + 63) / 64) * 64;
     a.line_offset = a.row_offset + sizeof(typename Prec<real>::row_t) * (ch + 1) * ctx->L;
     return MGR_OK;
+}
+
+// LDS of the field kernel: the window of each wave, then the line table.  With
+// many lines and waves a window holds fewer points than asked for.
+template <typename real>
+size_t field_lds(const mgr_ctx *ctx, RFArgs<real> &a)
+{
+    const size_t row = sizeof(typename Prec<real>::row_t) * ctx->L;
+    const size_t table = sizeof(double) * ctx->L;
+    const size_t fit = ((LDS_LIMIT - table) / a.nwg - Window<real>::fixed) / row;
+    a.ch = (int)std::max<size_t>(2, std::min<size_t>(a.ch, fit - 1));
+    a.wave_lds = (int)((Window<real>::fixed + row * (a.ch + 1) + 63) / 64 * 64);
+    a.line_offset = (size_t)a.wave_lds * a.nwg;
+    return a.line_offset + table;
 }
 
 template <typename real>
@@ -1443,37 +1804,38 @@ int launch_rf(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
         a.step_mask = (ctx->masks_valid && ctx->rf_window_skip) ? ctx->step_mask : nullptr;
     else
         a.step_mask = (ctx->masks64_valid && ctx->rf_window_skip) ? ctx->step_mask64 : nullptr;
+    a.noop_lo = INFINITY;   // never
+    a.noop_hi = 0.0f;
     if (sizeof(real) == 4 && a.step_mask && ctx->hdz32_max > 0.0f) {
-        // An out-of-window sub-point closes its row with c = chi_floor dz'_a + chi_floor dz'_b (each
-        // product rounded), at most cb = 2 chi_floor dz'_max (1 + 2^-20).  The no-op needs
-        // cb < y 2^-25 (then c is below half an ulp of y) and cb y < 2^-25 (then 1 + c y rounds to 1).
-        const double cb = 2.0 * (double)(float)(CHI_FLOOR * CHI_SCALE) * (double)ctx->hdz32_max * (1.0 + 0x1p-20);
+        // An out-of-window sub-point closes its row with c = chi dz'_a + chi' dz'_b (rounded twice),
+        // at most cb = 2 X dz'_max (1 + 2^-20).  The no-op needs cb < y 2^-25 (then c is below half an
+        // ulp of y) and cb y < 2^-25 (then 1 + c y rounds to 1).
+        const double cb = 2.0 * NEAR_X * (double)(float)(CHI_FLOOR * CHI_SCALE) * (double)ctx->hdz32_max * (1.0 + 0x1p-20);
         const double lo = cb * 0x1p25 * (1.0 + 0x1p-20), hi = 0x1p-25 / cb * (1.0 - 0x1p-20);
         if (lo < hi && lo < 3.0e38 && hi > 1.0e-37) {
             a.noop_lo = std::nextafter((float)lo, INFINITY);   // float(lo) may round below lo
             a.noop_hi = std::nextafter((float)hi, 0.0f);
         }
     }
+    a.span_stride = ctx->span_stride;
+    if (sizeof(real) == 8 && a.step_mask) a.span = ctx->span64;
+    if (sizeof(real) == 4 && a.step_mask && ctx->near_on) {
+        a.span = ctx->span32;
+        a.near_p = ctx->near_p;
+        a.near_bad = ctx->near_bad;
+    }
     a.root_major = ctx->root_major;
     a.far32 = (sizeof(real) == 4 && ctx->far_cache && ctx->far_valid[0]) ? ctx->far_I32 : nullptr;
     a.far64 = (sizeof(real) == 8 && ctx->far_cache && ctx->far_valid[1]) ? ctx->far_I64 : nullptr;
-    // FP32: one candidate line per bin when the lines' candidate ranges are disjoint
-    bool one = false;
-    if constexpr (sizeof(real) == 4) {
-        one = true;
-        for (int l = 0; l + 1 < ctx->h_tables.L; l++)
-            if (!(ctx->h_tables.line[l] * a.cand_lo <= ctx->h_tables.line[l + 1] * a.cand_hi)) one = false;
-        if (one) {
-            hipLaunchKernelGGL((k_radiation_field<real, true>), dim3(grid_of(a)), dim3(WAVE * a.nwg),
-                               lds_bytes(ctx, a), ctx->stream, a);
-            ctx->last_rf_kernel = "k_radiation_field<float, true>";
-        }
-    }
-    if (!one) {
-        hipLaunchKernelGGL((k_radiation_field<real, false>), dim3(grid_of(a)), dim3(WAVE * a.nwg),
-                           lds_bytes(ctx, a), ctx->stream, a);
-        ctx->last_rf_kernel = sizeof(real) == 4 ? "k_radiation_field<float, false>" : "k_radiation_field<double, false>";
-    }
+    // one candidate line per bin when the lines' candidate ranges are disjoint
+    bool one = true;
+    for (int l = 0; l + 1 < ctx->h_tables.L; l++)
+        if (!(ctx->h_tables.line[l] * a.cand_lo <= ctx->h_tables.line[l + 1] * a.cand_hi)) one = false;
+    const size_t lds = field_lds<real>(ctx, a);
+    auto kernel = one ? k_radiation_field<real, true> : k_radiation_field<real, false>;
+    hipLaunchKernelGGL(kernel, dim3(grid_of(a)), dim3(WAVE * a.nwg), lds, ctx->stream, a);
+    ctx->last_rf_kernel = sizeof(real) == 4 ? (one ? "k_radiation_field<float, true>" : "k_radiation_field<float, false>")
+                                            : (one ? "k_radiation_field<double, true>" : "k_radiation_field<double, false>");
     MGR_LAUNCH_CHECK();
     return MGR_OK;
 }

@@ -506,8 +506,9 @@ __global__ void k_step_masks(int64_t N, int Rmax, int nchunk, const int32_t *__r
                              const double *__restrict__ pw, const double *__restrict__ dshift_max,
                              const int64_t *__restrict__ seg_off, const int32_t *__restrict__ nseg,
                              const int32_t *__restrict__ seg_cell, const double *__restrict__ seg_shift,
-                             double window, const double *__restrict__ win,
-                             const int8_t *__restrict__ cnt, uint8_t *__restrict__ mask)
+                             double window, const double *__restrict__ near_pw, const double *__restrict__ win,
+                             const int8_t *__restrict__ cnt, uint8_t *__restrict__ mask,
+                             uint16_t *__restrict__ span, int64_t span_stride)
 {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= N * Rmax) return;
@@ -519,7 +520,8 @@ __global__ void k_step_masks(int64_t N, int Rmax, int nchunk, const int32_t *__r
     const int ns = nseg[q];
     const double dsm = dshift_max[o];
     int cn[STEP_MASK_CHUNKS];
-    for (int k = 0; k < nchunk; k++) cn[k] = cnt[(int64_t)o * STEP_MASK_CHUNKS + k];
+#pragma unroll
+    for (int k = 0; k < STEP_MASK_CHUNKS; k++) cn[k] = k < nchunk ? cnt[(int64_t)o * STEP_MASK_CHUNKS + k] : -1;
     const double *wo = win + (int64_t)o * STEP_MASK_CHUNKS * MAX_WIN * 2;
     int32_t c_prev = o;
     double s_prev = 1.0;   // co-moving shift of the origin
@@ -530,32 +532,107 @@ __global__ void k_step_masks(int64_t N, int Rmax, int nchunk, const int32_t *__r
         const int32_t cs[4] = {cb.x, cb.y, cb.z, cb.w};
         const double ss[4] = {sa.x, sa.y, sb.x, sb.y};
         unsigned word = 0;
+        ushort4 sp4[STEP_MASK_CHUNKS];
+#pragma unroll
+        for (int k = 0; k < STEP_MASK_CHUNKS; k++) sp4[k] = make_ushort4(SPAN_ALL, SPAN_ALL, SPAN_ALL, SPAN_ALL);
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             if (j0 + u >= ns) break;
             const int32_t c = cs[u];
             const double s = ss[u];
-            const bool interp = fabs(s - s_prev) > dsm;   // as split_step
+            const double ds = s - s_prev;
+            const bool interp = fabs(ds) > dsm;   // as split_step
             const double lo = interp ? fmin(s_prev, s) : s, hi = interp ? fmax(s_prev, s) : s;
             const double w = window * (interp ? fmax(pw[c_prev], pw[c]) : pw[c]);
+            const double v = near_pw ? (interp ? fmax(near_pw[c_prev], near_pw[c]) : near_pw[c]) : w;
             unsigned bits = 0;
-            for (int k = 0; k < nchunk; k++) {
+#pragma unroll
+            for (int k = 0; k < STEP_MASK_CHUNKS; k++) {
+                if (k >= nchunk) break;
                 const int n = cn[k];
                 if (n < 0) continue;
-                bool out = true;
+                bool out = true, span_out = true;
                 for (int i = 0; i < n; i++) {
                     const double a = wo[(k * MAX_WIN + i) * 2 + 0];
                     const double b = wo[(k * MAX_WIN + i) * 2 + 1];
                     if (hi >= (1.0 - w) * a && lo <= (1.0 + w) * b) out = false;
+                    if (hi >= (1.0 - v) * a && lo <= (1.0 + v) * b) span_out = false;
                 }
                 if (out) bits |= 1u << k;
+                if (!span) continue;
+                unsigned sp = span_out ? SPAN_NONE : SPAN_ALL;
+                if (!span_out && interp && n == 1) {
+                    // sub-point m lies at s_prev + m ds / np (split_step); those within
+                    // [x1, x2] can be in the window, with 1/100 of a sub-point (1/200 of a
+                    // width) for the rounding of the shifts
+                    const double x = fabs(ds) / dsm + 1;
+                    if (x < (double)(MAX_INTERPOLATION + 1)) {
+                        const int np = (int)x;
+                        const double e1 = ((1.0 - v) * wo[k * MAX_WIN * 2 + 0] - s_prev) * np / ds;
+                        const double e2 = ((1.0 + v) * wo[k * MAX_WIN * 2 + 1] - s_prev) * np / ds;
+                        const double x1 = fmin(e1, e2) - 0.01, x2 = fmax(e1, e2) + 0.01;
+                        const int m1 = x1 > 1.0 ? (x1 <= np ? (int)ceil(x1) : np + 1) : 1;
+                        const int m2 = x2 < np ? (x2 >= 1.0 ? (int)x2 : 0) : np;
+                        if (m2 < m1) sp = SPAN_NONE;
+                        else sp = (unsigned)((m1 - 1) * 256 / np) | (unsigned)min(255, (m2 * 256 + np - 1) / np - 1) << 8;
+                    }
+                }
+                if (u == 0) sp4[k].x = (uint16_t)sp;
+                else if (u == 1) sp4[k].y = (uint16_t)sp;
+                else if (u == 2) sp4[k].z = (uint16_t)sp;
+                else sp4[k].w = (uint16_t)sp;
             }
             word |= bits << (8 * u);
             c_prev = c;
             s_prev = s;
         }
         *reinterpret_cast<uint32_t *>(mask + s0 + j0) = word;
+        if (span) {
+#pragma unroll
+            for (int k = 0; k < STEP_MASK_CHUNKS; k++)
+                if (k < nchunk) *reinterpret_cast<ushort4 *>(span + k * span_stride + s0 + j0) = sp4[k];
+        }
     }
+}
+
+// Widths that the narrow window spans in each cell, times the cell's profile
+// width: the window of the cell with the largest total population over line
+// width (ratio, per sorted line), w2max = its square, less what the smaller
+// ratio of this cell allows, since its lines are that much weaker.
+__global__ void k_near_widths(int64_t N, const LineTables *__restrict__ tb, const double *__restrict__ pop_tot,
+                              const double *__restrict__ IW64, const double *__restrict__ pw_cmax,
+                              const double *__restrict__ ratio, double w2max, double *__restrict__ near_pw)
+{
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= N) return;
+    const int L = tb->L;
+    double rho = 0.0;
+    for (int l = 0; l < L; l++) {
+        const double r = pop_tot[(int64_t)tb->line_spec[tb->line_index[l]] * N + p] * IW64[p * L + l];
+        if (ratio[l] > 0.0) rho = fmax(rho, r / ratio[l]);
+    }
+    near_pw[p] = sqrt(fmax(rho > 0.0 ? w2max + log(rho) : 0.0, 4.0)) * pw_cmax[p];
+}
+
+// Largest total population over line width of every sorted line over all
+// cells (positive doubles order as their bits): with the line data it bounds
+// the emissivities and opacities that populations up to the total can give.
+__global__ void k_max_line(int64_t N, const LineTables *__restrict__ tb, const double *__restrict__ pop_tot,
+                           const double *__restrict__ IW64, uint64_t *__restrict__ out)
+{
+    __shared__ double sh[256];
+    const int l = blockIdx.y, L = tb->L;
+    const double *tot = pop_tot + (int64_t)tb->line_spec[tb->line_index[l]] * N;
+    double v = 0.0;
+    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < N; p += (int64_t)gridDim.x * blockDim.x)
+        v = fmax(v, tot[p] * IW64[p * L + l]);
+    sh[threadIdx.x] = v;
+    __syncthreads();
+    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + w]);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) atomicMax((unsigned long long *)&out[l], (unsigned long long)__double_as_longlong(sh[0]));
 }
 
 // Sums over the cached steps of (points x chunks) and of (points x chunks
@@ -807,7 +884,10 @@ int launch_trace(mgr_ctx *ctx)
         (void)hipFree(ctx->seg_cell); (void)hipFree(ctx->seg_shift); (void)hipFree(ctx->seg_dZ);
         (void)hipFree(ctx->seg_f32); (void)hipFree(ctx->seg_hdz32); (void)hipFree(ctx->step_mask);
         if (ctx->step_mask64) (void)hipFree(ctx->step_mask64);
+        if (ctx->span32) (void)hipFree(ctx->span32);
+        if (ctx->span64) (void)hipFree(ctx->span64);
         ctx->step_mask64 = nullptr;
+        ctx->span32 = ctx->span64 = nullptr;
         ctx->seg_cell = nullptr; ctx->seg_shift = nullptr; ctx->seg_dZ = nullptr;
         ctx->seg_f32 = nullptr; ctx->seg_hdz32 = nullptr; ctx->step_mask = nullptr;
     }
@@ -847,16 +927,59 @@ int launch_trace(mgr_ctx *ctx)
     return MGR_OK;
 }
 
+// The narrow window of the FP32 kernel's runs (Runs in the radiation unit) in
+// the cell with the widest profiles and largest possible rows: the square of
+// the smallest number of widths beyond which every line's opacity is below
+// NEAR_CHI / L of the floor and what its emission adds over a step is lost
+// against the boundary intensity of a 2.7 K background, so that a run that has
+// seen nothing else can be passed over.  Larger backgrounds and anything a ray
+// has picked up are above that; smaller ones fail the kernel's test and are
+// evaluated.  0: no such window narrower than the wide one.  p_min: what the
+// kernel holds p against (near_p).  ratio: k_max_line per sorted line; the
+// populations may reach twice the total in absolute value.
+static double near_window2(const mgr_ctx *ctx, const std::vector<double> &ratio, std::vector<float> &p_min)
+{
+    const LineTables &tb = ctx->h_tables;
+    const int L = tb.L;
+    const double slack = 1.05;   // rounding of x, exp2 and the sums in FP32
+    std::vector<double> add(L);
+    double w2 = 4.0;
+    for (int l = 0; l < L; l++) {
+        const int k = tb.line_index[l];
+        const double nu = tb.line[l] * (1.0 + 12.0 * ctx->pw_max);
+        const double pref = slack * nu * 2.0 * ratio[l] * HH_OVER_FOUR_PI * INVERSE_SQRT_PI * CHI_SCALE;
+        // the line's opacity over its share of the floor, and the intensity it can
+        // add over an interval times 2^25, both at the line's centre
+        const double chi = pref * (ctx->h_Ba[k] + ctx->h_Bs[k]) / (NEAR_CHI / L * CHI_FLOOR * CHI_SCALE);
+        add[l] = pref * I_SCALE * ctx->h_A[k] / (1.0 - NEAR_CHI) * 2.0 * NEAR_X * ctx->hdz32_max * 0x1p25;
+        const double I = SQRT2 * I_SCALE * TWO_HH_OVER_CC_SQUARED * tb.line[l] * tb.line[l] * tb.line[l] /
+                         std::expm1(HH_OVER_KB * tb.line[l] / T_CMB);
+        if (!std::isfinite(chi) || !std::isfinite(add[l])) return 0.0;
+        if (chi > 0.0) w2 = std::max(w2, std::log(chi));
+        if (add[l] > 0.0 && I > 0.0) w2 = std::max(w2, std::log(L * add[l] / (0.25 * I)));
+    }
+    double all = 0.0;
+    for (int l = 0; l < L; l++) {
+        const double x = add[l] * std::exp(-w2) * (1.0 + 0x1p-20);
+        all += x;
+        p_min[l] = std::nextafter((float)x, INFINITY);
+    }
+    p_min[L] = std::nextafter((float)all, INFINITY);
+    return std::sqrt(w2) < 0.97 * MASK_WINDOW ? w2 : 0.0;
+}
+
 // Computes the out-of-window bits of the cached steps for the current
-// frequencies (once per trace and spectral discretisation), for the FP32
-// kernel or (fp64) the FP64 one.  Models with more than STEP_MASK_CHUNKS
-// chunks of 64 bins get bits for the first ones only.
+// frequencies (once per trace and spectral discretisation), and the spans of
+// their sub-points in the window, for the FP32 kernel or (fp64) the FP64 one.
+// Models with more than STEP_MASK_CHUNKS chunks of 64 bins get them for the
+// first ones only.
 int launch_step_masks(mgr_ctx *ctx, bool fp64)
 {
     bool &valid = fp64 ? ctx->masks64_valid : ctx->masks_valid;
     if (valid || !ctx->traced || !ctx->spectral_set) return MGR_OK;
     uint8_t *&bits_out = fp64 ? ctx->step_mask64 : ctx->step_mask;
-    if (!bits_out) MGR_HIP(hipMalloc((void **)&bits_out, std::max<int64_t>(ctx->total_segments, 1)));
+    const int64_t T = std::max<int64_t>(ctx->total_segments, 1);
+    if (!bits_out) MGR_HIP(hipMalloc((void **)&bits_out, T));
     const double window = fp64 ? MASK_WINDOW64 : MASK_WINDOW;
     const int64_t N = ctx->N;
     const int nchunk = (int)std::min<int64_t>((ctx->F + WAVE - 1) / WAVE, STEP_MASK_CHUNKS);
@@ -873,36 +996,60 @@ int launch_step_masks(mgr_ctx *ctx, bool fp64)
     }
     if (rm != ctx->root_major) ctx->graph_precision = -1;   // captured launches hold the old order
     ctx->root_major = rm;
-    double *win = nullptr;
-    int8_t *cnt = nullptr;
-    MGR_HIP(hipMalloc((void **)&win, (size_t)N * STEP_MASK_CHUNKS * MAX_WIN * 2 * sizeof(double)));
-    if (hipMalloc((void **)&cnt, (size_t)N * STEP_MASK_CHUNKS) != hipSuccess) {
-        (void)hipFree(win);
-        return ctx->fail(MGR_ERR_DEVICE, "out of device memory");
+    DeviceBuffer red, win, cnt, near_pw;
+    MGR_HIP(hipMalloc(&win.p, (size_t)N * STEP_MASK_CHUNKS * MAX_WIN * 2 * sizeof(double)));
+    MGR_HIP(hipMalloc(&cnt.p, (size_t)N * STEP_MASK_CHUNKS));
+    // two bytes per chunk and step beside the trace's forty-odd; without memory
+    // for them the bits (FP32) or nothing (FP64) is left out
+    uint16_t *&span = fp64 ? ctx->span64 : ctx->span32;
+    ctx->span_stride = (T + 3) / 4 * 4;
+    if (!span && hipMalloc((void **)&span, (size_t)nchunk * ctx->span_stride * sizeof(uint16_t)) != hipSuccess) {
+        (void)hipGetLastError();
+        span = nullptr;
+    }
+    bool near = false;
+    if (!fp64) {
+        // the largest dz' bounds the row closings of out-of-window sub-points,
+        // the largest populations what they can add
+        std::vector<uint64_t> h(tb.L + 1, 0);
+        MGR_HIP(hipMalloc(&red.p, h.size() * sizeof(uint64_t)));
+        uint64_t *d = (uint64_t *)red.p;
+        MGR_HIP(hipMemsetAsync(d, 0, h.size() * sizeof(uint64_t), ctx->stream));
+        if (ctx->total_segments > 0)
+            hipLaunchKernelGGL(k_max_hdz, dim3(1024), dim3(256), 0, ctx->stream, ctx->total_segments, ctx->seg_hdz32,
+                               (unsigned *)(d + tb.L));
+        hipLaunchKernelGGL(k_max_line, dim3((unsigned)std::min<int64_t>((N + 255) / 256, 256), (unsigned)tb.L), dim3(256),
+                           0, ctx->stream, N, ctx->tables, ctx->pop_tot, ctx->IW64, d);
+        MGR_LAUNCH_CHECK();
+        MGR_HIP(hipMemcpyAsync(h.data(), d, h.size() * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+        MGR_HIP(hipStreamSynchronize(ctx->stream));
+        const unsigned bits = (unsigned)h[tb.L];
+        std::memcpy(&ctx->hdz32_max, &bits, sizeof(float));
+        std::vector<double> ratio(tb.L);
+        std::vector<float> p_min(tb.L + 1);
+        std::memcpy(ratio.data(), h.data(), tb.L * sizeof(double));
+        const double w2 = span && ctx->hdz32_max > 0.0f ? near_window2(ctx, ratio, p_min) : 0.0;
+        near = w2 > 0.0;
+        if (near) {
+            MGR_HIP(hipMalloc(&near_pw.p, (size_t)N * sizeof(double)));
+            hipLaunchKernelGGL(k_near_widths, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, ctx->stream, N,
+                               ctx->tables, ctx->pop_tot, ctx->IW64, ctx->pw_cmax, (const double *)d, w2,
+                               (double *)near_pw.p);
+            MGR_HIP(hipMemcpy(ctx->near_p, p_min.data(), p_min.size() * sizeof(float), hipMemcpyHostToDevice));
+        }
+        if (near != ctx->near_on) ctx->graph_precision = -1;   // captured launches hold the old choice
+        ctx->near_on = near;
     }
     hipLaunchKernelGGL(k_chunk_windows, dim3((unsigned)((N * nchunk + 3) / 4)), dim3(4 * WAVE), 0, ctx->stream, N,
                        (int)ctx->F, nchunk, rm, ctx->tables, ctx->nu, ctx->shift_min, ctx->shift_max, ctx->pw_max,
-                       window, win, cnt);
+                       window, (double *)win.p, (int8_t *)cnt.p);
     hipLaunchKernelGGL(k_step_masks, dim3((unsigned)((N * ctx->R + 127) / 128)), dim3(128), 0, ctx->stream, N,
                        (int)ctx->R, nchunk, ctx->d_cell_model, ctx->d_cell_qbase, ctx->d_m_R, ctx->pw_cmax,
                        ctx->dshift_max, ctx->seg_off,
-                       ctx->nseg, ctx->seg_cell, ctx->seg_shift, window, win, cnt, bits_out);
-    // the largest dz' bounds the row closings of out-of-window sub-points (FP32)
-    unsigned *dmax = reinterpret_cast<unsigned *>(cnt);   // N * STEP_MASK_CHUNKS >= 4 bytes, no longer read
-    hipError_t le = hipGetLastError();
-    if (le == hipSuccess) le = hipMemsetAsync(dmax, 0, sizeof(unsigned), ctx->stream);
-    if (le == hipSuccess && ctx->total_segments > 0 && !fp64) {
-        hipLaunchKernelGGL(k_max_hdz, dim3(1024), dim3(256), 0, ctx->stream, ctx->total_segments, ctx->seg_hdz32,
-                           dmax);
-        le = hipGetLastError();
-    }
-    unsigned bits = 0;
-    const hipError_t se = hipStreamSynchronize(ctx->stream);
-    if (le == hipSuccess && se == hipSuccess) le = hipMemcpy(&bits, dmax, sizeof(unsigned), hipMemcpyDeviceToHost);
-    (void)hipFree(win);
-    (void)hipFree(cnt);
-    if (le != hipSuccess || se != hipSuccess) return ctx->fail(MGR_ERR_DEVICE, "step-mask kernels failed");
-    if (!fp64) std::memcpy(&ctx->hdz32_max, &bits, sizeof(float));
+                       ctx->nseg, ctx->seg_cell, ctx->seg_shift, window, (const double *)near_pw.p, (double *)win.p,
+                       (int8_t *)cnt.p, bits_out, fp64 || near ? span : nullptr, ctx->span_stride);
+    MGR_LAUNCH_CHECK();
+    MGR_HIP(hipStreamSynchronize(ctx->stream));
     valid = true;
     return MGR_OK;
 }
