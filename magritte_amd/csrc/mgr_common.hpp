@@ -156,6 +156,7 @@ struct mgr_ctx {
     int64_t *d_cell_qbase = nullptr;   // [N] first (origin, ray) entry of the cell
     int32_t *d_m_R = nullptr, *d_m_rbase = nullptr, *d_m_active = nullptr;   // [M]
     int32_t *h_m_active = nullptr;     // pinned [M]
+    bool     all_active = true;        // the device's flags are all 1
     // segmented reductions: chunk c covers cells [chunk_cell[c], chunk_cell[c+1])
     // of one model; the chunks of model m are m_chunk_off[m] .. m_chunk_off[m+1]-1
     int64_t nchunks = 0;
@@ -383,19 +384,19 @@ int launch_emissivity_opacity(mgr_ctx *ctx);
 int clear_near_bad(mgr_ctx *ctx);   // before the rows of newly set populations (outside graph capture)
 int launch_trace(mgr_ctx *ctx);
 int launch_forward_masks(mgr_ctx *ctx);   // candidate neighbours of every (cell, ray), once
-int launch_radiation_field(mgr_ctx *ctx, int precision);   // kernel + Lambda*
 int launch_far_cache(mgr_ctx *ctx, int precision);   // outside graph capture
 int launch_rf_kernel(mgr_ctx *ctx, int precision);
 int tune_radiation_field(mgr_ctx *ctx, int precision);   // outside graph capture
 int launch_lambda(mgr_ctx *ctx);
 int launch_band(mgr_ctx *ctx);         // band elements of Lambda* (nband > 0)
 int launch_band_cells(mgr_ctx *ctx);   // band cells and their reverse map (at trace time)
-int launch_jeff(mgr_ctx *ctx);
+int launch_jeff(mgr_ctx *ctx, bool lambda);
 int launch_stateq(mgr_ctx *ctx);
 int launch_convergence(mgr_ctx *ctx);
 int launch_ng(mgr_ctx *ctx);
 int read_convergence(mgr_ctx *ctx, mgr_conv *conv);
 int set_active(mgr_ctx *ctx, bool all);   // all: every model of the batch iterates
+int clear_error(mgr_ctx *ctx);         // outside graph capture
 int launch_trace_image(mgr_ctx *ctx, int64_t ray);   // rest-frame trace of ray and its antipode
 int launch_step_masks(mgr_ctx *ctx, bool fp64);   // out-of-window bits of the cached steps (when stale)
 void free_image(mgr_ctx *ctx);

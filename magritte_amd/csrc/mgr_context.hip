@@ -673,6 +673,7 @@ int upload_models(mgr_ctx *ctx, const mgr_model_view *models, int64_t nmodels)
     {
         std::vector<int32_t> ones(Mm, 1);
         if ((rc = upload(ctx, &ctx->d_m_active, ones.data(), Mm))) return rc;
+        ctx->all_active = true;
     }
     if ((rc = dalloc(ctx, &ctx->d_mconv, Mm * 4))) return rc;
     if ((rc = dalloc(ctx, &ctx->d_mng, Mm * 4))) return rc;

@@ -12,6 +12,7 @@
 // cell, so the reference's global SparseLU<COLAMD> of size (N V)^2 is block
 // diagonal: here one thread solves one cell's V x V system with partial
 // pivoting in FP64 registers (V known at compile time for V <= 8).
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 #include <string>
@@ -47,30 +48,80 @@ __global__ void k_lambda_sum(int64_t N, int L, int nchunk, const double *__restr
 // With band elements (band_cell non-null) every element of (p, k) enters:
 // diff = Ls(p,k) n_i(p) + sum over the slots of p of Ls(slot, k) n_i(cell).
 // One species: its L lines are lines loff .. loff+L-1 of the per-line arrays
-// [N][Lst]; pop, qw and irad are the species' own.
-__global__ void k_jeff(int64_t N, int L, int Lst, int loff, int Q, int F, int V, const double *__restrict__ J,
-                       const int32_t *__restrict__ nr_line, const double *__restrict__ qw,
-                       const int32_t *__restrict__ irad, const double *__restrict__ pop,
-                       const double *__restrict__ Ls, double *__restrict__ Jlin,
-                       double *__restrict__ Jeff, double *__restrict__ Jdif, int64_t S,
-                       const int32_t *__restrict__ band_cell, const double *__restrict__ band_Ls)
+// [N][Lst]; pop, qw and irad are the species' own.  With Lpart given the lines'
+// Ls are first added up from the waves' shares, as k_lambda_sum does.
+struct JeffArgs {
+    int64_t N;
+    int L, Lst, loff, Q, F, V, nchunk;
+    const double *J;
+    const int32_t *nr_line;
+    const double *qw;
+    const int32_t *irad;
+    const double *pop, *Lpart;
+    double *Ls, *Jlin, *Jeff, *Jdif;
+    int64_t S;
+    const int32_t *band_cell;
+    const double *band_Ls;
+};
+
+__device__ __forceinline__ void jeff_finish(const JeffArgs &a, int64_t p, int k, double jl)
+{
+    const int64_t pk = p * a.Lst + a.loff + k;
+    double ls;
+    if (a.Lpart) {
+        ls = 0.0;
+        for (int c = 0; c < a.nchunk; c++) ls += a.Lpart[(p * a.nchunk + c) * a.Lst + a.loff + k];
+        a.Ls[pk] = ls;
+    } else {
+        ls = a.Ls[pk];
+    }
+    double diff = ls * a.pop[p * a.V + a.irad[k]];
+    if (a.band_cell)
+        for (int64_t sl = p * a.S; sl < (p + 1) * a.S; sl++) {
+            const int32_t c = a.band_cell[sl];
+            if (c >= 0) diff += a.band_Ls[sl * a.Lst + a.loff + k] * a.pop[(int64_t)c * a.V + a.irad[k]];
+        }
+    a.Jlin[pk] = jl;
+    a.Jeff[pk] = jl - HH_OVER_FOUR_PI * diff;
+    a.Jdif[pk] = HH_OVER_FOUR_PI * diff;
+}
+
+// One thread per (cell, line), for more bins than a cell's row of J in LDS.
+__global__ void k_jeff(JeffArgs a)
 {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= N * L) return;
-    const int64_t p = t / L;
-    const int k = (int)(t % L);
-    const int64_t pk = p * Lst + loff + k;
+    if (t >= a.N * a.L) return;
+    const int64_t p = t / a.L;
+    const int k = (int)(t % a.L);
+    const int64_t pk = p * a.Lst + a.loff + k;
     double jl = 0.0;
-    for (int z = 0; z < Q; z++) jl += qw[z] * J[p * F + nr_line[pk * Q + z]];
-    double diff = Ls[pk] * pop[p * V + irad[k]];
-    if (band_cell)
-        for (int64_t sl = p * S; sl < (p + 1) * S; sl++) {
-            const int32_t c = band_cell[sl];
-            if (c >= 0) diff += band_Ls[sl * Lst + loff + k] * pop[(int64_t)c * V + irad[k]];
-        }
-    Jlin[pk] = jl;
-    Jeff[pk] = jl - HH_OVER_FOUR_PI * diff;
-    Jdif[pk] = HH_OVER_FOUR_PI * diff;
+    for (int z = 0; z < a.Q; z++) jl += a.qw[z] * a.J[p * a.F + a.nr_line[pk * a.Q + z]];
+    jeff_finish(a, p, k, jl);
+}
+
+// The same with the rows of J of `cells` cells, and their bins of every root,
+// read in order into LDS and summed there.  One thread per (cell, line) on
+// global memory touched a cache line per lane and root: at 64^3 cells and 186
+// bins 1.71 ms for the 390 MB of J and 0.01 ms for the sum of Lambda*, here
+// 0.22 ms for both; at 1000 cells 13 + 5 us, here 7.
+__global__ __launch_bounds__(256) void k_jeff_rows(JeffArgs a, int cells)
+{
+    extern __shared__ double rows[];
+    const int64_t p0 = (int64_t)blockIdx.x * cells;
+    const int nc = (int)min((int64_t)cells, a.N - p0);
+    const int LQ = a.L * a.Q;
+    int32_t *bin = reinterpret_cast<int32_t *>(rows + cells * a.F);
+    for (int i = threadIdx.x; i < nc * a.F; i += blockDim.x) rows[i] = a.J[p0 * a.F + i];
+    for (int i = threadIdx.x; i < nc * LQ; i += blockDim.x) {
+        const int c = i / LQ;
+        bin[i] = c * a.F + a.nr_line[((p0 + c) * a.Lst + a.loff) * a.Q + (i - c * LQ)];
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < nc * a.L; i += blockDim.x) {
+        double jl = 0.0;
+        for (int z = 0; z < a.Q; z++) jl += a.qw[z] * rows[bin[i * a.Q + z]];
+        jeff_finish(a, p0 + i / a.L, i % a.L, jl);
+    }
 }
 
 // search (src/Functions/interpolation.tpp:14-54)
@@ -172,11 +223,10 @@ __device__ __forceinline__ void stateq_assemble(const StateqArgs &a, int64_t p, 
     y[Vn - 1] = a.pop_tot[p];
 }
 
-template <int VV>
-__device__ __forceinline__ void stateq_cell(const StateqArgs &a, int64_t p, int V, double *M, double *y)
+// Generic: one thread per cell, V levels known at run time.
+__device__ __forceinline__ void stateq_cell(const StateqArgs &a, int64_t p, int Vn, double *M, double *y)
 {
-    const int Vn = (VV > 0) ? VV : V;
-    stateq_assemble<VV>(a, p, Vn, M, y);
+    stateq_assemble<0>(a, p, Vn, M, y);
     // LU with partial pivoting
     for (int c = 0; c < Vn; c++) {
         int piv = c;
@@ -214,14 +264,148 @@ __device__ __forceinline__ void stateq_cell(const StateqArgs &a, int64_t p, int 
     for (int i = 0; i < Vn; i++) a.pop[p * Vn + i] = y[i];
 }
 
+// Eight lanes per cell, V = VV <= 8 levels: lane r owns row r of the system.
+// The rows are put together in LDS (the transitions' levels index their
+// columns), each entry from the same terms in the same order as
+// stateq_assemble, and eliminated in registers with partial pivoting, the
+// pivot row handed round by shuffles; the rows stay where they are and carry
+// their position in the pivoted order instead.  One thread per cell kept its
+// matrix in scratch memory (the pivot's row is not known at compile time) and
+// left a small model's cells to a few wavefronts: 1000 cells of 7 levels
+// 45 us, here 15; 262144 cells 336 us, here 138 (1.1 TB/s of the history's and
+// tables' bytes; the chain of the elimination's shuffles and divides).
+constexpr int SQ_LANES = 8, SQ_CELLS = 32;   // lanes per cell, cells per block
+__device__ __forceinline__ double from_row(double x, int r) { return __shfl(x, r, SQ_LANES); }
+
 template <int VV>
-__global__ void k_stateq(StateqArgs a)
+__global__ __launch_bounds__(SQ_LANES *SQ_CELLS) void k_stateq(StateqArgs a)
 {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double sM[SQ_CELLS][VV][VV];
+    const int r = threadIdx.x % SQ_LANES, slot = threadIdx.x / SQ_LANES;
+    const int64_t p = (int64_t)blockIdx.x * SQ_CELLS + slot;
     if (p >= a.N) return;
-    if (!a.m_active[a.cell_model[p]]) return;
-    double M[VV * VV], y[VV];
-    stateq_cell<VV>(a, p, VV, M, y);
+    if (!a.m_active[a.cell_model[p]]) return;   // whole groups of lanes: their shuffles stay among themselves
+    const bool lev = r < VV;
+    const int rr = lev ? r : VV - 1;
+    // history: prev3 <- prev2 <- prev1 <- population (lineProducingSpecies.tpp:260-262)
+    const int64_t ind = p * VV + rr;
+    const double x = a.pop[ind];
+    if (lev) {
+        a.prev3[ind] = a.prev2[ind];
+        a.prev2[ind] = a.prev1[ind];
+        a.prev1[ind] = x;
+    }
+    double *row = sM[slot][rr];
+    if (lev)
+#pragma unroll
+        for (int j = 0; j < VV; j++) row[j] = 0.0;
+    double diag = 0.0;
+    // a transition I -> J: rows J and I gain a term each off and on the diagonal
+    auto add = [&](int I, int J, double v_IJ, double v_JI) {
+        if (!lev || (r != I && r != J)) return;
+        row[r == J ? I : J] += r == J ? v_IJ : v_JI;
+        diag += r == J ? -v_JI : -v_IJ;
+    };
+    // radiative transitions (transpose convention of the reference)
+    for (int k = 0; k < a.L; k++) {
+        const double Je = a.Jeff[p * a.Lst + k];
+        const double v_IJ = a.A[k] + a.Bs[k] * Je;
+        const double v_JI = a.Ba[k] * Je;
+        add(a.irad[k], a.jrad[k], v_IJ, v_JI);
+    }
+    // approximated Lambda operator with the pre-solve opacity
+    for (int k = 0; k < a.L; k++) {
+        const int I = a.irad[k], J = a.jrad[k];
+        const double opacity = HH_OVER_FOUR_PI * (from_row(x, J) * a.Ba[k] - from_row(x, I) * a.Bs[k]);
+        const double v_IJ = -a.Ls[p * a.Lst + k] * opacity;
+        if (lev && r == J) row[I] += v_IJ;
+        if (r == I) diag += -v_IJ;
+    }
+    // collisional transitions (collisionPartner.tpp:15-72), eight at a time
+    const double Tp = a.T[p];
+    for (int c = 0; c < a.ncolpar; c++) {
+        double abn = a.abundance[p * a.nspecs + a.cp_num[c]];
+        if (a.cp_op[c] != 0) {
+            const double frac_H2_para = 1.0 / (1.0 + 9.0 * exp(-170.5 / Tp));
+            if (a.cp_op[c] == 1) abn *= (1.0 - frac_H2_para);
+            if (a.cp_op[c] == 2) abn *= frac_H2_para;
+        }
+        const int ncol = a.cp_ncol[c], ntmp = a.cp_ntmp[c];
+        const double *tmp = a.tmp + a.cp_toff[c];
+        const double *Cd = a.Cd + a.cp_coff[c];
+        const double *Ce = a.Ce + a.cp_coff[c];
+        const int t = search_table(tmp, ntmp, Tp);
+        const double step = (t == 0) ? 0.0 : (Tp - tmp[t - 1]) / (tmp[t] - tmp[t - 1]);
+        for (int k0 = 0; k0 < ncol; k0 += SQ_LANES) {
+            const int k = min(k0 + r, ncol - 1);
+            double ce, cd;
+            if (t == 0) {
+                ce = Ce[k];
+                cd = Cd[k];
+            } else {
+                ce = Ce[(t - 1) * ncol + k] + (Ce[t * ncol + k] - Ce[(t - 1) * ncol + k]) * step;
+                cd = Cd[(t - 1) * ncol + k] + (Cd[t * ncol + k] - Cd[(t - 1) * ncol + k]) * step;
+            }
+            const double down = cd * abn, up = ce * abn;
+            const int n = min(SQ_LANES, ncol - k0);
+            for (int u = 0; u < n; u++)
+                add(a.icol[a.cp_koff[c] + k0 + u], a.jcol[a.cp_koff[c] + k0 + u], from_row(down, u), from_row(up, u));
+        }
+    }
+    // conservation replaces the last level's equation
+    double m[VV], y = r == VV - 1 ? a.pop_tot[p] : 0.0;
+#pragma unroll
+    for (int j = 0; j < VV; j++) m[j] = r == VV - 1 ? 1.0 : j == r ? diag : row[j];
+    int at = lev ? r : VV;   // this row's place in the pivoted order
+    int lane_at[VV];         // and the row at each place, once fixed
+    bool singular = false;
+#pragma unroll
+    for (int c = 0; c < VV; c++) {
+        // the largest |entry| at or after place c, the first of equals
+        double best = at >= c && lev ? fabs(m[c]) : -1.0;
+        if (best != best) best = INFINITY;   // a NaN spreads to every row
+        int where = at << 3 | r;
+#pragma unroll
+        for (int off = 1; off < SQ_LANES; off <<= 1) {
+            const double v = __shfl_xor(best, off, SQ_LANES);
+            const int w = __shfl_xor(where, off, SQ_LANES);
+            if (v > best || (v == best && w < where)) { best = v; where = w; }
+        }
+        if (best == 0.0) singular = true;
+        const int piv = where & (SQ_LANES - 1), from = where >> 3;
+        // rows exchange places c and `from`
+        if (at == c) at = from;
+        if (r == piv) at = c;
+        lane_at[c] = piv;
+        double pr[VV];
+#pragma unroll
+        for (int j = c; j < VV; j++) pr[j] = from_row(m[j], piv);
+        const double yp = from_row(y, piv);
+        const double l = m[c] * (1.0 / pr[c]);
+        if (at > c && lev) {
+#pragma unroll
+            for (int j = c + 1; j < VV; j++) m[j] = __builtin_fma(-l, pr[j], m[j]);
+            y = __builtin_fma(-l, yp, y);
+        }
+    }
+    if (singular) {
+        if (r == 0) atomicOr(a.err_flag, ERR_SINGULAR);
+        return;
+    }
+    // back substitution: every lane follows, the one whose turn it is counts
+    double sol[VV];
+#pragma unroll
+    for (int c = VV - 1; c >= 0; c--) {
+        double acc = y;
+#pragma unroll
+        for (int j = c + 1; j < VV; j++) acc = __builtin_fma(-m[j], sol[j], acc);
+        sol[c] = from_row(acc / m[c], lane_at[c]);
+    }
+    double out = sol[0];
+#pragma unroll
+    for (int j = 1; j < VV; j++)
+        if (r == j) out = sol[j];
+    if (lev) a.pop[p * VV + r] = out;
 }
 
 constexpr int VMAX_GENERIC = 32;
@@ -232,7 +416,7 @@ __global__ void k_stateq_generic(StateqArgs a)
     if (p >= a.N) return;
     if (!a.m_active[a.cell_model[p]]) return;
     double M[VMAX_GENERIC * VMAX_GENERIC], y[VMAX_GENERIC];
-    stateq_cell<0>(a, p, a.V, M, y);
+    stateq_cell(a, p, a.V, M, y);
 }
 
 // ---- rate equations with band elements ----------------------------------------
@@ -417,83 +601,130 @@ __global__ void k_band_check(const int32_t *flags, int n, int32_t *err_flag)
     if (flags[n]) atomicOr(err_flag, ERR_BAND);
 }
 
+// Sum of RED_BLOCK = 256 values by one wave, in the order of a tree over halves.
+__device__ __forceinline__ double tree_sum(const double *sh, int t)
+{
+    double v = (sh[t] + sh[t + 128]) + (sh[t + 64] + sh[t + 192]);
+    for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_down(v, off);
+    return v;
+}
+
+// Sum of v over a block of RED_BLOCK threads, for every thread; sh: RED_BLOCK
+// doubles.
 __device__ __forceinline__ double block_sum(double v, double *sh)
 {
-    sh[threadIdx.x] = v;
+    const int t = threadIdx.x;
+    __syncthreads();   // sh is read no longer
+    sh[t] = v;
     __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-        __syncthreads();
+    if (t < WAVE) {
+        v = tree_sum(sh, t);
+        if (t == 0) sh[0] = v;
     }
-    const double r = sh[0];
     __syncthreads();
-    return r;
+    return sh[0];
 }
 
 __device__ __forceinline__ double block_max(double v, double *sh)
 {
-    sh[threadIdx.x] = v;
+    const int t = threadIdx.x;
     __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + s]);
-        __syncthreads();
+    sh[t] = v;
+    __syncthreads();
+    if (t < WAVE) {
+        v = fmax(fmax(sh[t], sh[t + 128]), fmax(sh[t + 64], sh[t + 192]));
+        for (int off = WAVE / 2; off > 0; off >>= 1) v = fmax(v, __shfl_down(v, off));
+        if (t == 0) sh[0] = v;
     }
-    const double r = sh[0];
     __syncthreads();
-    return r;
+    return sh[0];
 }
 
-// check_for_convergence (lineProducingSpecies.tpp:120-171): per block partial
-// sums of the not-converged weight and the mean relative change, and the
-// maximum relative change; levels with n <= 1e-10 n_tot are ignored.
 // check_for_convergence (lineProducingSpecies.tpp:120-171) per model: each
-// block reduces one chunk of cells of one model; the final kernel sums the
+// block reduces one chunk of cells of one model to its sums of the
+// not-converged weight and the mean relative change, and the maximum relative
+// change; levels with n <= 1e-10 n_tot are ignored.  The final kernel sums the
 // chunks of every model in order (deterministic) and reports, for the batch,
-// the worst model.
-__global__ void k_conv_partial(int V, double pop_prec, const int64_t *__restrict__ chunk_cell,
-                               const int32_t *__restrict__ cell_model, const int64_t *__restrict__ m_cell_off,
-                               const double *__restrict__ pop, const double *__restrict__ prev1,
-                               const double *__restrict__ pop_tot, double *__restrict__ partials,
-                               int32_t *__restrict__ err_flag)
+// the worst model.  One thread per cell of a chunk: with four cells each, a
+// small model's one chunk took 12.7 us, here 6.6.
+constexpr int CONV_BLOCK = CHUNK_CELLS;
+static_assert(CONV_BLOCK <= 1024, "one thread per cell of a chunk");
+__global__ __launch_bounds__(CONV_BLOCK) void k_conv_partial(
+    int V, double pop_prec, const int64_t *__restrict__ chunk_cell, const int32_t *__restrict__ cell_model,
+    const int64_t *__restrict__ m_cell_off, const double *__restrict__ pop, const double *__restrict__ prev1,
+    const double *__restrict__ pop_tot, double *__restrict__ partials, int32_t *__restrict__ err_flag)
 {
-    __shared__ double sh[RED_BLOCK];
+    __shared__ double sh[2][CONV_BLOCK / WAVE], tree[RED_BLOCK];
+    __shared__ int32_t over[CONV_BLOCK];
     const int64_t c0 = chunk_cell[blockIdx.x], c1 = chunk_cell[blockIdx.x + 1];
     const int32_t mdl = cell_model ? cell_model[c0] : 0;   // null: one model
     const double weight = 1.0 / (double)((m_cell_off[mdl + 1] - m_cell_off[mdl]) * V);
-    double fnc = 0.0, rcm = 0.0, rmax = 0.0;
+    double rcm = 0.0, rmax = 0.0;
+    int32_t n_over = 0;
     bool finite = true;
-    for (int64_t p = c0 + threadIdx.x; p < c1; p += blockDim.x) {
+    const int64_t p = c0 + threadIdx.x;
+    if (p < c1) {
         const double min_pop = 1.0E-10 * pop_tot[p];
         for (int i = 0; i < V; i++) {
             const int64_t ind = p * V + i;
+            const double n = pop[ind], n1 = prev1[ind];
             // the criterion passes over NaN populations (the comparison below
             // is false for them), so a diverged iteration would look converged:
             // it is reported instead (err_flag null: not checked)
-            finite = finite && __builtin_isfinite(pop[ind]);
-            if (pop[ind] > min_pop) {
+            finite = finite && __builtin_isfinite(n);
+            if (n > min_pop) {
                 double rc = 2.0;
-                rc *= fabs(pop[ind] - prev1[ind]);
-                rc /= (pop[ind] + prev1[ind]);
-                if (rc > pop_prec) fnc += weight;
+                rc *= fabs(n - n1);
+                rc /= (n + n1);
+                if (rc > pop_prec) n_over++;
                 rcm += weight * rc;
                 rmax = fmax(rmax, rc);
             }
         }
     }
     if (!finite && err_flag) atomicOr(err_flag, ERR_NONFINITE);
-    fnc = block_sum(fnc, sh);
-    rcm = block_sum(rcm, sh);
-    rmax = block_max(rmax, sh);
-    if (threadIdx.x == 0) {
-        partials[3 * blockIdx.x + 0] = fnc;
-        partials[3 * blockIdx.x + 1] = rcm;
-        partials[3 * blockIdx.x + 2] = rmax;
+    over[threadIdx.x] = n_over;
+    for (int off = WAVE / 2; off > 0; off >>= 1) {
+        rcm += __shfl_down(rcm, off);
+        rmax = fmax(rmax, __shfl_down(rmax, off));
+    }
+    if (threadIdx.x % WAVE == 0) {
+        sh[0][threadIdx.x / WAVE] = rcm;
+        sh[1][threadIdx.x / WAVE] = rmax;
+    }
+    __syncthreads();
+    // the weights are added in one fixed order, four cells and then a tree: the
+    // sum is compared with a round number, so its rounding decides at a tie
+    if (threadIdx.x < RED_BLOCK) {
+        double fnc = 0.0;
+        int n = 0;
+        for (int c = threadIdx.x; c < CONV_BLOCK; c += RED_BLOCK) n += over[c];
+        for (int i = 0; i < n; i++) fnc += weight;
+        tree[threadIdx.x] = fnc;
+    }
+    __syncthreads();
+    if (threadIdx.x < WAVE) {
+        const double v = tree_sum(tree, threadIdx.x);
+        if (threadIdx.x == 0) partials[3 * blockIdx.x + 0] = v;
+    } else if (threadIdx.x < WAVE + 2) {
+        const double *w = sh[threadIdx.x - WAVE];
+        double v = w[0];
+        for (int i = 1; i < CONV_BLOCK / WAVE; i++) v = threadIdx.x == WAVE ? v + w[i] : fmax(v, w[i]);
+        partials[3 * blockIdx.x + 1 + threadIdx.x - WAVE] = v;
     }
 }
 
+// Host copies of the results of an iteration: pinned memory that the last
+// kernel writes itself, instead of two copies behind it; that kernel also
+// clears the error word for the next iteration.
+struct ConvOut {
+    double  *out, *mconv;   // null: none
+    int32_t *err_clear;     // null: kept
+};
+
 __global__ void k_conv_final(int64_t M, const int64_t *__restrict__ m_chunk_off, const double *__restrict__ partials,
                              const int32_t *__restrict__ m_active, double *__restrict__ mconv,
-                             double *__restrict__ out, const int32_t *__restrict__ err_flag)
+                             double *__restrict__ out, const int32_t *err_flag, ConvOut host)
 {
     __shared__ double sh[RED_BLOCK];
     double a = 0.0, b = 0.0, c = 0.0;
@@ -508,6 +739,12 @@ __global__ void k_conv_final(int64_t M, const int64_t *__restrict__ m_chunk_off,
         mconv[4 * m + 1] = fb;
         mconv[4 * m + 2] = fc;
         mconv[4 * m + 3] = (double)m_active[m];
+        if (host.mconv) {
+            host.mconv[4 * m + 0] = fa;
+            host.mconv[4 * m + 1] = fb;
+            host.mconv[4 * m + 2] = fc;
+            host.mconv[4 * m + 3] = (double)m_active[m];
+        }
         if (m_active[m]) {
             a = fmax(a, fa);
             b = fmax(b, fb);
@@ -518,10 +755,18 @@ __global__ void k_conv_final(int64_t M, const int64_t *__restrict__ m_chunk_off,
     b = block_max(b, sh);
     c = block_max(c, sh);
     if (threadIdx.x == 0) {
+        const double e = (double)(*err_flag);
         out[0] = a;
         out[1] = b;
         out[2] = c;
-        out[3] = (double)(*err_flag);
+        out[3] = e;
+        if (host.out) {
+            host.out[0] = a;
+            host.out[1] = b;
+            host.out[2] = c;
+            host.out[3] = e;
+        }
+        if (host.err_clear) *host.err_clear = 0;
     }
 }
 
@@ -582,12 +827,10 @@ __global__ void k_ng_apply(int64_t N, int V, const int32_t *__restrict__ cell_mo
     x1[i] = xo;
 }
 
-__global__ void k_zero_flag(int32_t *flag) { *flag = 0; }
-
 // The driver's convergence words from the S species' words at 4 (l+1): the
 // largest fraction, mean and maximum change; the error word is shared.  The
 // context then holds one model, whose per-model words get the same figures.
-__global__ void k_conv_species(int S, double *reduced, double *mconv)
+__global__ void k_conv_species(int S, double *reduced, double *mconv, ConvOut host)
 {
     double a = 0.0, b = 0.0, c = 0.0;
     for (int l = 0; l < S; l++) {
@@ -602,6 +845,11 @@ __global__ void k_conv_species(int S, double *reduced, double *mconv)
     mconv[0] = a;
     mconv[1] = b;
     mconv[2] = c;
+    for (int i = 0; i < 4; i++) {
+        host.out[i] = reduced[i];
+        host.mconv[i] = mconv[i];
+    }
+    *host.err_clear = 0;
 }
 
 // ---- Ng acceleration without allocation ---------------------------------------
@@ -651,15 +899,42 @@ int launch_lambda(mgr_ctx *ctx)
     return MGR_OK;
 }
 
-int launch_jeff(mgr_ctx *ctx)
+// J_eff of every species; lambda: with the Lambda* sums from the waves' shares
+// (launch_lambda) in the same kernel.
+int launch_jeff(mgr_ctx *ctx, bool lambda)
 {
     for (int64_t l = 0; l < ctx->S; l++) {   // Simulation::compute_Jeff loops the species
-        const int64_t Ll = ctx->sp_L[l], lo = ctx->sp_loff[l];
-        hipLaunchKernelGGL(k_jeff, dim3(grid_for(ctx->N * Ll, 256)), dim3(256), 0, ctx->stream,
-                           ctx->N, (int)Ll, (int)ctx->L, (int)lo, (int)ctx->Q, (int)ctx->F, (int)ctx->sp_V[l],
-                           ctx->J, ctx->nr_line, ctx->qweights + l * ctx->Q, ctx->irad + lo,
-                           ctx->pop + ctx->N * ctx->sp_voff[l], ctx->Ls, ctx->Jlin, ctx->Jeff, ctx->Jdif,
-                           ctx->band_S, ctx->nband > 0 ? ctx->band_cell : nullptr, ctx->band_Ls);
+        JeffArgs a;
+        a.N = ctx->N;
+        a.L = (int)ctx->sp_L[l];
+        a.Lst = (int)ctx->L;
+        a.loff = (int)ctx->sp_loff[l];
+        a.Q = (int)ctx->Q;
+        a.F = (int)ctx->F;
+        a.V = (int)ctx->sp_V[l];
+        a.nchunk = (int)((ctx->F + WAVE - 1) / WAVE);
+        a.J = ctx->J;
+        a.nr_line = ctx->nr_line;
+        a.qw = ctx->qweights + l * ctx->Q;
+        a.irad = ctx->irad + a.loff;
+        a.pop = ctx->pop + ctx->N * ctx->sp_voff[l];
+        a.Lpart = lambda ? ctx->Lpart : nullptr;
+        a.Ls = ctx->Ls;
+        a.Jlin = ctx->Jlin;
+        a.Jeff = ctx->Jeff;
+        a.Jdif = ctx->Jdif;
+        a.S = ctx->band_S;
+        a.band_cell = ctx->nband > 0 ? ctx->band_cell : nullptr;
+        a.band_Ls = ctx->band_Ls;
+        const size_t cell_lds = (size_t)a.F * sizeof(double) + (size_t)a.L * a.Q * sizeof(int32_t);
+        if (cell_lds <= 48 * 1024) {
+            // rows of up to 8 cells in 18 KB of LDS (more in flight per CU than with fuller blocks)
+            const int cells = (int)std::min<size_t>(8, std::max<size_t>(1, 18 * 1024 / cell_lds));
+            hipLaunchKernelGGL(k_jeff_rows, dim3(grid_for(ctx->N, cells)), dim3(256), cells * cell_lds, ctx->stream, a,
+                               cells);
+        } else {
+            hipLaunchKernelGGL(k_jeff, dim3(grid_for(ctx->N * a.L, 256)), dim3(256), 0, ctx->stream, a);
+        }
         MGR_LAUNCH_CHECK();
     }
     return MGR_OK;
@@ -746,7 +1021,7 @@ int launch_stateq(mgr_ctx *ctx)
 
 static int launch_stateq_species(mgr_ctx *ctx, const StateqArgs &a)
 {
-    const dim3 g(grid_for(ctx->N, 128)), b(128);
+    const dim3 g(grid_for(ctx->N, SQ_CELLS)), b(SQ_LANES * SQ_CELLS);
     switch (a.V) {
         case 2: hipLaunchKernelGGL(k_stateq<2>, g, b, 0, ctx->stream, a); break;
         case 3: hipLaunchKernelGGL(k_stateq<3>, g, b, 0, ctx->stream, a); break;
@@ -758,7 +1033,7 @@ static int launch_stateq_species(mgr_ctx *ctx, const StateqArgs &a)
         default:
             if (a.V > VMAX_GENERIC)
                 return ctx->fail(MGR_ERR_UNSUPPORTED, "more than 32 levels");
-            hipLaunchKernelGGL(k_stateq_generic, g, b, 0, ctx->stream, a);
+            hipLaunchKernelGGL(k_stateq_generic, dim3(grid_for(ctx->N, 128)), dim3(128), 0, ctx->stream, a);
     }
     MGR_LAUNCH_CHECK();
     return MGR_OK;
@@ -768,21 +1043,25 @@ static int launch_stateq_species(mgr_ctx *ctx, const StateqArgs &a)
 // words go to reduced[4 (l+1) ..] and the driver's words are the largest over
 // the species (the ALI goes on while any species has not converged,
 // sim_lines.tpp:130-150).
+// The results also go to the pinned host words, and the error word is cleared.
 int launch_convergence(mgr_ctx *ctx)
 {
+    const ConvOut host{ctx->h_reduced, ctx->h_mconv, ctx->err_flag};
     for (int64_t l = 0; l < ctx->S; l++) {
         const int64_t vo = ctx->N * ctx->sp_voff[l];
-        hipLaunchKernelGGL(k_conv_partial, dim3((unsigned)ctx->nchunks), dim3(RED_BLOCK), 0, ctx->stream,
+        hipLaunchKernelGGL(k_conv_partial, dim3((unsigned)ctx->nchunks), dim3(CONV_BLOCK), 0, ctx->stream,
                            (int)ctx->sp_V[l], ctx->pop_prec, ctx->d_chunk_cell, ctx->d_cell_model, ctx->d_m_cell_off,
                            ctx->pop + vo, ctx->prev1 + vo, ctx->pop_tot + ctx->N * l, ctx->partials, ctx->err_flag);
         MGR_LAUNCH_CHECK();
         hipLaunchKernelGGL(k_conv_final, dim3(1), dim3(RED_BLOCK), 0, ctx->stream, ctx->M, ctx->d_m_chunk_off,
                            ctx->partials, ctx->d_m_active, ctx->d_mconv,
-                           ctx->S > 1 ? ctx->reduced + 4 * (l + 1) : ctx->reduced, ctx->err_flag);
+                           ctx->S > 1 ? ctx->reduced + 4 * (l + 1) : ctx->reduced, ctx->err_flag,
+                           ctx->S > 1 ? ConvOut{nullptr, nullptr, nullptr} : host);
         MGR_LAUNCH_CHECK();
     }
     if (ctx->S > 1) {
-        hipLaunchKernelGGL(k_conv_species, dim3(1), dim3(1), 0, ctx->stream, (int)ctx->S, ctx->reduced, ctx->d_mconv);
+        hipLaunchKernelGGL(k_conv_species, dim3(1), dim3(1), 0, ctx->stream, (int)ctx->S, ctx->reduced, ctx->d_mconv,
+                           host);
         MGR_LAUNCH_CHECK();
     }
     return MGR_OK;
@@ -808,24 +1087,26 @@ int launch_ng(mgr_ctx *ctx)
     return MGR_OK;
 }
 
-// Enqueue the copy of the convergence words to pinned host memory.
-static int enqueue_conv_copy(mgr_ctx *ctx)
-{
-    MGR_HIP(hipMemcpyAsync(ctx->h_reduced, ctx->reduced, 4 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    MGR_HIP(hipMemcpyAsync(ctx->h_mconv, ctx->d_mconv, ctx->M * 4 * sizeof(double), hipMemcpyDeviceToHost,
-                           ctx->stream));
-    return MGR_OK;
-}
-
 }  // namespace mgr
 
-// Copy the host's per-model activity flags to the device (outside graphs).
+// The host's per-model activity flags to the device, unless every model was
+// active there already; and no error yet (outside graphs).
 int mgr::set_active(mgr_ctx *ctx, bool all)
 {
     if (all)
         for (int64_t m = 0; m < ctx->M; m++) ctx->h_m_active[m] = 1;
-    MGR_HIP(hipMemcpyAsync(ctx->d_m_active, ctx->h_m_active, ctx->M * sizeof(int32_t), hipMemcpyHostToDevice,
-                           ctx->stream));
+    if (!(all && ctx->all_active)) {
+        MGR_HIP(hipMemcpyAsync(ctx->d_m_active, ctx->h_m_active, ctx->M * sizeof(int32_t), hipMemcpyHostToDevice,
+                               ctx->stream));
+        ctx->all_active = all;
+    }
+    return MGR_OK;
+}
+
+// A clean error word for what follows (outside graphs).
+int mgr::clear_error(mgr_ctx *ctx)
+{
+    MGR_HIP(hipMemsetAsync(ctx->err_flag, 0, sizeof(int32_t), ctx->stream));
     return MGR_OK;
 }
 
@@ -850,22 +1131,20 @@ int read_convergence(mgr_ctx *ctx, mgr_conv *conv)
 }
 
 // One ALI iteration, enqueued on the context stream (graph-capturable: no
-// memset nodes, the error word is cleared by a kernel).
+// memset nodes; the error word is clear before it and is cleared by it).
 static int enqueue_iteration(mgr_ctx *ctx, bool ng, int precision)
 {
     int rc;
-    hipLaunchKernelGGL(k_zero_flag, dim3(1), dim3(1), 0, ctx->stream, ctx->err_flag);
-    MGR_LAUNCH_CHECK();
     if (ng) {
         if ((rc = launch_ng(ctx))) return rc;
     } else {
-        if ((rc = launch_radiation_field(ctx, precision))) return rc;
-        if ((rc = launch_jeff(ctx))) return rc;
+        if ((rc = launch_rf_kernel(ctx, precision))) return rc;
+        if ((rc = launch_band(ctx))) return rc;
+        if ((rc = launch_jeff(ctx, true))) return rc;
         if ((rc = launch_stateq(ctx))) return rc;
     }
     if ((rc = launch_convergence(ctx))) return rc;
-    if ((rc = launch_emissivity_opacity(ctx))) return rc;
-    return enqueue_conv_copy(ctx);
+    return launch_emissivity_opacity(ctx);
 }
 
 static int build_graph(mgr_ctx *ctx, bool ng, int precision, hipGraphExec_t *out)
@@ -891,7 +1170,7 @@ int mgr_compute_Jeff(mgr_ctx *ctx)
     if (!ctx) return MGR_ERR_ARGUMENT;
     if (!ctx->J_set) return ctx->fail(MGR_ERR_STATE, "compute_radiation_field first");
     MGR_HIP(hipSetDevice(ctx->device));
-    int rc = launch_jeff(ctx);
+    int rc = launch_jeff(ctx, false);
     if (rc) return rc;
     MGR_HIP(hipStreamSynchronize(ctx->stream));
     return MGR_OK;
@@ -904,12 +1183,10 @@ int mgr_compute_level_populations_from_stateq(mgr_ctx *ctx, mgr_conv *conv)
     MGR_HIP(hipSetDevice(ctx->device));
     int rc;
     if ((rc = set_active(ctx, true))) return rc;
-    hipLaunchKernelGGL(k_zero_flag, dim3(1), dim3(1), 0, ctx->stream, ctx->err_flag);
-    MGR_LAUNCH_CHECK();
+    if ((rc = clear_error(ctx))) return rc;
     if ((rc = launch_stateq(ctx))) return rc;
     if ((rc = launch_convergence(ctx))) return rc;
     if ((rc = launch_emissivity_opacity(ctx))) return rc;
-    if ((rc = enqueue_conv_copy(ctx))) return rc;
     return read_convergence(ctx, conv);
 }
 
@@ -920,12 +1197,10 @@ int mgr_iteration_using_Ng_acceleration(mgr_ctx *ctx, mgr_conv *conv)
     MGR_HIP(hipSetDevice(ctx->device));
     int rc;
     if ((rc = set_active(ctx, true))) return rc;
-    hipLaunchKernelGGL(k_zero_flag, dim3(1), dim3(1), 0, ctx->stream, ctx->err_flag);
-    MGR_LAUNCH_CHECK();
+    if ((rc = clear_error(ctx))) return rc;
     if ((rc = launch_ng(ctx))) return rc;
     if ((rc = launch_convergence(ctx))) return rc;
     if ((rc = launch_emissivity_opacity(ctx))) return rc;
-    if ((rc = enqueue_conv_copy(ctx))) return rc;
     return read_convergence(ctx, conv);
 }
 
@@ -984,10 +1259,10 @@ int mgr_ng_acceleration_noalloc(int64_t ncells, int64_t nlev, double pop_prec, d
     hipLaunchKernelGGL(k_ng_final, dim3(1), dim3(64), 0, st, (int64_t)1, m_chunk_off, partials, coef);
     hipLaunchKernelGGL(k_ng_apply, dim3(grid_for(ncells * nlev, 256)), dim3(256), 0, st, ncells, V, nullptr,
                        m_active, coef, population, prev1, prev2, prev3);
-    hipLaunchKernelGGL(k_conv_partial, dim3((unsigned)nch), dim3(RED_BLOCK), 0, st, V, pop_prec, chunk_cell,
+    hipLaunchKernelGGL(k_conv_partial, dim3((unsigned)nch), dim3(CONV_BLOCK), 0, st, V, pop_prec, chunk_cell,
                        nullptr, m_cell_off, population, prev1, population_tot, partials, nullptr);
     hipLaunchKernelGGL(k_conv_final, dim3(1), dim3(RED_BLOCK), 0, st, (int64_t)1, m_chunk_off, partials, m_active,
-                       mconv, reduced, err_flag);
+                       mconv, reduced, err_flag, ConvOut{nullptr, nullptr, nullptr});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return noalloc_fail(MGR_ERR_DEVICE, std::string("kernel launch: ") + hipGetErrorString(e));
     if (conv) {
@@ -1050,7 +1325,7 @@ int mgr_ali_iteration(mgr_ctx *ctx, int ng, int precision, mgr_conv *conv)
     MGR_HIP(hipSetDevice(ctx->device));
     int rc = ensure_graphs(ctx, precision);
     if (rc) return rc;
-    if ((rc = set_active(ctx, true))) return rc;
+    if ((rc = clear_error(ctx))) return rc;
     MGR_HIP(hipGraphLaunch(ng ? ctx->graph_ng : ctx->graph_normal, ctx->stream));
     rc = read_convergence(ctx, conv);
     if (rc == MGR_OK && !ng) ctx->J_set = true;
@@ -1074,7 +1349,7 @@ int mgr_compute_level_populations(mgr_ctx *ctx, int use_Ng_acceleration, int64_t
     if (rc) return rc;
     // Every model of a batch iterates until it meets the criterion (its own
     // iteration count, as if solved alone); converged models are frozen.
-    if ((rc = set_active(ctx, true))) return rc;
+    if ((rc = clear_error(ctx))) return rc;
     for (int64_t m = 0; m < ctx->M; m++) ctx->m_iterations[m] = 0;
     int64_t iteration = 0, iteration_normal = 0;
     bool some_not_converged = true;

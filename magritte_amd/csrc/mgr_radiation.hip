@@ -2043,14 +2043,6 @@ int launch_rf_kernel(mgr_ctx *ctx, int precision)
               : launch_rf_shape<float>(ctx, ctx->rf_nwg[0], ctx->rf_ch[0], 0, ctx->N);
 }
 
-int launch_radiation_field(mgr_ctx *ctx, int precision)
-{
-    int rc = launch_rf_kernel(ctx, precision);
-    if (!rc) rc = launch_band(ctx);
-    if (rc) return rc;
-    return launch_lambda(ctx);   // update_Lambda's sums over the line bins
-}
-
 }  // namespace mgr
 
 extern "C" int mgr_compute_radiation_field(mgr_ctx *ctx, int precision)
@@ -2124,8 +2116,7 @@ extern "C" int mgr_first_pass(mgr_ctx *ctx, int precision, int pair_stride)
     rc = launch_rf_kernel(ctx, precision);
     ctx->rf_pair_stride = 1;
     if (!rc) rc = launch_band(ctx);
-    if (!rc) rc = launch_lambda(ctx);
-    if (!rc) rc = launch_jeff(ctx);
+    if (!rc) rc = launch_jeff(ctx, true);
     if (rc) return rc;
     MGR_HIP(hipStreamSynchronize(ctx->stream));
     int32_t errv = 0;
