@@ -1374,98 +1374,141 @@ __global__ __launch_bounds__(WAVE * MAX_WAVES) void k_image(RFArgs<real> a, doub
 
 // ---- banded Lambda* (n_off_diag >= 2) ------------------------------------------
 
-// Sub-points of traced step j of the entry at base: m = 1 .. n at shift
-// s0 + m ds with dZ dz, in cell c_prev for m < half and c_next otherwise
-// (Geometry::set_data, geometry.tpp:100-207).  step_raw loads what the split
-// needs, split_points forms it, so that the loads of a step can be issued
-// before the previous step's points are visited.
-struct StepPoints {
-    int     n, half;
-    double  s0, ds, dz;
-    int32_t c_prev, c_next;
-};
-
-struct StepRaw {
-    double  sc, sn, z;
-    int32_t c_prev, c_next;
-};
-
-__device__ __forceinline__ StepRaw step_raw(const RFArgs<double> &a, int64_t base, int j, int32_t o)
-{
-    StepRaw r;
-    r.sn = a.seg_shift[base + j];
-    r.sc = j > 0 ? a.seg_shift[base + j - 1] : 1.0;   // co-moving: the origin's shift is 1
-    r.z = a.seg_dZ[base + j];
-    r.c_prev = j > 0 ? a.seg_cell[base + j - 1] : o;
-    r.c_next = a.seg_cell[base + j];
-    return r;
-}
-
-__device__ __forceinline__ StepPoints split_points(const StepRaw &r, double dsm)
-{
-    StepPoints p;
-    const StepSplit sp = split_step(r.sc, r.sn, r.z, dsm);
-    p.n = sp.n;
-    p.half = sp.interp ? sp.half : 0;
-    p.s0 = sp.interp ? r.sc : r.sn;
-    p.ds = sp.dshift;
-    p.dz = sp.dZ;
-    p.c_prev = r.c_prev;
-    p.c_next = r.c_next;
-    return p;
-}
-
-__device__ __forceinline__ StepPoints step_points(const RFArgs<double> &a, int64_t base, int j, int32_t o,
-                                                  double dsm)
-{
-    return split_points(step_raw(a, base, j, o), dsm);
-}
-
 // The points of a ray pair in order: entry qx from its far end inwards, the
-// origin, then entry qy outwards, at most ny points of it.  visit(t, cell,
-// shift, dz, out) gets the visit count t and the dZ of the interval between
-// the point and the one visited before it, which is the dZ of the interval's
-// outer point (Simulation::setup, simulation.tpp:233-240, 292-299); out is
-// set when the step's out-of-window bit `cbit` (of a.step_mask) is set: no
-// line is then in the window of any bin of this wave (eta = 0, chi at the
-// floor).
-template <typename Visit>
-__device__ __forceinline__ void walk_pair(const RFArgs<double> &a, int32_t o, int64_t qx, int64_t qy, int ny,
-                                          double dsm, unsigned cbit, Visit &&visit)
+// origin, then entry qy outwards, at most ny points of it.  visit(t, chi, h, p)
+// gets the visit count t (uniform in the wave), the opacity of the lane's bin
+// there, the path factor h of the interval between the point and the one
+// visited before it, which is that of the interval's outer point
+// (Simulation::setup, simulation.tpp:233-240, 292-299; 0 for the first point),
+// and the point's place p in the window (its shift and cell in win.stage).
+//
+// As in sweep_pair, up to WAVE steps of the pair lie on the lanes, and their
+// points a window at a time, with the line rows of those inside the line
+// window in LDS; at the others (spans) chi is the floor.
+template <bool ONE, typename Visit>
+__device__ __forceinline__ void walk_pair(const RFArgs<double> &a, const LaneCtx<double> &lc, int32_t o, int64_t qx,
+                                          int64_t qy, int ny, double dsm, int chunk, const Window<double> &win,
+                                          Visit &&visit)
 {
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    const auto *ka = kernel_args<double>();
+    const int L = ka->L, W = ka->ch;
+    const int nsx = rfl_int(ka->nseg[qx]), nsy = rfl_int(ka->nseg[qy]);
+    const int T = nsx + 1 + (nsy < ny ? nsy : ny);   // steps; a step has at least one point
+    int left = rfl_int(ka->npts[qx]) + 1 + ny;       // points
+    const int64_t bx = ka->seg_off[qx], by = ka->seg_off[qy];
+    const bool spans = ka->span && chunk < STEP_MASK_CHUNKS;
     int t = 0;
-    double dz_prev = 0.0;
-    const int64_t bx = a.seg_off[qx];
-    // each step's loads are issued before the previous step's points are visited
-    int j = a.nseg[qx] - 1;
-    StepRaw nx;
-    uint8_t nmask = 0;
-    if (j >= 0) {
-        nx = step_raw(a, bx, j, o);
-        nmask = cbit ? a.step_mask[bx + j] : 0;
-    }
-    for (; j >= 0; --j) {
-        const StepPoints sp = split_points(nx, dsm);
-        const bool out = (nmask & cbit) != 0;
-        if (j > 0) {
-            nx = step_raw(a, bx, j - 1, o);
-            nmask = cbit ? a.step_mask[bx + j - 1] : 0;
+    double h_last = 0.0;   // path factor of the step before this batch
+    for (int g0 = 0; g0 < T; g0 += WAVE) {
+        const int g = g0 + lane;
+        const bool inward = g < nsx, outward = g > nsx && g < T;
+        const int j = inward ? nsx - 1 - g : g - nsx - 1;
+        const int64_t at = (inward ? bx : by) + j;
+        unsigned span = SPAN_ALL;
+        int32_t c_next = o, c_prev = o;
+        int n = g == nsx ? 1 : 0, half = 0;
+        double s0 = 1.0, ds = 0.0, h = 0.0;
+        if (inward || outward) {
+            if (spans) span = ka->span[ka->span_stride * chunk + at];
+            c_next = ka->seg_cell[at];
+            const double sn = ka->seg_shift[at];
+            double sc = 1.0;   // co-moving: the origin's shift is 1
+            if (j > 0) {
+                c_prev = ka->seg_cell[at - 1];
+                sc = ka->seg_shift[at - 1];
+            }
+            const StepSplit sp = split_step(sc, sn, ka->seg_dZ[at], dsm);
+            n = sp.n;
+            half = sp.interp ? sp.half : 0;
+            s0 = sp.interp ? sc : sn;
+            ds = sp.dshift;
+            h = sp.dZ * HDZ_SCALE;
         }
-        for (int m = sp.n; m >= 1; --m) {
-            visit(t++, m < sp.half ? sp.c_prev : sp.c_next, sub_point_shift(sp.s0, m, sp.ds), dz_prev, out);
-            dz_prev = sp.dz;
+        // the sub-points lo < m <= hi lie inside the window
+        const int lo = span == SPAN_NONE ? n : (int)(((span & 255) * (unsigned)n) >> 8);
+        const int hi = span == SPAN_NONE ? 0 : (int)((((span >> 8) + 1) * (unsigned)n + 255) >> 8);
+        // the interval before an inward step's first point, or the origin, is the previous step's
+        double h_in = from_lane(h, lane - 1);
+        if (lane == 0) h_in = h_last;
+        if (outward) h_in = h;
+        h_last = from_lane(h, WAVE - 1);
+        const int incl = scan_add(n), base = incl - n;
+        int total = __builtin_amdgcn_readlane(incl, WAVE - 1);
+        total = total < left ? total : left;
+        left -= total;
+        for (int w0 = 0; w0 < total; w0 += W) {
+            const int cw = total - w0 < W ? total - w0 : W;
+            wave_lds_fence();   // the previous window is consumed
+            win.owner[lane] = 0;
+            wave_lds_fence();
+            // (base, lane) of the step that begins at a point, or before the window and ends in it
+            if (n > 0 && base < w0 + W && base + n > w0) win.owner[base > w0 ? base - w0 : 0] = base << 6 | lane;
+            wave_lds_fence();
+            const int bl = scan_max(win.owner[lane]);
+            const int own = bl & (WAVE - 1);
+            const int k = w0 + lane - (bl >> 6);   // the point's number in its step, in visiting order
+            const int o_n = from_lane(n, own);
+            const int m = g0 + own < nsx ? o_n - k : k + 1;
+            Stage<double> sg;
+            sg.s = sub_point_shift(from_lane(s0, own), m, from_lane(ds, own));
+            const int32_t c_own = from_lane(c_next, own), c_before = from_lane(c_prev, own);
+            sg.cell = m < from_lane(half, own) ? c_before : c_own;
+            const int o_lo = from_lane(lo, own), o_hi = from_lane(hi, own);   // on every lane, before the || below
+            const uint64_t floors = __ballot(m <= o_lo || m > o_hi);
+            const double h_own = from_lane(h, own), h_first = from_lane(h_in, own);
+            win.hdz[lane] = k == 0 ? h_first : h_own;
+            win.stage[lane] = sg;
+            wave_lds_fence();
+            {
+                // the rows of WAVE / L points at a time, lane e L + l line l of point e
+                const int per = WAVE / L;
+                const int e0 = (int)(((uint64_t)(uint32_t)lane * ka->L_magic) >> 32), l = lane - e0 * L;
+                const double4 *src = ka->rows + l;
+                double4 *dst = win.rows + l * (W + 1);
+                if (e0 < per)
+                    for (int e = e0; e < cw; e += per) {
+                        if ((floors >> e) & 1) continue;
+                        const Stage<double> sg_e = win.stage[e];
+                        const double4 v = src[(uint32_t)sg_e.cell * (uint32_t)L];   // N L rows < 2^32
+                        dst[e] = make_double4(ONE ? sg_e.s : v.x, v.y, v.z, v.w);
+                    }
+            }
+            wave_lds_fence();
+            for (int p = 0; p < cw; ++p) {
+                double eta, chi = CHI_FLOOR * CHI_SCALE;
+                if (!((floors >> p) & 1)) eval_window<double, ONE>(a, lc, win, p, W, eta, chi);
+                visit(t++, chi, win.hdz[p], p);
+            }
         }
-    }
-    visit(t++, o, 1.0, dz_prev, false);
-    const int64_t by = a.seg_off[qy];
-    const int nsy = a.nseg[qy];
-    for (int jy = 0; jy < nsy && ny > 0; ++jy) {
-        const StepPoints sp = step_points(a, by, jy, o, dsm);
-        const bool out = cbit && (a.step_mask[by + jy] & cbit);
-        for (int m = 1; m <= sp.n && ny > 0; ++m, --ny)
-            visit(t++, m < sp.half ? sp.c_prev : sp.c_next, sub_point_shift(sp.s0, m, sp.ds), sp.dz, out);
     }
 }
+
+// The elimination's coefficients along one direction of a pair: close() takes
+// the next point and closes the row of the one before it.  With dt the closed
+// row's interval and dt' the one before it, c = dt / sqrt 2 and
+// F = 0.5 dt (dt + dt') (1 + F' / (0.5 dt' (dt + dt') (1 + F'))), the
+// reference's F (or G), is c x: the part of the sweeps' recurrence that no
+// source enters, without the divisions by the intervals.  The virtual start
+// gives F = dt + dt^2 / 2, the boundary row's.
+struct RowSweep {
+    double chi = 0.0, c = 0.0, c_prev = 0.0, y = SQRT2;
+    double F = 0.0, q = 1.0;   // of the closed row, q = 1 / (1 + F)
+
+    __device__ __forceinline__ void close(double chi_next, double h)
+    {
+#pragma clang fp contract(off)
+        c_prev = c;
+        c = (chi + chi_next) * h;
+        const double x = c + y;
+        F = c * x;
+        q = Prec<double>::rcp(1.0 + F);
+        y = __builtin_fma(x, q, c);
+        chi = chi_next;
+    }
+    // 1/A or 1/C of the closed row: 0.5 (dt + dt') dt
+    __device__ __forceinline__ double inverse_C() const { return (c_prev + c) * c; }
+};
 
 // Thermodynamics::profile (thermodynamics.tpp:16-29) of width `width` at
 // freq_diff, with the reference's scalar 1/exp.
@@ -1477,29 +1520,33 @@ __device__ __forceinline__ double profile64(double width, double freq_diff)
     return iw * INVERSE_SQRT_PI * (1.0 / exp(x * x));
 }
 
-// Per-lane window of the band kernel in LDS: array k, pair index n at
-// ((k W) + n - (n_ar - nband)) WAVE + lane, W = 3 (nband + 1), covering
-// n_ar - nband .. n_ar + 2 nband + 2.
-constexpr int BW_F = 0, BW_IC = 1, BW_G = 2, BW_FP = 3, BW_CHI = 4, BW_ARRAYS = 5;
-
 // The band elements of Lambda* (RayPair::update_Lambda, raypair_lambda.tpp:129-146,
 // with get_L_lower / get_L_upper, raypair_lambda.tpp:44-84) in FP64.  One wave
 // of 64 bins per (origin, chunk of bins).  Per ray pair the longer ray is the
-// low side (n_ar = nA points, sim_radiation.tpp:164-171), and the reference's
-// own variables are formed with its operation order (raypair_solver.tpp:200-388):
-//   pass 1, from index 0 up: dtau, F and 1/C up to index n_ar + 2 nband + 1;
-//   pass 2, from index last down: G down to index n_ar - nband + 1;
-// then for band m = 1 .. nband
+// low side (n_ar = nA points, sim_radiation.tpp:164-171), and for band
+// m = 1 .. nband
 //   lower: L_lower[m][n_ar-m] = L_diag[n_ar-m] prod_{q=n_ar-m+1}^{n_ar+1} 1/(1+G_q),
 //   upper: L_upper[m][n_ar+m] = L_diag[n_ar+2m+1] prod_{q=n_ar+2m}^{n_ar+m} 1/(1+F_q),
+//   L_diag[n] = 1/C_n / (F_n + G_{n+1} / (1 + G_{n+1})),
 // each times A_k (w_z 2 w_r) nu phi(nu) / chi at its own point, where the
-// pair's solve wrote it (the slots k_band_cells marks).  The wave sums its
-// lanes per transition; k_band_sum adds the waves of an origin.
-__global__ __launch_bounds__(WAVE) void k_lambda_band(RFArgs<double> a)
+// pair's solve wrote it (the slots k_band_cells marks).
+//   pass 1, from index last down to n_ar - nband: G, of which the products and
+//   the terms of L_diag that the elements need go to LDS;
+//   pass 2, from index 0 up to n_ar + 2 nband + 2: F and the elements.
+// Both passes walk the pair as the field kernel does (walk_pair), and the
+// lanes' elements are added per transition from LDS, one lane per (element,
+// transition); k_band_sum adds the waves of an origin.
+//
+// Bound by the FP64 profile and recurrence of every point, at 4 waves per SIMD
+// (125 VGPRs, 8 KB of LDS).  A walk with per-step scalar loads and divisions in
+// every lane, three rcp per point, five arrays of 3 (nband + 1) points in LDS
+// and butterfly sums per element and transition took 9.5 ms at 20^3 cells, 84
+// bins and one band; this one takes 3.4 ms.
+template <bool ONE>
+__global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_lambda_band(RFArgs<double> a)
 {
 #pragma clang fp contract(off)
     extern __shared__ __align__(16) unsigned char smem[];
-    double *win = reinterpret_cast<double *>(smem);
     const int G = gridDim.x;
     const int per = G >> 3;
     const int bid = blockIdx.x;
@@ -1509,7 +1556,17 @@ __global__ __launch_bounds__(WAVE) void k_lambda_band(RFArgs<double> a)
     const int chunk = logical - o * a.nchunk;
     const int lane = (int)threadIdx.x;
     const int F = a.F, L = a.L, nb = a.nband;
-    const int W = 3 * (nb + 1);
+    Window<double> win;
+    win.hdz = reinterpret_cast<double *>(smem);
+    win.stage = reinterpret_cast<Stage<double> *>(win.hdz + WAVE);
+    win.owner = reinterpret_cast<int *>(win.stage + WAVE);
+    win.rows = reinterpret_cast<double4 *>(win.owner + WAVE);
+    // per band and lane: elem [2 nb] the elements, lower ones first (before them
+    // the products over G or F so far), termG [2 nb] G / (1 + G) for their L_diag
+    double *elem = reinterpret_cast<double *>(win.rows + (size_t)L * (a.ch + 1));
+    double *termG = elem + 2 * nb * WAVE;
+    double *lt = termG + 2 * nb * WAVE;   // the line frequencies
+    int *first = reinterpret_cast<int *>(lt + L);   // [L + 1] of the transitions in elem's order of summation
     // the lane order of the field kernels (lane_bin), which the out-of-window bits follow
     const int slot = chunk * WAVE + lane;
     const bool active = slot < F;
@@ -1518,153 +1575,104 @@ __global__ __launch_bounds__(WAVE) void k_lambda_band(RFArgs<double> a)
     const double nu_f = a.nu[(int64_t)o * F + fa];
     const double dsm = a.dshift_max[o];
     LaneCtx<double> lc;
-    {
-        // the line frequencies the profile windows read at every point, in LDS after the window arrays
-        double *lt = win + (size_t)BW_ARRAYS * 3 * (nb + 1) * WAVE;
-        for (int i = lane; i < L; i += WAVE) lt[i] = a.tb->line[i];
-        __syncthreads();
-        lc.line = lt;
+    for (int i = lane; i < L; i += WAVE) lt[i] = a.tb->line[i];
+    lc.line = lt;
+    // lanes in order of their transition
+    int pos = 0, sorted = 0;
+    for (int kk = 0; kk <= L; kk++) {
+        const uint64_t same = __ballot(k == kk);
+        if (k == kk) pos = sorted + __builtin_popcountll(same & ((1ull << lane) - 1));
+        if (lane == 0) first[kk] = sorted;
+        sorted += __builtin_popcountll(same);
     }
+    wave_lds_fence();
     double S_o, chi_o;
-    origin_point<double>(a, nu_f, a.rows + (int64_t)o * L, lc, S_o, chi_o);
+    origin_point<double, false, ONE>(a, nu_f, a.rows + (int64_t)o * L, lc, S_o, chi_o);
     const double freq_line = k < L ? a.freq_k[k] : 1.0;
     const double A_k = k < L ? a.A_k[k] : 0.0;
     const double w_z = k < L ? a.qw[a.f_z[fa]] : 0.0;
-    auto wref = [&](int arr, int w) -> double & { return win[(arr * W + w) * WAVE + lane]; };
     const int64_t qb = a.cell_qbase[o];
     const int Rh = a.m_R[0] / 2;
     double *part = a.band_part + ((int64_t)o * a.nchunk + chunk) * a.band_S * L;
-    // this wave's out-of-window bit (the FP64 kernel's masks), none past the masked chunks
-    const unsigned cbit = (a.step_mask && chunk < STEP_MASK_CHUNKS) ? 1u << chunk : 0u;
-    // chi of a point: only the opacity enters dtau; at an out-of-window point the floor
-    auto opacity = [&](int32_t c, double s, bool out) -> double {
-        double eta, chi = CHI_FLOOR * CHI_SCALE;
-        if (!out) eval_point<double>(a, lc, a.rows + (int64_t)c * L, s, eta, chi);
-        return chi * (1.0 / CHI_SCALE);
-    };
 
     for (int r = 0; r < Rh; r++) {
         const int64_t qr = qb + r, qa = qb + a.antipod[r];
-        const int n_r = a.npts[qr], n_a = a.npts[qa];
+        const int n_r = rfl_int(a.npts[qr]), n_a = rfl_int(a.npts[qa]);
         const bool r_longer = n_r > n_a;
         const int64_t qA = r_longer ? qr : qa, qB = r_longer ? qa : qr;
         const int nA = r_longer ? n_r : n_a, nB = r_longer ? n_a : n_r;
         const int last = nA + nB;
-        const int w0 = nA - nb;
-        double dt0 = 0.0, dtL = 0.0;
+        const double factor = A_k * (w_z * 2.0 * a.ray_w[r]);
+        wave_lds_fence();   // the last pair's elements are summed
         if (nB >= 1) {
-            // pass 1: from index 0 (the far end of the longer ray) upwards
-            double chi_p = 0.0, dt_p = 0.0, F_p = 0.0, i1F_p = 0.0;
-            const int top = nA + 2 * nb + 2 < last ? nA + 2 * nb + 2 : last;
-            walk_pair(a, o, qA, qB, top - nA, dsm, cbit, [&](int n, int32_t c, double s, double dz, bool out) {
-                const double chi = opacity(c, s, out);
-                const int w = n - w0;
-                if (w >= 0 && w < W) {
-                    // nu phi(nu) at the point's own cell and frequency, and chi
-                    const double fs = s * nu_f;
-                    wref(BW_FP, w) = k < L ? fs * profile64(freq_line * a.pw[c], fs - freq_line) : 0.0;
-                    wref(BW_CHI, w) = chi;
+            RowSweep sw;
+            double prod = 1.0;
+            walk_pair<ONE>(a, lc, o, qB, qA, nA < nb ? nA : nb, dsm, chunk, win,
+                           [&](int t, double chi, double h, int) {
+                sw.close(chi, h);   // row last - t + 1 (none at t = 0)
+                const int i = last - t + 1 - nA;
+                if (i > 2 * nb + 2 || t == 0) return;
+                if (i >= 4 && !(i & 1)) termG[(nb + i / 2 - 2) * WAVE + lane] = sw.F * sw.q;   // of band i/2 - 1
+                if (i <= 1) {
+                    prod *= sw.q;
+                    if (i <= 0) {   // of band 1 - i
+                        elem[-i * WAVE + lane] = prod;
+                        termG[-i * WAVE + lane] = sw.F * sw.q;
+                    }
                 }
-                if (n >= 1) {
-                    const double dt = 0.5 * (chi_p + chi) * dz;   // dtau[n-1]
-                    if (n == 1) {
-                        dt0 = dt;
-                        const double B0_min_C0 = 1.0 + 2.0 * (1.0 / dt);
-                        F_p = 0.5 * B0_min_C0 * dt * dt;
-                        i1F_p = 1.0 / (1.0 + F_p);
-                        if (w - 1 >= 0 && w - 1 < W) wref(BW_F, w - 1) = F_p;
-                    } else {
-                        const double iA = 0.5 * (dt_p + dt) * dt_p;   // inverse_A[n-1]
-                        const double iC = 0.5 * (dt_p + dt) * dt;     // inverse_C[n-1]
-                        F_p = (1.0 + Prec<double>::rcp(iA) * F_p * i1F_p) * iC;  // F[n-1]
-                        i1F_p = Prec<double>::rcp(1.0 + F_p);
-                        if (w - 1 >= 0 && w - 1 < W) {
-                            wref(BW_F, w - 1) = F_p;
-                            wref(BW_IC, w - 1) = iC;
+            });
+            sw = RowSweep();
+            double fpc = 0.0;   // nu phi(nu) / chi of the last point, factor applied
+            const int ny = nB < 2 * nb + 2 ? nB : 2 * nb + 2;
+            walk_pair<ONE>(a, lc, o, qA, qB, ny, dsm, chunk, win, [&](int n, double chi, double h, int p) {
+                sw.close(chi, h);   // row n - 1 (none at n = 0)
+                const int i = n - 1 - nA;
+                if (i < -nb - 1) return;
+                if (i < 0) {
+                    if (i >= -nb && n > 0) {   // lower element of band -i
+                        const int at = (-i - 1) * WAVE;
+                        const double T = sw.inverse_C() / (sw.F + termG[at + lane]) * elem[at + lane];
+                        elem[at + pos] = fpc * T;
+                    }
+                } else if (i > 0) {
+                    // the products of the bands m with i in m .. 2 m
+                    for (int m = (i + 1) / 2; m <= nb && m <= i; m++) {
+                        double &e = elem[(nb + m - 1) * WAVE + lane];
+                        e = (m == i ? fpc : e) * sw.q;
+                    }
+                    const int m = i >> 1;
+                    if (m >= 1 && m <= nb) {
+                        const int at = (nb + m - 1) * WAVE;
+                        if (i & 1) {   // upper element of band m, from row n_ar + 2m + 1
+                            const double T = sw.inverse_C() / (sw.F + termG[at + lane]);
+                            elem[at + pos] = elem[at + lane] * T;
+                        } else if (n == last) {   // which is the last row
+                            const double c2 = sw.c * sw.c;
+                            const double T = c2 / (c2 + SQRT2 * sw.c + sw.F * sw.q);
+                            elem[at + pos] = elem[at + lane] * T;
                         }
                     }
-                    dt_p = dt;
                 }
-                chi_p = chi;
-            });
-            // pass 2: from index last (the far end of the shorter ray) downwards
-            double G_p = 0.0, i1G_p = 0.0;
-            chi_p = 0.0;
-            dt_p = 0.0;
-            const int bottom = nA - nb > 0 ? nA - nb : 0;
-            walk_pair(a, o, qB, qA, nA - bottom, dsm, cbit, [&](int t, int32_t c, double s, double dz, bool out) {
-                const int n = last - t;
-                const double chi = opacity(c, s, out);
-                if (t >= 1) {
-                    const double dt = 0.5 * (chi + chi_p) * dz;   // dtau[n]
-                    if (n == last - 1) {
-                        dtL = dt;
-                        const double Bd_min_Ad = 1.0 + 2.0 * (1.0 / dt);
-                        G_p = 0.5 * Bd_min_Ad * dt * dt;              // G[last]
-                    } else {
-                        const double iA = 0.5 * (dt + dt_p) * dt;     // inverse_A[n+1]
-                        const double iC = 0.5 * (dt + dt_p) * dt_p;   // inverse_C[n+1]
-                        G_p = (1.0 + Prec<double>::rcp(iC) * G_p * i1G_p) * iA;  // G[n+1]
-                    }
-                    i1G_p = Prec<double>::rcp(1.0 + G_p);
-                    const int w = n + 1 - w0;
-                    if (w >= 0 && w < W) wref(BW_G, w) = G_p;
-                    dt_p = dt;
+                if (i < nb) {   // nu phi(nu) / chi at the point's own cell and frequency
+                    const Stage<double> sg = win.stage[p];
+                    const double fs = sg.s * nu_f;
+                    fpc = k < L ? factor * (fs * profile64(freq_line * a.pw[sg.cell], fs - freq_line)) /
+                                      (chi * (1.0 / CHI_SCALE))
+                                : 0.0;
                 }
-                chi_p = chi;
             });
         }
-        // per slot of the pair: this lane's element, then the wave's sum per transition
-        int kmin = k, kmax = k < L ? k : -1;
-        for (int off = WAVE / 2; off >= 1; off >>= 1) {
-            kmin = min(kmin, __shfl_xor(kmin, off));
-            kmax = max(kmax, __shfl_xor(kmax, off));
+        // elements that the pair does not have
+        for (int m = 1; m <= nb; m++) {
+            if (nB < 1 || nA < m) elem[(m - 1) * WAVE + lane] = 0.0;
+            if (nB <= 2 * m) elem[(nb + m - 1) * WAVE + lane] = 0.0;
         }
-        const double factor = A_k * (w_z * 2.0 * a.ray_w[r]);
-        for (int i = 0; i < 2 * nb; i++) {
-            const bool upper = i >= nb;
-            const int m = upper ? i - nb + 1 : i + 1;
-            double v = 0.0;
-            if (!upper && nB >= 1 && nA >= m) {
-                // L_lower[m][n] = T^-1[n_ar+1][n], n = n_ar - m
-                const int n = nA - m, w = n - w0;
-                double T;
-                if (n == 0) {
-                    const double B0_min_C0 = 1.0 + 2.0 * (1.0 / dt0);
-                    const double B0 = B0_min_C0 + 2.0 * (1.0 / dt0) * (1.0 / dt0);
-                    const double G1 = wref(BW_G, 1 - w0);
-                    T = (1.0 + G1) / (B0_min_C0 + B0 * G1);
-                } else {
-                    const double G1 = wref(BW_G, w + 1);
-                    T = wref(BW_IC, w) / (wref(BW_F, w) + G1 * (1.0 / (1.0 + G1)));
-                }
-                for (int q = n + 1; q <= nA + 1; q++) T = T * (1.0 / (1.0 + wref(BW_G, q - w0)));
-                v = factor * (wref(BW_FP, w) * T / wref(BW_CHI, w));
-            } else if (upper && nB > 2 * m) {
-                // L_upper[m][n] = T^-1[n][n_ar+2m+1], n = n_ar + m
-                const int n = nA + m, j = nA + 2 * m + 1;
-                double T;
-                if (j == last) {
-                    const double Fl = wref(BW_F, j - 1 - w0);
-                    const double Bd_min_Ad = 1.0 + 2.0 * (1.0 / dtL);
-                    const double Bd = Bd_min_Ad + 2.0 * (1.0 / dtL) * (1.0 / dtL);
-                    T = (1.0 + Fl) / (Bd_min_Ad + Bd * Fl);
-                } else {
-                    const double Gj = wref(BW_G, j + 1 - w0);
-                    T = wref(BW_IC, j - w0) / (wref(BW_F, j - w0) + Gj * (1.0 / (1.0 + Gj)));
-                }
-                for (int q = j - 1; q >= n; q--) T = T * (1.0 / (1.0 + wref(BW_F, q - w0)));
-                v = factor * (wref(BW_FP, n - w0) * T / wref(BW_CHI, n - w0));
-            }
-            if (k >= L) v = 0.0;
-            double mine = 0.0;
-            for (int kk = kmin; kk <= kmax; kk++) {
-                double x = (k == kk) ? v : 0.0;
-                for (int off = WAVE / 2; off >= 1; off >>= 1) x += __shfl_xor(x, off);
-                x = __shfl(x, 0);   // lane 0's order for every lane
-                if (lane == kk) mine = x;
-            }
-            if (lane < L) part[((int64_t)r * 2 * nb + i) * L + lane] = mine;
+        wave_lds_fence();
+        for (int s = lane; s < 2 * nb * L; s += WAVE) {
+            const int i = s / L, kk = s - i * L;
+            double sum = 0.0;
+            for (int u = first[kk]; u < first[kk + 1]; u++) sum += elem[i * WAVE + u];
+            part[(int64_t)r * 2 * nb * L + s] = sum;
         }
     }
 }
@@ -1765,6 +1773,15 @@ size_t field_lds(const mgr_ctx *ctx, RFArgs<real> &a)
     return a.line_offset + table;
 }
 
+// One candidate line per bin: the lines' candidate ranges are disjoint.
+template <typename real>
+bool one_line(const mgr_ctx *ctx, const RFArgs<real> &a)
+{
+    for (int l = 0; l + 1 < ctx->h_tables.L; l++)
+        if (!(ctx->h_tables.line[l] * a.cand_lo <= ctx->h_tables.line[l + 1] * a.cand_hi)) return false;
+    return true;
+}
+
 template <typename real>
 size_t lds_bytes(const mgr_ctx *ctx, const RFArgs<real> &a)
 {
@@ -1827,10 +1844,7 @@ int launch_rf(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
     a.root_major = ctx->root_major;
     a.far32 = (sizeof(real) == 4 && ctx->far_cache && ctx->far_valid[0]) ? ctx->far_I32 : nullptr;
     a.far64 = (sizeof(real) == 8 && ctx->far_cache && ctx->far_valid[1]) ? ctx->far_I64 : nullptr;
-    // one candidate line per bin when the lines' candidate ranges are disjoint
-    bool one = true;
-    for (int l = 0; l + 1 < ctx->h_tables.L; l++)
-        if (!(ctx->h_tables.line[l] * a.cand_lo <= ctx->h_tables.line[l + 1] * a.cand_hi)) one = false;
+    const bool one = one_line(ctx, a);
     const size_t lds = field_lds<real>(ctx, a);
     auto kernel = one ? k_radiation_field<real, true> : k_radiation_field<real, false>;
     hipLaunchKernelGGL(kernel, dim3(grid_of(a)), dim3(WAVE * a.nwg), lds, ctx->stream, a);
@@ -1889,9 +1903,15 @@ int launch_band(mgr_ctx *ctx)
     a.nband = ctx->nband;
     a.band_S = ctx->band_S;
     a.band_part = ctx->band_part;
-    a.step_mask = (ctx->masks64_valid && ctx->rf_window_skip) ? ctx->step_mask64 : nullptr;
-    const size_t lds = ((size_t)BW_ARRAYS * 3 * (ctx->nband + 1) * WAVE + ctx->L) * sizeof(double);
-    hipLaunchKernelGGL(k_lambda_band, dim3(grid_of(a)), dim3(WAVE), lds, ctx->stream, a);
+    a.root_major = ctx->root_major;
+    a.span_stride = ctx->span_stride;
+    if (ctx->masks64_valid && ctx->rf_window_skip) a.span = ctx->span64;
+    // windows of at most 32 points: rows of up to 8 KB, so that 4 waves fit a SIMD
+    a.ch = (int)std::max<int64_t>(2, std::min<int64_t>(32, 8 * 1024 / (int64_t)(sizeof(double4) * ctx->L) - 1));
+    const size_t lds = Window<double>::fixed + sizeof(double4) * ctx->L * (a.ch + 1) +
+                       sizeof(double) * (4 * (size_t)ctx->nband * WAVE + ctx->L) + sizeof(int) * (ctx->L + 1);
+    auto kernel = one_line(ctx, a) ? k_lambda_band<true> : k_lambda_band<false>;
+    hipLaunchKernelGGL(kernel, dim3(grid_of(a)), dim3(WAVE), lds, ctx->stream, a);
     MGR_LAUNCH_CHECK();
     const int64_t SL = ctx->band_S * ctx->L;
     hipLaunchKernelGGL(k_band_sum, dim3((unsigned)((ctx->N * SL + 255) / 256)), dim3(256), 0, ctx->stream, ctx->N,
