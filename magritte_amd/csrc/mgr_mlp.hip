@@ -22,14 +22,18 @@
 // walking, keyed per epoch), Adam's step count and the epoch's loss live in
 // device memory, and each epoch is one hipGraph replay.
 //
-// Work mapping: a workgroup of 4 wavefronts takes tiles of 64 rows (cells);
-// wave w owns rows 16w..16w+15 of the tile for the forward pass and the
-// back-propagation of activations, keeping its pre-activations Z1, Z2 in
-// registers in the MFMA result layout; the weight gradients, which reduce
-// over rows, are split by output tile over the 4 waves with the 64 rows of
-// the tile as the MFMA K dimension, and accumulate in registers over all the
-// tiles a workgroup takes.  Per-workgroup partial gradients are reduced in a
-// fixed order by the Adam kernel, so training is deterministic.
+// Work mapping: a workgroup of 4 wavefronts takes tiles of 64 rows (cells), a
+// wave 16 of them.  The products are formed transposed, neurons by rows
+// (D = W^T H^T): a lane's results, four consecutive neurons of one row, are
+// then K values of the next product's right operand as they stand.  The M
+// rows of two tiles take the neurons of 32 in alternate fours (neuron), which
+// puts the operand's eight values in order.  So the forward pass and the back-propagation of activations
+// stay in registers.  The weight gradients reduce over rows: the operands are
+// transposed on the matrix cores (a product with the unit matrix, exact) and
+// exchanged through LDS, and each wave forms a quarter of the gradients over
+// the 64 rows, accumulating in registers over all the tiles a workgroup takes.
+// Per-workgroup partial gradients are reduced in a fixed order by the Adam
+// kernel, so training is deterministic.
 //
 // MFMA operand layouts (lane l, r = l % 16, g = l / 16):
 //   16x16x16: A[m = r][k = 4g + j], B[k = 4g + j][n = r], j = 0..3;
@@ -63,33 +67,53 @@ constexpr int OFF_W3 = OFF_B2 + HID;
 constexpr int OFF_B3 = OFF_W3 + HID * OUT;
 constexpr int NPAR = OFF_B3 + OUT;
 
-// bf16 weight layouts, each laid out so that one lane reads its 4 operand
-// values as one 8-byte word:
-//   W1f [HID][KIN]   forward B of layer 1 (transposed, input padded)
-//   W2f [HID][HID]   forward B of layer 2 (transposed)
-//   W2b [HID][HID]   backward B of dH1 = dZ2 W2^T (as stored, [in][out])
-//   W3f [NOUT][HID]  forward B of layer 3 (transposed, output padded)
-//   W3b [HID][NOUT]  backward B of dH2 = dY W3^T ([in][out], output padded)
+// bf16 weights as left operands A[m][k], one word per lane and MFMA: frag16
+// for K = 16 (8 bytes), frag32 for K = 32 (16 bytes)
+//   W1F  m = neuron, k = input (padded)     forward, layer 1
+//   W2F  m = neuron, k = neuron of layer 1  forward, layer 2
+//   W2B  m = neuron of layer 1, k = neuron  backward, dH1 = dZ2 W2^T
+//   W3F  m = output (padded), k = neuron    forward, layer 3
+//   W3B  m = neuron, k = output (padded)    backward, dH2 = dY W3^T
+// neurons in m in the order of neuron_row, in k as they are.
+// The padding entries are zero from the network's creation on.
 constexpr int BF_W1F = 0;
 constexpr int BF_W2F = BF_W1F + HID * KIN;
-constexpr int BF_W2B = BF_W2F + HID * HID;
-constexpr int BF_W3F = BF_W2B + HID * HID;
-constexpr int BF_W3B = BF_W3F + NOUT * HID;
+constexpr int BF_W3F = BF_W2F + HID * HID;
+constexpr int BF_FORWARD = BF_W3F + NOUT * HID;   // what the forward pass needs
+constexpr int BF_W2B = BF_FORWARD;
+constexpr int BF_W3B = BF_W2B + HID * HID;
 constexpr int BF_TOTAL = BF_W3B + HID * NOUT;
 
-// LDS of the training kernel (bf16 elements)
-constexpr int L_X = BF_TOTAL;                 // [ROWS][KIN]
-constexpr int L_H1 = L_X + ROWS * KIN;        // [ROWS][HID]
-constexpr int L_H2 = L_H1 + ROWS * HID;       // [ROWS][HID]
-constexpr int L_DY = L_H2 + ROWS * HID;       // [ROWS][NOUT]
-constexpr int L_DZ2 = L_DY + ROWS * NOUT;     // [ROWS][HID]
-constexpr int L_DZ1 = L_DZ2 + ROWS * HID;     // [ROWS][HID]
-constexpr int L_TOTAL = L_DZ1 + ROWS * HID;
-constexpr size_t LDS_TRAIN = (size_t)L_TOTAL * 2;   // 147,456 bytes
+__device__ __forceinline__ int frag16(int m, int k) { return m / 16 * 256 + (k / 4 * 16 + m % 16) * 4 + k % 4; }
+__device__ __forceinline__ int frag32(int m, int k)
+{
+    return ((m / 16 * (HID / 32) + k / 32) * 64 + k % 32 / 8 * 16 + m % 16) * 8 + k % 8;
+}
+// The neuron in row m of tile t, and the row (16 t + m) of a neuron.
+__device__ __forceinline__ int neuron(int t, int m) { return t / 2 * 32 + m / 4 * 8 + t % 2 * 4 + m % 4; }
+__device__ __forceinline__ int neuron_row(int u) { return (u / 32 * 2 + u % 8 / 4) * 16 + u % 32 / 8 * 4 + u % 4; }
+
+// Partial gradients of a workgroup: the words as the threads hold them, so that
+// they are written whole, with the loss at NPAR
+//   W2 [q][ot][thread][4], W1 [q][wave][g < 2][r][4], W3 [q][wave][g][r < OUT][4], b1, b2, b3
+constexpr int PG_W1 = HID * HID;
+constexpr int PG_W3 = PG_W1 + IN * HID;
+constexpr int PG_B = PG_W3 + HID * OUT;
+
+// LDS of the training kernel: the weights, the biases, and the transposed
+// operands of the weight gradients, tile t of two waves' 32 rows at
+// ((t 2 + wave / 2) 64 + lane) 8 + (wave % 2) 4
+constexpr int T_H1 = 0, T_DZ2 = 8, T_H2 = 16, T_DZ1 = 24, T_X = 32, T_DY = 33, T_TILES = 34;
+constexpr int NBIAS = HID + HID + NOUT;
+constexpr size_t LDS_BIAS = (size_t)BF_TOTAL * 2;                  // bytes before the biases
+constexpr size_t LDS_TILES = LDS_BIAS + NBIAS * sizeof(float);
+constexpr size_t LDS_TRAIN = LDS_TILES + (size_t)T_TILES * 2 * 64 * 16;   // 148,544 bytes
+constexpr size_t LDS_FORWARD = (size_t)BF_FORWARD * 2 + NBIAS * sizeof(float) + ROWS * NOUT * sizeof(float);
 
 typedef short s4 __attribute__((ext_vector_type(4)));
 typedef short s8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint16_t f2bf(float x)
@@ -99,15 +123,12 @@ __device__ __forceinline__ uint16_t f2bf(float x)
     return (uint16_t)(u >> 16);
 }
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
-
 __device__ __forceinline__ s4 ld4(const uint16_t *p) { return *reinterpret_cast<const s4 *>(p); }
 __device__ __forceinline__ s8 ld8(const uint16_t *p) { return *reinterpret_cast<const s8 *>(p); }
-__device__ __forceinline__ s8 ld8s(const uint16_t *p, int stride)
-{
-    s8 r;
-    for (int j = 0; j < 8; j++) r[j] = (short)p[j * stride];
-    return r;
-}
+// the same rounding (to nearest even) of four values
+__device__ __forceinline__ s4 to_bf(f4 x) { return __builtin_bit_cast(s4, __builtin_convertvector(x, bf4)); }
+__device__ __forceinline__ s8 join(s4 a, s4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+
 __device__ __forceinline__ f4 mfma(s4 a, s4 b, f4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
@@ -120,22 +141,23 @@ __device__ __forceinline__ f4 mfma32(s8 a, s8 b, f4 c)
 constexpr float SQRT_2_OVER_PI = 0.7978845608028654f;
 constexpr float GELU_C = 0.044715f;
 
-__device__ __forceinline__ float tanh_f(float u)
+// GELU (tanh form) and its derivative.  With p = 1 / (exp(2u) + 1),
+// u = sqrt(2/pi) (z + c z^3) held to +-15, t = tanh u = 1 - 2 p, gelu =
+// z (1 + t) / 2 and gelu' = (1 + t) / 2 + z (1 - t^2) u' / 2.  The reciprocal
+// is the correctly rounded one.
+__device__ __forceinline__ void gelu(float z, float &h, float &grad)
 {
-    // tanh u = 1 - 2 / (exp(2u) + 1), saturating for large |u|
-    const float e = __expf(2.0f * fminf(fmaxf(u, -15.0f), 15.0f));
-    return 1.0f - 2.0f / (e + 1.0f);
-}
-__device__ __forceinline__ float gelu(float z)
-{
-    const float t = tanh_f(SQRT_2_OVER_PI * (z + GELU_C * z * z * z));
-    return 0.5f * z * (1.0f + t);
-}
-__device__ __forceinline__ float gelu_grad(float z)
-{
-    const float t = tanh_f(SQRT_2_OVER_PI * (z + GELU_C * z * z * z));
-    const float du = SQRT_2_OVER_PI * (1.0f + 3.0f * GELU_C * z * z);
-    return 0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * du;
+#pragma clang fp contract(off)
+    float u = SQRT_2_OVER_PI * fmaf(z, z * (GELU_C * z), z);
+    u = __builtin_amdgcn_fmed3f(u, -15.0f, 15.0f);
+    const float d = __builtin_amdgcn_exp2f(u * (2.0f * 1.44269504f)) + 1.0f;
+    float p = __builtin_amdgcn_rcpf(d);
+    p = fmaf(fmaf(-d, p, 1.0f), p, p);   // the quotient 1 / d for every d in [1, 2^48)
+    const float t = fmaf(-2.0f, p, 1.0f);
+    const float w = fmaf(0.5f, t, 0.5f);
+    h = z * w;
+    const float du = 0.5f * SQRT_2_OVER_PI * fmaf(z, 3.0f * GELU_C * z, 1.0f);
+    grad = du * (z * fmaf(-t, t, 1.0f)) + w;
 }
 
 struct Norm {
@@ -202,217 +224,285 @@ __device__ __forceinline__ int64_t source_row(const TrainState *st, const int64_
     return idx ? idx[row] : row;
 }
 
-// Copy the bf16 weight layouts (all of them, or the forward ones) into LDS.
-__device__ __forceinline__ void load_weights(uint16_t *s, const uint16_t *__restrict__ wbf, bool fwd_only)
+// The parameter of word e of the partial gradients.
+__device__ __forceinline__ int param_of(int e)
+{
+    const int j = e % 4;
+    if (e < PG_W1) {
+        const int lane = e / 4 % 64, wave = e / 256 % 4, ot = e / 1024 % 8, q = e / 8192;
+        return OFF_W2 + neuron(2 * wave + q, lane / 16 * 4 + j) * HID + neuron(ot, lane % 16);
+    }
+    if (e < PG_W3) {
+        const int i = (e - PG_W1) / 4, lane = i % 32, wave = i / 32 % 4, q = i / 128;
+        return OFF_W1 + (lane / 16 * 4 + j) * HID + neuron(2 * wave + q, lane % 16);
+    }
+    if (e < PG_B) {
+        const int i = (e - PG_W3) / 4, r = i % OUT, g = i / OUT % 4, wave = i / (4 * OUT) % 4, q = i / (16 * OUT);
+        return OFF_W3 + neuron(2 * wave + q, 4 * g + j) * OUT + r;
+    }
+    const int b = e - PG_B;
+    return b < HID ? OFF_B1 + b : b < 2 * HID ? OFF_B2 + b - HID : OFF_B3 + b - 2 * HID;
+}
+
+// Copy the first `total` bf16 weights and the biases (outputs padded) into LDS.
+__device__ __forceinline__ void load_weights(uint16_t *s, float *sB, const uint16_t *__restrict__ wbf,
+                                             const float *__restrict__ P, int total)
 {
     const uint4 *src = reinterpret_cast<const uint4 *>(wbf);
     uint4 *dst = reinterpret_cast<uint4 *>(s);
-    const int n = BF_TOTAL / 8;   // 8 bf16 per uint4
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const int e = i * 8;
-        if (fwd_only && e >= BF_W2B && e < BF_W3F) continue;
-        if (fwd_only && e >= BF_W3B) continue;
-        dst[i] = src[i];
-    }
+#pragma unroll 10
+    for (int i = threadIdx.x; i < total / 8; i += THREADS) dst[i] = src[i];
+    for (int i = threadIdx.x; i < NBIAS; i += THREADS)
+        sB[i] = i < HID ? P[OFF_B1 + i] : i < 2 * HID ? P[OFF_B2 + i - HID] : i - 2 * HID < OUT ? P[OFF_B3 + i - 2 * HID] : 0.0f;
 }
 
-// Forward pass of the 16 rows of one wave (tile rows R0..R0+15).  sX holds
-// the normalised, bf16 inputs.  Leaves H1, H2 in LDS, Z1, Z2 in registers
-// and returns the output tile y (row R0 + 4g + j, column r).
-__device__ __forceinline__ f4 forward_rows(const uint16_t *s, uint16_t *sH1, uint16_t *sH2, int R0,
-                                           const float *__restrict__ P, f4 z1[8], f4 z2[8])
+// The lane's inputs 4g .. 4g+3 normalised, as right operand: zeros in the
+// padding and for a row that is not in the batch.
+__device__ __forceinline__ s4 input_operand(f4 x, bool valid, f4 xm, f4 xs)
 {
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const uint16_t *sX = s + L_X;
-    const s4 ax = ld4(sX + (R0 + r) * KIN + 4 * g);
-    for (int nt = 0; nt < 8; nt++) {
-        f4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = mfma(ax, ld4(s + BF_W1F + (nt * 16 + r) * KIN + 4 * g), acc);
-        const float b = P[OFF_B1 + nt * 16 + r];
+    const f4 v = (x - xm) / xs;
+    return to_bf(valid ? v : f4{0.f, 0.f, 0.f, 0.f});
+}
+
+// Forward pass of the 16 rows of one wave, row r of lane (r, g) and neurons
+// neuron(mt, 4g + j): the activations, as operands of the next product, and the
+// derivatives of GELU go to layer1 and layer2, the outputs 4g + j are returned.
+template <typename Layer1, typename Layer2>
+__device__ __forceinline__ f4 forward_rows(const uint16_t *s, const float *sB, s4 x, Layer1 &&layer1, Layer2 &&layer2)
+{
+    s4 h1[8], h2[8];
+    const int lane = threadIdx.x & 63, g = lane >> 4;
+#pragma unroll
+    for (int mt = 0; mt < 8; mt++) {
+        const f4 z = mfma(ld4(s + BF_W1F + (mt * 64 + lane) * 4), x, f4{0.f, 0.f, 0.f, 0.f}) +
+                     *reinterpret_cast<const f4 *>(sB + neuron(mt, 4 * g));
+        f4 h, d;
+#pragma unroll
         for (int j = 0; j < 4; j++) {
-            acc[j] += b;
-            sH1[(R0 + 4 * g + j) * HID + nt * 16 + r] = f2bf(gelu(acc[j]));
+            float hj, dj;
+            gelu(z[j], hj, dj);
+            h[j] = hj;
+            d[j] = dj;
         }
-        z1[nt] = acc;
+        h1[mt] = to_bf(h);
+        layer1(mt, h1[mt], d);
     }
-    __syncthreads();
-    for (int nt = 0; nt < 8; nt++) {
-        f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int mt = 0; mt < 8; mt++) {
+        f4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
         for (int kt = 0; kt < 4; kt++)
-            acc = mfma32(ld8(sH1 + (R0 + r) * HID + kt * 32 + 8 * g),
-                         ld8(s + BF_W2F + (nt * 16 + r) * HID + kt * 32 + 8 * g), acc);
-        const float b = P[OFF_B2 + nt * 16 + r];
+            z = mfma32(ld8(s + BF_W2F + ((mt * 4 + kt) * 64 + lane) * 8), join(h1[2 * kt], h1[2 * kt + 1]), z);
+        z += *reinterpret_cast<const f4 *>(sB + HID + neuron(mt, 4 * g));
+        f4 h, d;
+#pragma unroll
         for (int j = 0; j < 4; j++) {
-            acc[j] += b;
-            sH2[(R0 + 4 * g + j) * HID + nt * 16 + r] = f2bf(gelu(acc[j]));
+            float hj, dj;
+            gelu(z[j], hj, dj);
+            h[j] = hj;
+            d[j] = dj;
         }
-        z2[nt] = acc;
+        h2[mt] = to_bf(h);
+        layer2(mt, h2[mt], d);
     }
-    __syncthreads();
     f4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
     for (int kt = 0; kt < 4; kt++)
-        y = mfma32(ld8(sH2 + (R0 + r) * HID + kt * 32 + 8 * g), ld8(s + BF_W3F + r * HID + kt * 32 + 8 * g), y);
-    const float b3 = r < OUT ? P[OFF_B3 + r] : 0.0f;
-    for (int j = 0; j < 4; j++) y[j] += b3;
-    return y;
-}
-
-// Stage the normalised inputs of tile rows into sX (zeros past n and in the
-// padding columns).
-__device__ __forceinline__ void stage_inputs(uint16_t *sX, const float *__restrict__ X, const TrainState *st,
-                                             const int64_t *__restrict__ idx, int64_t b0, int64_t row0, int64_t n,
-                                             const Norm &nm)
-{
-    for (int e = threadIdx.x; e < ROWS * KIN; e += blockDim.x) {
-        const int rr = e / KIN, c = e - rr * KIN;
-        const int64_t row = row0 + rr;
-        float v = 0.0f;
-        if (row < n && c < IN) {
-            const int64_t src = source_row(st, idx, b0, row);
-            v = (X[src * IN + c] - nm.xm[c]) / nm.xs[c];
-        }
-        sX[e] = f2bf(v);
-    }
+        y = mfma32(ld8(s + BF_W3F + (kt * 64 + lane) * 8), join(h2[2 * kt], h2[2 * kt + 1]), y);
+    return y + *reinterpret_cast<const f4 *>(sB + 2 * HID + 4 * g);
 }
 
 // Loss and gradients over rows [0, n) of a batch of X/T (rows b0 .. b0+n-1 of
 // the epoch's permutation with st, else through idx when given, else the
 // rows themselves): grid-stride over 64-row tiles; per-workgroup partial
-// gradients (packed like the parameters) and partial loss go to
-// part[blockIdx.x * (NPAR + 1)].
-__global__ __launch_bounds__(THREADS) void k_mlp_grad(const float *__restrict__ X, const float *__restrict__ T,
-                                                      const TrainState *st, const int64_t *__restrict__ idx,
-                                                      int64_t b0, int64_t n, int64_t n_total,
-                                                      const uint16_t *__restrict__ wbf, const float *__restrict__ P,
-                                                      const Norm *__restrict__ norm, float *__restrict__ part)
+// gradients (PG_W1) and partial loss go to part[blockIdx.x * (NPAR + 1)].
+//
+// Bound by vector instructions, most of them the GELUs', at one wave per SIMD
+// (9 us per tile), and per launch by the weights' way into LDS and the 74 KB of
+// partial gradients (7 us alone, 16 with a workgroup on every CU).  With activations in row-major LDS (16-way bank
+// conflicts on every operand) and gradient operands gathered two bytes at a
+// time a 16384-row batch took 40 us and 400000 rows 590 us; here 24 and
+// 250.
+__global__ __launch_bounds__(THREADS, 1) void k_mlp_grad(const float *__restrict__ X, const float *__restrict__ T,
+                                                         const TrainState *st, const int64_t *__restrict__ idx,
+                                                         int64_t b0, int64_t n, int64_t n_total,
+                                                         const uint16_t *__restrict__ wbf, const float *__restrict__ P,
+                                                         const Norm *__restrict__ norm, float *__restrict__ part)
 {
     extern __shared__ __align__(16) uint16_t s[];
-    uint16_t *sX = s + L_X, *sH1 = s + L_H1, *sH2 = s + L_H2, *sDY = s + L_DY, *sDZ2 = s + L_DZ2,
-             *sDZ1 = s + L_DZ1;
-    const Norm &nm = *norm;
-    load_weights(s, wbf, false);
+    float *sB = reinterpret_cast<float *>(reinterpret_cast<char *>(s) + LDS_BIAS);
+    uint16_t *sT = reinterpret_cast<uint16_t *>(reinterpret_cast<char *>(s) + LDS_TILES);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const int R0 = wave * 16;
     const float inv = 2.0f / ((float)n_total * (float)OUT);
+    f4 xm{}, xs{1.f, 1.f, 1.f, 1.f}, ym{}, ys{1.f, 1.f, 1.f, 1.f};
+    for (int j = 0; j < 4; j++) {
+        if (g < 2) {
+            xm[j] = norm->xm[4 * g + j];
+            xs[j] = norm->xs[4 * g + j];
+        }
+        if (4 * g + j < OUT) {
+            ym[j] = norm->ym[4 * g + j];
+            ys[j] = norm->ys[4 * g + j];
+        }
+    }
+    s4 unit;   // the unit matrix as right operand
+    for (int j = 0; j < 4; j++) unit[j] = 4 * g + j == r ? 0x3F80 : 0;
+    auto put = [&](int t, s4 operand) {
+        const f4 zero = {0.f, 0.f, 0.f, 0.f};
+        // rows 4g + j of neuron r: exact, the values are bf16
+        const s4 v = to_bf(mfma(operand, unit, zero));
+        *reinterpret_cast<s4 *>(sT + ((t * 2 + (wave >> 1)) * 64 + lane) * 8 + (wave & 1) * 4) = v;
+    };
+    auto get = [&](int t, int p) { return ld8(sT + ((t * 2 + p) * 64 + lane) * 8); };
 
-    f4 gW2[16], gW1[2], gW3[2];
-    for (int t = 0; t < 16; t++) gW2[t] = f4{0.f, 0.f, 0.f, 0.f};
-    for (int t = 0; t < 2; t++) gW1[t] = gW3[t] = f4{0.f, 0.f, 0.f, 0.f};
+    f4 gW2[2][8], gW1[2], gW3[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        gW1[q] = gW3[q] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 8; t++) gW2[q][t] = gW1[q];
+    }
     float gb = 0.0f, gb3 = 0.0f, loss = 0.0f;
+    // the sum of a transposed operand's column m over the tile's rows, in their order
+    auto column = [&](int t, int m, float sum) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const s8 v = ld8(sT + ((t * 2 + i / 4) * 64 + i % 4 * 16 + m) * 8);
+            for (int j = 0; j < 8; j++) sum += bf2f((uint16_t)v[j]);
+        }
+        return sum;
+    };
+    const int column_row = neuron_row(threadIdx.x % HID);   // bias gradients: dZ1 of threads 0..127, dZ2 of the others
+    const int column_tile = (threadIdx.x < HID ? T_DZ1 : T_DZ2) + column_row / 16;
+
+    // a tile's inputs and targets are read before the weights, or the tile before, are dealt with
+    f4 next_x = xm, next_t = ym;
+    bool next_valid = false;
+    auto fetch = [&](int64_t tile) {
+        // the rows of two waves alternate in fours, as the neurons of two tiles do
+        const int64_t row = tile * ROWS + neuron(wave, r);
+        next_valid = row < n;
+        if (!next_valid || g > 1) return;
+        const int64_t src = source_row(st, idx, b0, row);
+        next_x = *reinterpret_cast<const f4 *>(X + src * IN + 4 * g);
+        for (int j = 0; j < 4; j++)
+            if (4 * g + j < OUT) next_t[j] = T[src * OUT + 4 * g + j];
+    };
+    fetch(blockIdx.x);
+    load_weights(s, sB, wbf, P, BF_TOTAL);
 
     const int64_t ntiles = (n + ROWS - 1) / ROWS;
     for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int64_t row0 = tile * ROWS;
-        __syncthreads();   // the previous tile's activations are consumed
-        stage_inputs(sX, X, st, idx, b0, row0, n, nm);
-        __syncthreads();
-        f4 z1[8], z2[8];
-        const f4 y = forward_rows(s, sH1, sH2, R0, P, z1, z2);
+        const bool valid = next_valid && g < 2;
+        const s4 x = input_operand(next_x, valid, xm, xs);
+        const f4 t = next_t;
+        __syncthreads();   // the weights are in place, the previous tile's operands consumed
+        fetch(tile + gridDim.x);
+        f4 g1[8], g2[8];
+        const f4 y = forward_rows(
+            s, sB, x,
+            [&](int mt, s4 h, f4 d) {
+                g1[mt] = d;
+                put(T_H1 + mt, h);
+            },
+            [&](int mt, s4 h, f4 d) {
+                g2[mt] = d;
+                put(T_H2 + mt, h);
+            });
         // dY = 2 (y - t) / (n_total OUT) on valid rows and outputs
-        for (int j = 0; j < 4; j++) {
-            const int rr = R0 + 4 * g + j;
-            const int64_t row = row0 + rr;
-            float d = 0.0f;
-            if (row < n && r < OUT) {
-                const int64_t src = source_row(st, idx, b0, row);
-                const float t = (T[src * OUT + r] - nm.ym[r]) / nm.ys[r];
-                d = y[j] - t;
-                loss += d * d;
-                d *= inv;
+        f4 d = {0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < 4; j++)
+            if (valid && 4 * g + j < OUT) {
+                const float e = y[j] - (t[j] - ym[j]) / ys[j];
+                loss += e * e;
+                d[j] = e * inv;
             }
-            sDY[rr * NOUT + r] = f2bf(d);
-        }
-        __syncthreads();
+        const s4 dy = to_bf(d);
+        put(T_X, x);
+        put(T_DY, dy);
         // dH2 = dY W3^T, dZ2 = dH2 * gelu'(Z2)
-        {
-            const s4 a = ld4(sDY + (R0 + r) * NOUT + 4 * g);
-            for (int nt = 0; nt < 8; nt++) {
-                f4 acc = {0.f, 0.f, 0.f, 0.f};
-                acc = mfma(a, ld4(s + BF_W3B + (nt * 16 + r) * NOUT + 4 * g), acc);
-                for (int j = 0; j < 4; j++)
-                    sDZ2[(R0 + 4 * g + j) * HID + nt * 16 + r] = f2bf(acc[j] * gelu_grad(z2[nt][j]));
-            }
+        s4 dz2[8];
+#pragma unroll
+        for (int mt = 0; mt < 8; mt++) {
+            const f4 zero = {0.f, 0.f, 0.f, 0.f};
+            dz2[mt] = to_bf(mfma(ld4(s + BF_W3B + (mt * 64 + lane) * 4), dy, zero) * g2[mt]);
+            put(T_DZ2 + mt, dz2[mt]);
         }
-        __syncthreads();
         // dH1 = dZ2 W2^T, dZ1 = dH1 * gelu'(Z1)
-        for (int nt = 0; nt < 8; nt++) {
+#pragma unroll
+        for (int mt = 0; mt < 8; mt++) {
             f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
             for (int kt = 0; kt < 4; kt++)
-                acc = mfma32(ld8(sDZ2 + (R0 + r) * HID + kt * 32 + 8 * g),
-                             ld8(s + BF_W2B + (nt * 16 + r) * HID + kt * 32 + 8 * g), acc);
-            for (int j = 0; j < 4; j++)
-                sDZ1[(R0 + 4 * g + j) * HID + nt * 16 + r] = f2bf(acc[j] * gelu_grad(z1[nt][j]));
+                acc = mfma32(ld8(s + BF_W2B + ((mt * 4 + kt) * 64 + lane) * 8), join(dz2[2 * kt], dz2[2 * kt + 1]), acc);
+            put(T_DZ1 + mt, to_bf(acc * g1[mt]));
         }
         __syncthreads();
-        // weight gradients over the 64 rows of the tile (MFMA K = rows)
-        for (int ks = 0; ks < 2; ks++) {
-            const int rb = 32 * ks + 8 * g;
+        // the gradients of neurons 32 wave .. 32 wave + 31 (of layer 1 for W2) over the tile's rows
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const s8 xt = get(T_X, p), dyt = get(T_DY, p);
+            const s8 h0 = get(T_H1 + 2 * wave, p), h1t = get(T_H1 + 2 * wave + 1, p);
+#pragma unroll
+            for (int ot = 0; ot < 8; ot++) {
+                const s8 dz = get(T_DZ2 + ot, p);
+                gW2[0][ot] = mfma32(h0, dz, gW2[0][ot]);
+                gW2[1][ot] = mfma32(h1t, dz, gW2[1][ot]);
+            }
+#pragma unroll
             for (int q = 0; q < 2; q++) {
-                const int it = 2 * wave + q;
-                const s8 aH1 = ld8s(sH1 + rb * HID + it * 16 + r, HID);
-                for (int ot = 0; ot < 8; ot++)
-                    gW2[q * 8 + ot] = mfma32(aH1, ld8s(sDZ2 + rb * HID + ot * 16 + r, HID), gW2[q * 8 + ot]);
-                gW1[q] = mfma32(ld8s(sX + rb * KIN + r, KIN), ld8s(sDZ1 + rb * HID + it * 16 + r, HID), gW1[q]);
-                gW3[q] = mfma32(ld8s(sH2 + rb * HID + it * 16 + r, HID), ld8s(sDY + rb * NOUT + r, NOUT), gW3[q]);
+                gW1[q] = mfma32(xt, get(T_DZ1 + 2 * wave + q, p), gW1[q]);
+                gW3[q] = mfma32(get(T_H2 + 2 * wave + q, p), dyt, gW3[q]);
             }
         }
-        // bias gradients: column sums of dZ1 (threads 0..127), dZ2 (128..255), dY (0..6)
-        {
-            const int c = threadIdx.x & (HID - 1);
-            const uint16_t *src = threadIdx.x < HID ? sDZ1 : sDZ2;
-            for (int rr = 0; rr < ROWS; rr++) gb += bf2f(src[rr * HID + c]);
-            if (threadIdx.x < OUT)
-                for (int rr = 0; rr < ROWS; rr++) gb3 += bf2f(sDY[rr * NOUT + threadIdx.x]);
-        }
+        gb = column(column_tile, column_row % 16, gb);
+        if (wave == 3) gb3 = column(T_DY, r, gb3);
     }
 
-    // partial gradients of this workgroup, packed like the parameters
     float *out = part + (int64_t)blockIdx.x * (NPAR + 1);
+#pragma unroll
     for (int q = 0; q < 2; q++) {
-        const int it = 2 * wave + q;
+#pragma unroll
         for (int ot = 0; ot < 8; ot++)
-            for (int j = 0; j < 4; j++)
-                out[OFF_W2 + (it * 16 + 4 * g + j) * HID + ot * 16 + r] = gW2[q * 8 + ot][j];
-        for (int j = 0; j < 4; j++) {
-            const int i = 4 * g + j;   // input feature (padded to 16)
-            if (i < IN) out[OFF_W1 + i * HID + it * 16 + r] = gW1[q][j];
-            if (r < OUT) out[OFF_W3 + (it * 16 + 4 * g + j) * OUT + r] = gW3[q][j];
-        }
+            *reinterpret_cast<f4 *>(out + ((q * 8 + ot) * THREADS + threadIdx.x) * 4) = gW2[q][ot];
+        if (g < 2) *reinterpret_cast<f4 *>(out + PG_W1 + ((q * 4 + wave) * 32 + lane) * 4) = gW1[q];
+        if (r < OUT) *reinterpret_cast<f4 *>(out + PG_W3 + (((q * 4 + wave) * 4 + g) * OUT + r) * 4) = gW3[q];
     }
-    if (threadIdx.x < HID) out[OFF_B1 + threadIdx.x] = gb;
-    else out[OFF_B2 + threadIdx.x - HID] = gb;
-    if (threadIdx.x < OUT) out[OFF_B3 + threadIdx.x] = gb3;
-    // loss: wave sums, then one lane per wave adds into LDS-free slots in order
+    out[PG_B + threadIdx.x] = gb;
+    if (wave == 3 && g == 0 && r < OUT) out[PG_B + 2 * HID + r] = gb3;
+    // loss: wave sums, then one lane adds the waves' in order
     for (int off = 32; off > 0; off >>= 1) loss += __shfl_down(loss, off, 64);
-    __shared__ float wl[4];
+    __syncthreads();   // the operands are consumed
+    float *wl = reinterpret_cast<float *>(sT);
     if (lane == 0) wl[wave] = loss;
     __syncthreads();
     if (threadIdx.x == 0) out[NPAR] = (wl[0] + wl[1]) + (wl[2] + wl[3]);
 }
 
-// bf16 copies of master parameter p in the weight layouts (the padding
-// entries stay zero from the first k_mlp_pack).
+// bf16 copies of master parameter p in the weight layouts.
 __device__ __forceinline__ void repack_param(int p, float x, uint16_t *__restrict__ wbf)
 {
     const uint16_t h = f2bf(x);
     if (p < OFF_B1) {                        // W1 [i][o]
         const int i = (p - OFF_W1) / HID, o = (p - OFF_W1) % HID;
-        wbf[BF_W1F + o * KIN + i] = h;
+        wbf[BF_W1F + frag16(neuron_row(o), i)] = h;
     } else if (p >= OFF_W2 && p < OFF_B2) {  // W2 [i][o]
         const int k = p - OFF_W2, i = k / HID, o = k % HID;
-        wbf[BF_W2F + o * HID + i] = h;
-        wbf[BF_W2B + k] = h;
+        wbf[BF_W2F + frag32(neuron_row(o), i)] = h;
+        wbf[BF_W2B + frag32(neuron_row(i), o)] = h;
     } else if (p >= OFF_W3 && p < OFF_B3) {  // W3 [i][o]
         const int k = p - OFF_W3, i = k / OUT, o = k % OUT;
-        wbf[BF_W3F + o * HID + i] = h;
-        wbf[BF_W3B + i * NOUT + o] = h;
+        wbf[BF_W3F + frag32(o, i)] = h;
+        wbf[BF_W3B + frag16(neuron_row(i), o)] = h;
     }
 }
 
 // Sum the G partials of each parameter in a fixed order (8 interleaved
 // sequential sums, then a fixed tree: deterministic), optionally apply one
 // Adam step and refresh the parameter's bf16 copies.  Blocks of 256 threads
-// cover 32 parameters (p = NPAR is the loss).  In a training run (st given)
+// cover 32 parameters (p = NPAR is the loss); with 16 loads of a thread in
+// flight, 256 partials (19 MB) take 7.9 us, with the compiler's
+// choice 13.  In a training run (st given)
 // the step is step0 + epoch * nbatch + batch + 1 and the loss sum is added to
 // loss_acc[epoch]; otherwise c1, c2 are given.
 constexpr int RED_P = 32, RED_W = 8;
@@ -423,13 +513,16 @@ __global__ __launch_bounds__(RED_P * RED_W) void k_mlp_reduce_adam(
 {
     __shared__ float sh[RED_W][RED_P];
     const int pi = threadIdx.x % RED_P, wi = threadIdx.x / RED_P;
-    const int p = blockIdx.x * RED_P + pi;
+    const int e = blockIdx.x * RED_P + pi;
     float s = 0.0f;
-    if (p <= NPAR)
-        for (int w = wi; w < G; w += RED_W) s += part[(int64_t)w * (NPAR + 1) + p];
+    if (e <= NPAR) {
+#pragma unroll 16
+        for (int w = wi; w < G; w += RED_W) s += part[(int64_t)w * (NPAR + 1) + e];
+    }
     sh[wi][pi] = s;
     __syncthreads();
-    if (wi != 0 || p > NPAR) return;
+    if (wi != 0 || e > NPAR) return;
+    const int p = e < NPAR ? param_of(e) : NPAR;
     const float gsum = ((sh[0][pi] + sh[1][pi]) + (sh[2][pi] + sh[3][pi])) +
                        ((sh[4][pi] + sh[5][pi]) + (sh[6][pi] + sh[7][pi]));
     if (grad_out) grad_out[p] = gsum;
@@ -453,25 +546,8 @@ __global__ __launch_bounds__(RED_P * RED_W) void k_mlp_reduce_adam(
 // FP32 master parameters -> the bf16 layouts.
 __global__ void k_mlp_pack(const float *__restrict__ P, uint16_t *__restrict__ wbf)
 {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= BF_TOTAL) return;
-    float v = 0.0f;
-    if (e < BF_W2F) {                       // W1f [HID][KIN]
-        const int o = e / KIN, i = e % KIN;
-        v = i < IN ? P[OFF_W1 + i * HID + o] : 0.0f;
-    } else if (e < BF_W2B) {                // W2f [HID out][HID in]
-        const int k = e - BF_W2F, o = k / HID, i = k % HID;
-        v = P[OFF_W2 + i * HID + o];
-    } else if (e < BF_W3F) {                // W2b [in][out]
-        v = P[OFF_W2 + (e - BF_W2B)];
-    } else if (e < BF_W3B) {                // W3f [NOUT][HID]
-        const int k = e - BF_W3F, o = k / HID, i = k % HID;
-        v = o < OUT ? P[OFF_W3 + i * OUT + o] : 0.0f;
-    } else {                                // W3b [HID][NOUT]
-        const int k = e - BF_W3B, i = k / NOUT, o = k % NOUT;
-        v = o < OUT ? P[OFF_W3 + i * OUT + o] : 0.0f;
-    }
-    wbf[e] = f2bf(v);
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < NPAR) repack_param(p, P[p], wbf);
 }
 
 // Forward only: Y (de-normalised) for rows [0, n), or, with pop != null, the
@@ -484,30 +560,37 @@ __global__ __launch_bounds__(THREADS) void k_mlp_forward(const float *__restrict
                                                          double *__restrict__ pop)
 {
     extern __shared__ __align__(16) uint16_t s[];
-    uint16_t *sX = s + L_X, *sH1 = s + L_H1, *sH2 = s + L_H2;
-    const Norm &nm = *norm;
-    load_weights(s, wbf, true);
+    float *sB = reinterpret_cast<float *>(s + BF_FORWARD);
+    float(*sy)[NOUT] = reinterpret_cast<float(*)[NOUT]>(sB + NBIAS);
+    load_weights(s, sB, wbf, P, BF_FORWARD);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const int R0 = wave * 16;
-    __shared__ float sy[ROWS][NOUT];
+    f4 xm{}, xs{1.f, 1.f, 1.f, 1.f}, ym{}, ys{};
+    for (int j = 0; j < 4; j++) {
+        if (g < 2) {
+            xm[j] = norm->xm[4 * g + j];
+            xs[j] = norm->xs[4 * g + j];
+        }
+        if (4 * g + j < OUT) {
+            ym[j] = norm->ym[4 * g + j];
+            ys[j] = norm->ys[4 * g + j];
+        }
+    }
     const int64_t ntiles = (n + ROWS - 1) / ROWS;
     for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int64_t row0 = tile * ROWS;
-        __syncthreads();
-        stage_inputs(sX, X, nullptr, nullptr, 0, row0, n, nm);
-        __syncthreads();
-        f4 z1[8], z2[8];
-        const f4 y = forward_rows(s, sH1, sH2, R0, P, z1, z2);
+        const int64_t row = tile * ROWS + wave * 16 + r;
+        const bool valid = row < n && g < 2;
+        const s4 x = input_operand(valid ? *reinterpret_cast<const f4 *>(X + row * IN + 4 * g) : xm, valid, xm, xs);
+        __syncthreads();   // the weights are in place, the previous tile's outputs read
+        const f4 y = forward_rows(s, sB, x, [](int, s4, f4) {}, [](int, s4, f4) {});
         for (int j = 0; j < 4; j++) {
-            const int rr = R0 + 4 * g + j;
-            const float v = r < OUT ? y[j] * nm.ys[r] + nm.ym[r] : 0.0f;
-            sy[rr][r] = v;
-            const int64_t row = row0 + rr;
-            if (Y && row < n && r < OUT) Y[row * OUT + r] = v;
+            const int i = 4 * g + j;
+            const float v = y[j] * ys[j] + ym[j];
+            sy[wave * 16 + r][i] = v;
+            if (Y && row < n && i < OUT) Y[row * OUT + i] = v;
         }
         __syncthreads();
         if (pop && threadIdx.x < ROWS) {
-            const int64_t row = row0 + threadIdx.x;
+            const int64_t row = tile * ROWS + threadIdx.x;
             if (row < n) {
                 double f[OUT], sum = 0.0;
                 double mx = -1e300;
@@ -616,7 +699,7 @@ struct mgr_mlp {
 
 static int mlp_pack(mgr_mlp *mlp)
 {
-    hipLaunchKernelGGL(k_mlp_pack, dim3((BF_TOTAL + 255) / 256), dim3(256), 0, mlp->stream, mlp->P, mlp->wbf);
+    hipLaunchKernelGGL(k_mlp_pack, dim3((NPAR + 255) / 256), dim3(256), 0, mlp->stream, mlp->P, mlp->wbf);
     MLP_HIP(hipGetLastError());
     return MGR_OK;
 }
@@ -624,7 +707,7 @@ static int mlp_pack(mgr_mlp *mlp)
 static int mlp_lds_attr(mgr_mlp *mlp)
 {
     MLP_HIP(hipFuncSetAttribute((const void *)k_mlp_grad, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_TRAIN));
-    MLP_HIP(hipFuncSetAttribute((const void *)k_mlp_forward, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_TRAIN));
+    MLP_HIP(hipFuncSetAttribute((const void *)k_mlp_forward, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_FORWARD));
     return MGR_OK;
 }
 
@@ -665,6 +748,7 @@ extern "C" int mgr_mlp_create(int device, uint64_t seed, mgr_mlp **out)
     if (hipMemcpy(mlp->P, P.data(), NPAR * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(mlp->m, 0, NPAR * sizeof(float)) != hipSuccess ||
         hipMemset(mlp->v, 0, NPAR * sizeof(float)) != hipSuccess ||
+        hipMemset(mlp->wbf, 0, BF_TOTAL * sizeof(uint16_t)) != hipSuccess ||
         hipMemcpy(mlp->norm, &mlp->h_norm, sizeof(Norm), hipMemcpyHostToDevice) != hipSuccess)
         return bail(MGR_ERR_DEVICE);
     int rc = mlp_lds_attr(mlp);
@@ -729,10 +813,15 @@ extern "C" int mgr_mlp_set_normalisation(mgr_mlp *mlp, const float *x_mean, cons
     return MGR_OK;
 }
 
-static int grid_for_rows(int64_t n)
+// Workgroups for n rows: one per tile up to `most`.  The gradient kernel fills
+// a CU with one workgroup, and each costs 74 KB of partial gradients: more
+// than one per CU only adds to both (400000 rows: the reduction takes 6 us
+// after 256 workgroups, 40 after 1024).
+constexpr int GRAD_GROUPS = 256;
+static int grid_for_rows(int64_t n, int most)
 {
     const int64_t tiles = (n + ROWS - 1) / ROWS;
-    return (int)(tiles < 1024 ? (tiles > 0 ? tiles : 1) : 1024);
+    return (int)std::min<int64_t>(std::max<int64_t>(tiles, 1), most);
 }
 
 extern "C" int mgr_mlp_forward(mgr_mlp *mlp, const float *X, int64_t n, float *Y)
@@ -749,7 +838,7 @@ extern "C" int mgr_mlp_forward(mgr_mlp *mlp, const float *X, int64_t n, float *Y
     int rc = MGR_OK;
     if (hipMemcpy(dX, X, n * IN * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) rc = MGR_ERR_DEVICE;
     if (!rc) {
-        hipLaunchKernelGGL(k_mlp_forward, dim3(grid_for_rows(n)), dim3(THREADS), LDS_TRAIN, mlp->stream, dX, n,
+        hipLaunchKernelGGL(k_mlp_forward, dim3(grid_for_rows(n, 1024)), dim3(THREADS), LDS_FORWARD, mlp->stream, dX, n,
                            mlp->wbf, mlp->P, mlp->norm, dY, (const double *)nullptr, (double *)nullptr);
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(mlp->stream) != hipSuccess) rc = MGR_ERR_DEVICE;
     }
@@ -779,7 +868,7 @@ extern "C" int mgr_mlp_loss_grad(mgr_mlp *mlp, const float *X, const float *T, i
 {
     if (!mlp || !X || !T || n <= 0) return MGR_ERR_ARGUMENT;
     MLP_HIP(hipSetDevice(mlp->device));
-    const int G = grid_for_rows(n);
+    const int G = grid_for_rows(n, GRAD_GROUPS);
     float *dX = nullptr, *dT = nullptr, *dpart = nullptr, *dgrad = nullptr;
     int rc = MGR_OK;
     if (hipMalloc(&dX, n * IN * sizeof(float)) != hipSuccess || hipMalloc(&dT, n * OUT * sizeof(float)) != hipSuccess ||
@@ -812,7 +901,7 @@ extern "C" int mgr_mlp_train(mgr_mlp *mlp, const float *X, const float *T, int64
     if (n > (int64_t)1 << 31) return mlp->fail(MGR_ERR_ARGUMENT, "more than 2^31 training rows");
     MLP_HIP(hipSetDevice(mlp->device));
     const int64_t nbatch = (n + batch - 1) / batch;
-    const int Gmax = grid_for_rows(std::min(batch, n));
+    const int Gmax = grid_for_rows(std::min(batch, n), GRAD_GROUPS);
     float *dX = nullptr, *dT = nullptr, *dpart = nullptr, *dloss = nullptr;
     TrainState *dst = nullptr;
     int rc = MGR_OK;
@@ -840,7 +929,7 @@ extern "C" int mgr_mlp_train(mgr_mlp *mlp, const float *X, const float *T, int64
         hipLaunchKernelGGL(k_epoch_begin, dim3(1), dim3(1), 0, mlp->stream, dst);
         for (int64_t b = 0; b < nbatch; b++) {
             const int64_t b0 = b * batch, nb = std::min(batch, n - b0);
-            const int G = grid_for_rows(nb);
+            const int G = grid_for_rows(nb, GRAD_GROUPS);
             hipLaunchKernelGGL(k_mlp_grad, dim3(G), dim3(THREADS), LDS_TRAIN, mlp->stream, dX, dT,
                                (const TrainState *)dst, (const int64_t *)nullptr, b0, nb, nb, mlp->wbf, mlp->P,
                                mlp->norm, dpart);
@@ -928,7 +1017,7 @@ extern "C" int mgr_warm_start(mgr_ctx *ctx, mgr_mlp *mlp)
                 hipMemsetAsync(dCount, 0, sizeof(unsigned long long), ctx->stream) != hipSuccess))
         rc = ctx->fail(MGR_ERR_DEVICE, "warm start: copy failed");
     if (!rc) {
-        hipLaunchKernelGGL(k_mlp_forward, dim3(grid_for_rows(ctx->N)), dim3(THREADS), LDS_TRAIN, ctx->stream, dX,
+        hipLaunchKernelGGL(k_mlp_forward, dim3(grid_for_rows(ctx->N, 1024)), dim3(THREADS), LDS_FORWARD, ctx->stream, dX,
                            ctx->N, mlp->wbf, mlp->P, mlp->norm, (float *)nullptr, ctx->pop_tot, ctx->pop);
         hipLaunchKernelGGL(k_warm_guard, dim3((unsigned)((ctx->N + 255) / 256)), dim3(256), 0, ctx->stream, ctx->N,
                            (int)OUT, (int)ctx->L, ctx->irad, ctx->jrad, ctx->Ba, ctx->Bs, dPrev, ctx->pop, dCount);
