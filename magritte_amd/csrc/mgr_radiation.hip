@@ -81,6 +81,7 @@ constexpr int32_t ERR_NOT_BOUNDARY = 2;   // ray ends on a non-boundary cell
 constexpr int32_t ERR_EMPTY_SIDE   = 4;   // empty ray at a non-boundary origin
 constexpr int CH_MAX = 64;                // traced steps staged per chunk (at most)
 constexpr size_t LDS_LIMIT = 64 * 1024;   // dynamic LDS per workgroup
+constexpr int64_t WAVES_IN_FLIGHT = 8192;  // of the field kernels: 256 CUs, 8 waves per SIMD
 constexpr int MAX_WAVES = 4;              // frequency chunks per workgroup
 
 template <typename real> struct Prec;
@@ -1929,13 +1930,18 @@ static int launch_rf_shape(mgr_ctx *ctx, int nwg, int ch, int64_t o_begin, int64
         return launch_rf<float>(ctx, ctx->row32, nwg, ch, o_begin, o_count);
 }
 
-struct TuneCand { int nwg, ch; float ms; };
-
-// Launch-shape autotuner: waves (64-bin chunks) per workgroup and steps per
-// staged chunk, timed on up to 16384 origins of the model; the fastest shape
-// (or the one with the fewest waves among near-ties) is kept for the context
-// and precision.  Runs
+// Launch-shape autotuner: points per window first, with one wave (a 64-bin
+// chunk) per workgroup, then waves per workgroup with the best window.  Timed
+// on two slices of origins, around 1/8 and 5/8 of the model's cells, so that
+// outer and inner cells are seen, each with the waves the chip holds at once;
+// smaller models are timed whole.  The fastest shape (or the one with the
+// fewest waves among near-ties) is kept for the context and precision.  Runs
 // outside graph capture, before the first radiation field of a precision.
+//
+// The windows differ by up to 20 %, the waves, which share only the line
+// table, by 2 % (9 % where bins meet several lines): all combinations on 16384
+// origins, and the best ones again on the whole model, took 20 ms of a
+// 27^3-cell solve of 48 and chose the same shapes; this takes 4.
 template <typename real>
 static int tune(mgr_ctx *ctx, int pi)
 {
@@ -1943,99 +1949,48 @@ static int tune(mgr_ctx *ctx, int pi)
     const int chmax = max_chunk<real>(ctx);
     if (chmax < 2) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
     std::vector<int> nwgs;
-    for (int w = 1; w <= MAX_WAVES; w++)
-        if (w == 1 || w == nchunk || (nchunk % w) == 0 || w == std::min(nchunk, MAX_WAVES)) nwgs.push_back(w);
+    for (int w = 2; w <= MAX_WAVES; w++)
+        if (w == nchunk || (nchunk % w) == 0 || w == std::min(nchunk, MAX_WAVES)) nwgs.push_back(w);
     std::vector<int> chs;
     for (int c : {16, 32, 64})
         if (c <= chmax) chs.push_back(c);
     if (chs.empty() || chs.back() != chmax) chs.push_back(chmax);
-    // up to 16384 origins in four slices spread over the model (at 1/8, 3/8,
-    // 5/8 and 7/8 of its cells), so that the timing sees inner and outer cells
-    const int64_t cnt = std::min<int64_t>(ctx->N, 16384);
-    const int nslice = cnt >= 4096 ? 4 : 1;
-    const int64_t per = cnt / nslice;
-    int64_t os[4];
-    for (int k = 0; k < nslice; k++)
-        os[k] = nslice == 1 ? (ctx->N - cnt) / 2
-                            : std::min<int64_t>(std::max<int64_t>((2 * k + 1) * ctx->N / 8 - per / 2, 0), ctx->N - per);
+    const int64_t fill = (WAVES_IN_FLIGHT + nchunk - 1) / nchunk;   // origins that fill the chip
+    const int nslice = ctx->N > 2 * fill ? 2 : 1;
+    const int64_t per = nslice == 2 ? fill : ctx->N;
     auto launch_slices = [&](int w, int c) {
-        int r = MGR_OK;
-        for (int k = 0; k < nslice && !r; k++) r = launch_rf_shape<real>(ctx, w, c, os[k], per);
+        if (nslice == 1) return launch_rf_shape<real>(ctx, w, c, 0, ctx->N);
+        int r = launch_rf_shape<real>(ctx, w, c, std::max<int64_t>(ctx->N / 8 - per / 2, 0), per);
+        if (!r) r = launch_rf_shape<real>(ctx, w, c, std::min(ctx->N * 5 / 8 - per / 2, ctx->N - per), per);
         return r;
     };
-    int best_w = std::min(nchunk, MAX_WAVES), best_c = chmax;
-    float best = 1e30f;
     hipEvent_t e0, e1;
     MGR_HIP(hipEventCreate(&e0));
     MGR_HIP(hipEventCreate(&e1));
-    int rc = launch_slices(best_w, best_c);   // warm-up
+    int best_w = 1, best_c = chs.front();
+    float best = 1e30f;
+    int rc = launch_slices(1, chs.back());   // warm-up
     ctx->tune_log.clear();
-    for (int w : nwgs) {
-        for (int c : chs) {
-            if (rc) break;
-            float ms = 0.0f;
-            if (hipEventRecord(e0, ctx->stream) != hipSuccess) { rc = MGR_ERR_DEVICE; break; }
-            rc = launch_slices(w, c);
-            if (rc) break;
-            if (hipEventRecord(e1, ctx->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-                hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-                rc = MGR_ERR_DEVICE;
-                break;
-            }
-            ctx->tune_log.push_back({w, c, ms});
-            if (ms < best) { best = ms; best_w = w; best_c = c; }
+    auto time_shape = [&](int w, int c) {
+        float ms = 0.0f;
+        if (hipEventRecord(e0, ctx->stream) != hipSuccess) return MGR_ERR_DEVICE;
+        const int r = launch_slices(w, c);
+        if (r) return r;
+        if (hipEventRecord(e1, ctx->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
+            hipEventElapsedTime(&ms, e0, e1) != hipSuccess)
+            return MGR_ERR_DEVICE;
+        ctx->tune_log.push_back({w, c, ms});
+        // more waves only for 2 % (fewer schedule the end of a full launch more evenly)
+        if (ms < best * (w > best_w ? 0.98f : 1.0f)) {
+            best = ms;
+            best_w = w;
+            best_c = c;
         }
-    }
-    if (rc) {
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
-        return rc == MGR_ERR_DEVICE ? ctx->fail(MGR_ERR_DEVICE, "radiation-field tuning failed") : rc;
-    }
-    // Shapes within 2 % of the fastest are a tie on the slice; the one with
-    // fewer waves per workgroup schedules the end of a full launch more evenly
-    // (measured ~3 % faster on full launches where the slice could not tell).
-    float pick = best;
-    for (const auto &t : ctx->tune_log)
-        if (t.ms <= best * 1.02f && (t.nwg < best_w || (t.nwg == best_w && t.ms < pick))) {
-            best_w = t.nwg;
-            best_c = t.ch;
-            pick = t.ms;
-        }
-    // The slices do not always rank shapes as full launches do: when a full
-    // launch is cheap (under ~0.4 s by the slice timing), the fastest slice
-    // shape of each wave count within 5 % of the best is timed on the whole
-    // model once, and the fastest full launch is kept.
-    const double full_est = (double)best * (double)ctx->N / (double)(per * nslice);
-    if (nslice > 1 && full_est < 400.0) {
-        std::vector<TuneCand> cands;
-        for (int w : nwgs) {
-            float bw = 1e30f;
-            int bc = 0;
-            for (const auto &t : ctx->tune_log)
-                if (t.nwg == w && t.ms < bw) { bw = t.ms; bc = t.ch; }
-            if (bc && bw <= best * 1.05f) cands.push_back({w, bc, 0.0f});
-        }
-        if (cands.size() > 1) {
-            float full_best = 1e30f;
-            for (auto &cd : cands) {
-                float ms = 0.0f;
-                if (hipEventRecord(e0, ctx->stream) != hipSuccess) { rc = MGR_ERR_DEVICE; break; }
-                rc = launch_rf_shape<real>(ctx, cd.nwg, cd.ch, 0, ctx->N);
-                if (rc) break;
-                if (hipEventRecord(e1, ctx->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-                    hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-                    rc = MGR_ERR_DEVICE;
-                    break;
-                }
-                // ties within 1 % go to the fewer waves (the candidates come in that order)
-                if (ms < full_best * 0.99f) {
-                    full_best = ms;
-                    best_w = cd.nwg;
-                    best_c = cd.ch;
-                }
-            }
-        }
-    }
+        return MGR_OK;
+    };
+    for (size_t i = 0; i < chs.size() && !rc; i++) rc = time_shape(1, chs[i]);
+    const int window = best_c;
+    for (size_t i = 0; i < nwgs.size() && !rc; i++) rc = time_shape(nwgs[i], window);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc == MGR_ERR_DEVICE ? ctx->fail(MGR_ERR_DEVICE, "radiation-field tuning failed") : rc;
