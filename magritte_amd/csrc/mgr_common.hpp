@@ -6,6 +6,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -136,9 +137,14 @@ __host__ __device__ inline int lane_bin(int i, int L, int F, bool root_major)
 // Device-resident model and state (SoA).  Indices follow the reference:
 // J(p,f) at f + p*F (radiation.tpp:11-15), populations at i + p*V
 // (lineProducingSpecies.tpp:24-30), emissivity/opacity at k + p*L (lines.tpp:19-34).
+namespace mgr {
+struct Bounce;
+}
+
 struct mgr_ctx {
     int         device = 0;
     hipStream_t stream = nullptr;
+    std::shared_ptr<mgr::Bounce> bounce;   // staging of large copies to the host
     std::string err;
     int         status_sticky = MGR_OK;
 
@@ -390,6 +396,11 @@ int tune_radiation_field(mgr_ctx *ctx, int precision);   // outside graph captur
 int launch_lambda(mgr_ctx *ctx);
 int launch_band(mgr_ctx *ctx);         // band elements of Lambda* (nband > 0)
 int launch_band_cells(mgr_ctx *ctx);   // band cells and their reverse map (at trace time)
+int copy_to_host(mgr_ctx *ctx, void *dst, const void *src, size_t bytes);
+hipError_t block_malloc(mgr_ctx *ctx, void **p, size_t bytes);
+void block_free(mgr_ctx *ctx, void *p);
+void free_trace(mgr_ctx *ctx);         // the trace's arrays and what is computed from them per step
+void free_far(mgr_ctx *ctx);           // the far-end intensity caches
 int launch_jeff(mgr_ctx *ctx, bool lambda);
 int launch_stateq(mgr_ctx *ctx);
 int launch_convergence(mgr_ctx *ctx);

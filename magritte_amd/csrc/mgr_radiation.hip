@@ -2177,8 +2177,8 @@ extern "C" int mgr_compute_image(mgr_ctx *ctx, int64_t ray, int precision, doubl
     int32_t errv = 0;
     MGR_HIP(hipMemcpy(&errv, ctx->err_flag, sizeof(int32_t), hipMemcpyDeviceToHost));
     if (errv) return ctx->fail(MGR_ERR_TRACE, "an image ray ended off the boundary or an interior origin has an empty ray");
-    if (I_m) MGR_HIP(hipMemcpy(I_m, g.I_m, NF * sizeof(double), hipMemcpyDeviceToHost));
-    if (I_p) MGR_HIP(hipMemcpy(I_p, g.I_p, NF * sizeof(double), hipMemcpyDeviceToHost));
+    if (I_m && (rc = copy_to_host(ctx, I_m, g.I_m, NF * sizeof(double)))) return rc;
+    if (I_p && (rc = copy_to_host(ctx, I_p, g.I_p, NF * sizeof(double)))) return rc;
     return MGR_OK;
 }
 
@@ -2221,7 +2221,7 @@ int launch_far_cache(mgr_ctx *ctx, int precision)
     if (!*buf) {
         size_t fr = 0, tot = 0;
         if (hipMemGetInfo(&fr, &tot) != hipSuccess || bytes > fr / 4 * 3 ||
-            hipMalloc(buf, std::max<size_t>(bytes, 8)) != hipSuccess) {
+            block_malloc(ctx, buf, std::max<size_t>(bytes, 8)) != hipSuccess) {
             (void)hipGetLastError();
             *buf = nullptr;
             ctx->far_bad[pi] = true;
@@ -2267,10 +2267,7 @@ extern "C" int mgr_set_far_cache(mgr_ctx *ctx, int enable)
     MGR_HIP(hipStreamSynchronize(ctx->stream));
     ctx->far_cache = enable != 0;
     if (!ctx->far_cache) {
-        if (ctx->far_I32) (void)hipFree(ctx->far_I32);
-        if (ctx->far_I64) (void)hipFree(ctx->far_I64);
-        ctx->far_I32 = nullptr;
-        ctx->far_I64 = nullptr;
+        free_far(ctx);
     }
     ctx->far_invalidate();
     ctx->graph_precision = -1;   // captured launches hold the old choice
@@ -2291,7 +2288,5 @@ extern "C" int mgr_get_u(mgr_ctx *ctx, double *u)
     if (!ctx->u_store) return ctx->fail(MGR_ERR_STATE, "scattering is off (mgr_set_scattering)");
     MGR_HIP(hipSetDevice(ctx->device));
     MGR_HIP(hipStreamSynchronize(ctx->stream));
-    MGR_HIP(hipMemcpy(u, ctx->u_store, (size_t)(ctx->R / 2) * ctx->N * ctx->F * sizeof(double),
-                      hipMemcpyDeviceToHost));
-    return MGR_OK;
+    return copy_to_host(ctx, u, ctx->u_store, (size_t)(ctx->R / 2) * ctx->N * ctx->F * sizeof(double));
 }

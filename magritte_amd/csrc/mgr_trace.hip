@@ -146,6 +146,15 @@ __device__ __forceinline__ Walk trace_walk(int64_t N, const double *__restrict__
         }
         shift_nxt = REST ? rest_shift(vel, nxt, sx, sy, sz) : doppler_shift(vel, o, nxt, nx, ny, nz);
     }
+    // a co-moving walk owns its last block of four slots: those past its end are empty
+    if (FILL && !REST)
+        for (; w & 3; w++) {
+            seg_cell[w] = 0;
+            seg_shift[w] = 0.0;
+            seg_dZ[w] = 0.0;
+            seg_f32[w] = make_int4(0, 0, 0, 0);
+            seg_hdz32[w] = 0.0f;
+        }
     // the last, partly filled block of the record
     if (!FILL && rec && k.steps <= cap) rec[(k.steps - 1) >> 2] = acc;
     return k;
@@ -778,6 +787,13 @@ struct DeviceBuffer {
     ~DeviceBuffer() { release(); }
 };
 
+struct BlockBuffer {
+    mgr_ctx *ctx;
+    void    *p = nullptr;
+    void release() { block_free(ctx, p); p = nullptr; }
+    ~BlockBuffer() { release(); }
+};
+
 static int trace_error(mgr_ctx *ctx, int32_t errv)
 {
     if (errv & ERR_TOO_MANY) return ctx->fail(MGR_ERR_TRACE, "Too many (> 10 000) interpolations needed!");
@@ -814,14 +830,14 @@ int launch_trace(mgr_ctx *ctx)
     // The counting pass records the cells of every walk of up to `cap` steps
     // (a multiple of 4) in a buffer of at most a quarter of the free memory;
     // the filling pass replays them.  Longer walks are scanned again.
-    DeviceBuffer cells;
+    BlockBuffer cells{ctx};
     int cap = 0;
     if (NR > 0) {
         size_t freeb = 0, totb = 0;
         if (hipMemGetInfo(&freeb, &totb) == hipSuccess) {
             const int64_t budget = std::min<int64_t>((int64_t)(freeb / 4), TRACE_RECORD_BYTES);
             cap = (int)std::min<int64_t>(ctx->trace_record_steps, budget / NR / (int64_t)sizeof(int32_t) / 4 * 4);
-            if (cap < 4 || hipMalloc(&cells.p, (size_t)NR * cap * sizeof(int32_t)) != hipSuccess) {
+            if (cap < 4 || block_malloc(ctx, &cells.p, (size_t)NR * cap * sizeof(int32_t)) != hipSuccess) {
                 (void)hipGetLastError();
                 cells.p = nullptr;
                 cap = 0;
@@ -880,24 +896,14 @@ int launch_trace(mgr_ctx *ctx)
     ctx->masks_valid = false;
     ctx->masks64_valid = false;
     ctx->far_invalidate();
-    if (ctx->seg_cell) {
-        (void)hipFree(ctx->seg_cell); (void)hipFree(ctx->seg_shift); (void)hipFree(ctx->seg_dZ);
-        (void)hipFree(ctx->seg_f32); (void)hipFree(ctx->seg_hdz32); (void)hipFree(ctx->step_mask);
-        if (ctx->step_mask64) (void)hipFree(ctx->step_mask64);
-        if (ctx->span32) (void)hipFree(ctx->span32);
-        if (ctx->span64) (void)hipFree(ctx->span64);
-        ctx->step_mask64 = nullptr;
-        ctx->span32 = ctx->span64 = nullptr;
-        ctx->seg_cell = nullptr; ctx->seg_shift = nullptr; ctx->seg_dZ = nullptr;
-        ctx->seg_f32 = nullptr; ctx->seg_hdz32 = nullptr; ctx->step_mask = nullptr;
-    }
+    free_trace(ctx);
     const int64_t T = std::max<int64_t>(ctx->total_segments, 1);
-    MGR_HIP(hipMalloc((void **)&ctx->step_mask, T * sizeof(uint8_t)));
-    MGR_HIP(hipMalloc((void **)&ctx->seg_cell, T * sizeof(int32_t)));
-    MGR_HIP(hipMalloc((void **)&ctx->seg_shift, T * sizeof(double)));
-    MGR_HIP(hipMalloc((void **)&ctx->seg_dZ, T * sizeof(double)));
-    MGR_HIP(hipMalloc((void **)&ctx->seg_f32, T * sizeof(int4)));
-    MGR_HIP(hipMalloc((void **)&ctx->seg_hdz32, T * sizeof(float)));
+    MGR_HIP(block_malloc(ctx, (void **)&ctx->step_mask, T * sizeof(uint8_t)));
+    MGR_HIP(block_malloc(ctx, (void **)&ctx->seg_cell, T * sizeof(int32_t)));
+    MGR_HIP(block_malloc(ctx, (void **)&ctx->seg_shift, T * sizeof(double)));
+    MGR_HIP(block_malloc(ctx, (void **)&ctx->seg_dZ, T * sizeof(double)));
+    MGR_HIP(block_malloc(ctx, (void **)&ctx->seg_f32, T * sizeof(int4)));
+    MGR_HIP(block_malloc(ctx, (void **)&ctx->seg_hdz32, T * sizeof(float)));
     if (!ctx->far_cell) {
         MGR_HIP(hipMalloc((void **)&ctx->far_cell, std::max<int64_t>(NR, 1) * sizeof(int32_t)));
         MGR_HIP(hipMalloc((void **)&ctx->far_shift, std::max<int64_t>(NR, 1) * sizeof(double)));
@@ -979,7 +985,7 @@ int launch_step_masks(mgr_ctx *ctx, bool fp64)
     if (valid || !ctx->traced || !ctx->spectral_set) return MGR_OK;
     uint8_t *&bits_out = fp64 ? ctx->step_mask64 : ctx->step_mask;
     const int64_t T = std::max<int64_t>(ctx->total_segments, 1);
-    if (!bits_out) MGR_HIP(hipMalloc((void **)&bits_out, T));
+    if (!bits_out) MGR_HIP(block_malloc(ctx, (void **)&bits_out, T));
     const double window = fp64 ? MASK_WINDOW64 : MASK_WINDOW;
     const int64_t N = ctx->N;
     const int nchunk = (int)std::min<int64_t>((ctx->F + WAVE - 1) / WAVE, STEP_MASK_CHUNKS);
@@ -1003,7 +1009,7 @@ int launch_step_masks(mgr_ctx *ctx, bool fp64)
     // for them the bits (FP32) or nothing (FP64) is left out
     uint16_t *&span = fp64 ? ctx->span64 : ctx->span32;
     ctx->span_stride = (T + 3) / 4 * 4;
-    if (!span && hipMalloc((void **)&span, (size_t)nchunk * ctx->span_stride * sizeof(uint16_t)) != hipSuccess) {
+    if (!span && block_malloc(ctx, (void **)&span, (size_t)nchunk * ctx->span_stride * sizeof(uint16_t)) != hipSuccess) {
         (void)hipGetLastError();
         span = nullptr;
     }
