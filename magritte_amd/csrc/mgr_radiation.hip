@@ -103,7 +103,7 @@ template <> struct Prec<double> {
     }
 };
 
-// One traced step in LDS (image kernels).  Sub-point m = 1..n of the step lies
+// One traced step in LDS (FP32 image kernel).  Sub-point m = 1..n of the step lies
 // at shift s0 + m ds with path-length factor dz = dZ HDZ_SCALE and belongs to
 // the current cell for m < half, to `cell` otherwise.
 struct alignas(32) Step {
@@ -350,7 +350,7 @@ __device__ __forceinline__ double fmad(double a, double b, double c) { return __
 template <typename real>
 struct Sweep {
     real S_q, chi_q, hdz_q, cq;   // pending (outer) point: S, chi, its dz' and chi dz'
-    real c, y, z, p;              // last closed interval and the scaled state
+    real c, y, z, p, q;           // last closed interval and the scaled state, q = 1 / (1 + F) of the closed row
 
     // Virtual start.  With hdz_q = cq = 0 a step closes nothing: c = 0,
     // x = y, q = 1 exactly, so the first point may be stepped like any other.
@@ -394,7 +394,7 @@ struct Sweep {
     {
 #pragma clang fp contract(off)
         const real x = c + y;
-        const real q = Prec<real>::rcp(fmad(c, x, (real)1));
+        q = Prec<real>::rcp(fmad(c, x, (real)1));
         y = fmad(x, q, c);
         z = fmad(S_q, c, p) * q;
     }
@@ -404,10 +404,9 @@ struct Sweep {
 
 // Stage the entries e = 0..cnt-1 of chunk [a, b): entry e holds step j = a-1+e
 // (j = -1 is the origin) and the line rows of its cell.
-template <typename real>
-__device__ __forceinline__ void stage_chunk(const RFArgs<real> &a, int32_t o, int64_t q, int j0,
+__device__ __forceinline__ void stage_chunk(const RFArgs<float> &a, int32_t o, int64_t q, int j0,
                                             int cnt, double dsm, Step *__restrict__ st,
-                                            typename Prec<real>::row_t *__restrict__ rw)
+                                            float4 *__restrict__ rw)
 {
     const int64_t s0 = a.seg_off[q];
     const int nthr = blockDim.x;
@@ -420,7 +419,7 @@ __device__ __forceinline__ void stage_chunk(const RFArgs<real> &a, int32_t o, in
             const int32_t c = a.seg_cell[s0 + j];
             const double sn = a.seg_shift[s0 + j];
             const double z = a.seg_dZ[s0 + j];
-            const double sc = (j > 0) ? a.seg_shift[s0 + j - 1] : (a.origin_shift ? a.origin_shift[q] : 1.0);
+            const double sc = (j > 0) ? a.seg_shift[s0 + j - 1] : a.origin_shift[q];
             const StepSplit sp = split_step(sc, sn, z, dsm);
             s.cell = c;
             s.nh = sp.n | ((sp.interp ? sp.half : 0) << STEP_HALF_SHIFT);
@@ -481,17 +480,6 @@ __device__ __forceinline__ void eval_point<double>(const RFArgs<double> &a, cons
         fs = s * lc.nu_f;
     }
     eta_chi64(a, row, 1, lc.line, fs, lc.lstart, eta, chi);
-}
-
-// The point evaluation of a kernel: eval_point, or the FP32 image variant
-// with FP64 shifts.
-template <typename real, bool X64, typename SR>
-__device__ __forceinline__ void eval_at(const RFArgs<real> &a, const LaneCtx<real> &lc,
-                                        const typename Prec<real>::row_t *__restrict__ row, SR s,
-                                        real &eta, real &chi)
-{
-    if constexpr (X64) eta_chi32x(a, row, lc.ln, s, eta, chi);
-    else eval_point<real>(a, lc, row, s, eta, chi);
 }
 
 // shift of sub-point m: FP64 exactly s0 + m ds as Geometry::set_data;
@@ -584,15 +572,13 @@ __global__ __launch_bounds__(256) void k_far_cache(RFArgs<float> a, int Rmax, T 
 
 // One ray of an image pair, eliminated from its boundary end (incoming intensity
 // I_far, scaled) inwards to the origin, which it leaves pending.
-template <typename real, bool X64>
-__device__ __forceinline__ Sweep<real> sweep_side(const RFArgs<real> &a, const LaneCtx<real> &lc,
-                                                  int32_t o, int64_t q, real I_far, real S_o,
-                                                  real chi_o, double dsm,
+__device__ __forceinline__ Sweep<float> sweep_side(const RFArgs<float> &a, const LaneCtx<float> &lc,
+                                                  int32_t o, int64_t q, float I_far, float S_o,
+                                                  float chi_o, double dsm,
                                                   Step *__restrict__ st,
-                                                  typename Prec<real>::row_t *__restrict__ rw)
+                                                  float4 *__restrict__ rw)
 {
-    using row_t = typename Prec<real>::row_t;
-    Sweep<real> sw;
+    Sweep<float> sw;
     sw.init(I_far);
     const int ns = a.nseg[q];
     const int L = a.L;
@@ -601,37 +587,37 @@ __device__ __forceinline__ Sweep<real> sweep_side(const RFArgs<real> &a, const L
         const int a_ = b_ > CH ? b_ - CH : 0;
         const int cnt = b_ - a_ + 1;
         __syncthreads();   // the previous chunk is consumed by every wave
-        stage_chunk<real>(a, o, q, a_ - 1, cnt, dsm, st, rw);
+        stage_chunk(a, o, q, a_ - 1, cnt, dsm, st, rw);
         for (int e = cnt - 1; e >= 1; --e) {
             const int nh = rfl_int(st[e].nh);   // one readfirstlane: n and half are wave-uniform
             const int n = nh & STEP_N_MASK;
             const int half = (nh >> STEP_HALF_SHIFT) & STEP_HALF_MASK;
             const double s0 = st[e].s0, ds = st[e].ds;
-            const real hdz = (real)st[e].dz;
+            const float hdz = (float)st[e].dz;
             // sub-points m >= half lie in the step's cell (row e), m < half in
             // the previous one (row e-1); two loops keep each row's address
             // loop-invariant
-            const row_t *rn = rw + e * L;
-            const row_t *rc = rw + (e - 1) * L;
+            const float4 *rn = rw + e * L;
+            const float4 *rc = rw + (e - 1) * L;
             const int mlo = half > 1 ? half : 1;
             for (int m = n; m >= mlo; --m) {
-                real eta, chi;
-                eval_at<real, X64>(a, lc, rn, sub_point_shift(s0, m, ds), eta, chi);
-                const real S = eta * Prec<real>::rcp(chi);
+                float eta, chi;
+                eta_chi32x(a, rn, lc.ln, sub_point_shift(s0, m, ds), eta, chi);
+                const float S = eta * Prec<float>::rcp(chi);
                 sw.step(chi);   // on the first point an exact no-op (c = 0, q = 1)
                 sw.pend(S, chi, hdz);
             }
             for (int m = (half - 1 < n ? half - 1 : n); m >= 1; --m) {
-                real eta, chi;
-                eval_at<real, X64>(a, lc, rc, sub_point_shift(s0, m, ds), eta, chi);
-                const real S = eta * Prec<real>::rcp(chi);
+                float eta, chi;
+                eta_chi32x(a, rc, lc.ln, sub_point_shift(s0, m, ds), eta, chi);
+                const float S = eta * Prec<float>::rcp(chi);
                 sw.step(chi);
                 sw.pend(S, chi, hdz);
             }
         }
     }
     sw.step(chi_o);   // the origin closes the innermost row and is left pending
-    sw.pend(S_o, chi_o, (real)0);
+    sw.pend(S_o, chi_o, (float)0);
     return sw;
 }
 
@@ -640,13 +626,11 @@ __device__ __forceinline__ Sweep<real> sweep_side(const RFArgs<real> &a, const L
 // pending row with its own dZ (the outer point's, as Simulation::setup pairs
 // them, simulation.tpp:306) and becomes the pending point; on return the
 // far-end point is pending.
-template <typename real, bool X64 = false>
-__device__ __forceinline__ void sweep_outward(const RFArgs<real> &a, const LaneCtx<real> &lc, int32_t o,
-                                              int64_t q, double dsm, Sweep<real> &sw,
+__device__ __forceinline__ void sweep_outward(const RFArgs<float> &a, const LaneCtx<float> &lc, int32_t o,
+                                              int64_t q, double dsm, Sweep<float> &sw,
                                               Step *__restrict__ st,
-                                              typename Prec<real>::row_t *__restrict__ rw)
+                                              float4 *__restrict__ rw)
 {
-    using row_t = typename Prec<real>::row_t;
     const int ns = a.nseg[q];
     const int L = a.L;
     const int CH = a.ch;
@@ -654,27 +638,27 @@ __device__ __forceinline__ void sweep_outward(const RFArgs<real> &a, const LaneC
         const int b_ = a_ + CH < ns ? a_ + CH : ns;
         const int cnt = b_ - a_ + 1;
         __syncthreads();   // the previous chunk is consumed by every wave
-        stage_chunk<real>(a, o, q, a_ - 1, cnt, dsm, st, rw);
+        stage_chunk(a, o, q, a_ - 1, cnt, dsm, st, rw);
         for (int e = 1; e < cnt; ++e) {
             const int nh = rfl_int(st[e].nh);   // one readfirstlane: n and half are wave-uniform
             const int n = nh & STEP_N_MASK;
             const int half = (nh >> STEP_HALF_SHIFT) & STEP_HALF_MASK;
             const double s0 = st[e].s0, ds = st[e].ds;
-            const real hdz = (real)st[e].dz;
-            const row_t *rn = rw + e * L;
-            const row_t *rc = rw + (e - 1) * L;
+            const float hdz = (float)st[e].dz;
+            const float4 *rn = rw + e * L;
+            const float4 *rc = rw + (e - 1) * L;
             const int mhi = half - 1 < n ? half - 1 : n;
             for (int m = 1; m <= mhi; ++m) {
-                real eta, chi;
-                eval_at<real, X64>(a, lc, rc, sub_point_shift(s0, m, ds), eta, chi);
-                const real S = eta * Prec<real>::rcp(chi);
+                float eta, chi;
+                eta_chi32x(a, rc, lc.ln, sub_point_shift(s0, m, ds), eta, chi);
+                const float S = eta * Prec<float>::rcp(chi);
                 sw.step_out(chi, hdz);
                 sw.pend(S, chi, hdz);
             }
             for (int m = half > 1 ? half : 1; m <= n; ++m) {
-                real eta, chi;
-                eval_at<real, X64>(a, lc, rn, sub_point_shift(s0, m, ds), eta, chi);
-                const real S = eta * Prec<real>::rcp(chi);
+                float eta, chi;
+                eta_chi32x(a, rn, lc.ln, sub_point_shift(s0, m, ds), eta, chi);
+                const float S = eta * Prec<float>::rcp(chi);
                 sw.step_out(chi, hdz);
                 sw.pend(S, chi, hdz);
             }
@@ -775,6 +759,14 @@ struct Window {
     Stage<real> *stage;
     int         *owner;
     static constexpr size_t fixed = WAVE * (sizeof(real) + sizeof(Stage<real>) + sizeof(int));   // bytes beside the rows
+    static constexpr size_t bytes(int64_t L, int points) { return fixed + sizeof(row_t) * L * (points + 1); }
+    __device__ __forceinline__ void place(unsigned char *smem)
+    {
+        hdz = reinterpret_cast<real *>(smem);
+        stage = reinterpret_cast<Stage<real> *>(hdz + WAVE);
+        owner = reinterpret_cast<int *>(stage + WAVE);
+        rows = reinterpret_cast<row_t *>(owner + WAVE);
+    }
 };
 
 constexpr int BATCH = WAVE - 1;   // steps per batch: one lane each, the last lane for the cell before them
@@ -1170,10 +1162,7 @@ void k_radiation_field(RFArgs<real> a)
     extern __shared__ __align__(16) unsigned char smem[];
     const int wave = rfl_int((int)(threadIdx.x / WAVE));
     Window<real> win;
-    win.hdz = reinterpret_cast<real *>(smem + wave * a.wave_lds);
-    win.stage = reinterpret_cast<Stage<real> *>(win.hdz + WAVE);
-    win.owner = reinterpret_cast<int *>(win.stage + WAVE);
-    win.rows = reinterpret_cast<row_t *>(win.owner + WAVE);
+    win.place(smem + wave * a.wave_lds);
 
     // XCD-aware order: consecutive workgroups go to different XCDs, so hand
     // each XCD a contiguous range of origins.
@@ -1278,114 +1267,17 @@ void k_radiation_field(RFArgs<real> a)
     lambda_partials(a, o, chunk, active, f, nu_f, lam_f);
 }
 
-// Image of ray r (Simulation::compute_and_write_image, sim_radiation.tpp:345-478;
-// RayPair::solve_for_image, raypair_solver.tpp:523-579).  Entries 2o (the
-// antipode, index 0 end of the pair) and 2o + 1 (ray r, index ndep-1 end) of
-// the rest-frame trace.  The intensities leaving the pair are
-// I_p = 2 u(ndep-1) - I_bdy_n and I_m = 2 u(0) - I_bdy_0 (RayPair::get_Ip_at_end,
-// get_Im_at_front, raypair.tpp:212-229).  Instead of a stored forward
-// elimination and back-substitution, each end's u comes from one full sweep
-// that starts at the other end, passes the origin and closes at the end
-// itself with its boundary row: two sweeps, no per-point storage.
-template <typename real, bool X64>
-__global__ __launch_bounds__(WAVE * MAX_WAVES) void k_image(RFArgs<real> a, double *__restrict__ I_m,
-                                                            double *__restrict__ I_p)
-{
-    using row_t = typename Prec<real>::row_t;
-    extern __shared__ __align__(16) unsigned char smem[];
-    Step *st = reinterpret_cast<Step *>(smem);
-    row_t *rw = reinterpret_cast<row_t *>(smem + a.row_offset);
-
-    const int G = gridDim.x;
-    const int per = G >> 3;
-    const int bid = blockIdx.x;
-    const int logical = (bid & 7) * per + (bid >> 3);
-    if (logical >= a.grid_real) return;   // whole workgroup: before any barrier
-    const int32_t o = a.o_begin + (int32_t)(logical / a.ngroups);
-    const int group = logical - (o - a.o_begin) * a.ngroups;
-    const int wave = threadIdx.x / WAVE;
-    const int chunk = rfl_int(group * a.nwg + wave);   // wave-uniform: scalar skip tests
-    const int F = a.F;
-    const int f = chunk * WAVE + (int)(threadIdx.x & (WAVE - 1));
-    const bool active = f < F;
-    const int fa = active ? f : F - 1;
-    const double nu_f = a.nu[(int64_t)o * F + fa];
-    const double dsm = a.dshift_max[o];
-    const int32_t bo = a.cell2bdy[o];
-    const row_t *orow = a.rows + (int64_t)o * a.L;
-
-    LaneCtx<real> lc;
-    if constexpr (sizeof(real) == 8) lc.line = a.tb->line;
-    real S_o, chi_o;
-    origin_point<real, X64>(a, nu_f, orow, lc, S_o, chi_o);
-
-    int32_t err = 0;
-    const int64_t qa = 2 * (int64_t)o, qr = qa + 1;
-    const int n_a = a.npts[qa];
-    const int n_r = a.npts[qr];
-    double Im = 0.0, Ip = 0.0;
-    if (n_a == 0 && n_r == 0) {
-        // too short a ray: both intensities are I_bdy of the origin's boundary entry
-        if (bo < 0) err |= ERR_EMPTY_SIDE;
-        else Im = Ip = a.I_bdy[(int64_t)bo * F + fa];
-    } else {
-        double I_o = 0.0;   // an empty side takes I_bdy of the origin's boundary entry
-        if (n_a == 0 || n_r == 0) {
-            if (bo < 0) err |= ERR_EMPTY_SIDE;
-            else I_o = a.I_bdy[(int64_t)bo * F + fa];
-        }
-        const double I0 = n_a > 0 ? far_intensity(a, qa, nu_f, F, err) : I_o;
-        const double In = n_r > 0 ? far_intensity(a, qr, nu_f, F, err) : I_o;
-        const real I0s = (real)(I0 * I_SCALE);
-        const real Ins = (real)(In * I_SCALE);
-        real u_n, u_0;
-        {
-            // from the antipode's far end through the origin to ray r's end
-            Sweep<real> A;
-            if (n_a > 0) {
-                A = sweep_side<real, X64>(a, lc, o, qa, I0s, S_o, chi_o, dsm, st, rw);
-            } else {
-                A.init(I0s);
-                A.pend(S_o, chi_o, (real)0);
-            }
-            sweep_outward<real, X64>(a, lc, o, qr, dsm, A, st, rw);
-            u_n = end_u(A, Ins);
-        }
-        {
-            // and back
-            Sweep<real> B;
-            if (n_r > 0) {
-                B = sweep_side<real, X64>(a, lc, o, qr, Ins, S_o, chi_o, dsm, st, rw);
-            } else {
-                B.init(Ins);
-                B.pend(S_o, chi_o, (real)0);
-            }
-            sweep_outward<real, X64>(a, lc, o, qa, dsm, B, st, rw);
-            u_0 = end_u(B, I0s);
-        }
-        Ip = 2.0 * ((double)u_n * (1.0 / I_SCALE)) - In;
-        Im = 2.0 * ((double)u_0 * (1.0 / I_SCALE)) - I0;
-    }
-    if (err) atomicOr(a.err_flag, err);
-    if (active) {
-        I_m[(int64_t)o * F + f] = Im;
-        I_p[(int64_t)o * F + f] = Ip;
-    }
-}
-
-// ---- banded Lambda* (n_off_diag >= 2) ------------------------------------------
-
 // The points of a ray pair in order: entry qx from its far end inwards, the
-// origin, then entry qy outwards, at most ny points of it.  visit(t, chi, h, p)
-// gets the visit count t (uniform in the wave), the opacity of the lane's bin
-// there, the path factor h of the interval between the point and the one
+// origin, then entry qy outwards, at most ny points of it.  visit(t, eta, chi,
+// h, p) gets the visit count t (uniform in the wave), the emissivity and opacity
+// of the lane's bin there, the path factor h of the interval between the point and the one
 // visited before it, which is that of the interval's outer point
 // (Simulation::setup, simulation.tpp:233-240, 292-299; 0 for the first point),
 // and the point's place p in the window (its shift and cell in win.stage).
 //
 // As in sweep_pair, up to WAVE steps of the pair lie on the lanes, and their
 // points a window at a time, with the line rows of those inside the line
-// window in LDS; at the others (spans) chi is the floor.
+// window in LDS; at the others (spans) eta = 0 and chi is the floor.
 template <bool ONE, typename Visit>
 __device__ __forceinline__ void walk_pair(const RFArgs<double> &a, const LaneCtx<double> &lc, int32_t o, int64_t qx,
                                           int64_t qy, int ny, double dsm, int chunk, const Window<double> &win,
@@ -1414,7 +1306,7 @@ __device__ __forceinline__ void walk_pair(const RFArgs<double> &a, const LaneCtx
             if (spans) span = ka->span[ka->span_stride * chunk + at];
             c_next = ka->seg_cell[at];
             const double sn = ka->seg_shift[at];
-            double sc = 1.0;   // co-moving: the origin's shift is 1
+            double sc = ka->origin_shift ? ka->origin_shift[inward ? qx : qy] : 1.0;   // co-moving: the origin's is 1
             if (j > 0) {
                 c_prev = ka->seg_cell[at - 1];
                 sc = ka->seg_shift[at - 1];
@@ -1477,13 +1369,194 @@ __device__ __forceinline__ void walk_pair(const RFArgs<double> &a, const LaneCtx
             }
             wave_lds_fence();
             for (int p = 0; p < cw; ++p) {
-                double eta, chi = CHI_FLOOR * CHI_SCALE;
+                double eta = 0.0, chi = CHI_FLOOR * CHI_SCALE;
                 if (!((floors >> p) & 1)) eval_window<double, ONE>(a, lc, win, p, W, eta, chi);
-                visit(t++, chi, win.hdz[p], p);
+                visit(t++, eta, chi, win.hdz[p], p);
             }
         }
     }
 }
+
+// Image of ray r (Simulation::compute_and_write_image, sim_radiation.tpp:345-478;
+// RayPair::solve_for_image, raypair_solver.tpp:523-579).  Entries 2o (the
+// antipode, index 0 end of the pair) and 2o + 1 (ray r, index ndep-1 end) of
+// the rest-frame trace.  The intensities leaving the pair are
+// I_p = 2 u(ndep-1) - I_bdy_n and I_m = 2 u(0) - I_bdy_0 (RayPair::get_Ip_at_end,
+// get_Im_at_front, raypair.tpp:212-229).
+// u at the end of the elimination is its boundary row's.  The rows say
+// u_n = q_n u_{n+1} + c_n z_n, so u_0 = U + P u_n with P the product of the q
+// and U the sum of P c z: one sweep for both ends, no per-point storage.
+//
+// FP64: one wave per (origin, chunk of bins), at 4 per SIMD.  Bound by the
+// evaluation of every point, most of them outside the window of most bins.  Two
+// sweeps by workgroups that staged 64 steps at a time (as k_image32) took 5.2 ms
+// at 36^3 cells and 186 bins, this takes 2.3.
+__global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_image64(RFArgs<double> a,
+                                                                                          double *__restrict__ I_m,
+                                                                                          double *__restrict__ I_p)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int G = gridDim.x;
+    const int per = G >> 3;
+    const int bid = blockIdx.x;
+    const int logical = (bid & 7) * per + (bid >> 3);
+    if (logical >= a.grid_real) return;
+    const int32_t o = a.o_begin + (int32_t)(logical / a.nchunk);
+    const int chunk = logical - (o - a.o_begin) * a.nchunk;
+    const int lane = (int)threadIdx.x;
+    Window<double> win;
+    win.place(smem);
+    const int F = a.F;
+    const int f = chunk * WAVE + lane;
+    const bool active = f < F;
+    const int fa = active ? f : F - 1;
+    const double nu_f = a.nu[(int64_t)o * F + fa];
+    const double dsm = a.dshift_max[o];
+    const int32_t bo = a.cell2bdy[o];
+    LaneCtx<double> lc;
+    {
+        // the line frequencies, read at every point
+        double *lt = reinterpret_cast<double *>(smem + a.line_offset);
+        for (int i = lane; i < a.L; i += WAVE) lt[i] = a.tb->line[i];
+        wave_lds_fence();
+        lc.line = lt;
+    }
+    double S_o, chi_o;
+    origin_point<double>(a, nu_f, a.rows + (int64_t)o * a.L, lc, S_o, chi_o);
+
+    int32_t err = 0;
+    const int64_t qa = 2 * (int64_t)o, qr = qa + 1;
+    const int n_a = rfl_int(a.npts[qa]);
+    const int n_r = rfl_int(a.npts[qr]);
+    double Im = 0.0, Ip = 0.0;
+    if (n_a == 0 && n_r == 0) {
+        // too short a ray: both intensities are I_bdy of the origin's boundary entry
+        if (bo < 0) err |= ERR_EMPTY_SIDE;
+        else Im = Ip = a.I_bdy[(int64_t)bo * F + fa];
+    } else {
+        double I_o = 0.0;   // an empty side takes I_bdy of the origin's boundary entry
+        if (n_a == 0 || n_r == 0) {
+            if (bo < 0) err |= ERR_EMPTY_SIDE;
+            else I_o = a.I_bdy[(int64_t)bo * F + fa];
+        }
+        const double I0 = n_a > 0 ? far_intensity(a, qa, nu_f, F, err) : I_o;
+        const double In = n_r > 0 ? far_intensity(a, qr, nu_f, F, err) : I_o;
+        Sweep<double> sw;
+        sw.init(I0 * I_SCALE);
+        double U = 0.0, P = 1.0;
+        walk_pair<false>(a, lc, o, qa, qr, n_r, dsm, chunk, win, [&](int t, double eta, double chi, double h, int) {
+            const double S = eta * Prec<double>::rcp(chi);
+            if (t <= n_a) {   // inwards and to the origin, with the pending point's path factor
+                sw.hdz_q = h;
+                sw.cq = sw.chi_q * h;
+                sw.step(chi);
+            } else {
+                sw.step_out(chi, h);
+            }
+            sw.pend(S, chi, h);
+            U = fmad(P, sw.c * sw.z, U);
+            P *= sw.q;
+        });
+        const double u_n = end_u(sw, In * I_SCALE), u_0 = fmad(P, u_n, U);
+        Ip = 2.0 * (u_n * (1.0 / I_SCALE)) - In;
+        Im = 2.0 * (u_0 * (1.0 / I_SCALE)) - I0;
+    }
+    if (err) atomicOr(a.err_flag, err);
+    if (active) {
+        I_m[(int64_t)o * F + f] = Im;
+        I_p[(int64_t)o * F + f] = Ip;
+    }
+}
+
+// The same in FP32, with shifts and profile arguments in FP64 (eta_chi32x).
+// Instead of a stored forward elimination and back-substitution, each end's u
+// comes from one full sweep that starts at the other end, passes the origin and
+// closes at the end itself with its boundary row: two sweeps, no per-point
+// storage.  (36^3 cells, 186 bins: 1.18 ms; on walk_pair 1.35.)
+__global__ __launch_bounds__(WAVE * MAX_WAVES) void k_image32(RFArgs<float> a, double *__restrict__ I_m,
+                                                              double *__restrict__ I_p)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    Step *st = reinterpret_cast<Step *>(smem);
+    float4 *rw = reinterpret_cast<float4 *>(smem + a.row_offset);
+
+    const int G = gridDim.x;
+    const int per = G >> 3;
+    const int bid = blockIdx.x;
+    const int logical = (bid & 7) * per + (bid >> 3);
+    if (logical >= a.grid_real) return;   // whole workgroup: before any barrier
+    const int32_t o = a.o_begin + (int32_t)(logical / a.ngroups);
+    const int group = logical - (o - a.o_begin) * a.ngroups;
+    const int wave = threadIdx.x / WAVE;
+    const int chunk = rfl_int(group * a.nwg + wave);   // wave-uniform: scalar skip tests
+    const int F = a.F;
+    const int f = chunk * WAVE + (int)(threadIdx.x & (WAVE - 1));
+    const bool active = f < F;
+    const int fa = active ? f : F - 1;
+    const double nu_f = a.nu[(int64_t)o * F + fa];
+    const double dsm = a.dshift_max[o];
+    const int32_t bo = a.cell2bdy[o];
+    const float4 *orow = a.rows + (int64_t)o * a.L;
+
+    LaneCtx<float> lc;
+    float S_o, chi_o;
+    origin_point<float, true>(a, nu_f, orow, lc, S_o, chi_o);
+
+    int32_t err = 0;
+    const int64_t qa = 2 * (int64_t)o, qr = qa + 1;
+    const int n_a = a.npts[qa];
+    const int n_r = a.npts[qr];
+    double Im = 0.0, Ip = 0.0;
+    if (n_a == 0 && n_r == 0) {
+        // too short a ray: both intensities are I_bdy of the origin's boundary entry
+        if (bo < 0) err |= ERR_EMPTY_SIDE;
+        else Im = Ip = a.I_bdy[(int64_t)bo * F + fa];
+    } else {
+        double I_o = 0.0;   // an empty side takes I_bdy of the origin's boundary entry
+        if (n_a == 0 || n_r == 0) {
+            if (bo < 0) err |= ERR_EMPTY_SIDE;
+            else I_o = a.I_bdy[(int64_t)bo * F + fa];
+        }
+        const double I0 = n_a > 0 ? far_intensity(a, qa, nu_f, F, err) : I_o;
+        const double In = n_r > 0 ? far_intensity(a, qr, nu_f, F, err) : I_o;
+        const float I0s = (float)(I0 * I_SCALE);
+        const float Ins = (float)(In * I_SCALE);
+        float u_n, u_0;
+        {
+            // from the antipode's far end through the origin to ray r's end
+            Sweep<float> A;
+            if (n_a > 0) {
+                A = sweep_side(a, lc, o, qa, I0s, S_o, chi_o, dsm, st, rw);
+            } else {
+                A.init(I0s);
+                A.pend(S_o, chi_o, (float)0);
+            }
+            sweep_outward(a, lc, o, qr, dsm, A, st, rw);
+            u_n = end_u(A, Ins);
+        }
+        {
+            // and back
+            Sweep<float> B;
+            if (n_r > 0) {
+                B = sweep_side(a, lc, o, qr, Ins, S_o, chi_o, dsm, st, rw);
+            } else {
+                B.init(Ins);
+                B.pend(S_o, chi_o, (float)0);
+            }
+            sweep_outward(a, lc, o, qa, dsm, B, st, rw);
+            u_0 = end_u(B, I0s);
+        }
+        Ip = 2.0 * ((double)u_n * (1.0 / I_SCALE)) - In;
+        Im = 2.0 * ((double)u_0 * (1.0 / I_SCALE)) - I0;
+    }
+    if (err) atomicOr(a.err_flag, err);
+    if (active) {
+        I_m[(int64_t)o * F + f] = Im;
+        I_p[(int64_t)o * F + f] = Ip;
+    }
+}
+
+// ---- banded Lambda* (n_off_diag >= 2) ------------------------------------------
 
 // The elimination's coefficients along one direction of a pair: close() takes
 // the next point and closes the row of the one before it.  With dt the closed
@@ -1558,10 +1631,7 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4))) void 
     const int lane = (int)threadIdx.x;
     const int F = a.F, L = a.L, nb = a.nband;
     Window<double> win;
-    win.hdz = reinterpret_cast<double *>(smem);
-    win.stage = reinterpret_cast<Stage<double> *>(win.hdz + WAVE);
-    win.owner = reinterpret_cast<int *>(win.stage + WAVE);
-    win.rows = reinterpret_cast<double4 *>(win.owner + WAVE);
+    win.place(smem);
     // per band and lane: elem [2 nb] the elements, lower ones first (before them
     // the products over G or F so far), termG [2 nb] G / (1 + G) for their L_diag
     double *elem = reinterpret_cast<double *>(win.rows + (size_t)L * (a.ch + 1));
@@ -1609,7 +1679,7 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4))) void 
             RowSweep sw;
             double prod = 1.0;
             walk_pair<ONE>(a, lc, o, qB, qA, nA < nb ? nA : nb, dsm, chunk, win,
-                           [&](int t, double chi, double h, int) {
+                           [&](int t, double, double chi, double h, int) {
                 sw.close(chi, h);   // row last - t + 1 (none at t = 0)
                 const int i = last - t + 1 - nA;
                 if (i > 2 * nb + 2 || t == 0) return;
@@ -1625,7 +1695,7 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4))) void 
             sw = RowSweep();
             double fpc = 0.0;   // nu phi(nu) / chi of the last point, factor applied
             const int ny = nB < 2 * nb + 2 ? nB : 2 * nb + 2;
-            walk_pair<ONE>(a, lc, o, qA, qB, ny, dsm, chunk, win, [&](int n, double chi, double h, int p) {
+            walk_pair<ONE>(a, lc, o, qA, qB, ny, dsm, chunk, win, [&](int n, double, double chi, double h, int p) {
                 sw.close(chi, h);   // row n - 1 (none at n = 0)
                 const int i = n - 1 - nA;
                 if (i < -nb - 1) return;
@@ -1756,7 +1826,6 @@ int make_args(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
     if (ch < 2 || ch > max_chunk<real, X64>(ctx)) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
     a.ch = ch;
     a.row_offset = ((sizeof(Step) * (ch + 1) + 63) / 64) * 64;
-    a.line_offset = a.row_offset + sizeof(typename Prec<real>::row_t) * (ch + 1) * ctx->L;
     return MGR_OK;
 }
 
@@ -1783,10 +1852,12 @@ bool one_line(const mgr_ctx *ctx, const RFArgs<real> &a)
     return true;
 }
 
-template <typename real>
-size_t lds_bytes(const mgr_ctx *ctx, const RFArgs<real> &a)
+// Points per window of walk_pair: at most 32, with rows of up to 8 KB, so that 4
+// waves fit a SIMD.
+int walk_window(const mgr_ctx *ctx)
 {
-    return a.line_offset + (sizeof(real) == 8 ? sizeof(double) * ctx->L : 0);
+    const int64_t row = sizeof(double4) * ctx->L;
+    return (int)std::max<int64_t>(2, std::min<int64_t>(32, 8 * 1024 / row - 1));
 }
 
 template <typename real>
@@ -1855,14 +1926,16 @@ int launch_rf(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
     return MGR_OK;
 }
 
-// Image kernel over every origin, on the rest-frame trace of ctx->img.
-template <typename real, bool X64>
+// Image kernel over every origin, on the rest-frame trace of ctx->img.  FP32: the
+// sweep and profiles in FP32, shifts and profile arguments in FP64.
+template <typename real>
 int launch_image(mgr_ctx *ctx, const typename Prec<real>::row_t *rows)
 {
+    constexpr bool F32 = sizeof(real) == 4;
     const int nchunk = (int)((ctx->F + WAVE - 1) / WAVE);
     const mgr_ctx::ImageTrace &g = ctx->img;
     RFArgs<real> a;
-    int rc = make_args<real, X64>(ctx, rows, std::min(nchunk, MAX_WAVES), max_chunk<real, X64>(ctx), 0,
+    int rc = make_args<real, F32>(ctx, rows, F32 ? std::min(nchunk, MAX_WAVES) : 1, max_chunk<real, F32>(ctx), 0,
                                   ctx->N, g.shift_min, g.shift_max, a);
     if (rc) return rc;
     a.step_mask = nullptr;   // the masks index the co-moving cache, not the image's trace
@@ -1872,13 +1945,18 @@ int launch_image(mgr_ctx *ctx, const typename Prec<real>::row_t *rows)
     a.seg_cell = g.seg_cell;
     a.seg_shift = g.seg_shift;
     a.seg_dZ = g.seg_dZ;
-    a.seg_f32 = g.seg_f32;
-    a.seg_hdz32 = g.seg_hdz32;
     a.far_cell = g.far_cell;
     a.far_shift = g.far_shift;
     a.origin_shift = g.origin_shift;
-    hipLaunchKernelGGL((k_image<real, X64>), dim3(grid_of(a)), dim3(WAVE * a.nwg), lds_bytes(ctx, a), ctx->stream, a,
-                       g.I_m, g.I_p);
+    if constexpr (F32) {
+        const size_t lds = a.row_offset + sizeof(float4) * (a.ch + 1) * ctx->L;
+        hipLaunchKernelGGL(k_image32, dim3(grid_of(a)), dim3(WAVE * a.nwg), lds, ctx->stream, a, g.I_m, g.I_p);
+    } else {
+        a.ch = walk_window(ctx);
+        a.line_offset = Window<double>::bytes(ctx->L, a.ch);
+        const size_t lds = a.line_offset + sizeof(double) * ctx->L;
+        hipLaunchKernelGGL(k_image64, dim3(grid_of(a)), dim3(WAVE), lds, ctx->stream, a, g.I_m, g.I_p);
+    }
     MGR_LAUNCH_CHECK();
     return MGR_OK;
 }
@@ -1907,9 +1985,8 @@ int launch_band(mgr_ctx *ctx)
     a.root_major = ctx->root_major;
     a.span_stride = ctx->span_stride;
     if (ctx->masks64_valid && ctx->rf_window_skip) a.span = ctx->span64;
-    // windows of at most 32 points: rows of up to 8 KB, so that 4 waves fit a SIMD
-    a.ch = (int)std::max<int64_t>(2, std::min<int64_t>(32, 8 * 1024 / (int64_t)(sizeof(double4) * ctx->L) - 1));
-    const size_t lds = Window<double>::fixed + sizeof(double4) * ctx->L * (a.ch + 1) +
+    a.ch = walk_window(ctx);
+    const size_t lds = Window<double>::bytes(ctx->L, a.ch) +
                        sizeof(double) * (4 * (size_t)ctx->nband * WAVE + ctx->L) + sizeof(int) * (ctx->L + 1);
     auto kernel = one_line(ctx, a) ? k_lambda_band<true> : k_lambda_band<false>;
     hipLaunchKernelGGL(kernel, dim3(grid_of(a)), dim3(WAVE), lds, ctx->stream, a);
@@ -2169,9 +2246,7 @@ extern "C" int mgr_compute_image(mgr_ctx *ctx, int64_t ray, int precision, doubl
         MGR_HIP(hipMalloc((void **)&g.I_p, NF * sizeof(double)));
     }
     MGR_HIP(hipMemsetAsync(ctx->err_flag, 0, sizeof(int32_t), ctx->stream));
-    // FP32: the sweep and profiles in FP32, shifts and profile arguments in FP64
-    rc = precision == MGR_FP64 ? launch_image<double, false>(ctx, ctx->row64)
-                               : launch_image<float, true>(ctx, ctx->row32);
+    rc = precision == MGR_FP64 ? launch_image<double>(ctx, ctx->row64) : launch_image<float>(ctx, ctx->row32);
     if (rc) return rc;
     MGR_HIP(hipStreamSynchronize(ctx->stream));
     int32_t errv = 0;
