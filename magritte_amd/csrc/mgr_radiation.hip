@@ -7,8 +7,8 @@
 // (raypair_solver.tpp:200-388, n_off_diag 0 or 1: the same diagonal operator)
 // and RayPair::update_Lambda (raypair_lambda.tpp:94-149); with scattering it
 // also keeps each pair's u (Radiation::u, sim_radiation.tpp:226-262).  The
-// image kernel (Simulation::compute_and_write_image) reuses the same staging
-// and elimination on a rest-frame trace.
+// image kernels (Simulation::compute_and_write_image) run the same elimination
+// along a rest-frame trace.
 //
 // Work mapping (CDNA4, 64-wide wavefronts): one wavefront per origin cell and
 // chunk of 64 frequency bins (lane = bin).  The wave loops over the nrays/2 ray
@@ -27,7 +27,7 @@
 // and recurrences are 19.5 per point and wave, 65 % of all.  Decoding each
 // step in the elimination loop and stepping every point took 49 ms; on the
 // stress envelope (36^3, ~10 points per step) 44 against 19 ms.  FP64: 221
-// against 167 ms and 192 against 105 ms.
+// against 148 ms and 192 against 94 ms.
 //
 // The tridiagonal Feautrier system of a ray pair is solved two-sided: each ray
 // of the pair is eliminated from its boundary inwards in the Rybicki-Hummer
@@ -1033,10 +1033,9 @@ __device__ __forceinline__ void sweep_pair(const RFArgs<real> &a, const LaneCtx<
                     for (int e = e0; e < cw; e += per) {
                         if (!F32 && ((marks >> e) & 1)) continue;
                         const Stage<real> sg_e = win.stage[e];
-                        row_t v = src[(uint32_t)sg_e.cell * (uint32_t)L];   // N L rows < 2^32
-                        if constexpr (F32) v.w = sg_e.s;
-                        else if constexpr (INROW) v.x = sg_e.s;
-                        dst[e] = v;
+                        const row_t v = src[(uint32_t)sg_e.cell * (uint32_t)L];   // N L rows < 2^32
+                        if constexpr (F32) dst[e] = make_float4(v.x, v.y, v.z, sg_e.s);
+                        else dst[e] = make_double4(INROW ? sg_e.s : v.x, v.y, v.z, v.w);
                     }
             }
             wave_lds_fence();
