@@ -2006,6 +2006,25 @@ static int launch_rf_shape(mgr_ctx *ctx, int nwg, int ch, int64_t o_begin, int64
         return launch_rf<float>(ctx, ctx->row32, nwg, ch, o_begin, o_count);
 }
 
+// The largest window whose LDS still admits the waves that the kernel's
+// registers do, 8, 6 or 4 per SIMD: a pair's points take the fewest windows
+// there.  FP32 at 64^3 cells (6 lines, 41 points): 31.4 ms against 31.9 with 32
+// points, and 34.1 with 48, which only 26 waves per CU have room for.
+template <typename real>
+static int fitting_window(mgr_ctx *ctx)
+{
+    constexpr size_t CU_LDS = 160 * 1024, GRANULE = 1280;
+    RFArgs<real> a;
+    const typename Prec<real>::row_t *none = nullptr;
+    if (make_args<real>(ctx, none, 1, 2, 0, 1, ctx->shift_min, ctx->shift_max, a) != MGR_OK) return 2;
+    const size_t waves = 4 * (sizeof(real) == 8 ? 4 : one_line(ctx, a) ? 8 : 6);
+    const size_t room = CU_LDS / waves / GRANULE * GRANULE, table = sizeof(double) * ctx->L;
+    const size_t row = sizeof(typename Prec<real>::row_t) * ctx->L;
+    // a wave's LDS is rounded up to 64 bytes
+    if (room < Window<real>::fixed + table + 64 + 3 * row) return 2;
+    return (int)std::min<size_t>(64, (room - table - Window<real>::fixed) / 64 * 64 / row - 1);
+}
+
 // Launch-shape autotuner: points per window first, with one wave (a 64-bin
 // chunk) per workgroup, then waves per workgroup with the best window.  Timed
 // on two slices of origins, around 1/8 and 5/8 of the model's cells, so that
@@ -2028,8 +2047,8 @@ static int tune(mgr_ctx *ctx, int pi)
     for (int w = 2; w <= MAX_WAVES; w++)
         if (w == nchunk || (nchunk % w) == 0 || w == std::min(nchunk, MAX_WAVES)) nwgs.push_back(w);
     std::vector<int> chs;
-    for (int c : {16, 32, 64})
-        if (c <= chmax) chs.push_back(c);
+    for (int c : {16, fitting_window<real>(ctx), 64})
+        if (c <= chmax && (chs.empty() || c > chs.back())) chs.push_back(c);
     if (chs.empty() || chs.back() != chmax) chs.push_back(chmax);
     const int64_t fill = (WAVES_IN_FLIGHT + nchunk - 1) / nchunk;   // origins that fill the chip
     const int nslice = ctx->N > 2 * fill ? 2 : 1;
