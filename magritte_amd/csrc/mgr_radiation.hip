@@ -168,7 +168,7 @@ struct RFArgs {
 // exp(-t) for t >= 0: reduced by multiples of ln 2, whose double is taken in
 // two parts, to |r| <= ln 2 / 2, and there the polynomial of degree 11 that
 // meets exp at the 12 Chebyshev nodes of that interval (relative error below
-// 1.7e-17), scaled by ldexp; 0 from t = 745 on.  18 instructions, without the
+// 1.7e-17), scaled by ldexp; 0 from t = 745 up to 1e15 at least.  18 instructions, without the
 // range and sign handling of the library's exp.
 __device__ __forceinline__ double exp_neg(double t)
 {
@@ -451,7 +451,7 @@ struct LaneCtx<double> {
     double nu_f;
     int    lstart;
     const double *line;   // line frequencies (a copy in LDS in the field kernel)
-    double nu_l;          // frequency of the bin's only candidate line l (-1e30: none)
+    double nu_l;          // frequency of the bin's only candidate line l (none: one far away)
     int    l;
 };
 
@@ -729,7 +729,7 @@ __device__ __forceinline__ void origin_point(const RFArgs<real> &a, double nu_f,
         lc.lstart = ls;
         if constexpr (ONE) {
             const bool cand = a.tb->line[ls] * a.cand_lo >= nu_f && a.tb->line[ls] * a.cand_hi <= nu_f;
-            lc.nu_l = cand ? a.tb->line[ls] : -1.0e30;
+            lc.nu_l = cand ? a.tb->line[ls] : 0.9 * nu_f;   // 0.1 nu is thousands of widths: exp_neg gives 0
             lc.l = ls;
         }
         if constexpr (ONE) eta_chi_one(lc, orow[ls], 1.0, eta_o, chi_o);

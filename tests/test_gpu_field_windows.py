@@ -102,3 +102,20 @@ def test_populations_beyond_the_spans_bound(scale):
     ctx.compute_radiation_field("fp32")
     assert np.array_equal(ctx.J(), J1) and np.array_equal(ctx.lambda_diag(), L1)
     ctx.close()
+
+
+@pytest.mark.parametrize("name", ["regular", "envelope"])
+def test_fp64_bins_that_meet_no_line(name):
+    """Roots up to 30 widths: the outer bins of a static model have no candidate
+    line at any point, and the FP64 profile must still come out as exactly 0."""
+    from magritte_amd.hip import Context
+    m = (synthetic.regular_grid_model(n=6, nquads=41) if name == "regular" else
+         synthetic.envelope_model(n=6, seed=8, nside=1, nquads=41))
+    m.roots = m.roots * 6.0
+    orc, ctx = Oracle(m).setup(), Context(m).setup()
+    orc.compute_radiation_field()
+    ctx.compute_radiation_field("fp64")
+    J, Jo = ctx.J(), orc.J()
+    assert np.all(np.isfinite(J))
+    assert float(np.max(np.abs(J - Jo) / Jo)) < 1e-10
+    assert np.all(np.isfinite(ctx.lambda_diag()))
