@@ -1584,13 +1584,13 @@ struct RowSweep {
 };
 
 // Thermodynamics::profile (thermodynamics.tpp:16-29) of width `width` at
-// freq_diff, with the reference's scalar 1/exp.
+// freq_diff.
 __device__ __forceinline__ double profile64(double width, double freq_diff)
 {
 #pragma clang fp contract(off)
-    const double iw = 1.0 / width;
+    const double iw = Prec<double>::rcp(width);
     const double x = iw * freq_diff;
-    return iw * INVERSE_SQRT_PI * (1.0 / exp(x * x));
+    return iw * INVERSE_SQRT_PI * exp_neg(x * x);
 }
 
 // The band elements of Lambda* (RayPair::update_Lambda, raypair_lambda.tpp:129-146,
@@ -1614,7 +1614,7 @@ __device__ __forceinline__ double profile64(double width, double freq_diff)
 // (125 VGPRs, 8 KB of LDS).  A walk with per-step scalar loads and divisions in
 // every lane, three rcp per point, five arrays of 3 (nband + 1) points in LDS
 // and butterfly sums per element and transition took 9.5 ms at 20^3 cells, 84
-// bins and one band; this one takes 3.4 ms.
+// bins and one band; this one takes 3.3 ms.
 template <bool ONE>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_lambda_band(RFArgs<double> a)
 {
@@ -1658,7 +1658,7 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4))) void 
     wave_lds_fence();
     double S_o, chi_o;
     origin_point<double, false, ONE>(a, nu_f, a.rows + (int64_t)o * L, lc, S_o, chi_o);
-    const double freq_line = k < L ? a.freq_k[k] : 1.0;
+    const double freq_line = k < L ? a.freq_k[k] : nu_f;
     const double A_k = k < L ? a.A_k[k] : 0.0;
     const double w_z = k < L ? a.qw[a.f_z[fa]] : 0.0;
     const int64_t qb = a.cell_qbase[o];
@@ -1701,7 +1701,7 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4))) void 
                 if (i < 0) {
                     if (i >= -nb && n > 0) {   // lower element of band -i
                         const int at = (-i - 1) * WAVE;
-                        const double T = sw.inverse_C() / (sw.F + termG[at + lane]) * elem[at + lane];
+                        const double T = sw.inverse_C() * Prec<double>::rcp(sw.F + termG[at + lane]) * elem[at + lane];
                         elem[at + pos] = fpc * T;
                     }
                 } else if (i > 0) {
@@ -1714,21 +1714,21 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4))) void 
                     if (m >= 1 && m <= nb) {
                         const int at = (nb + m - 1) * WAVE;
                         if (i & 1) {   // upper element of band m, from row n_ar + 2m + 1
-                            const double T = sw.inverse_C() / (sw.F + termG[at + lane]);
+                            const double T = sw.inverse_C() * Prec<double>::rcp(sw.F + termG[at + lane]);
                             elem[at + pos] = elem[at + lane] * T;
                         } else if (n == last) {   // which is the last row
                             const double c2 = sw.c * sw.c;
-                            const double T = c2 / (c2 + SQRT2 * sw.c + sw.F * sw.q);
+                            const double T = c2 * Prec<double>::rcp(c2 + SQRT2 * sw.c + sw.F * sw.q);
                             elem[at + pos] = elem[at + lane] * T;
                         }
                     }
                 }
-                if (i < nb) {   // nu phi(nu) / chi at the point's own cell and frequency
+                // nu phi(nu) / chi at the point's own cell and frequency, where an element needs it
+                if (i < -1 || (i >= 0 && i < nb && nB > 2 * (i + 1))) {
                     const Stage<double> sg = win.stage[p];
                     const double fs = sg.s * nu_f;
-                    fpc = k < L ? factor * (fs * profile64(freq_line * a.pw[sg.cell], fs - freq_line)) /
-                                      (chi * (1.0 / CHI_SCALE))
-                                : 0.0;
+                    fpc = factor * (fs * profile64(freq_line * a.pw[sg.cell], fs - freq_line)) *
+                          Prec<double>::rcp(chi * (1.0 / CHI_SCALE));
                 }
             });
         }
