@@ -22,15 +22,17 @@
 // walking, keyed per epoch), Adam's step count and the epoch's loss live in
 // device memory, and each epoch is one hipGraph replay.
 //
-// Work mapping: a workgroup of 4 wavefronts takes tiles of 64 rows (cells), a
-// wave 16 of them.  The products are formed transposed, neurons by rows
-// (D = W^T H^T): a lane's results, four consecutive neurons of one row, are
-// then K values of the next product's right operand as they stand.  The M
-// rows of two tiles take the neurons of 32 in alternate fours (neuron), which
-// puts the operand's eight values in order.  So the forward pass and the back-propagation of activations
-// stay in registers.  The weight gradients reduce over rows: the operands are
-// transposed on the matrix cores (a product with the unit matrix, exact) and
-// exchanged through LDS, and each wave forms a quarter of the gradients over
+// Work mapping: the products are formed transposed, neurons by rows
+// (D = W^T H^T), 16 rows (cells) to a wavefront: a lane's results, four
+// consecutive neurons of one row, are then K values of the next product's
+// right operand as they stand.  The M rows of two tiles take the neurons of 32
+// in alternate fours (neuron), which puts the operand's eight values in order.
+// Prediction: a wave's rows stay in its registers from the inputs to the outputs.
+// Training: a workgroup takes tiles of 64 rows with 8 waves, two for the same 16
+// rows, which form one half of the neurons each and hand each other their
+// operands through LDS.  The weight gradients reduce over rows: their operands
+// are transposed on the matrix cores (a product with the unit matrix, exact)
+// and pass through LDS too, and each wave forms an eighth of the gradients over
 // the 64 rows, accumulating in registers over all the tiles a workgroup takes.
 // Per-workgroup partial gradients are reduced in a fixed order by the Adam
 // kernel, so training is deterministic.
@@ -56,7 +58,8 @@ constexpr int OUT = MGR_MLP_OUT;      // 7 levels
 constexpr int KIN = 16;               // IN padded to one MFMA K step
 constexpr int NOUT = 16;              // OUT padded to one MFMA N tile
 constexpr int ROWS = 64;              // rows per workgroup tile
-constexpr int THREADS = 256;
+constexpr int THREADS = 256;           // of the forward kernel
+constexpr int GRAD_THREADS = 512;      // of the gradient kernel
 
 // packed FP32 parameters: W1 [IN][HID], b1, W2 [HID][HID], b2, W3 [HID][OUT], b3
 constexpr int OFF_W1 = 0;
@@ -95,19 +98,22 @@ __device__ __forceinline__ int neuron_row(int u) { return (u / 32 * 2 + u % 8 / 
 
 // Partial gradients of a workgroup: the words as the threads hold them, so that
 // they are written whole, with the loss at NPAR
-//   W2 [q][ot][thread][4], W1 [q][wave][g < 2][r][4], W3 [q][wave][g][r < OUT][4], b1, b2, b3
+//   W2 [q][i][thread][4], W1 [wave][g < 2][r][4], W3 [wave][g][r < OUT][4], b1, b2, b3
 constexpr int PG_W1 = HID * HID;
 constexpr int PG_W3 = PG_W1 + IN * HID;
 constexpr int PG_B = PG_W3 + HID * OUT;
 
-// LDS of the training kernel: the weights, the biases, and the transposed
-// operands of the weight gradients, tile t of two waves' 32 rows at
-// ((t 2 + wave / 2) 64 + lane) 8 + (wave % 2) 4
+// LDS of the training kernel, 160 KB: the weights; the transposed operands of the
+// weight gradients, tile t of two waves' 32 rows at ((t 2 + rows / 32) 64 + lane) 8
+// + (rows / 16 % 2) 4; and one layer's right operands of the next product, K step
+// kt of rows / 16 at ((rows / 16 4 + kt) 64 + lane) 8 (layer 2's pass through
+// the tiles T_DZ1, which are written last)
 constexpr int T_H1 = 0, T_DZ2 = 8, T_H2 = 16, T_DZ1 = 24, T_X = 32, T_DY = 33, T_TILES = 34;
+constexpr int L_TILES = BF_TOTAL;                       // bf16 elements before the tiles
+constexpr int L_PASS = L_TILES + T_TILES * 2 * 64 * 8;
+constexpr size_t LDS_TRAIN = (size_t)(L_PASS + ROWS * HID) * 2;
+static_assert(LDS_TRAIN <= 160 * 1024, "a CU's LDS");
 constexpr int NBIAS = HID + HID + NOUT;
-constexpr size_t LDS_BIAS = (size_t)BF_TOTAL * 2;                  // bytes before the biases
-constexpr size_t LDS_TILES = LDS_BIAS + NBIAS * sizeof(float);
-constexpr size_t LDS_TRAIN = LDS_TILES + (size_t)T_TILES * 2 * 64 * 16;   // 148,544 bytes
 constexpr size_t LDS_FORWARD = (size_t)BF_FORWARD * 2 + NBIAS * sizeof(float) + ROWS * NOUT * sizeof(float);
 
 typedef short s4 __attribute__((ext_vector_type(4)));
@@ -229,31 +235,28 @@ __device__ __forceinline__ int param_of(int e)
 {
     const int j = e % 4;
     if (e < PG_W1) {
-        const int lane = e / 4 % 64, wave = e / 256 % 4, ot = e / 1024 % 8, q = e / 8192;
-        return OFF_W2 + neuron(2 * wave + q, lane / 16 * 4 + j) * HID + neuron(ot, lane % 16);
+        const int lane = e / 4 % 64, wave = e / 256 % 8, i = e / 2048 % 4, q = e / 8192;
+        return OFF_W2 + neuron(wave % 4 * 2 + q, lane / 16 * 4 + j) * HID + neuron(wave / 4 * 4 + i, lane % 16);
     }
     if (e < PG_W3) {
-        const int i = (e - PG_W1) / 4, lane = i % 32, wave = i / 32 % 4, q = i / 128;
-        return OFF_W1 + (lane / 16 * 4 + j) * HID + neuron(2 * wave + q, lane % 16);
+        const int i = (e - PG_W1) / 4, lane = i % 32, wave = i / 32;
+        return OFF_W1 + (lane / 16 * 4 + j) * HID + neuron(wave, lane % 16);
     }
     if (e < PG_B) {
-        const int i = (e - PG_W3) / 4, r = i % OUT, g = i / OUT % 4, wave = i / (4 * OUT) % 4, q = i / (16 * OUT);
-        return OFF_W3 + neuron(2 * wave + q, 4 * g + j) * OUT + r;
+        const int i = (e - PG_W3) / 4, r = i % OUT, g = i / OUT % 4, wave = i / (4 * OUT);
+        return OFF_W3 + neuron(wave, 4 * g + j) * OUT + r;
     }
     const int b = e - PG_B;
     return b < HID ? OFF_B1 + b : b < 2 * HID ? OFF_B2 + b - HID : OFF_B3 + b - 2 * HID;
 }
 
-// Copy the first `total` bf16 weights and the biases (outputs padded) into LDS.
-__device__ __forceinline__ void load_weights(uint16_t *s, float *sB, const uint16_t *__restrict__ wbf,
-                                             const float *__restrict__ P, int total)
+// Copy the first `total` bf16 weights into LDS.
+__device__ __forceinline__ void load_weights(uint16_t *s, const uint16_t *__restrict__ wbf, int total)
 {
     const uint4 *src = reinterpret_cast<const uint4 *>(wbf);
     uint4 *dst = reinterpret_cast<uint4 *>(s);
 #pragma unroll 10
-    for (int i = threadIdx.x; i < total / 8; i += THREADS) dst[i] = src[i];
-    for (int i = threadIdx.x; i < NBIAS; i += THREADS)
-        sB[i] = i < HID ? P[OFF_B1 + i] : i < 2 * HID ? P[OFF_B2 + i - HID] : i - 2 * HID < OUT ? P[OFF_B3 + i - 2 * HID] : 0.0f;
+    for (int i = threadIdx.x; i < total / 8; i += blockDim.x) dst[i] = src[i];
 }
 
 // The lane's inputs 4g .. 4g+3 normalised, as right operand: zeros in the
@@ -264,52 +267,52 @@ __device__ __forceinline__ s4 input_operand(f4 x, bool valid, f4 xm, f4 xs)
     return to_bf(valid ? v : f4{0.f, 0.f, 0.f, 0.f});
 }
 
-// Forward pass of the 16 rows of one wave, row r of lane (r, g) and neurons
-// neuron(mt, 4g + j): the activations, as operands of the next product, and the
-// derivatives of GELU go to layer1 and layer2, the outputs 4g + j are returned.
-template <typename Layer1, typename Layer2>
-__device__ __forceinline__ f4 forward_rows(const uint16_t *s, const float *sB, s4 x, Layer1 &&layer1, Layer2 &&layer2)
+// GELU of four pre-activations as an operand, and its derivatives.
+__device__ __forceinline__ s4 activate(f4 z, f4 &grad)
 {
-    s4 h1[8], h2[8];
+    f4 h;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        float hj, dj;
+        gelu(z[j], hj, dj);
+        h[j] = hj;
+        grad[j] = dj;
+    }
+    return to_bf(h);
+}
+
+// A K = 128 product of one M tile: its four operands w ((kt 64 + lane) 8) by b.
+__device__ __forceinline__ f4 product(const uint16_t *w, const s8 b[4])
+{
+    const int lane = threadIdx.x & 63;
+    f4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kt = 0; kt < 4; kt++) z = mfma32(ld8(w + (kt * 64 + lane) * 8), b[kt], z);
+    return z;
+}
+
+// Outputs 4g + j of the 16 rows of one wave, row r of lane (r, g), with biases sB.
+__device__ __forceinline__ f4 forward_rows(const uint16_t *s, const float *sB, s4 x)
+{
     const int lane = threadIdx.x & 63, g = lane >> 4;
+    f4 none;
+    s4 h[8];
+    s8 b[4];
 #pragma unroll
-    for (int mt = 0; mt < 8; mt++) {
-        const f4 z = mfma(ld4(s + BF_W1F + (mt * 64 + lane) * 4), x, f4{0.f, 0.f, 0.f, 0.f}) +
-                     *reinterpret_cast<const f4 *>(sB + neuron(mt, 4 * g));
-        f4 h, d;
+    for (int mt = 0; mt < 8; mt++)
+        h[mt] = activate(mfma(ld4(s + BF_W1F + (mt * 64 + lane) * 4), x, f4{0.f, 0.f, 0.f, 0.f}) +
+                             *reinterpret_cast<const f4 *>(sB + neuron(mt, 4 * g)),
+                         none);
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            float hj, dj;
-            gelu(z[j], hj, dj);
-            h[j] = hj;
-            d[j] = dj;
-        }
-        h1[mt] = to_bf(h);
-        layer1(mt, h1[mt], d);
-    }
+    for (int kt = 0; kt < 4; kt++) b[kt] = join(h[2 * kt], h[2 * kt + 1]);
 #pragma unroll
-    for (int mt = 0; mt < 8; mt++) {
-        f4 z = {0.f, 0.f, 0.f, 0.f};
+    for (int mt = 0; mt < 8; mt++)
+        h[mt] = activate(product(s + BF_W2F + mt * 4 * 64 * 8, b) +
+                             *reinterpret_cast<const f4 *>(sB + HID + neuron(mt, 4 * g)),
+                         none);
 #pragma unroll
-        for (int kt = 0; kt < 4; kt++)
-            z = mfma32(ld8(s + BF_W2F + ((mt * 4 + kt) * 64 + lane) * 8), join(h1[2 * kt], h1[2 * kt + 1]), z);
-        z += *reinterpret_cast<const f4 *>(sB + HID + neuron(mt, 4 * g));
-        f4 h, d;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            float hj, dj;
-            gelu(z[j], hj, dj);
-            h[j] = hj;
-            d[j] = dj;
-        }
-        h2[mt] = to_bf(h);
-        layer2(mt, h2[mt], d);
-    }
-    f4 y = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kt = 0; kt < 4; kt++)
-        y = mfma32(ld8(s + BF_W3F + (kt * 64 + lane) * 8), join(h2[2 * kt], h2[2 * kt + 1]), y);
-    return y + *reinterpret_cast<const f4 *>(sB + 2 * HID + 4 * g);
+    for (int kt = 0; kt < 4; kt++) b[kt] = join(h[2 * kt], h[2 * kt + 1]);
+    return product(s + BF_W3F, b) + *reinterpret_cast<const f4 *>(sB + 2 * HID + 4 * g);
 }
 
 // Loss and gradients over rows [0, n) of a batch of X/T (rows b0 .. b0+n-1 of
@@ -317,52 +320,48 @@ __device__ __forceinline__ f4 forward_rows(const uint16_t *s, const float *sB, s
 // rows themselves): grid-stride over 64-row tiles; per-workgroup partial
 // gradients (PG_W1) and partial loss go to part[blockIdx.x * (NPAR + 1)].
 //
-// Bound by vector instructions, most of them the GELUs', at one wave per SIMD
-// (9 us per tile), and per launch by the weights' way into LDS and the 74 KB of
-// partial gradients (7 us alone, 16 with a workgroup on every CU).  With activations in row-major LDS (16-way bank
-// conflicts on every operand) and gradient operands gathered two bytes at a
-// time a 16384-row batch took 40 us and 400000 rows 590 us; here 24 and
-// 250.
-__global__ __launch_bounds__(THREADS, 1) void k_mlp_grad(const float *__restrict__ X, const float *__restrict__ T,
-                                                         const TrainState *st, const int64_t *__restrict__ idx,
-                                                         int64_t b0, int64_t n, int64_t n_total,
-                                                         const uint16_t *__restrict__ wbf, const float *__restrict__ P,
-                                                         const Norm *__restrict__ norm, float *__restrict__ part)
+// Bound by vector instructions, most of them the GELUs', and per launch by the
+// weights' way into LDS and the 74 KB of partial gradients.  With activations in
+// row-major LDS (16-way bank conflicts on every operand) and gradient operands
+// gathered two bytes at a time a 16384-row batch took 40 us and 400000 rows 590
+// us; with 4 waves that hold all 128 neurons of their rows (413 registers, of
+// which the upper half is moved in and out) 24 and 251; here 22 and 215.
+__global__ __launch_bounds__(GRAD_THREADS) void k_mlp_grad(const float *__restrict__ X, const float *__restrict__ T,
+                                                           const TrainState *st, const int64_t *__restrict__ idx,
+                                                           int64_t b0, int64_t n, int64_t n_total,
+                                                           const uint16_t *__restrict__ wbf,
+                                                           const float *__restrict__ P,
+                                                           const Norm *__restrict__ norm, float *__restrict__ part)
 {
     extern __shared__ __align__(16) uint16_t s[];
-    float *sB = reinterpret_cast<float *>(reinterpret_cast<char *>(s) + LDS_BIAS);
-    uint16_t *sT = reinterpret_cast<uint16_t *>(reinterpret_cast<char *>(s) + LDS_TILES);
+    uint16_t *sT = s + L_TILES, *pass = s + L_PASS, *pass2 = sT + T_DZ1 * 2 * 64 * 8;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int rb = wave & 3, mt0 = wave / 4 * 4;   // the wave's 16 rows and its first tile of neurons
     const float inv = 2.0f / ((float)n_total * (float)OUT);
-    f4 xm{}, xs{1.f, 1.f, 1.f, 1.f}, ym{}, ys{1.f, 1.f, 1.f, 1.f};
-    for (int j = 0; j < 4; j++) {
-        if (g < 2) {
-            xm[j] = norm->xm[4 * g + j];
-            xs[j] = norm->xs[4 * g + j];
-        }
-        if (4 * g + j < OUT) {
-            ym[j] = norm->ym[4 * g + j];
-            ys[j] = norm->ys[4 * g + j];
-        }
-    }
     s4 unit;   // the unit matrix as right operand
     for (int j = 0; j < 4; j++) unit[j] = 4 * g + j == r ? 0x3F80 : 0;
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
     auto put = [&](int t, s4 operand) {
-        const f4 zero = {0.f, 0.f, 0.f, 0.f};
         // rows 4g + j of neuron r: exact, the values are bf16
         const s4 v = to_bf(mfma(operand, unit, zero));
-        *reinterpret_cast<s4 *>(sT + ((t * 2 + (wave >> 1)) * 64 + lane) * 8 + (wave & 1) * 4) = v;
+        *reinterpret_cast<s4 *>(sT + ((t * 2 + (rb >> 1)) * 64 + lane) * 8 + (rb & 1) * 4) = v;
     };
     auto get = [&](int t, int p) { return ld8(sT + ((t * 2 + p) * 64 + lane) * 8); };
+    // this wave's half of a layer to the rows' two waves, and the whole of it
+    auto give = [&](uint16_t *to, const s4 h[4]) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            *reinterpret_cast<s8 *>(to + ((rb * 4 + mt0 / 2 + i) * 64 + lane) * 8) = join(h[2 * i], h[2 * i + 1]);
+    };
+    auto take = [&](const uint16_t *from, s8 b[4]) {
+#pragma unroll
+        for (int kt = 0; kt < 4; kt++) b[kt] = ld8(from + ((rb * 4 + kt) * 64 + lane) * 8);
+    };
 
-    f4 gW2[2][8], gW1[2], gW3[2];
+    f4 gW2[2][4], gW1 = zero, gW3 = zero;
 #pragma unroll
-    for (int q = 0; q < 2; q++) {
-        gW1[q] = gW3[q] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int t = 0; t < 8; t++) gW2[q][t] = gW1[q];
-    }
-    float gb = 0.0f, gb3 = 0.0f, loss = 0.0f;
+    for (int i = 0; i < 4; i++) gW2[0][i] = gW2[1][i] = zero;
+    float gb = 0.0f, loss = 0.0f;
     // the sum of a transposed operand's column m over the tile's rows, in their order
     auto column = [&](int t, int m, float sum) {
 #pragma unroll
@@ -372,15 +371,17 @@ __global__ __launch_bounds__(THREADS, 1) void k_mlp_grad(const float *__restrict
         }
         return sum;
     };
-    const int column_row = neuron_row(threadIdx.x % HID);   // bias gradients: dZ1 of threads 0..127, dZ2 of the others
-    const int column_tile = (threadIdx.x < HID ? T_DZ1 : T_DZ2) + column_row / 16;
+    // bias gradients: dZ1 of threads 0..127, dZ2 of 128..255, dY of wave 4
+    const int column_row = neuron_row(threadIdx.x % HID);
+    const int column_tile = wave == 4 ? T_DY : (threadIdx.x < HID ? T_DZ1 : T_DZ2) + column_row / 16;
+    const int column_m = wave == 4 ? r : column_row % 16;
 
     // a tile's inputs and targets are read before the weights, or the tile before, are dealt with
-    f4 next_x = xm, next_t = ym;
+    f4 next_x = zero, next_t = zero;
     bool next_valid = false;
     auto fetch = [&](int64_t tile) {
         // the rows of two waves alternate in fours, as the neurons of two tiles do
-        const int64_t row = tile * ROWS + neuron(wave, r);
+        const int64_t row = tile * ROWS + neuron(rb, r);
         next_valid = row < n;
         if (!next_valid || g > 1) return;
         const int64_t src = source_row(st, idx, b0, row);
@@ -389,87 +390,98 @@ __global__ __launch_bounds__(THREADS, 1) void k_mlp_grad(const float *__restrict
             if (4 * g + j < OUT) next_t[j] = T[src * OUT + 4 * g + j];
     };
     fetch(blockIdx.x);
-    load_weights(s, sB, wbf, P, BF_TOTAL);
+    load_weights(s, wbf, BF_TOTAL);
 
     const int64_t ntiles = (n + ROWS - 1) / ROWS;
     for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        // the biases and the normalisation are read again for every tile (out of
+        // the cache): kept in registers they would push others out to memory
+        const float *Pt = P;
+        const Norm *nt = norm;
+        asm volatile("" : "+s"(Pt), "+s"(nt));
+        auto bias = [&](int layer, int i) {
+            return *reinterpret_cast<const f4 *>(Pt + layer + neuron(mt0 + i, 4 * g));
+        };
         const bool valid = next_valid && g < 2;
-        const s4 x = input_operand(next_x, valid, xm, xs);
-        const f4 t = next_t;
+        f4 xn = next_x, t = next_t;   // normalised
+        for (int j = 0; j < 4; j++) {
+            if (g < 2) xn[j] = (xn[j] - nt->xm[4 * g + j]) / nt->xs[4 * g + j];
+            if (4 * g + j < OUT) t[j] = (t[j] - nt->ym[4 * g + j]) / nt->ys[4 * g + j];
+        }
+        const s4 x = to_bf(valid ? xn : zero);
         __syncthreads();   // the weights are in place, the previous tile's operands consumed
         fetch(tile + gridDim.x);
-        f4 g1[8], g2[8];
-        const f4 y = forward_rows(
-            s, sB, x,
-            [&](int mt, s4 h, f4 d) {
-                g1[mt] = d;
-                put(T_H1 + mt, h);
-            },
-            [&](int mt, s4 h, f4 d) {
-                g2[mt] = d;
-                put(T_H2 + mt, h);
-            });
+        s4 h[4];
+        s8 b[4];
+        f4 g1[4], g2[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            h[i] = activate(mfma(ld4(s + BF_W1F + ((mt0 + i) * 64 + lane) * 4), x, zero) + bias(OFF_B1, i), g1[i]);
+            put(T_H1 + mt0 + i, h[i]);
+        }
+        give(pass, h);
+        __syncthreads();
+        take(pass, b);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            h[i] = activate(product(s + BF_W2F + (mt0 + i) * 4 * 64 * 8, b) + bias(OFF_B2, i), g2[i]);
+            put(T_H2 + mt0 + i, h[i]);
+        }
+        give(pass2, h);
+        __syncthreads();
+        take(pass2, b);
+        const f4 y = product(s + BF_W3F, b);
         // dY = 2 (y - t) / (n_total OUT) on valid rows and outputs
-        f4 d = {0.f, 0.f, 0.f, 0.f};
+        f4 d = zero;
         for (int j = 0; j < 4; j++)
             if (valid && 4 * g + j < OUT) {
-                const float e = y[j] - (t[j] - ym[j]) / ys[j];
-                loss += e * e;
+                const float e = y[j] + Pt[OFF_B3 + 4 * g + j] - t[j];
+                if (wave < 4) loss += e * e;
                 d[j] = e * inv;
             }
         const s4 dy = to_bf(d);
-        put(T_X, x);
-        put(T_DY, dy);
+        if (wave < 4) put(T_X, x);
+        else put(T_DY, dy);
         // dH2 = dY W3^T, dZ2 = dH2 * gelu'(Z2)
-        s4 dz2[8];
 #pragma unroll
-        for (int mt = 0; mt < 8; mt++) {
-            const f4 zero = {0.f, 0.f, 0.f, 0.f};
-            dz2[mt] = to_bf(mfma(ld4(s + BF_W3B + (mt * 64 + lane) * 4), dy, zero) * g2[mt]);
-            put(T_DZ2 + mt, dz2[mt]);
+        for (int i = 0; i < 4; i++) {
+            h[i] = to_bf(mfma(ld4(s + BF_W3B + ((mt0 + i) * 64 + lane) * 4), dy, zero) * g2[i]);
+            put(T_DZ2 + mt0 + i, h[i]);
         }
+        give(pass, h);
+        __syncthreads();
+        take(pass, b);
         // dH1 = dZ2 W2^T, dZ1 = dH1 * gelu'(Z1)
 #pragma unroll
-        for (int mt = 0; mt < 8; mt++) {
-            f4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kt = 0; kt < 4; kt++)
-                acc = mfma32(ld8(s + BF_W2B + ((mt * 4 + kt) * 64 + lane) * 8), join(dz2[2 * kt], dz2[2 * kt + 1]), acc);
-            put(T_DZ1 + mt, to_bf(acc * g1[mt]));
-        }
+        for (int i = 0; i < 4; i++)
+            put(T_DZ1 + mt0 + i, to_bf(product(s + BF_W2B + (mt0 + i) * 4 * 64 * 8, b) * g1[i]));
         __syncthreads();
-        // the gradients of neurons 32 wave .. 32 wave + 31 (of layer 1 for W2) over the tile's rows
+        // an eighth of the gradients over the tile's rows: W2 of 32 neurons by 64, W1 and W3 of 16
 #pragma unroll
         for (int p = 0; p < 2; p++) {
-            const s8 xt = get(T_X, p), dyt = get(T_DY, p);
-            const s8 h0 = get(T_H1 + 2 * wave, p), h1t = get(T_H1 + 2 * wave + 1, p);
+            const s8 ha = get(T_H1 + 2 * rb, p), hb = get(T_H1 + 2 * rb + 1, p);
 #pragma unroll
-            for (int ot = 0; ot < 8; ot++) {
-                const s8 dz = get(T_DZ2 + ot, p);
-                gW2[0][ot] = mfma32(h0, dz, gW2[0][ot]);
-                gW2[1][ot] = mfma32(h1t, dz, gW2[1][ot]);
+            for (int i = 0; i < 4; i++) {
+                const s8 dz = get(T_DZ2 + mt0 + i, p);
+                gW2[0][i] = mfma32(ha, dz, gW2[0][i]);
+                gW2[1][i] = mfma32(hb, dz, gW2[1][i]);
             }
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                gW1[q] = mfma32(xt, get(T_DZ1 + 2 * wave + q, p), gW1[q]);
-                gW3[q] = mfma32(get(T_H2 + 2 * wave + q, p), dyt, gW3[q]);
-            }
+            gW1 = mfma32(get(T_X, p), get(T_DZ1 + wave, p), gW1);
+            gW3 = mfma32(get(T_H2 + wave, p), get(T_DY, p), gW3);
         }
-        gb = column(column_tile, column_row % 16, gb);
-        if (wave == 3) gb3 = column(T_DY, r, gb3);
+        if (wave < 5) gb = column(column_tile, column_m, gb);
     }
 
     float *out = part + (int64_t)blockIdx.x * (NPAR + 1);
 #pragma unroll
-    for (int q = 0; q < 2; q++) {
+    for (int q = 0; q < 2; q++)
 #pragma unroll
-        for (int ot = 0; ot < 8; ot++)
-            *reinterpret_cast<f4 *>(out + ((q * 8 + ot) * THREADS + threadIdx.x) * 4) = gW2[q][ot];
-        if (g < 2) *reinterpret_cast<f4 *>(out + PG_W1 + ((q * 4 + wave) * 32 + lane) * 4) = gW1[q];
-        if (r < OUT) *reinterpret_cast<f4 *>(out + PG_W3 + (((q * 4 + wave) * 4 + g) * OUT + r) * 4) = gW3[q];
-    }
-    out[PG_B + threadIdx.x] = gb;
-    if (wave == 3 && g == 0 && r < OUT) out[PG_B + 2 * HID + r] = gb3;
+        for (int i = 0; i < 4; i++)
+            *reinterpret_cast<f4 *>(out + ((q * 4 + i) * GRAD_THREADS + threadIdx.x) * 4) = gW2[q][i];
+    if (g < 2) *reinterpret_cast<f4 *>(out + PG_W1 + (wave * 32 + lane) * 4) = gW1;
+    if (r < OUT) *reinterpret_cast<f4 *>(out + PG_W3 + ((wave * 4 + g) * OUT + r) * 4) = gW3;
+    if (wave < 4) out[PG_B + threadIdx.x] = gb;
+    if (wave == 4 && g == 0 && r < OUT) out[PG_B + 2 * HID + r] = gb;
     // loss: wave sums, then one lane adds the waves' in order
     for (int off = 32; off > 0; off >>= 1) loss += __shfl_down(loss, off, 64);
     __syncthreads();   // the operands are consumed
@@ -562,7 +574,12 @@ __global__ __launch_bounds__(THREADS) void k_mlp_forward(const float *__restrict
     extern __shared__ __align__(16) uint16_t s[];
     float *sB = reinterpret_cast<float *>(s + BF_FORWARD);
     float(*sy)[NOUT] = reinterpret_cast<float(*)[NOUT]>(sB + NBIAS);
-    load_weights(s, sB, wbf, P, BF_FORWARD);
+    load_weights(s, wbf, BF_FORWARD);
+    for (int i = threadIdx.x; i < NBIAS; i += THREADS)
+        sB[i] = i < HID           ? P[OFF_B1 + i]
+                : i < 2 * HID     ? P[OFF_B2 + i - HID]
+                : i < 2 * HID + OUT ? P[OFF_B3 + i - 2 * HID]
+                                  : 0.0f;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     f4 xm{}, xs{1.f, 1.f, 1.f, 1.f}, ym{}, ys{};
     for (int j = 0; j < 4; j++) {
@@ -581,7 +598,7 @@ __global__ __launch_bounds__(THREADS) void k_mlp_forward(const float *__restrict
         const bool valid = row < n && g < 2;
         const s4 x = input_operand(valid ? *reinterpret_cast<const f4 *>(X + row * IN + 4 * g) : xm, valid, xm, xs);
         __syncthreads();   // the weights are in place, the previous tile's outputs read
-        const f4 y = forward_rows(s, sB, x, [](int, s4, f4) {}, [](int, s4, f4) {});
+        const f4 y = forward_rows(s, sB, x);
         for (int j = 0; j < 4; j++) {
             const int i = 4 * g + j;
             const float v = y[j] * ys[j] + ym[j];
@@ -853,7 +870,7 @@ extern "C" int mgr_mlp_forward(mgr_mlp *mlp, const float *X, int64_t n, float *Y
 static int mlp_grad_device(mgr_mlp *mlp, const float *dX, const float *dT, int64_t n, float *dpart, int G,
                            float *dgrad)
 {
-    hipLaunchKernelGGL(k_mlp_grad, dim3(G), dim3(THREADS), LDS_TRAIN, mlp->stream, dX, dT,
+    hipLaunchKernelGGL(k_mlp_grad, dim3(G), dim3(GRAD_THREADS), LDS_TRAIN, mlp->stream, dX, dT,
                        (const TrainState *)nullptr, (const int64_t *)nullptr, (int64_t)0, n, n, mlp->wbf, mlp->P,
                        mlp->norm, dpart);
     MLP_HIP(hipGetLastError());
@@ -930,7 +947,7 @@ extern "C" int mgr_mlp_train(mgr_mlp *mlp, const float *X, const float *T, int64
         for (int64_t b = 0; b < nbatch; b++) {
             const int64_t b0 = b * batch, nb = std::min(batch, n - b0);
             const int G = grid_for_rows(nb, GRAD_GROUPS);
-            hipLaunchKernelGGL(k_mlp_grad, dim3(G), dim3(THREADS), LDS_TRAIN, mlp->stream, dX, dT,
+            hipLaunchKernelGGL(k_mlp_grad, dim3(G), dim3(GRAD_THREADS), LDS_TRAIN, mlp->stream, dX, dT,
                                (const TrainState *)dst, (const int64_t *)nullptr, b0, nb, nb, mlp->wbf, mlp->P,
                                mlp->norm, dpart);
             hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((NPAR + 1 + RED_P - 1) / RED_P), dim3(RED_P * RED_W), 0,
