@@ -58,7 +58,7 @@ constexpr int WAVE = 64;                 // CDNA wavefront width
 // the FP32 profile exp2(-x^2 log2 e) is then exactly zero, since x >= 10.5
 // gives exp2 of less than -159, below the smallest denormal 2^-149 (zero from
 // x > 10.2; the FP32 rounding of x is ~1e-6 widths).
-constexpr int STEP_N_MASK = 0x3FFF, STEP_HALF_SHIFT = 14, STEP_HALF_MASK = 0x1FFF, STEP_OUT_SHIFT = 27;
+constexpr int STEP_N_MASK = 0x3FFF, STEP_HALF_SHIFT = 14, STEP_HALF_MASK = 0x1FFF;
 constexpr int STEP_MASK_CHUNKS = 5;
 constexpr double MASK_WINDOW = 10.5;
 // The FP64 kernel's bits: more than 11 (1 + 1e-6) widths from every line, so

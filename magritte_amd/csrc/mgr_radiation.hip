@@ -540,33 +540,34 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_far_cache(RFArgs<float> a, int Rmax, T *__restrict__ out,
                                                    int32_t *__restrict__ err_flag)
 {
-    const int64_t e = (int64_t)blockIdx.x * (blockDim.x / WAVE) + rfl_int((int)(threadIdx.x / WAVE));
-    if (e >= a.N * Rmax) return;
-    const int32_t o = (int32_t)(e / Rmax);
-    const int r = (int)(e - (int64_t)o * Rmax);
-    if (r >= a.m_R[a.cell_model[o]]) return;
-    const int64_t q = a.cell_qbase[o] + r;
     const int F = a.F;
     const int lane = (int)(threadIdx.x & (WAVE - 1));
-    T *dst = out + q * F;
-    const int32_t cf = a.far_cell[q];
-    const int32_t b = cf < 0 ? -1 : a.cell2bdy[cf];
-    if (b < 0) {   // no points (0), or a far cell off the boundary (0 and an error)
-        if (cf >= 0 && lane == 0) atomicOr(err_flag, ERR_NOT_BOUNDARY);
-        for (int f = lane; f < F; f += WAVE) dst[f] = (T)(0.0 * I_SCALE);
-        return;
-    }
-    const double fsh = a.far_shift[q];
-    const double *nup = a.nu + (int64_t)cf * F;
-    const double *Ib = a.I_bdy + (int64_t)b * F;
-    const double *nuo = a.nu + (int64_t)o * F;
-    for (int f = lane; f < F; f += WAVE) {
-        double fs;
-        {
-#pragma clang fp contract(off)
-            fs = fsh * nuo[f];
+    const int64_t first = (int64_t)blockIdx.x * (blockDim.x / WAVE) + rfl_int((int)(threadIdx.x / WAVE));
+    for (int64_t e = first; e < a.N * Rmax; e += (int64_t)gridDim.x * (blockDim.x / WAVE)) {
+        const int32_t o = (int32_t)(e / Rmax);
+        const int r = (int)(e - (int64_t)o * Rmax);
+        if (r >= a.m_R[a.cell_model[o]]) continue;
+        const int64_t q = a.cell_qbase[o] + r;
+        T *dst = out + q * F;
+        const int32_t cf = a.far_cell[q];
+        const int32_t b = cf < 0 ? -1 : a.cell2bdy[cf];
+        if (b < 0) {   // no points (0), or a far cell off the boundary (0 and an error)
+            if (cf >= 0 && lane == 0) atomicOr(err_flag, ERR_NOT_BOUNDARY);
+            for (int f = lane; f < F; f += WAVE) dst[f] = (T)(0.0 * I_SCALE);
+            continue;
         }
-        dst[f] = (T)(rescale_I_bdy(nup, Ib, F, fs) * I_SCALE);
+        const double fsh = a.far_shift[q];
+        const double *nup = a.nu + (int64_t)cf * F;
+        const double *Ib = a.I_bdy + (int64_t)b * F;
+        const double *nuo = a.nu + (int64_t)o * F;
+        for (int f = lane; f < F; f += WAVE) {
+            double fs;
+            {
+#pragma clang fp contract(off)
+                fs = fsh * nuo[f];
+            }
+            dst[f] = (T)(rescale_I_bdy(nup, Ib, F, fs) * I_SCALE);
+        }
     }
 }
 
@@ -2333,8 +2334,10 @@ int launch_far_cache(mgr_ctx *ctx, int precision)
     a.I_bdy = ctx->I_bdy;
     a.far_cell = ctx->far_cell;
     a.far_shift = ctx->far_shift;
-    const int64_t entries = ctx->N * ctx->R;   // one wave each, four to a workgroup
-    const dim3 grid((unsigned)((entries + 3) / 4));
+    // one wave per entry, four to a workgroup; a launch holds fewer than 2^32
+    // threads, larger models' waves take several entries
+    const int64_t entries = ctx->N * ctx->R;
+    const dim3 grid((unsigned)std::min<int64_t>((entries + 3) / 4, 1 << 23));
     MGR_HIP(hipMemsetAsync(ctx->err_flag, 0, sizeof(int32_t), ctx->stream));
     if (pi)
         hipLaunchKernelGGL(k_far_cache<double>, grid, dim3(256), 0, ctx->stream, a, (int)ctx->R, ctx->far_I64,
