@@ -923,6 +923,16 @@ hipError_t mgr::block_malloc(mgr_ctx *ctx, void **p, size_t bytes)
     }
 }
 
+size_t mgr::blocks_kept(const mgr_ctx *ctx)
+{
+    Blocks &b = Blocks::get();
+    std::lock_guard<std::mutex> lock(b.m);
+    size_t bytes = 0;
+    for (const auto &k : b.kept)
+        if (k.device == ctx->device) bytes += k.bytes;
+    return bytes;
+}
+
 void mgr::block_free(mgr_ctx *ctx, void *p)
 {
     if (!p) return;

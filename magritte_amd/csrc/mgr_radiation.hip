@@ -2313,8 +2313,12 @@ int launch_far_cache(mgr_ctx *ctx, int precision)
     void **buf = pi ? (void **)&ctx->far_I64 : (void **)&ctx->far_I32;
     const size_t bytes = (size_t)ctx->NQ * (size_t)ctx->F * (pi ? sizeof(double) : sizeof(float));
     if (!*buf) {
+        // of the memory free without the spans, which are worth less, and kept blocks
         size_t fr = 0, tot = 0;
-        if (hipMemGetInfo(&fr, &tot) != hipSuccess || bytes > fr / 4 * 3 ||
+        const int64_t nspan = std::min<int64_t>((ctx->F + WAVE - 1) / WAVE, STEP_MASK_CHUNKS) *
+                              ((ctx->span32 ? 1 : 0) + (ctx->span64 ? 1 : 0));
+        const size_t spans = (size_t)(nspan * ctx->span_stride) * sizeof(uint16_t);
+        if (hipMemGetInfo(&fr, &tot) != hipSuccess || bytes > (fr + spans + blocks_kept(ctx)) / 4 * 3 ||
             block_malloc(ctx, buf, std::max<size_t>(bytes, 8)) != hipSuccess) {
             (void)hipGetLastError();
             *buf = nullptr;
