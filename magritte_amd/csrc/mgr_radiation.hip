@@ -2012,12 +2012,9 @@ static int launch_rf_shape(mgr_ctx *ctx, int nwg, int ch, int64_t o_begin, int64
 // there.  FP32 at 64^3 cells (6 lines, 41 points): 31.4 ms against 31.9 with 32
 // points, and 34.1 with 48, which only 26 waves per CU have room for.
 template <typename real>
-static int fitting_window(mgr_ctx *ctx)
+static int fitting_window(const mgr_ctx *ctx, const RFArgs<real> &a)
 {
     constexpr size_t CU_LDS = 160 * 1024, GRANULE = 1280;
-    RFArgs<real> a;
-    const typename Prec<real>::row_t *none = nullptr;
-    if (make_args<real>(ctx, none, 1, 2, 0, 1, ctx->shift_min, ctx->shift_max, a) != MGR_OK) return 2;
     const size_t waves = 4 * (sizeof(real) == 8 ? 4 : one_line(ctx, a) ? 8 : 6);
     const size_t room = CU_LDS / waves / GRANULE * GRANULE, table = sizeof(double) * ctx->L;
     const size_t row = sizeof(typename Prec<real>::row_t) * ctx->L;
@@ -2034,26 +2031,33 @@ static int fitting_window(mgr_ctx *ctx)
 // fewest waves among near-ties) is kept for the context and precision.  Runs
 // outside graph capture, before the first radiation field of a precision.
 //
-// The windows differ by up to 20 %, the waves, which share only the line
-// table, by 2 % (9 % where bins meet several lines): all combinations on 16384
-// origins, and the best ones again on the whole model, took 20 ms of a
-// 27^3-cell solve of 48 and chose the same shapes; this takes 4.
+// What is tried is what has won somewhere: 64-point windows only where the
+// waves do not fill the chip twice (56 against 59 us at 10^3 cells; 10 to 25 %
+// behind on every larger model), and several waves per workgroup, which share
+// only the line table, only where bins meet several lines (6 % ahead on the
+// blended model; with one line equal or up to 12 % behind).  A 27^3-cell solve
+// takes 24 to 25 ms with these 2 shapes, 27 with 4, and 48 with all combinations
+// on 16384 origins and the best ones again on the whole model.
 template <typename real>
 static int tune(mgr_ctx *ctx, int pi)
 {
     const int nchunk = (int)((ctx->F + WAVE - 1) / WAVE);
     const int chmax = max_chunk<real>(ctx);
     if (chmax < 2) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
-    std::vector<int> nwgs;
-    for (int w = 2; w <= MAX_WAVES; w++)
-        if (w == nchunk || (nchunk % w) == 0 || w == std::min(nchunk, MAX_WAVES)) nwgs.push_back(w);
-    std::vector<int> chs;
-    for (int c : {16, fitting_window<real>(ctx), 64})
-        if (c <= chmax && (chs.empty() || c > chs.back())) chs.push_back(c);
-    if (chs.empty() || chs.back() != chmax) chs.push_back(chmax);
+    RFArgs<real> a;
+    const typename Prec<real>::row_t *none = nullptr;
+    int rc = make_args<real>(ctx, none, 1, 2, 0, 1, ctx->shift_min, ctx->shift_max, a);
+    if (rc) return rc;
     const int64_t fill = (WAVES_IN_FLIGHT + nchunk - 1) / nchunk;   // origins that fill the chip
     const int nslice = ctx->N > 2 * fill ? 2 : 1;
     const int64_t per = nslice == 2 ? fill : ctx->N;
+    const int fit = std::min(fitting_window(ctx, a), chmax);
+    std::vector<int> chs{std::min(16, chmax)}, nwgs;
+    if (fit > chs.back()) chs.push_back(fit);
+    if (nslice == 1 && chmax > chs.back()) chs.push_back(chmax);
+    if (!one_line(ctx, a))
+        for (int w = 2; w <= MAX_WAVES; w++)
+            if (w == nchunk || (nchunk % w) == 0 || w == std::min(nchunk, MAX_WAVES)) nwgs.push_back(w);
     auto launch_slices = [&](int w, int c) {
         if (nslice == 1) return launch_rf_shape<real>(ctx, w, c, 0, ctx->N);
         int r = launch_rf_shape<real>(ctx, w, c, std::max<int64_t>(ctx->N / 8 - per / 2, 0), per);
@@ -2065,7 +2069,7 @@ static int tune(mgr_ctx *ctx, int pi)
     MGR_HIP(hipEventCreate(&e1));
     int best_w = 1, best_c = chs.front();
     float best = 1e30f;
-    int rc = launch_slices(1, chs.back());   // warm-up
+    rc = launch_slices(1, chs.back());   // warm-up
     ctx->tune_log.clear();
     auto time_shape = [&](int w, int c) {
         float ms = 0.0f;
