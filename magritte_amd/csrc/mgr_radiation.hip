@@ -71,6 +71,7 @@
 #include <vector>
 
 #include "mgr_common.hpp"
+#include "mgr_lds.hpp"
 #include "mgr_ray.hpp"
 
 using namespace mgr;
@@ -80,7 +81,6 @@ namespace {
 constexpr int32_t ERR_NOT_BOUNDARY = 2;   // ray ends on a non-boundary cell
 constexpr int32_t ERR_EMPTY_SIDE   = 4;   // empty ray at a non-boundary origin
 constexpr int CH_MAX = 64;                // traced steps staged per chunk (at most)
-constexpr size_t LDS_LIMIT = 64 * 1024;   // dynamic LDS per workgroup
 constexpr int64_t WAVES_IN_FLIGHT = 8192;  // of the field kernels: 256 CUs, 8 waves per SIMD
 constexpr int MAX_WAVES = 4;              // frequency chunks per workgroup
 
@@ -1829,18 +1829,13 @@ int make_args(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
     return MGR_OK;
 }
 
-// LDS of the field kernel: the window of each wave, then the line table.  With
-// many lines and waves a window holds fewer points than asked for.
+// LDS of the field kernel with nwg waves per workgroup: the window of each wave
+// (of up to `points` points), then the line table.
 template <typename real>
-size_t field_lds(const mgr_ctx *ctx, RFArgs<real> &a)
+FieldLds window_lds(const mgr_ctx *ctx, int nwg, int points)
 {
-    const size_t row = sizeof(typename Prec<real>::row_t) * ctx->L;
-    const size_t table = sizeof(double) * ctx->L;
-    const size_t fit = ((LDS_LIMIT - table) / a.nwg - Window<real>::fixed) / row;
-    a.ch = (int)std::max<size_t>(2, std::min<size_t>(a.ch, fit - 1));
-    a.wave_lds = (int)((Window<real>::fixed + row * (a.ch + 1) + 63) / 64 * 64);
-    a.line_offset = (size_t)a.wave_lds * a.nwg;
-    return a.line_offset + table;
+    return field_lds(Window<real>::fixed, sizeof(typename Prec<real>::row_t) * ctx->L, sizeof(double) * ctx->L, nwg,
+                     points);
 }
 
 // One candidate line per bin: the lines' candidate ranges are disjoint.
@@ -1917,9 +1912,13 @@ int launch_rf(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
     a.far32 = (sizeof(real) == 4 && ctx->far_cache && ctx->far_valid[0]) ? ctx->far_I32 : nullptr;
     a.far64 = (sizeof(real) == 8 && ctx->far_cache && ctx->far_valid[1]) ? ctx->far_I64 : nullptr;
     const bool one = one_line(ctx, a);
-    const size_t lds = field_lds<real>(ctx, a);
+    const FieldLds lds = window_lds<real>(ctx, a.nwg, a.ch);
+    if (lds.points < 2) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
+    a.ch = lds.points;
+    a.wave_lds = (int)lds.wave;
+    a.line_offset = lds.wave * a.nwg;
     auto kernel = one ? k_radiation_field<real, true> : k_radiation_field<real, false>;
-    hipLaunchKernelGGL(kernel, dim3(grid_of(a)), dim3(WAVE * a.nwg), lds, ctx->stream, a);
+    hipLaunchKernelGGL(kernel, dim3(grid_of(a)), dim3(WAVE * a.nwg), lds.total, ctx->stream, a);
     ctx->last_rf_kernel = sizeof(real) == 4 ? (one ? "k_radiation_field<float, true>" : "k_radiation_field<float, false>")
                                             : (one ? "k_radiation_field<double, true>" : "k_radiation_field<double, false>");
     MGR_LAUNCH_CHECK();
