@@ -369,15 +369,18 @@ int mgr_compute_image(mgr_ctx *ctx, int64_t ray, int precision, double *I_m, dou
  * counterpart in the reference): waves of 64 frequency bins per workgroup and
  * points staged per window, 0 before the first radiation field of that
  * precision; with capacity > 0 also the shapes tried by the last tuning and
- * their times on the tuning slice (ms).                                       */
+ * their times on the tuning slice (ms).  The points are those used: fewer than
+ * asked for where a workgroup's windows would not fit its LDS.                */
 int mgr_radiation_field_shape(mgr_ctx *ctx, int precision, int *waves_per_group, int *steps_per_chunk,
                               int capacity, int *n_tried, int *tried_waves, int *tried_steps,
                               float *tried_ms);
 /* Forces that launch shape for later radiation fields of that precision
  * instead of tuning (no counterpart in the reference): 1..4 waves per
- * workgroup, 2..(the model's LDS limit, at most 64) steps per chunk; both 0
- * hands the choice back to the autotuner.  J and Lambda* do not depend on
- * the shape.                                                                  */
+ * workgroup, 2..(the model's LDS limit for one wave, at most 64) points per
+ * window; both 0 hands the choice back to the autotuner.  Where the windows of
+ * that many waves do not fit a workgroup's LDS they hold the points that do,
+ * which mgr_radiation_field_shape reports.  J and Lambda* do not depend on the
+ * shape.                                                                      */
 int mgr_set_radiation_field_shape(mgr_ctx *ctx, int precision, int waves_per_group, int steps_per_chunk);
 
 /* Out-of-window skip of the radiation-field kernels (no counterpart in the

@@ -2070,7 +2070,9 @@ static int tune(mgr_ctx *ctx, int pi)
     float best = 1e30f;
     rc = launch_slices(1, chs.back());   // warm-up
     ctx->tune_log.clear();
-    auto time_shape = [&](int w, int c) {
+    auto time_shape = [&](int w, int points) {
+        const int c = window_lds<real>(ctx, w, points).points;
+        if (c < 2) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
         float ms = 0.0f;
         if (hipEventRecord(e0, ctx->stream) != hipSuccess) return MGR_ERR_DEVICE;
         const int r = launch_slices(w, c);
@@ -2233,8 +2235,11 @@ extern "C" int mgr_set_radiation_field_shape(mgr_ctx *ctx, int precision, int wa
         if (steps_per_chunk < 2 || steps_per_chunk > chmax)
             return ctx->fail(MGR_ERR_ARGUMENT, "steps_per_chunk must be 2.." + std::to_string(chmax) +
                                                    " for this model's line rows");
+        const FieldLds lds = pi ? window_lds<double>(ctx, waves_per_group, steps_per_chunk)
+                                : window_lds<float>(ctx, waves_per_group, steps_per_chunk);
+        if (lds.points < 2) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
         ctx->rf_nwg[pi] = waves_per_group;
-        ctx->rf_ch[pi] = steps_per_chunk;
+        ctx->rf_ch[pi] = lds.points;
     }
     // the ALI graphs were captured with the previous shape
     if (ctx->graph_precision == precision) {

@@ -402,7 +402,7 @@ class Context:
         return buf.value.decode()
 
     def radiation_field_shape(self, precision="fp32"):
-        """(waves per workgroup, steps per chunk) chosen by the autotuner, and
+        """(waves per workgroup, points per window) chosen by the autotuner, and
         the shapes it tried with their times (ms)."""
         w, c, n = C.c_int(0), C.c_int(0), C.c_int(0)
         cap = 32
@@ -413,7 +413,8 @@ class Context:
         return (w.value, c.value), [(int(tw[i]), int(tc[i]), float(tm[i])) for i in range(k)]
 
     def set_radiation_field_shape(self, precision="fp32", waves_per_group=0, steps_per_chunk=0):
-        """Force the launch shape (0, 0: back to the autotuner)."""
+        """Force the launch shape (0, 0: back to the autotuner); the points per window
+        are cut to what the waves' LDS holds (radiation_field_shape)."""
         self._check(self.lib.mgr_set_radiation_field_shape(self.h, _prec(precision), int(waves_per_group),
                                                            int(steps_per_chunk)), "set_radiation_field_shape")
 

@@ -27,3 +27,24 @@ def test_shapes_at_the_lds_limit(nlev, precision, waves, points):
     ctx.compute_radiation_field(precision)
     assert np.array_equal(ctx.J(), J) and np.array_equal(ctx.lambda_diag(), Lam)
     ctx.close()
+
+
+@pytest.mark.parametrize("nlev,waves,points", [(8, 4, 64), (8, 4, 63), (14, 4, 34), (14, 2, 64), (36, 4, 32)])
+def test_reported_shape_is_the_used_one(nlev, waves, points):
+    """FP64 windows that do not fit are reported with the points they hold: as many
+    as 64 KB have room for beside the line table, each wave's share (1792 bytes and
+    32 per line of points + 1) in whole 64 bytes."""
+    from magritte_amd.hip import Context
+    ctx = Context(synthetic.envelope_model(n=4, seed=3, nside=1, nlev=nlev, nquads=5)).setup()
+    ctx.set_radiation_field_shape("fp64", waves, points)
+    w, c = ctx.radiation_field_shape("fp64")[0]
+    L = nlev - 1
+
+    def lds(n):
+        return -(-(1792 + 32 * L * (n + 1)) // 64) * 64 * waves + 8 * L
+
+    assert w == waves and 2 <= c <= points
+    assert lds(c) <= 65536 and (c == points or lds(c + 1) > 65536)
+    ctx.compute_radiation_field("fp64")
+    assert ctx.radiation_field_shape("fp64")[0] == (w, c)
+    ctx.close()
