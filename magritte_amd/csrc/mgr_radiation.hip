@@ -168,9 +168,10 @@ struct RFArgs {
 // exp(-t) for t >= 0: reduced by multiples of ln 2, whose double is taken in
 // two parts, to |r| <= ln 2 / 2, and there the polynomial of degree 11 that
 // meets exp at the 12 Chebyshev nodes of that interval (relative error below
-// 1.7e-17), scaled by ldexp; 0 from t = 745 up to 1e15 at least.  18 instructions, without the
-// range and sign handling of the library's exp.
-__device__ __forceinline__ double exp_neg(double t)
+// 1.7e-17), scaled by ldexp; 0 from t = 745.2 up to 1e15 at least, and where `in`
+// is false.  18 instructions, without the range and sign handling of the
+// library's exp.
+__device__ __forceinline__ double exp_neg(double t, bool in = true)
 {
     const double n = __builtin_rint(t * -1.4426950408889634);
     // ln 2 = 0x1.62e42fee00000p-1 (n times it is exact) + 1.9082149292705877e-10
@@ -187,7 +188,7 @@ __device__ __forceinline__ double exp_neg(double t)
     p = __builtin_fma(p, r, 0.5000000000000019);
     p = __builtin_fma(p, r, 1.0);
     p = __builtin_fma(p, r, 1.0);
-    return __builtin_ldexp(p, (int)n);
+    return __builtin_ldexp(p, in ? (int)n : -4000);
 }
 
 // FP64: get_eta_and_chi (simulation.tpp:385-481) for one lane with the exact
@@ -453,6 +454,7 @@ struct LaneCtx<double> {
     const double *line;   // line frequencies (a copy in LDS in the field kernel)
     double nu_l;          // frequency of the bin's only candidate line l (none: one far away)
     int    l;
+    double top;           // upper end of that line's window (eta_chi_one)
 };
 
 template <typename real>
@@ -677,8 +679,9 @@ __device__ __forceinline__ real end_u(const Sweep<real> &sw, real I)
 }
 
 // FP64 with one candidate line per bin: get_eta_and_chi's window holds at most
-// that line, and a bin further than 11 widths from it gets exp(-x^2) < 3e-53
-// of it instead of nothing, which neither chi's floor nor any sum can feel.
+// that line, x widths away: -11 <= x <= 11, or any x >= -11 of the last of all
+// lines, which the reference's search never passes (top = 746, where exp(-x^2)
+// is 0).  Beyond, eta is exactly 0, and so is J behind a dark boundary.
 // v: (anything, 1/width, E, K) of the line.
 __device__ __forceinline__ void eta_chi_one(const LaneCtx<double> &lc, const double4 v, double s, double &eta,
                                             double &chi)
@@ -686,7 +689,8 @@ __device__ __forceinline__ void eta_chi_one(const LaneCtx<double> &lc, const dou
 #pragma clang fp contract(off)
     const double fs = s * lc.nu_f;
     const double x = (fs - lc.nu_l) * v.y;
-    const double g = fs * exp_neg(x * x);
+    const double t = x * fabs(x);
+    const double g = fs * exp_neg(fabs(t), t >= -LINE_WINDOW * LINE_WINDOW && t <= lc.top);
     eta = v.z * g;
     chi = __builtin_fma(v.w, g, CHI_FLOOR * CHI_SCALE);
 }
@@ -729,8 +733,11 @@ __device__ __forceinline__ void origin_point(const RFArgs<real> &a, double nu_f,
         lc.nu_f = nu_f;
         lc.lstart = ls;
         if constexpr (ONE) {
-            const bool cand = a.tb->line[ls] * a.cand_lo >= nu_f && a.tb->line[ls] * a.cand_hi <= nu_f;
-            lc.nu_l = cand ? a.tb->line[ls] : 0.9 * nu_f;   // 0.1 nu is thousands of widths: exp_neg gives 0
+            // a bin below its line's reach at every point has none: 0.1 nu is thousands of widths
+            const double line = a.tb->line[ls];
+            const bool last = ls == a.L - 1;
+            lc.nu_l = line * a.cand_hi <= nu_f && (last || line * a.cand_lo >= nu_f) ? line : 0.9 * nu_f;
+            lc.top = last && lc.nu_l == line ? 746.0 : LINE_WINDOW * LINE_WINDOW;
             lc.l = ls;
         }
         if constexpr (ONE) eta_chi_one(lc, orow[ls], 1.0, eta_o, chi_o);
