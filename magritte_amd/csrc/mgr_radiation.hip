@@ -168,10 +168,12 @@ struct RFArgs {
 // exp(-t) for t >= 0: reduced by multiples of ln 2, whose double is taken in
 // two parts, to |r| <= ln 2 / 2, and there the polynomial of degree 11 that
 // meets exp at the 12 Chebyshev nodes of that interval (relative error below
-// 1.7e-17), scaled by ldexp; 0 from t = 745.2 up to 1e15 at least, and where `in`
-// is false.  18 instructions, without the range and sign handling of the
-// library's exp.
-__device__ __forceinline__ double exp_neg(double t, bool in = true)
+// 1.7e-17), scaled by ldexp; 0 from t = 745.2 on.  18 instructions, without the
+// range and sign handling of the library's exp: a t above 1e9, whose n an int
+// does not hold, needs `in` false, which gives 0 (up to 1e40; above, the
+// polynomial overflows) and keeps a NaN.
+constexpr double EXP_NEG_END = 746.0;   // 0 from here on
+__device__ __forceinline__ double exp_neg(double t, bool in)
 {
     const double n = __builtin_rint(t * -1.4426950408889634);
     // ln 2 = 0x1.62e42fee00000p-1 (n times it is exact) + 1.9082149292705877e-10
@@ -212,8 +214,8 @@ __device__ __forceinline__ void eta_chi64(const RFArgs<double> &a, const double4
     }
     double e_acc = 0.0, c_acc = CHI_FLOOR * CHI_SCALE;
     while (fd >= -v.x) {
-        const double x = fd * v.y;
-        const double g = fs * exp_neg(x * x);
+        const double x = fd * v.y, t = x * x;
+        const double g = fs * exp_neg(t, t <= EXP_NEG_END);   // the last line's window has no upper end
         e_acc += v.z * g;
         c_acc += v.w * g;
         if (left <= 0) break;
@@ -680,9 +682,9 @@ __device__ __forceinline__ real end_u(const Sweep<real> &sw, real I)
 
 // FP64 with one candidate line per bin: get_eta_and_chi's window holds at most
 // that line, x widths away: -11 <= x <= 11, or any x >= -11 of the last of all
-// lines, which the reference's search never passes (top = 746, where exp(-x^2)
-// is 0).  Beyond, eta is exactly 0, and so is J behind a dark boundary.
-// v: (anything, 1/width, E, K) of the line.
+// lines, which the reference's search never passes (top = EXP_NEG_END).  Beyond,
+// eta is exactly 0, and so is J behind a dark boundary.  v: (anything, 1/width,
+// E, K) of the line.
 __device__ __forceinline__ void eta_chi_one(const LaneCtx<double> &lc, const double4 v, double s, double &eta,
                                             double &chi)
 {
@@ -737,7 +739,7 @@ __device__ __forceinline__ void origin_point(const RFArgs<real> &a, double nu_f,
             const double line = a.tb->line[ls];
             const bool last = ls == a.L - 1;
             lc.nu_l = line * a.cand_hi <= nu_f && (last || line * a.cand_lo >= nu_f) ? line : 0.9 * nu_f;
-            lc.top = last && lc.nu_l == line ? 746.0 : LINE_WINDOW * LINE_WINDOW;
+            lc.top = last && lc.nu_l == line ? EXP_NEG_END : LINE_WINDOW * LINE_WINDOW;
             lc.l = ls;
         }
         if constexpr (ONE) eta_chi_one(lc, orow[ls], 1.0, eta_o, chi_o);
@@ -1597,8 +1599,8 @@ __device__ __forceinline__ double profile64(double width, double freq_diff)
 {
 #pragma clang fp contract(off)
     const double iw = Prec<double>::rcp(width);
-    const double x = iw * freq_diff;
-    return iw * INVERSE_SQRT_PI * exp_neg(x * x);
+    const double x = iw * freq_diff, t = x * x;
+    return iw * INVERSE_SQRT_PI * exp_neg(t, t <= EXP_NEG_END);
 }
 
 // The band elements of Lambda* (RayPair::update_Lambda, raypair_lambda.tpp:129-146,
