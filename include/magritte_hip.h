@@ -393,8 +393,9 @@ int mgr_set_radiation_field_shape(mgr_ctx *ctx, int precision, int waves_per_gro
  * points are eliminated with eta = 0 and chi at its floor.  Results are
  * bit-identical either way, but for the last line's wing above 11 widths in
  * FP64, which get_eta_and_chi's window does not end (below 3e-53 of the line's
- * opacity: to be seen behind a boundary without radiation only).  Off evaluates
- * every point.                                                                */
+ * opacity: to be seen behind a boundary without radiation only).  0: every point
+ * is evaluated; 2: only whole steps are passed over, as where there is no memory
+ * for the spans of sub-points; else on.                                       */
 int mgr_set_window_skip(mgr_ctx *ctx, int enable);
 /* Far-end intensity cache (no counterpart in the reference; on by default):
  * the rescaled boundary intensity entering every (origin, ray) and bin,

@@ -324,6 +324,7 @@ struct mgr_ctx {
     bool     masks64_valid = false;
     float    hdz32_max = 0.0f;      // largest dz' of the cached steps (set with the masks)
     bool     rf_window_skip = true;
+    bool     rf_spans = true;       // by sub-points, not whole steps only
     // lane order of the radiation-field kernel (lane_bin), chosen with the
     // masks: root-major when no bin can meet a second line's window
     bool     root_major = false;

@@ -864,8 +864,9 @@ __device__ __forceinline__ void eval_window(const RFArgs<real> &a, const LaneCtx
 //   WIDE   steps beyond MASK_WINDOW widths (step_mask): profiles are 0,
 //          X = floor, S = 0 and any p will do;
 //   NONE   every point is evaluated.
-// The FP64 kernel (SPAN or NONE) steps every point, but evaluates only those
-// within MASK_WINDOW64 widths: beyond, eta = 0 and chi is the floor exactly.
+// The FP64 kernel steps every point, but evaluates only those within
+// MASK_WINDOW64 widths (SPAN, or the steps that have one: WIDE): beyond, eta = 0
+// and chi is the floor exactly.
 struct Runs {
     enum { SPAN = 0, WIDE = 1, NONE = 2 };
 };
@@ -920,7 +921,7 @@ __device__ __forceinline__ void sweep_pair(const RFArgs<real> &a, const LaneCtx<
         unsigned span = SPAN_ALL;
         if (lane < nb) {
             if (mode == Runs::SPAN) span = ka->span[ka->span_stride * chunk + at];
-            else if (F32 && mode == Runs::WIDE) span = (ka->step_mask[at] >> chunk) & 1 ? SPAN_NONE : SPAN_ALL;
+            else if (mode == Runs::WIDE) span = (ka->step_mask[at] >> chunk) & 1 ? SPAN_NONE : SPAN_ALL;
         }
         const uint64_t valid = (1ull << nb) - 1;   // nb <= 63
         const uint64_t outm = __ballot(span == SPAN_NONE) & valid;
@@ -1216,8 +1217,8 @@ void k_radiation_field(RFArgs<real> a)
                 mode = Runs::SPAN;
                 p_near = lc.ln.nc > 1 ? a.near_p[a.L] : a.near_p[lc.ln.la];
             }
-        } else if (a.span) {
-            mode = Runs::SPAN;
+        } else if (a.step_mask) {
+            mode = a.span ? Runs::SPAN : Runs::WIDE;
         }
     }
     mode = rfl_int(mode);
@@ -1286,7 +1287,8 @@ void k_radiation_field(RFArgs<real> a)
 //
 // As in sweep_pair, up to WAVE steps of the pair lie on the lanes, and their
 // points a window at a time, with the line rows of those inside the line
-// window in LDS; at the others (spans) eta = 0 and chi is the floor.
+// window in LDS; at the others (by the spans, or by the steps' bits without them)
+// eta = 0 and chi is the floor.
 template <bool ONE, typename Visit>
 __device__ __forceinline__ void walk_pair(const RFArgs<double> &a, const LaneCtx<double> &lc, int32_t o, int64_t qx,
                                           int64_t qy, int ny, double dsm, int chunk, const Window<double> &win,
@@ -1299,7 +1301,7 @@ __device__ __forceinline__ void walk_pair(const RFArgs<double> &a, const LaneCtx
     const int T = nsx + 1 + (nsy < ny ? nsy : ny);   // steps; a step has at least one point
     int left = rfl_int(ka->npts[qx]) + 1 + ny;       // points
     const int64_t bx = ka->seg_off[qx], by = ka->seg_off[qy];
-    const bool spans = ka->span && chunk < STEP_MASK_CHUNKS;
+    const bool spans = ka->span && chunk < STEP_MASK_CHUNKS, bits = !spans && ka->step_mask && chunk < STEP_MASK_CHUNKS;
     int t = 0;
     double h_last = 0.0;   // path factor of the step before this batch
     for (int g0 = 0; g0 < T; g0 += WAVE) {
@@ -1313,6 +1315,7 @@ __device__ __forceinline__ void walk_pair(const RFArgs<double> &a, const LaneCtx
         double s0 = 1.0, ds = 0.0, h = 0.0;
         if (inward || outward) {
             if (spans) span = ka->span[ka->span_stride * chunk + at];
+            else if (bits) span = (ka->step_mask[at] >> chunk) & 1 ? SPAN_NONE : SPAN_ALL;
             c_next = ka->seg_cell[at];
             const double sn = ka->seg_shift[at];
             double sc = ka->origin_shift ? ka->origin_shift[inward ? qx : qy] : 1.0;   // co-moving: the origin's is 1
@@ -1911,8 +1914,8 @@ int launch_rf(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
         }
     }
     a.span_stride = ctx->span_stride;
-    if (sizeof(real) == 8 && a.step_mask) a.span = ctx->span64;
-    if (sizeof(real) == 4 && a.step_mask && ctx->near_on) {
+    if (sizeof(real) == 8 && a.step_mask && ctx->rf_spans) a.span = ctx->span64;
+    if (sizeof(real) == 4 && a.step_mask && ctx->near_on && ctx->rf_spans) {
         a.span = ctx->span32;
         a.near_p = ctx->near_p;
         a.near_bad = ctx->near_bad;
@@ -1992,7 +1995,10 @@ int launch_band(mgr_ctx *ctx)
     a.band_part = ctx->band_part;
     a.root_major = ctx->root_major;
     a.span_stride = ctx->span_stride;
-    if (ctx->masks64_valid && ctx->rf_window_skip) a.span = ctx->span64;
+    if (ctx->masks64_valid && ctx->rf_window_skip) {
+        a.step_mask = ctx->step_mask64;
+        if (ctx->rf_spans) a.span = ctx->span64;
+    }
     a.ch = walk_window(ctx);
     const size_t lds = Window<double>::bytes(ctx->L, a.ch) +
                        sizeof(double) * (4 * (size_t)ctx->nband * WAVE + ctx->L) + sizeof(int) * (ctx->L + 1);
@@ -2395,6 +2401,7 @@ extern "C" int mgr_set_window_skip(mgr_ctx *ctx, int enable)
 {
     if (!ctx) return MGR_ERR_ARGUMENT;
     ctx->rf_window_skip = enable != 0;
+    ctx->rf_spans = enable != 2;
     ctx->graph_precision = -1;   // captured launches hold the old choice
     return MGR_OK;
 }

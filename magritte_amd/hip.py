@@ -349,10 +349,11 @@ class Context:
     def set_scattering(self, use_scattering=True):
         self._check(self.lib.mgr_set_scattering(self.h, 1 if use_scattering else 0), "set_scattering")
 
-    def set_window_skip(self, enable=True):
-        """Both kernels: eliminate steps out of every line window without
-        evaluating their profiles (bit-identical; on by default)."""
-        self._check(self.lib.mgr_set_window_skip(self.h, 1 if enable else 0), "set_window_skip")
+    def set_window_skip(self, enable=True, spans=True):
+        """Both kernels: eliminate points out of every line window without
+        evaluating their profiles (bit-identical; on by default); without
+        spans only those of whole steps."""
+        self._check(self.lib.mgr_set_window_skip(self.h, (1 if spans else 2) if enable else 0), "set_window_skip")
 
     def set_trace_options(self, record_steps=-1, candidate_masks=True):
         """Options of the next trace: cells recorded per walk for the filling
