@@ -168,14 +168,13 @@ struct RFArgs {
 // exp(-t) for t >= 0: reduced by multiples of ln 2, whose double is taken in
 // two parts, to |r| <= ln 2 / 2, and there the polynomial of degree 11 that
 // meets exp at the 12 Chebyshev nodes of that interval (relative error below
-// 1.7e-17), scaled by ldexp; 0 from t = 745.2 on.  18 instructions, without the
-// range and sign handling of the library's exp: a t above 1e9, whose n an int
-// does not hold, needs `in` false, which gives 0 (up to 1e40; above, the
-// polynomial overflows) and keeps a NaN.
+// 1.7e-17), scaled by ldexp; 0 from t = 745.2 up to 1e40, where the polynomial
+// overflows, and NaN for NaN.  18 instructions, without the range and sign
+// handling of the library's exp.
 constexpr double EXP_NEG_END = 746.0;   // 0 from here on
-__device__ __forceinline__ double exp_neg(double t, bool in)
+__device__ __forceinline__ double exp_neg_parts(double t, double &n)
 {
-    const double n = __builtin_rint(t * -1.4426950408889634);
+    n = __builtin_rint(t * -1.4426950408889634);
     // ln 2 = 0x1.62e42fee00000p-1 (n times it is exact) + 1.9082149292705877e-10
     const double r = __builtin_fma(n, -1.9082149292705877e-10, __builtin_fma(n, -0x1.62e42fee00000p-1, -t));
     double p = 2.511003761756205e-08;
@@ -189,7 +188,29 @@ __device__ __forceinline__ double exp_neg(double t, bool in)
     p = __builtin_fma(p, r, 0.1666666666666668);
     p = __builtin_fma(p, r, 0.5000000000000019);
     p = __builtin_fma(p, r, 1.0);
-    p = __builtin_fma(p, r, 1.0);
+    return __builtin_fma(p, r, 1.0);
+}
+
+// From t = 1.5e9 on an int does not hold n: the instruction gives the nearest
+// one, where a conversion in C++ is undefined.
+__device__ __forceinline__ int nearest_int(double x)
+{
+    int i;
+    asm("v_cvt_i32_f64 %0, %1" : "=v"(i) : "v"(x));
+    return i;
+}
+__device__ __forceinline__ double exp_neg(double t)
+{
+    double n;
+    const double p = exp_neg_parts(t, n);
+    return __builtin_ldexp(p, nearest_int(n));
+}
+
+// 0 where `in` is false, which it is to be beyond EXP_NEG_END.
+__device__ __forceinline__ double exp_neg(double t, bool in)
+{
+    double n;
+    const double p = exp_neg_parts(t, n);
     return __builtin_ldexp(p, in ? (int)n : -4000);
 }
 
@@ -214,8 +235,8 @@ __device__ __forceinline__ void eta_chi64(const RFArgs<double> &a, const double4
     }
     double e_acc = 0.0, c_acc = CHI_FLOOR * CHI_SCALE;
     while (fd >= -v.x) {
-        const double x = fd * v.y, t = x * x;
-        const double g = fs * exp_neg(t, t <= EXP_NEG_END);   // the last line's window has no upper end
+        const double x = fd * v.y;
+        const double g = fs * exp_neg(x * x);   // the last line's window has no upper end
         e_acc += v.z * g;
         c_acc += v.w * g;
         if (left <= 0) break;
@@ -894,6 +915,7 @@ __device__ __forceinline__ void sweep_pair(const RFArgs<real> &a, const LaneCtx<
     using row_t = typename Prec<real>::row_t;
     constexpr bool F32 = sizeof(real) == 4;
     constexpr bool INROW = F32 || ONE;   // the rows have a component to spare for the shift
+    constexpr int UNROLL = F32 || ONE ? 2 : 1;
     Sweep<real> sw;
     sw.init(ns_a > 0 ? I_a : I_r);
     const real chi_floor = (real)(CHI_FLOOR * CHI_SCALE);
@@ -1055,7 +1077,7 @@ __device__ __forceinline__ void sweep_pair(const RFArgs<real> &a, const LaneCtx<
                 const int e = marks ? (int)__builtin_ctzll(marks) : cw;
                 const bool turns = pending && turn - w0 <= e;
                 const int stop = turns ? turn - w0 : e;
-#pragma unroll 2
+#pragma unroll UNROLL
                 for (; p < stop; ++p) {
                     real eta, chi;
                     eval_window<real, ONE>(a, lc, win, p, W, eta, chi);
@@ -1602,8 +1624,8 @@ __device__ __forceinline__ double profile64(double width, double freq_diff)
 {
 #pragma clang fp contract(off)
     const double iw = Prec<double>::rcp(width);
-    const double x = iw * freq_diff, t = x * x;
-    return iw * INVERSE_SQRT_PI * exp_neg(t, t <= EXP_NEG_END);
+    const double x = iw * freq_diff;
+    return iw * INVERSE_SQRT_PI * exp_neg(x * x);
 }
 
 // The band elements of Lambda* (RayPair::update_Lambda, raypair_lambda.tpp:129-146,
