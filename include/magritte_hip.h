@@ -370,7 +370,10 @@ int mgr_compute_image(mgr_ctx *ctx, int64_t ray, int precision, double *I_m, dou
  * points staged per window, 0 before the first radiation field of that
  * precision; with capacity > 0 also the shapes tried by the last tuning and
  * their times on the tuning slice (ms).  The points are those used: fewer than
- * asked for where a workgroup's windows would not fit its LDS.                */
+ * asked for where a workgroup's windows would not fit its LDS.  FP32 models of
+ * many lines or bins, behind dark boundaries, with very long steps or with the
+ * skip off run a kernel of staged steps, whose second number is the traced steps
+ * staged per chunk (mgr_last_radiation_field_kernel names it).                */
 int mgr_radiation_field_shape(mgr_ctx *ctx, int precision, int *waves_per_group, int *steps_per_chunk,
                               int capacity, int *n_tried, int *tried_waves, int *tried_steps,
                               float *tried_ms);

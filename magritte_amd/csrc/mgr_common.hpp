@@ -58,7 +58,7 @@ constexpr int WAVE = 64;                 // CDNA wavefront width
 // the FP32 profile exp2(-x^2 log2 e) is then exactly zero, since x >= 10.5
 // gives exp2 of less than -159, below the smallest denormal 2^-149 (zero from
 // x > 10.2; the FP32 rounding of x is ~1e-6 widths).
-constexpr int STEP_N_MASK = 0x3FFF, STEP_HALF_SHIFT = 14, STEP_HALF_MASK = 0x1FFF;
+constexpr int STEP_N_MASK = 0x3FFF, STEP_HALF_SHIFT = 14, STEP_HALF_MASK = 0x1FFF, STEP_OUT_SHIFT = 27;
 constexpr int STEP_MASK_CHUNKS = 5;
 constexpr double MASK_WINDOW = 10.5;
 // The FP64 kernel's bits: more than 11 (1 + 1e-6) widths from every line, so
@@ -283,10 +283,10 @@ struct mgr_ctx {
     bool     J_set = false;
     float    last_rf_ms = 0.0f;
     const char *last_rf_kernel = "";   // name of the radiation-field kernel last launched
-    // radiation-field launch shape per precision (FP32, FP64): waves per
-    // workgroup and staged steps per chunk; 0 until chosen
-    int      rf_nwg[2] = {0, 0}, rf_ch[2] = {0, 0};
-    bool     rf_autotune = true;
+    // radiation-field launch shape of each kernel (FP32 by points, FP64, FP32 of
+    // staged steps): waves per workgroup and points per window, or steps per
+    // chunk; 0 until chosen
+    int      rf_nwg[3] = {0, 0, 0}, rf_ch[3] = {0, 0, 0};
     int      rf_pair_stride = 1;    // every k-th ray pair (weights times k): the warm start's first pass only
     int64_t  warm_fallbacks = 0;    // cells that kept their populations in the last warm start
     struct TuneEntry { int nwg, ch; float ms; };
@@ -318,6 +318,7 @@ struct mgr_ctx {
     uint16_t *span32 = nullptr, *span64 = nullptr;
     int64_t  span_stride = 0;
     bool     near_on = false;
+    bool     bdy_dark = false;      // a boundary fails the FP32 kernel's test behind the spans
     float   *near_p = nullptr;      // [L + 1] bound on p behind span32, per sorted line and for bins of several
     int32_t *near_bad = nullptr;    // set when a population exceeds twice its cell's total (until they are set anew)
     uint8_t *step_mask64 = nullptr; // [total segments] the FP64 kernel's bits (MASK_WINDOW64)

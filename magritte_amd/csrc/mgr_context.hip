@@ -1210,6 +1210,19 @@ int mgr_compute_spectral_discretisation_image(mgr_ctx *ctx, double width)
     return spectral_discretisation(ctx, true, width);
 }
 
+// Whether a boundary is darker than the spans of the FP32 kernel allow for, a
+// quarter of the 2.7 K background at every line (near_window2); with T_CMB itself
+// where temperatures is null.
+static bool dark_boundary(const mgr_ctx *ctx, const double *temperatures)
+{
+    if (!temperatures) return false;
+    double T = INFINITY;
+    for (int64_t b = 0; b < ctx->NB; b++) T = temperatures[b] >= T ? T : temperatures[b];
+    if (T >= T_CMB) return false;
+    const double x = HH_OVER_KB * ctx->h_tables.line[ctx->h_tables.L - 1];
+    return !(T > 0.0 && std::expm1(x / T_CMB) >= 0.3 * std::expm1(x / T));
+}
+
 int mgr_compute_boundary_intensities(mgr_ctx *ctx, const double *temperatures)
 {
     if (!ctx) return MGR_ERR_ARGUMENT;
@@ -1229,6 +1242,9 @@ int mgr_compute_boundary_intensities(mgr_ctx *ctx, const double *temperatures)
         return ctx->fail(MGR_ERR_DEVICE, "boundary intensities kernel failed");
     ctx->bdy_set = true;
     ctx->far_invalidate();
+    const bool dark = dark_boundary(ctx, temperatures);
+    if (dark != ctx->bdy_dark) ctx->graph_precision = -1;   // captured launches hold the old choice
+    ctx->bdy_dark = dark;
     return MGR_OK;
 }
 

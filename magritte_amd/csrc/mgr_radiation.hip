@@ -68,6 +68,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "mgr_common.hpp"
@@ -103,12 +104,18 @@ template <> struct Prec<double> {
     }
 };
 
-// One traced step in LDS (FP32 image kernel).  Sub-point m = 1..n of the step lies
-// at shift s0 + m ds with path-length factor dz = dZ HDZ_SCALE and belongs to
-// the current cell for m < half, to `cell` otherwise.
+// One traced step in LDS.  Sub-point m = 1..n of the step lies at shift s0 + m ds
+// with path-length factor dz = dZ HDZ_SCALE and belongs to the current cell for
+// m < half, to `cell` otherwise.  FP32 image kernel: Step; FP32 field kernel of
+// staged steps: Step32, whose s0 is shift - 1.
 struct alignas(32) Step {
     double  s0, ds, dz;
     int32_t nh;           // n | half << 14 (STEP_*)
+    int32_t cell;
+};
+struct alignas(32) Step32 {
+    float   s0, ds, dz;
+    int32_t nh;           // n | half << 14 | out-of-window bits << 27: one 16-byte read with the above
     int32_t cell;
 };
 
@@ -263,13 +270,15 @@ struct Lane32 {
     const double *line;   // line frequencies (a copy in LDS in the field kernel)
 };
 
-// rows: the first line's row, the others `stride` apart; their w is the shift - 1.
+// rows: the first line's row, the others `stride` apart; the shift - 1 is their w,
+// or `delta` (GIVEN).
+template <bool GIVEN = false>
 __device__ __forceinline__ void eta_chi32(const RFArgs<float> &a, const Lane32 &ln, const float4 *__restrict__ rows,
-                                          int stride, float &eta, float &chi)
+                                          int stride, float &eta, float &chi, float delta = 0.0f)
 {
 #pragma clang fp contract(off)
     const float4 v0 = rows[ln.la * stride];
-    const float delta = v0.w;
+    if constexpr (!GIVEN) delta = v0.w;
     // nu_f (1 + delta) and (nu_f delta + nu_f - nu_l), each with one rounding
     const float nus = fmaf(delta, ln.nuf, ln.nuf);
     const float x0 = fmaf(delta, ln.nuf, ln.A0) * v0.x;
@@ -428,17 +437,26 @@ struct Sweep {
 
 // Stage the entries e = 0..cnt-1 of chunk [a, b): entry e holds step j = a-1+e
 // (j = -1 is the origin) and the line rows of its cell.
+template <typename S>
 __device__ __forceinline__ void stage_chunk(const RFArgs<float> &a, int32_t o, int64_t q, int j0,
-                                            int cnt, double dsm, Step *__restrict__ st,
+                                            int cnt, double dsm, S *__restrict__ st,
                                             float4 *__restrict__ rw)
 {
     const int64_t s0 = a.seg_off[q];
     const int nthr = blockDim.x;
     for (int e = threadIdx.x; e < cnt; e += nthr) {
         const int j = j0 + e;
-        Step s;
+        S s;
         if (j < 0) {
             s.cell = o; s.nh = 0; s.s0 = 0; s.ds = 0; s.dz = 0;
+        } else if constexpr (std::is_same_v<S, Step32>) {
+            // split at trace time with the same FP64 arithmetic as below
+            const int4 v = a.seg_f32[s0 + j];
+            s.cell = v.x;
+            s.nh = v.y | (a.step_mask ? (int)a.step_mask[s0 + j] << STEP_OUT_SHIFT : 0);
+            s.s0 = __int_as_float(v.z);
+            s.ds = __int_as_float(v.w);
+            s.dz = a.seg_hdz32[s0 + j];
         } else {
             const int32_t c = a.seg_cell[s0 + j];
             const double sn = a.seg_shift[s0 + j];
@@ -1143,6 +1161,100 @@ __device__ __forceinline__ void sweep_pair(const RFArgs<real> &a, const LaneCtx<
     if (ns_r > 0) finish();
 }
 
+// One ray of a pair (entry q, which has points) by steps staged for the whole
+// workgroup (FP32): eliminated from its boundary end inwards to the origin, which
+// it leaves pending.  Out-of-window steps (step_mask) have eta = 0 and chi at the
+// floor at every sub-point, which are stepped but not evaluated; while y passes the
+// test (Runs) only the run's first one is.
+__device__ __forceinline__ Sweep<float> sweep_staged(const RFArgs<float> &a, const LaneCtx<float> &lc, int32_t o,
+                                                    int64_t q, float I_far, float S_o, float chi_o, int chunk,
+                                                    Step32 *__restrict__ st, float4 *__restrict__ rw)
+{
+    Sweep<float> sw;
+    sw.init(I_far);
+    const float chi_floor = (float)(CHI_FLOOR * CHI_SCALE);
+    // this wave's out-of-window bit in a staged nh word (none past the masked chunks)
+    const unsigned cbit = chunk < STEP_MASK_CHUNKS ? 1u << (STEP_OUT_SHIFT + chunk) : 0u;
+    const int L = a.L, CH = a.ch;
+    auto uniform = [](float x) { return __int_as_float(rfl_int(__float_as_int(x))); };
+    // s0 and ds stay in vector registers: one scalar operand per FMA
+    auto read = [&](int e) { return reinterpret_cast<const float4 *>(st + e)[0]; };
+    const int ns = rfl_int(a.nseg[q]);
+    bool noop = false;   // y is in range since the run's first point
+    for (int b_ = ns; b_ > 0; b_ -= CH) {
+        const int a_ = b_ > CH ? b_ - CH : 0;
+        const int cnt = b_ - a_ + 1;
+        __syncthreads();   // the previous chunk is consumed by every wave
+        stage_chunk(a, o, q, a_ - 1, cnt, 0.0, st, rw);
+        int e = cnt - 1;
+        while (e >= 1) {
+            float4 v = read(e);
+            int nh = rfl_int(__float_as_int(v.w));   // n, half and the bits are wave-uniform
+            if (!((unsigned)nh & cbit)) {
+                noop = false;
+                // a run of steps with points inside a line window, in a loop of its
+                // own so that the sweep state keeps its registers
+                for (;;) {
+                    const int n = nh & STEP_N_MASK;
+                    __builtin_assume(n >= 1);   // a traced step emits 1 .. 10000 points
+                    const int half = (nh >> STEP_HALF_SHIFT) & STEP_HALF_MASK;
+                    const float hdz = uniform(v.z);
+                    // sub-points m >= half lie in the step's cell (row e), m < half in
+                    // the previous one (row e-1)
+                    const float4 *rn = rw + e * L, *rc = rw + (e - 1) * L;
+                    const int mlo = half > 1 ? half : 1;
+                    for (int m = n; m >= mlo; --m) {
+                        float eta, chi;
+                        eta_chi32<true>(a, lc.ln, rn, 1, eta, chi, sub_point_shift(v.x, m, v.y));
+                        sw.step(chi);   // on the first point an exact no-op (c = 0, q = 1)
+                        const float S = eta * Prec<float>::rcp(chi);   // after the step: no copy of the last one
+                        sw.pend(S, chi, hdz);
+                    }
+                    for (int m = (half - 1 < n ? half - 1 : n); m >= 1; --m) {
+                        float eta, chi;
+                        eta_chi32<true>(a, lc.ln, rc, 1, eta, chi, sub_point_shift(v.x, m, v.y));
+                        sw.step(chi);
+                        const float S = eta * Prec<float>::rcp(chi);
+                        sw.pend(S, chi, hdz);
+                    }
+                    if (--e < 1) break;
+                    v = read(e);
+                    nh = rfl_int(__float_as_int(v.w));
+                    if ((unsigned)nh & cbit) break;
+                }
+                if (e < 1) break;
+            }
+            // an out-of-window step: its first sub-point closes the row of the last evaluated point
+            const int n = nh & STEP_N_MASK;
+            __builtin_assume(n >= 1);
+            const float hdz = uniform(v.z);
+            if (!noop) {
+                sw.step(chi_floor);
+                sw.pend(0.0f, chi_floor, hdz);
+                noop = __all(sw.y > a.noop_lo && sw.y < a.noop_hi);
+                if (!noop) {
+                    for (int m = n - 1; m >= 1; --m) {
+                        sw.step(chi_floor);
+                        sw.pend(0.0f, chi_floor, hdz);
+                    }
+                    --e;
+                    continue;
+                }
+            }
+            // pass over the out-of-window steps that follow in the chunk, keeping the last one's dz'
+            int last = e;
+            while (last > 1 && ((unsigned)rfl_int(st[last - 1].nh) & cbit)) last--;
+            const float hdz_l = last == e ? hdz : uniform(st[last].dz);
+            sw.hdz_q = hdz_l;
+            sw.cq = chi_floor * hdz_l;
+            e = last - 1;
+        }
+    }
+    sw.step(chi_o);   // the origin closes the innermost row and is left pending
+    sw.pend(S_o, chi_o, 0.0f);
+    return sw;
+}
+
 // This wave's share of the Lambda* diagonal per transition
 // (RayPair::update_Lambda, raypair_lambda.tpp:94-149, n_off_diag 0):
 // Ls(p,k) = sum over the bins f of transition k of
@@ -1182,19 +1294,16 @@ __device__ __forceinline__ void lambda_partials(const RFArgs<real> &a, int32_t o
         a.Lpart[((int64_t)o * a.nchunk + chunk) * L + lane] = mine;
 }
 
-// FP32: at least 8 waves per SIMD (at most 64 VGPRs), which hide the LDS
-// latency of the line rows; 6 where bins have several lines, whose second
-// line's registers spill at 64; FP64: 4.  The waves of a workgroup
-// share nothing but the line table.
-template <typename real, bool ONE>
-__global__ __launch_bounds__(WAVE * MAX_WAVES) __attribute__((amdgpu_waves_per_eu(sizeof(real) == 4 ? (ONE ? 8 : 6) : 4)))
-void k_radiation_field(RFArgs<real> a)
+// One wave's bins of one origin: the pairs by sweep_pair, each wave with a window
+// of its own, or by sweep_staged (STAGED).
+template <typename real, bool ONE, bool STAGED>
+__device__ __forceinline__ void field_of_origin(RFArgs<real> a)
 {
     using row_t = typename Prec<real>::row_t;
     extern __shared__ __align__(16) unsigned char smem[];
     const int wave = rfl_int((int)(threadIdx.x / WAVE));
     Window<real> win;
-    win.place(smem + wave * a.wave_lds);
+    if constexpr (!STAGED) win.place(smem + wave * a.wave_lds);
 
     // XCD-aware order: consecutive workgroups go to different XCDs, so hand
     // each XCD a contiguous range of origins.
@@ -1217,7 +1326,7 @@ void k_radiation_field(RFArgs<real> a)
         if constexpr (sizeof(real) == 4) lc.ln.line = lt;
         else lc.line = lt;
     }
-    if (chunk >= a.nchunk) return;        // a wave without bins: no barrier follows
+    if (!STAGED && chunk >= a.nchunk) return;   // a wave without bins: no barrier follows
     const int F = a.F;
     const int slot = chunk * WAVE + (int)(threadIdx.x & (WAVE - 1));
     const bool active = slot < F;
@@ -1232,7 +1341,7 @@ void k_radiation_field(RFArgs<real> a)
     // how out-of-window runs are passed over (Runs)
     int mode = Runs::NONE;
     float p_near = -FLT_MAX;
-    if (chunk < STEP_MASK_CHUNKS) {
+    if (!STAGED && chunk < STEP_MASK_CHUNKS) {
         if constexpr (sizeof(real) == 4) {
             if (a.step_mask) mode = Runs::WIDE;
             if (a.step_mask && a.span && *a.near_bad == 0) {
@@ -1274,10 +1383,24 @@ void k_radiation_field(RFArgs<real> a)
             else z_o = (real)SQRT2 * (real)(a.I_bdy[(int64_t)bo * F + f] * I_SCALE);
             y2 = (real)SQRT2;
         }
-        const real I_a = ns_a > 0 ? far_in<real>(a, qa, nu_f, F, f, err) : (real)0;
-        const real I_r = ns_r > 0 ? far_in<real>(a, qr, nu_f, F, f, err) : (real)0;
-        sweep_pair<real, ONE>(a, lc, o, qa, ns_a, qr, ns_r, I_a, I_r, S_o, chi_o, dsm, p_near, chunk, mode, win, y2,
-                              p2, c2);
+        if constexpr (STAGED) {
+            Step32 *st = reinterpret_cast<Step32 *>(smem);
+            float4 *rw = reinterpret_cast<float4 *>(smem + a.row_offset);
+            // one call for both rays, the antipode's first
+            for (int64_t q = ns_a > 0 ? qa : qr;; q = qr) {
+                const float I = far_in<float>(a, q, nu_f, F, f, err);
+                const Sweep<float> sw = sweep_staged(a, lc, o, q, I, S_o, chi_o, chunk, st, rw);
+                y2 += sw.y;
+                p2 += sw.p;
+                c2 += sw.c;
+                if (q == qr || ns_r == 0) break;
+            }
+        } else {
+            const real I_a = ns_a > 0 ? far_in<real>(a, qa, nu_f, F, f, err) : (real)0;
+            const real I_r = ns_r > 0 ? far_in<real>(a, qr, nu_f, F, f, err) : (real)0;
+            sweep_pair<real, ONE>(a, lc, o, qa, ns_a, qr, ns_r, I_a, I_r, S_o, chi_o, dsm, p_near, chunk, mode, win,
+                                  y2, p2, c2);
+        }
         const real den = Prec<real>::rcp(y2);
         real u;
         {
@@ -1297,6 +1420,27 @@ void k_radiation_field(RFArgs<real> a)
         a.Lam[(int64_t)o * F + f] = lam_f;
     }
     lambda_partials(a, o, chunk, active, f, nu_f, lam_f);
+}
+
+// FP32: at least 8 waves per SIMD (at most 64 VGPRs), which hide the LDS
+// latency of the line rows; 6 where bins have several lines, whose second
+// line's registers spill at 64; FP64: 4.  The waves of a workgroup
+// share nothing but the line table.
+template <typename real, bool ONE>
+__global__ __launch_bounds__(WAVE * MAX_WAVES) __attribute__((amdgpu_waves_per_eu(sizeof(real) == 4 ? (ONE ? 8 : 6) : 4)))
+void k_radiation_field(RFArgs<real> a)
+{
+    field_of_origin<real, ONE, false>(a);
+}
+
+// The same with steps and their line rows staged for the workgroup's waves, which
+// is the faster way where a point's rows are many or few points are passed over
+// (per_point).
+template <bool ONE>
+__global__ __launch_bounds__(WAVE * MAX_WAVES) __attribute__((amdgpu_waves_per_eu(8)))
+void k_field_staged(RFArgs<float> a)
+{
+    field_of_origin<float, ONE, true>(a);
 }
 
 // The points of a ray pair in order: entry qx from its far end inwards, the
@@ -1804,6 +1948,17 @@ int max_chunk(const mgr_ctx *ctx)
     return ch < CH_MAX ? ch : CH_MAX;
 }
 
+// A line can be inside the window of bin nu_f at some point only if
+// nu_l (1 - 11 pw_max) <= s_max nu_f and nu_l (1 + 11 pw_max) >= s_min nu_f, with
+// shifts in [shift_min, shift_max]: line * lo < nu_f is below the bin's reach,
+// line * hi <= nu_f a candidate.  The margins cover rounding of the shifts and widths.
+void candidate_bounds(const mgr_ctx *ctx, double shift_min, double shift_max, double &lo, double &hi)
+{
+    const double w = LINE_WINDOW * ctx->pw_max;
+    lo = (1.0 + w) * (1.0 + 1.0e-9) / shift_min;
+    hi = (1.0 - w) * (1.0 - 1.0e-9) / shift_max;
+}
+
 // Arguments shared by the radiation-field and image kernels: model tables,
 // rows, candidate-line bounds for shifts in [shift_min, shift_max], launch
 // shape (nwg waves of 64 bins per workgroup, chunks of ch staged steps) over
@@ -1835,12 +1990,7 @@ int make_args(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
     a.I_bdy = ctx->I_bdy;
     a.ray_w = ctx->ray_w;
     a.dshift_max = ctx->dshift_max;
-    // A line can be inside the window of bin nu_f at some point only if
-    // nu_l (1 - 11 pw_max) <= s_max nu_f and nu_l (1 + 11 pw_max) >= s_min nu_f;
-    // the margins cover rounding of the shifts and widths.
-    const double w = LINE_WINDOW * ctx->pw_max;
-    a.cand_lo = (1.0 + w) * (1.0 + 1.0e-9) / shift_min;   // line * cand_lo < nu_f: below
-    a.cand_hi = (1.0 - w) * (1.0 - 1.0e-9) / shift_max;   // line * cand_hi <= nu_f: candidate
+    candidate_bounds(ctx, shift_min, shift_max, a.cand_lo, a.cand_hi);
     a.lstart_threshold = a.cand_lo;
     a.J = ctx->J;
     a.Lam = ctx->Lam;
@@ -1872,12 +2022,14 @@ FieldLds window_lds(const mgr_ctx *ctx, int nwg, int points)
                      points);
 }
 
-// One candidate line per bin: the lines' candidate ranges are disjoint.
-template <typename real>
-bool one_line(const mgr_ctx *ctx, const RFArgs<real> &a)
+// One candidate line per bin of the co-moving frame: the lines' candidate ranges
+// are disjoint.
+bool one_line(const mgr_ctx *ctx)
 {
+    double lo, hi;
+    candidate_bounds(ctx, ctx->shift_min, ctx->shift_max, lo, hi);
     for (int l = 0; l + 1 < ctx->h_tables.L; l++)
-        if (!(ctx->h_tables.line[l] * a.cand_lo <= ctx->h_tables.line[l + 1] * a.cand_hi)) return false;
+        if (!(ctx->h_tables.line[l] * lo <= ctx->h_tables.line[l + 1] * hi)) return false;
     return true;
 }
 
@@ -1895,8 +2047,55 @@ unsigned grid_of(const RFArgs<real> &a)
     return (unsigned)(((int64_t)a.grid_real + 7) / 8) * 8;
 }
 
+// The range of y in which the points of an out-of-window run change nothing
+// (Runs), with chi at most X times the floor there; empty (lo > hi) if there is
+// none.  Such a point closes its row with c = chi dz'_a + chi' dz'_b (rounded
+// twice), at most cb = 2 X dz'_max (1 + 2^-20).  The no-op needs cb < y 2^-25
+// (then c is below half an ulp of y) and cb y < 2^-25 (then 1 + c y rounds to 1).
+void noop_range(const mgr_ctx *ctx, double X, float &lo_out, float &hi_out)
+{
+    lo_out = INFINITY;   // never
+    hi_out = 0.0f;
+    if (!(ctx->hdz32_max > 0.0f)) return;
+    const double cb = 2.0 * X * (double)(float)(CHI_FLOOR * CHI_SCALE) * (double)ctx->hdz32_max * (1.0 + 0x1p-20);
+    const double lo = cb * 0x1p25 * (1.0 + 0x1p-20), hi = 0x1p-25 / cb * (1.0 - 0x1p-20);
+    if (lo < hi && lo < 3.0e38 && hi > 1.0e-37) {
+        lo_out = std::nextafter((float)lo, INFINITY);   // float(lo) may round below lo
+        hi_out = std::nextafter((float)hi, 0.0f);
+    }
+}
+
+// FP32: whether the points are laid out per lane (k_radiation_field) or the steps
+// staged for the workgroup (k_field_staged).  By points a wave brings the rows of
+// all lines to LDS for every point that it evaluates, by steps the workgroup does
+// once per step.  By points is the faster way where most points are passed over
+// and the rows are few, steps staged
+//   - where runs cannot be passed over by their spans: behind a dark boundary (36^3
+//     envelope at 0.05 K 6.8 ms, by points 7.1), with steps beyond 1e18 m (24^3
+//     envelope 2.06, 2.82), and with the skip off (16^3 stress 2.26, 2.65);
+//   - from 15 lines on (24^3 envelope, 31 lines 1.11 ms, by points 1.88; 15 lines
+//     0.55, 0.59; 14 and 13 lines 0.55, 0.55 and 0.55, 0.54);
+//   - with more than 16 chunks of bins, of which five are passed over at all (7 lines,
+//     22 chunks 1.49 ms, by points 1.55; 17 chunks 1.15, 1.17; 11 chunks 0.78, 0.76),
+//     or with more than those five and 12 lines (6 chunks 0.59, 0.63) or bins of
+//     several lines (8 chunks 0.76, 0.91).
+bool per_point(const mgr_ctx *ctx)
+{
+    if (!ctx->masks_valid || !ctx->rf_window_skip || !ctx->rf_spans || !ctx->near_on || ctx->bdy_dark) return false;
+    const int64_t nchunk = (ctx->F + WAVE - 1) / WAVE;
+    if (ctx->L >= 15 || nchunk > 16) return false;
+    if (nchunk > STEP_MASK_CHUNKS && (ctx->L >= 12 || !one_line(ctx))) return false;
+    float lo, hi;
+    noop_range(ctx, NEAR_X, lo, hi);
+    return lo < hi;
+}
+
+// The launch shape's place in the context: of the FP32 kernel by points, the FP64
+// kernel or the FP32 kernel of staged steps.
+int shape_of(const mgr_ctx *ctx, int precision) { return precision == MGR_FP64 ? 1 : per_point(ctx) ? 0 : 2; }
+
 // Launch over origins [o_begin, o_begin + o_count) with nwg waves (64 bins
-// each) per workgroup and chunks of ch staged steps.
+// each) per workgroup and windows of ch points, or chunks of ch staged steps.
 template <typename real>
 int launch_rf(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int ch, int64_t o_begin,
               int64_t o_count)
@@ -1922,22 +2121,14 @@ int launch_rf(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
         a.step_mask = (ctx->masks_valid && ctx->rf_window_skip) ? ctx->step_mask : nullptr;
     else
         a.step_mask = (ctx->masks64_valid && ctx->rf_window_skip) ? ctx->step_mask64 : nullptr;
-    a.noop_lo = INFINITY;   // never
-    a.noop_hi = 0.0f;
-    if (sizeof(real) == 4 && a.step_mask && ctx->hdz32_max > 0.0f) {
-        // An out-of-window sub-point closes its row with c = chi dz'_a + chi' dz'_b (rounded twice),
-        // at most cb = 2 X dz'_max (1 + 2^-20).  The no-op needs cb < y 2^-25 (then c is below half an
-        // ulp of y) and cb y < 2^-25 (then 1 + c y rounds to 1).
-        const double cb = 2.0 * NEAR_X * (double)(float)(CHI_FLOOR * CHI_SCALE) * (double)ctx->hdz32_max * (1.0 + 0x1p-20);
-        const double lo = cb * 0x1p25 * (1.0 + 0x1p-20), hi = 0x1p-25 / cb * (1.0 - 0x1p-20);
-        if (lo < hi && lo < 3.0e38 && hi > 1.0e-37) {
-            a.noop_lo = std::nextafter((float)lo, INFINITY);   // float(lo) may round below lo
-            a.noop_hi = std::nextafter((float)hi, 0.0f);
-        }
+    bool by_point = true;
+    if constexpr (sizeof(real) == 4) {
+        by_point = per_point(ctx);
+        noop_range(ctx, by_point ? NEAR_X : 1.0, a.noop_lo, a.noop_hi);
     }
     a.span_stride = ctx->span_stride;
     if (sizeof(real) == 8 && a.step_mask && ctx->rf_spans) a.span = ctx->span64;
-    if (sizeof(real) == 4 && a.step_mask && ctx->near_on && ctx->rf_spans) {
+    if (sizeof(real) == 4 && by_point) {
         a.span = ctx->span32;
         a.near_p = ctx->near_p;
         a.near_bad = ctx->near_bad;
@@ -1945,7 +2136,18 @@ int launch_rf(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
     a.root_major = ctx->root_major;
     a.far32 = (sizeof(real) == 4 && ctx->far_cache && ctx->far_valid[0]) ? ctx->far_I32 : nullptr;
     a.far64 = (sizeof(real) == 8 && ctx->far_cache && ctx->far_valid[1]) ? ctx->far_I64 : nullptr;
-    const bool one = one_line(ctx, a);
+    const bool one = one_line(ctx);
+    if constexpr (sizeof(real) == 4) {
+        if (!by_point) {
+            a.line_offset = a.row_offset + sizeof(float4) * (a.ch + 1) * ctx->L;
+            const size_t lds = a.line_offset + sizeof(double) * ctx->L;
+            auto kernel = one ? k_field_staged<true> : k_field_staged<false>;
+            hipLaunchKernelGGL(kernel, dim3(grid_of(a)), dim3(WAVE * a.nwg), lds, ctx->stream, a);
+            ctx->last_rf_kernel = one ? "k_field_staged<true>" : "k_field_staged<false>";
+            MGR_LAUNCH_CHECK();
+            return MGR_OK;
+        }
+    }
     const FieldLds lds = window_lds<real>(ctx, a.nwg, a.ch);
     if (lds.points < 2) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
     a.ch = lds.points;
@@ -2024,7 +2226,7 @@ int launch_band(mgr_ctx *ctx)
     a.ch = walk_window(ctx);
     const size_t lds = Window<double>::bytes(ctx->L, a.ch) +
                        sizeof(double) * (4 * (size_t)ctx->nband * WAVE + ctx->L) + sizeof(int) * (ctx->L + 1);
-    auto kernel = one_line(ctx, a) ? k_lambda_band<true> : k_lambda_band<false>;
+    auto kernel = one_line(ctx) ? k_lambda_band<true> : k_lambda_band<false>;
     hipLaunchKernelGGL(kernel, dim3(grid_of(a)), dim3(WAVE), lds, ctx->stream, a);
     MGR_LAUNCH_CHECK();
     const int64_t SL = ctx->band_S * ctx->L;
@@ -2048,10 +2250,10 @@ static int launch_rf_shape(mgr_ctx *ctx, int nwg, int ch, int64_t o_begin, int64
 // there.  FP32 at 64^3 cells (6 lines, 41 points): 31.4 ms against 31.9 with 32
 // points, and 34.1 with 48, which only 26 waves per CU have room for.
 template <typename real>
-static int fitting_window(const mgr_ctx *ctx, const RFArgs<real> &a)
+static int fitting_window(const mgr_ctx *ctx)
 {
     constexpr size_t CU_LDS = 160 * 1024, GRANULE = 1280;
-    const size_t waves = 4 * (sizeof(real) == 8 ? 4 : one_line(ctx, a) ? 8 : 6);
+    const size_t waves = 4 * (sizeof(real) == 8 ? 4 : one_line(ctx) ? 8 : 6);
     const size_t room = CU_LDS / waves / GRANULE * GRANULE, table = sizeof(double) * ctx->L;
     const size_t row = sizeof(typename Prec<real>::row_t) * ctx->L;
     // a wave's LDS is rounded up to 64 bytes
@@ -2077,21 +2279,23 @@ static int fitting_window(const mgr_ctx *ctx, const RFArgs<real> &a)
 template <typename real>
 static int tune(mgr_ctx *ctx, int pi)
 {
+    const bool staged = pi == 2;
     const int nchunk = (int)((ctx->F + WAVE - 1) / WAVE);
     const int chmax = max_chunk<real>(ctx);
     if (chmax < 2) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
-    RFArgs<real> a;
-    const typename Prec<real>::row_t *none = nullptr;
-    int rc = make_args<real>(ctx, none, 1, 2, 0, 1, ctx->shift_min, ctx->shift_max, a);
-    if (rc) return rc;
     const int64_t fill = (WAVES_IN_FLIGHT + nchunk - 1) / nchunk;   // origins that fill the chip
     const int nslice = ctx->N > 2 * fill ? 2 : 1;
     const int64_t per = nslice == 2 ? fill : ctx->N;
-    const int fit = std::min(fitting_window(ctx, a), chmax);
+    const int fit = std::min(fitting_window<real>(ctx), chmax);
     std::vector<int> chs{std::min(16, chmax)}, nwgs;
-    if (fit > chs.back()) chs.push_back(fit);
-    if (nslice == 1 && chmax > chs.back()) chs.push_back(chmax);
-    if (!one_line(ctx, a))
+    if (staged) {
+        if (chmax > 16) chs.push_back(std::min(32, chmax));
+        if (chmax > 32) chs.push_back(chmax);
+    } else {
+        if (fit > chs.back()) chs.push_back(fit);
+        if (nslice == 1 && chmax > chs.back()) chs.push_back(chmax);
+    }
+    if (staged || !one_line(ctx))
         for (int w = 2; w <= MAX_WAVES; w++)
             if (w == nchunk || (nchunk % w) == 0 || w == std::min(nchunk, MAX_WAVES)) nwgs.push_back(w);
     auto launch_slices = [&](int w, int c) {
@@ -2105,10 +2309,10 @@ static int tune(mgr_ctx *ctx, int pi)
     MGR_HIP(hipEventCreate(&e1));
     int best_w = 1, best_c = chs.front();
     float best = 1e30f;
-    rc = launch_slices(1, chs.back());   // warm-up
+    int rc = launch_slices(1, chs.back());   // warm-up
     ctx->tune_log.clear();
     auto time_shape = [&](int w, int points) {
-        const int c = window_lds<real>(ctx, w, points).points;
+        const int c = staged ? points : window_lds<real>(ctx, w, points).points;
         if (c < 2) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
         float ms = 0.0f;
         if (hipEventRecord(e0, ctx->stream) != hipSuccess) return MGR_ERR_DEVICE;
@@ -2128,7 +2332,11 @@ static int tune(mgr_ctx *ctx, int pi)
     };
     for (size_t i = 0; i < chs.size() && !rc; i++) rc = time_shape(1, chs[i]);
     const int window = best_c;
-    for (size_t i = 0; i < nwgs.size() && !rc; i++) rc = time_shape(nwgs[i], window);
+    for (size_t i = 0; i < nwgs.size() && !rc; i++) {
+        if (!staged) rc = time_shape(nwgs[i], window);
+        else   // the waves share the steps: every size
+            for (size_t k = 0; k < chs.size() && !rc; k++) rc = time_shape(nwgs[i], chs[k]);
+    }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc == MGR_ERR_DEVICE ? ctx->fail(MGR_ERR_DEVICE, "radiation-field tuning failed") : rc;
@@ -2139,21 +2347,17 @@ static int tune(mgr_ctx *ctx, int pi)
 
 int tune_radiation_field(mgr_ctx *ctx, int precision)
 {
-    const int pi = precision == MGR_FP64 ? 1 : 0;
+    const int pi = shape_of(ctx, precision);
     if (ctx->rf_nwg[pi] > 0) return MGR_OK;
-    if (ctx->rf_autotune) return pi ? tune<double>(ctx, 1) : tune<float>(ctx, 0);
-    const int nchunk = (int)((ctx->F + WAVE - 1) / WAVE);
-    ctx->rf_nwg[pi] = std::min(nchunk, MAX_WAVES);
-    ctx->rf_ch[pi] = pi ? max_chunk<double>(ctx) : max_chunk<float>(ctx);
-    return MGR_OK;
+    return pi == 1 ? tune<double>(ctx, pi) : tune<float>(ctx, pi);
 }
 
 int launch_rf_kernel(mgr_ctx *ctx, int precision)
 {
-    const int pi = precision == MGR_FP64 ? 1 : 0;
+    const int pi = shape_of(ctx, precision);
     if (ctx->rf_nwg[pi] <= 0) return ctx->fail(MGR_ERR_STATE, "radiation-field launch shape not chosen");
-    return pi ? launch_rf_shape<double>(ctx, ctx->rf_nwg[1], ctx->rf_ch[1], 0, ctx->N)
-              : launch_rf_shape<float>(ctx, ctx->rf_nwg[0], ctx->rf_ch[0], 0, ctx->N);
+    return pi == 1 ? launch_rf_shape<double>(ctx, ctx->rf_nwg[pi], ctx->rf_ch[pi], 0, ctx->N)
+                   : launch_rf_shape<float>(ctx, ctx->rf_nwg[pi], ctx->rf_ch[pi], 0, ctx->N);
 }
 
 }  // namespace mgr
@@ -2245,7 +2449,7 @@ extern "C" int mgr_radiation_field_shape(mgr_ctx *ctx, int precision, int *waves
 {
     if (!ctx) return MGR_ERR_ARGUMENT;
     if (precision != MGR_FP32 && precision != MGR_FP64) return ctx->fail(MGR_ERR_ARGUMENT, "bad precision");
-    const int pi = precision == MGR_FP64 ? 1 : 0;
+    const int pi = shape_of(ctx, precision);
     if (waves_per_group) *waves_per_group = ctx->rf_nwg[pi];
     if (steps_per_chunk) *steps_per_chunk = ctx->rf_ch[pi];
     const int n = (int)ctx->tune_log.size();
@@ -2262,21 +2466,27 @@ extern "C" int mgr_set_radiation_field_shape(mgr_ctx *ctx, int precision, int wa
 {
     if (!ctx) return MGR_ERR_ARGUMENT;
     if (precision != MGR_FP32 && precision != MGR_FP64) return ctx->fail(MGR_ERR_ARGUMENT, "bad precision");
-    const int pi = precision == MGR_FP64 ? 1 : 0;
+    const bool fp64 = precision == MGR_FP64;
+    const int pi = fp64 ? 1 : 0;
     if (waves_per_group == 0 && steps_per_chunk == 0) {
         ctx->rf_nwg[pi] = ctx->rf_ch[pi] = 0;   // the next radiation field tunes again
+        if (!fp64) ctx->rf_nwg[2] = ctx->rf_ch[2] = 0;
     } else {
-        const int chmax = pi ? max_chunk<double>(ctx) : max_chunk<float>(ctx);
+        const int chmax = fp64 ? max_chunk<double>(ctx) : max_chunk<float>(ctx);
         if (waves_per_group < 1 || waves_per_group > MAX_WAVES)
             return ctx->fail(MGR_ERR_ARGUMENT, "waves_per_group must be 1.." + std::to_string(MAX_WAVES));
         if (steps_per_chunk < 2 || steps_per_chunk > chmax)
             return ctx->fail(MGR_ERR_ARGUMENT, "steps_per_chunk must be 2.." + std::to_string(chmax) +
                                                    " for this model's line rows");
-        const FieldLds lds = pi ? window_lds<double>(ctx, waves_per_group, steps_per_chunk)
-                                : window_lds<float>(ctx, waves_per_group, steps_per_chunk);
+        const FieldLds lds = fp64 ? window_lds<double>(ctx, waves_per_group, steps_per_chunk)
+                                  : window_lds<float>(ctx, waves_per_group, steps_per_chunk);
         if (lds.points < 2) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
         ctx->rf_nwg[pi] = waves_per_group;
         ctx->rf_ch[pi] = lds.points;
+        if (!fp64) {
+            ctx->rf_nwg[2] = waves_per_group;
+            ctx->rf_ch[2] = steps_per_chunk;
+        }
     }
     // the ALI graphs were captured with the previous shape
     if (ctx->graph_precision == precision) {
