@@ -2140,7 +2140,7 @@ int launch_rf(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
     if constexpr (sizeof(real) == 4) {
         if (!by_point) {
             a.line_offset = a.row_offset + sizeof(float4) * (a.ch + 1) * ctx->L;
-            const size_t lds = a.line_offset + sizeof(double) * ctx->L;
+            const size_t lds = a.line_offset + (one ? 0 : sizeof(double) * ctx->L);
             auto kernel = one ? k_field_staged<true> : k_field_staged<false>;
             hipLaunchKernelGGL(kernel, dim3(grid_of(a)), dim3(WAVE * a.nwg), lds, ctx->stream, a);
             ctx->last_rf_kernel = one ? "k_field_staged<true>" : "k_field_staged<false>";
@@ -2322,8 +2322,8 @@ static int tune(mgr_ctx *ctx, int pi)
             hipEventElapsedTime(&ms, e0, e1) != hipSuccess)
             return MGR_ERR_DEVICE;
         ctx->tune_log.push_back({w, c, ms});
-        // more waves only for 2 % (fewer schedule the end of a full launch more evenly)
-        if (ms < best * (w > best_w ? 0.98f : 1.0f)) {
+        // more waves only for 2 % (fewer schedule the end of a full launch more evenly), and more staged steps
+        if (ms < best * (w > best_w || (staged && c > best_c) ? 0.98f : 1.0f)) {
             best = ms;
             best_w = w;
             best_c = c;
