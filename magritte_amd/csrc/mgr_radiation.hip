@@ -2248,7 +2248,9 @@ static int launch_rf_shape(mgr_ctx *ctx, int nwg, int ch, int64_t o_begin, int64
 // The largest window whose LDS still admits the waves that the kernel's
 // registers do, 8, 6 or 4 per SIMD: a pair's points take the fewest windows
 // there.  FP32 at 64^3 cells (6 lines, 41 points): 31.4 ms against 31.9 with 32
-// points, and 34.1 with 48, which only 26 waves per CU have room for.
+// points, and 34.1 with 48, which only 26 waves per CU have room for.  FP64 at
+// 24^3 cells with 31 lines (7 points): 3.75 ms with 6 points, 5.2 with 16, and 6.95
+// with 7, whose rows lie 8 apart and meet in the same banks.
 template <typename real>
 static int fitting_window(const mgr_ctx *ctx)
 {
@@ -2292,8 +2294,10 @@ static int tune(mgr_ctx *ctx, int pi)
         if (chmax > 16) chs.push_back(std::min(32, chmax));
         if (chmax > 32) chs.push_back(chmax);
     } else {
-        if (fit > chs.back()) chs.push_back(fit);
-        if (nslice == 1 && chmax > chs.back()) chs.push_back(chmax);
+        // smaller with many lines, then even: the lines' rows are points + 1 apart
+        if (fit > chs.front()) chs.push_back(fit);
+        else if (fit < chs.front()) chs.push_back(std::max(fit / 2 * 2, 2));
+        if (nslice == 1 && chmax > std::max(fit, chs.front())) chs.push_back(chmax);
     }
     if (staged || !one_line(ctx))
         for (int w = 2; w <= MAX_WAVES; w++)

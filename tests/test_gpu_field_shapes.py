@@ -48,3 +48,17 @@ def test_reported_shape_is_the_used_one(nlev, waves, points):
     ctx.compute_radiation_field("fp64")
     assert ctx.radiation_field_shape("fp64")[0] == (w, c)
     ctx.close()
+
+
+@pytest.mark.parametrize("nlev,fit", [(8, 36), (21, 10), (32, 6)])
+def test_the_tuner_tries_the_window_that_fits(nlev, fit):
+    """The FP64 windows timed: 16 points and as many as four waves per SIMD have LDS
+    for (a sixteenth of 160 KB in multiples of 1280 bytes each: 10240), fewer than
+    16 and even with many lines."""
+    from magritte_amd.hip import Context
+    ctx = Context(synthetic.envelope_model(n=6, seed=3, nside=1, nlev=nlev, nquads=7)).setup()
+    ctx.compute_radiation_field("fp64")
+    tried = {c for w, c, _ in ctx.radiation_field_shape("fp64")[1] if w == 1}
+    assert {16, fit} <= tried
+    assert ctx.radiation_field_shape("fp64")[0][1] in tried
+    ctx.close()
