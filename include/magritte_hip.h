@@ -195,7 +195,14 @@ int  mgr_species_info(mgr_ctx *ctx, int64_t *nlspecs, int64_t *nlev, int64_t *nr
  * relative_change_max; lineProducingSpecies.tpp:120-171); the mgr_conv of the
  * driver entry points holds the largest over the species.                   */
 int  mgr_species_convergence(mgr_ctx *ctx, int64_t l, mgr_conv *conv);
+/* Frees a context.  Of its memory the large arrays of the trace, 2 GB per process
+ * at most, stay allocated for the next trace or context, until an allocation of
+ * this library fails or mgr_release_memory is called: before other libraries of
+ * the process need that memory, call it.                                    */
 void mgr_destroy(mgr_ctx *ctx);
+/* Gives back the device memory kept for later contexts; how many bytes it was.
+ * Contexts in use keep theirs.  Any thread may call it at any time.          */
+int64_t mgr_release_memory(void);
 const char *mgr_last_error(const mgr_ctx *ctx);   /* ctx may be NULL (create errors) */
 int  mgr_device_count(int *count);
 

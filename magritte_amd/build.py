@@ -31,6 +31,7 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}", "-Wall",
           "-fno-gpu-rdc", "-munsafe-fp-atomics"]
 
 UNITS = {
+    "mgr_blocks.hip": [],
     "mgr_context.hip": ["-ffp-contract=off"],
     "mgr_trace.hip": ["-ffp-contract=off"],
     "mgr_radiation.hip": [],

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../../include/magritte_hip.h"
+#include "mgr_blocks.hpp"
 
 namespace mgr {
 
@@ -399,9 +400,6 @@ int launch_lambda(mgr_ctx *ctx);
 int launch_band(mgr_ctx *ctx);         // band elements of Lambda* (nband > 0)
 int launch_band_cells(mgr_ctx *ctx);   // band cells and their reverse map (at trace time)
 int copy_to_host(mgr_ctx *ctx, void *dst, const void *src, size_t bytes);
-hipError_t block_malloc(mgr_ctx *ctx, void **p, size_t bytes);
-void block_free(mgr_ctx *ctx, void *p);
-size_t blocks_kept(const mgr_ctx *ctx);   // bytes that block_malloc gives or frees before it fails
 void free_trace(mgr_ctx *ctx);         // the trace's arrays and what is computed from them per step
 void free_far(mgr_ctx *ctx);           // the far-end intensity caches
 int launch_jeff(mgr_ctx *ctx, bool lambda);

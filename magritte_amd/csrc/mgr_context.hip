@@ -36,7 +36,7 @@ int dalloc(mgr_ctx *ctx, T **p, size_t n)
 {
     *p = nullptr;
     if (n == 0) n = 1;
-    hipError_t e = hipMalloc((void **)p, n * sizeof(T));
+    hipError_t e = mgr::device_malloc((void **)p, n * sizeof(T));
     if (e != hipSuccess) {
         *p = nullptr;
         return ctx->fail(MGR_ERR_NOMEM, std::string("hipMalloc of ") + std::to_string(n * sizeof(T)) +
@@ -648,7 +648,7 @@ int upload_models(mgr_ctx *ctx, const mgr_model_view *models, int64_t nmodels)
             rec[q].z = m->position[3 * c + 2];
             rec[q].c = c;
         }
-        MGR_HIP(hipMalloc((void **)&ctx->nb_rec, rec.size() * sizeof(NbRec)));
+        MGR_HIP(mgr::device_malloc((void **)&ctx->nb_rec, rec.size() * sizeof(NbRec)));
         MGR_HIP(hipMemcpy(ctx->nb_rec, rec.data(), rec.size() * sizeof(NbRec), hipMemcpyHostToDevice));
         // the tracer's candidate masks: list lengths, and a margin of 1e-9 of
         // the largest |p - o|_1 |n|_inf over cells and rays
@@ -791,7 +791,7 @@ int upload_models(mgr_ctx *ctx, const mgr_model_view *models, int64_t nmodels)
 template <typename T>
 static void bfree(mgr_ctx *ctx, T *&p)
 {
-    mgr::block_free(ctx, p);
+    mgr::block_free(ctx->stream, p);
     p = nullptr;
 }
 
@@ -856,110 +856,6 @@ int free_model(mgr_ctx *ctx)
 }  // namespace mgr
 
 // ---- C-ABI -------------------------------------------------------------------
-
-// Device memory of the trace and its caches, kept for the next trace or context
-// of the process when it is given back: a model's arrays are a few large blocks,
-// allocated and freed once per model, and the runtime clears and unmaps every
-// one: a 27^3-cell solve frees 1.6 GB and takes 30 ms, 66 to 96 while the
-// clearing of larger models freed before holds the frees up; with the blocks
-// kept 27 in both cases.  At most KEPT bytes are kept,
-// the oldest go first; all go when an allocation fails.  A block is given back
-// when the context's stream, on which alone it is used, is idle; its next
-// owner writes all that it reads.
-namespace {
-struct Blocks {
-    static constexpr size_t LEAST = 4 << 20;     // smaller ones are not kept
-    static constexpr size_t KEPT = (size_t)2 << 30;
-    struct Block {
-        void  *p;
-        size_t bytes;
-        int    device;
-    };
-    std::mutex         m;
-    std::vector<Block> kept;   // oldest first
-    std::vector<Block> used;
-    size_t             held = 0;
-
-    static Blocks &get()
-    {
-        static Blocks *b = new Blocks;   // never destroyed: the runtime may be gone by then
-        return *b;
-    }
-};
-}  // namespace
-
-hipError_t mgr::block_malloc(mgr_ctx *ctx, void **p, size_t bytes)
-{
-    if (bytes < Blocks::LEAST) return hipMalloc(p, bytes);
-    Blocks &b = Blocks::get();
-    std::vector<Blocks::Block> old;
-    try {
-        std::lock_guard<std::mutex> lock(b.m);
-        b.used.reserve(b.used.size() + 1);
-        size_t best = b.kept.size();
-        for (size_t i = 0; i < b.kept.size(); i++)
-            if (b.kept[i].device == ctx->device && b.kept[i].bytes >= bytes && b.kept[i].bytes <= bytes + bytes / 4 &&
-                (best == b.kept.size() || b.kept[i].bytes < b.kept[best].bytes))
-                best = i;
-        if (best < b.kept.size()) {
-            *p = b.kept[best].p;
-            b.used.push_back(b.kept[best]);
-            b.held -= b.kept[best].bytes;
-            b.kept.erase(b.kept.begin() + best);
-            return hipSuccess;
-        }
-        hipError_t e = hipMalloc(p, bytes);
-        if (e != hipSuccess && !b.kept.empty()) {
-            (void)hipGetLastError();
-            for (const auto &k : b.kept) (void)hipFree(k.p);
-            b.kept.clear();
-            b.held = 0;
-            e = hipMalloc(p, bytes);
-        }
-        if (e == hipSuccess) b.used.push_back({*p, bytes, ctx->device});
-        return e;
-    } catch (const std::bad_alloc &) {
-        return hipErrorOutOfMemory;
-    }
-}
-
-size_t mgr::blocks_kept(const mgr_ctx *ctx)
-{
-    Blocks &b = Blocks::get();
-    std::lock_guard<std::mutex> lock(b.m);
-    size_t bytes = 0;
-    for (const auto &k : b.kept)
-        if (k.device == ctx->device) bytes += k.bytes;
-    return bytes;
-}
-
-void mgr::block_free(mgr_ctx *ctx, void *p)
-{
-    if (!p) return;
-    Blocks &b = Blocks::get();
-    const bool idle = hipStreamSynchronize(ctx->stream) == hipSuccess;
-    try {
-        std::lock_guard<std::mutex> lock(b.m);
-        for (size_t i = 0; i < b.used.size(); i++) {
-            if (b.used[i].p != p) continue;
-            const Blocks::Block mine = b.used[i];
-            if (idle && mine.bytes <= Blocks::KEPT) {
-                while (b.held + mine.bytes > Blocks::KEPT) {
-                    (void)hipFree(b.kept.front().p);
-                    b.held -= b.kept.front().bytes;
-                    b.kept.erase(b.kept.begin());
-                }
-                b.kept.push_back(mine);
-                b.held += mine.bytes;
-                p = nullptr;
-            }
-            b.used.erase(b.used.begin() + i);
-            break;
-        }
-    } catch (const std::bad_alloc &) {
-    }
-    if (p) (void)hipFree(p);
-}
 
 // Pinned staging memory of a context for large copies to the host, allocated by
 // the first one: a slot and an event for each worker.
@@ -1131,6 +1027,8 @@ int mgr_species_convergence(mgr_ctx *ctx, int64_t l, mgr_conv *conv)
     conv->relative_change_max = w[2];
     return MGR_OK;
 }
+
+int64_t mgr_release_memory(void) { return (int64_t)blocks_release(); }
 
 void mgr_destroy(mgr_ctx *ctx)
 {

@@ -744,10 +744,10 @@ extern "C" int mgr_mlp_create(int device, uint64_t seed, mgr_mlp **out)
     };
     if (hipSetDevice(device) != hipSuccess) return bail(MGR_ERR_DEVICE);
     if (hipStreamCreate(&mlp->stream) != hipSuccess) return bail(MGR_ERR_DEVICE);
-    if (hipMalloc(&mlp->P, NPAR * sizeof(float)) != hipSuccess || hipMalloc(&mlp->m, NPAR * sizeof(float)) != hipSuccess ||
-        hipMalloc(&mlp->v, NPAR * sizeof(float)) != hipSuccess ||
-        hipMalloc(&mlp->wbf, BF_TOTAL * sizeof(uint16_t)) != hipSuccess ||
-        hipMalloc(&mlp->norm, sizeof(Norm)) != hipSuccess)
+    if (mgr::device_malloc(&mlp->P, NPAR * sizeof(float)) != hipSuccess || mgr::device_malloc(&mlp->m, NPAR * sizeof(float)) != hipSuccess ||
+        mgr::device_malloc(&mlp->v, NPAR * sizeof(float)) != hipSuccess ||
+        mgr::device_malloc(&mlp->wbf, BF_TOTAL * sizeof(uint16_t)) != hipSuccess ||
+        mgr::device_malloc(&mlp->norm, sizeof(Norm)) != hipSuccess)
         return bail(MGR_ERR_NOMEM);
     // He-style initialisation from a 64-bit LCG + Box-Muller, zero biases
     std::vector<float> P(NPAR, 0.0f);
@@ -847,8 +847,8 @@ extern "C" int mgr_mlp_forward(mgr_mlp *mlp, const float *X, int64_t n, float *Y
     if (n == 0) return MGR_OK;
     MLP_HIP(hipSetDevice(mlp->device));
     float *dX = nullptr, *dY = nullptr;
-    MLP_HIP(hipMalloc(&dX, n * IN * sizeof(float)));
-    if (hipMalloc(&dY, n * OUT * sizeof(float)) != hipSuccess) {
+    MLP_HIP(mgr::device_malloc(&dX, n * IN * sizeof(float)));
+    if (mgr::device_malloc(&dY, n * OUT * sizeof(float)) != hipSuccess) {
         (void)hipFree(dX);
         return mlp->fail(MGR_ERR_NOMEM, "forward: output allocation");
     }
@@ -888,9 +888,9 @@ extern "C" int mgr_mlp_loss_grad(mgr_mlp *mlp, const float *X, const float *T, i
     const int G = grid_for_rows(n, GRAD_GROUPS);
     float *dX = nullptr, *dT = nullptr, *dpart = nullptr, *dgrad = nullptr;
     int rc = MGR_OK;
-    if (hipMalloc(&dX, n * IN * sizeof(float)) != hipSuccess || hipMalloc(&dT, n * OUT * sizeof(float)) != hipSuccess ||
-        hipMalloc(&dpart, (size_t)G * (NPAR + 1) * sizeof(float)) != hipSuccess ||
-        hipMalloc(&dgrad, (NPAR + 1) * sizeof(float)) != hipSuccess)
+    if (mgr::device_malloc(&dX, n * IN * sizeof(float)) != hipSuccess || mgr::device_malloc(&dT, n * OUT * sizeof(float)) != hipSuccess ||
+        mgr::device_malloc(&dpart, (size_t)G * (NPAR + 1) * sizeof(float)) != hipSuccess ||
+        mgr::device_malloc(&dgrad, (NPAR + 1) * sizeof(float)) != hipSuccess)
         rc = MGR_ERR_NOMEM;
     if (!rc && (hipMemcpy(dX, X, n * IN * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
                 hipMemcpy(dT, T, n * OUT * sizeof(float), hipMemcpyHostToDevice) != hipSuccess))
@@ -922,9 +922,9 @@ extern "C" int mgr_mlp_train(mgr_mlp *mlp, const float *X, const float *T, int64
     float *dX = nullptr, *dT = nullptr, *dpart = nullptr, *dloss = nullptr;
     TrainState *dst = nullptr;
     int rc = MGR_OK;
-    if (hipMalloc(&dX, n * IN * sizeof(float)) != hipSuccess || hipMalloc(&dT, n * OUT * sizeof(float)) != hipSuccess ||
-        hipMalloc(&dpart, (size_t)Gmax * (NPAR + 1) * sizeof(float)) != hipSuccess ||
-        hipMalloc(&dloss, epochs * sizeof(float)) != hipSuccess || hipMalloc(&dst, sizeof(TrainState)) != hipSuccess)
+    if (mgr::device_malloc(&dX, n * IN * sizeof(float)) != hipSuccess || mgr::device_malloc(&dT, n * OUT * sizeof(float)) != hipSuccess ||
+        mgr::device_malloc(&dpart, (size_t)Gmax * (NPAR + 1) * sizeof(float)) != hipSuccess ||
+        mgr::device_malloc(&dloss, epochs * sizeof(float)) != hipSuccess || mgr::device_malloc(&dst, sizeof(TrainState)) != hipSuccess)
         rc = MGR_ERR_NOMEM;
     TrainState h{};
     h.epoch = -1;
@@ -998,7 +998,7 @@ extern "C" int mgr_features(mgr_ctx *ctx, float *X)
     if (ctx->S > 1) return ctx->fail(MGR_ERR_UNSUPPORTED, "the warm-start features are defined for one line-producing species");
     MGR_HIP(hipSetDevice(ctx->device));
     float *dX = nullptr;
-    MGR_HIP(hipMalloc(&dX, ctx->N * IN * sizeof(float)));
+    MGR_HIP(mgr::device_malloc(&dX, ctx->N * IN * sizeof(float)));
     int rc = mgr::launch_features(ctx, dX, ctx->J_set);   // before any radiation field the J inputs are 0
     if (!rc && (hipStreamSynchronize(ctx->stream) != hipSuccess ||
                 hipMemcpy(X, dX, ctx->N * IN * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess))
@@ -1022,9 +1022,9 @@ extern "C" int mgr_warm_start(mgr_ctx *ctx, mgr_mlp *mlp)
     double *dPrev = nullptr;
     unsigned long long *dCount = nullptr;
     const size_t npop = (size_t)ctx->N * OUT;
-    if (hipMalloc(&dX, ctx->N * IN * sizeof(float)) != hipSuccess ||
-        hipMalloc(&dPrev, npop * sizeof(double)) != hipSuccess ||
-        hipMalloc(&dCount, sizeof(unsigned long long)) != hipSuccess) {
+    if (mgr::device_malloc(&dX, ctx->N * IN * sizeof(float)) != hipSuccess ||
+        mgr::device_malloc(&dPrev, npop * sizeof(double)) != hipSuccess ||
+        mgr::device_malloc(&dCount, sizeof(unsigned long long)) != hipSuccess) {
         (void)hipFree(dX);
         (void)hipFree(dPrev);
         return ctx->fail(MGR_ERR_NOMEM, "warm start: device allocation failed");

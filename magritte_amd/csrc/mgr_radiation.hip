@@ -2520,8 +2520,8 @@ extern "C" int mgr_compute_image(mgr_ctx *ctx, int64_t ray, int precision, doubl
     mgr_ctx::ImageTrace &g = ctx->img;
     const int64_t NF = ctx->N * ctx->F;
     if (!g.I_m) {
-        MGR_HIP(hipMalloc((void **)&g.I_m, NF * sizeof(double)));
-        MGR_HIP(hipMalloc((void **)&g.I_p, NF * sizeof(double)));
+        MGR_HIP(device_malloc((void **)&g.I_m, NF * sizeof(double)));
+        MGR_HIP(device_malloc((void **)&g.I_p, NF * sizeof(double)));
     }
     MGR_HIP(hipMemsetAsync(ctx->err_flag, 0, sizeof(int32_t), ctx->stream));
     rc = precision == MGR_FP64 ? launch_image<double>(ctx, ctx->row64) : launch_image<float>(ctx, ctx->row32);
@@ -2546,7 +2546,7 @@ extern "C" int mgr_set_scattering(mgr_ctx *ctx, int use_scattering)
     MGR_HIP(hipStreamSynchronize(ctx->stream));
     if (use_scattering && !ctx->u_store) {
         const size_t n = (size_t)(ctx->R / 2) * ctx->N * ctx->F;
-        MGR_HIP(hipMalloc((void **)&ctx->u_store, std::max<size_t>(n, 1) * sizeof(double)));
+        MGR_HIP(device_malloc((void **)&ctx->u_store, std::max<size_t>(n, 1) * sizeof(double)));
         MGR_HIP(hipMemset(ctx->u_store, 0, std::max<size_t>(n, 1) * sizeof(double)));
     } else if (!use_scattering && ctx->u_store) {
         (void)hipFree(ctx->u_store);
@@ -2577,8 +2577,8 @@ int launch_far_cache(mgr_ctx *ctx, int precision)
         const int64_t nspan = std::min<int64_t>((ctx->F + WAVE - 1) / WAVE, STEP_MASK_CHUNKS) *
                               ((ctx->span32 ? 1 : 0) + (ctx->span64 ? 1 : 0));
         const size_t spans = (size_t)(nspan * ctx->span_stride) * sizeof(uint16_t);
-        if (hipMemGetInfo(&fr, &tot) != hipSuccess || bytes > (fr + spans + blocks_kept(ctx)) / 4 * 3 ||
-            block_malloc(ctx, buf, std::max<size_t>(bytes, 8)) != hipSuccess) {
+        if (hipMemGetInfo(&fr, &tot) != hipSuccess || bytes > (fr + spans + blocks_kept(ctx->device)) / 4 * 3 ||
+            block_malloc(ctx->device, buf, std::max<size_t>(bytes, 8)) != hipSuccess) {
             (void)hipGetLastError();
             *buf = nullptr;
             ctx->far_bad[pi] = true;

@@ -773,8 +773,8 @@ int launch_band_cells(mgr_ctx *ctx)
     if (ctx->band_rev) (void)hipFree(ctx->band_rev);
     ctx->band_rev_off = nullptr;
     ctx->band_rev = nullptr;
-    MGR_HIP(hipMalloc((void **)&ctx->band_rev_off, (N + 1) * sizeof(int64_t)));
-    MGR_HIP(hipMalloc((void **)&ctx->band_rev, rev.size() * sizeof(int64_t)));
+    MGR_HIP(device_malloc((void **)&ctx->band_rev_off, (N + 1) * sizeof(int64_t)));
+    MGR_HIP(device_malloc((void **)&ctx->band_rev, rev.size() * sizeof(int64_t)));
     MGR_HIP(hipMemcpy(ctx->band_rev_off, off.data(), (N + 1) * sizeof(int64_t), hipMemcpyHostToDevice));
     MGR_HIP(hipMemcpy(ctx->band_rev, rev.data(), rev.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     return MGR_OK;
@@ -790,7 +790,7 @@ struct DeviceBuffer {
 struct BlockBuffer {
     mgr_ctx *ctx;
     void    *p = nullptr;
-    void release() { block_free(ctx, p); p = nullptr; }
+    void release() { block_free(ctx->stream, p); p = nullptr; }
     ~BlockBuffer() { release(); }
 };
 
@@ -807,7 +807,7 @@ int launch_forward_masks(mgr_ctx *ctx)
 {
     const int64_t n = ctx->N * ctx->R;
     if (ctx->fwd_mask || !ctx->trace_masks || ctx->nb_kmax > 63 || n == 0) return MGR_OK;
-    MGR_HIP(hipMalloc((void **)&ctx->fwd_mask, n * sizeof(uint64_t)));
+    MGR_HIP(device_malloc((void **)&ctx->fwd_mask, n * sizeof(uint64_t)));
     hipLaunchKernelGGL(k_forward_masks, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, ctx->stream, ctx->N,
                        (int)ctx->R, ctx->d_cell_model, ctx->d_m_R, ctx->d_m_rbase, ctx->pos, ctx->nb_off, ctx->nb_rec,
                        ctx->is_boundary, ctx->rays, ctx->fwd_tau, ctx->fwd_mask);
@@ -820,9 +820,9 @@ int launch_trace(mgr_ctx *ctx)
     const int64_t N = ctx->N, R = ctx->R, NR = ctx->NQ;
     const unsigned grid = (unsigned)((N * R + 127) / 128);
     if (!ctx->nseg) {
-        MGR_HIP(hipMalloc((void **)&ctx->nseg, NR * sizeof(int32_t)));
-        MGR_HIP(hipMalloc((void **)&ctx->npts, NR * sizeof(int32_t)));
-        MGR_HIP(hipMalloc((void **)&ctx->seg_off, (NR + 1) * sizeof(int64_t)));
+        MGR_HIP(device_malloc((void **)&ctx->nseg, NR * sizeof(int32_t)));
+        MGR_HIP(device_malloc((void **)&ctx->npts, NR * sizeof(int32_t)));
+        MGR_HIP(device_malloc((void **)&ctx->seg_off, (NR + 1) * sizeof(int64_t)));
     }
     static const uint64_t one_bits[2] = {0x3FF0000000000000ull, 0x3FF0000000000000ull};   // 1.0, 1.0
     MGR_HIP(hipMemcpyAsync(ctx->shift_bits, one_bits, 2 * sizeof(uint64_t), hipMemcpyHostToDevice, ctx->stream));
@@ -835,9 +835,9 @@ int launch_trace(mgr_ctx *ctx)
     if (NR > 0) {
         size_t freeb = 0, totb = 0;
         if (hipMemGetInfo(&freeb, &totb) == hipSuccess) {
-            const int64_t budget = std::min<int64_t>((int64_t)(freeb / 4), TRACE_RECORD_BYTES);
+            const int64_t budget = std::min<int64_t>((int64_t)((freeb + blocks_kept(ctx->device)) / 4), TRACE_RECORD_BYTES);
             cap = (int)std::min<int64_t>(ctx->trace_record_steps, budget / NR / (int64_t)sizeof(int32_t) / 4 * 4);
-            if (cap < 4 || block_malloc(ctx, &cells.p, (size_t)NR * cap * sizeof(int32_t)) != hipSuccess) {
+            if (cap < 4 || block_malloc(ctx->device, &cells.p, (size_t)NR * cap * sizeof(int32_t)) != hipSuccess) {
                 (void)hipGetLastError();
                 cells.p = nullptr;
                 cap = 0;
@@ -898,15 +898,15 @@ int launch_trace(mgr_ctx *ctx)
     ctx->far_invalidate();
     free_trace(ctx);
     const int64_t T = std::max<int64_t>(ctx->total_segments, 1);
-    MGR_HIP(block_malloc(ctx, (void **)&ctx->step_mask, T * sizeof(uint8_t)));
-    MGR_HIP(block_malloc(ctx, (void **)&ctx->seg_cell, T * sizeof(int32_t)));
-    MGR_HIP(block_malloc(ctx, (void **)&ctx->seg_shift, T * sizeof(double)));
-    MGR_HIP(block_malloc(ctx, (void **)&ctx->seg_dZ, T * sizeof(double)));
-    MGR_HIP(block_malloc(ctx, (void **)&ctx->seg_f32, T * sizeof(int4)));
-    MGR_HIP(block_malloc(ctx, (void **)&ctx->seg_hdz32, T * sizeof(float)));
+    MGR_HIP(block_malloc(ctx->device, (void **)&ctx->step_mask, T * sizeof(uint8_t)));
+    MGR_HIP(block_malloc(ctx->device, (void **)&ctx->seg_cell, T * sizeof(int32_t)));
+    MGR_HIP(block_malloc(ctx->device, (void **)&ctx->seg_shift, T * sizeof(double)));
+    MGR_HIP(block_malloc(ctx->device, (void **)&ctx->seg_dZ, T * sizeof(double)));
+    MGR_HIP(block_malloc(ctx->device, (void **)&ctx->seg_f32, T * sizeof(int4)));
+    MGR_HIP(block_malloc(ctx->device, (void **)&ctx->seg_hdz32, T * sizeof(float)));
     if (!ctx->far_cell) {
-        MGR_HIP(hipMalloc((void **)&ctx->far_cell, std::max<int64_t>(NR, 1) * sizeof(int32_t)));
-        MGR_HIP(hipMalloc((void **)&ctx->far_shift, std::max<int64_t>(NR, 1) * sizeof(double)));
+        MGR_HIP(device_malloc((void **)&ctx->far_cell, std::max<int64_t>(NR, 1) * sizeof(int32_t)));
+        MGR_HIP(device_malloc((void **)&ctx->far_shift, std::max<int64_t>(NR, 1) * sizeof(double)));
     }
     MGR_HIP(hipMemcpy(ctx->seg_off, off.data(), (NR + 1) * sizeof(int64_t), hipMemcpyHostToDevice));
     if (cells.p)
@@ -985,7 +985,7 @@ int launch_step_masks(mgr_ctx *ctx, bool fp64)
     if (valid || !ctx->traced || !ctx->spectral_set) return MGR_OK;
     uint8_t *&bits_out = fp64 ? ctx->step_mask64 : ctx->step_mask;
     const int64_t T = std::max<int64_t>(ctx->total_segments, 1);
-    if (!bits_out) MGR_HIP(block_malloc(ctx, (void **)&bits_out, T));
+    if (!bits_out) MGR_HIP(block_malloc(ctx->device, (void **)&bits_out, T));
     const double window = fp64 ? MASK_WINDOW64 : MASK_WINDOW;
     const int64_t N = ctx->N;
     const int nchunk = (int)std::min<int64_t>((ctx->F + WAVE - 1) / WAVE, STEP_MASK_CHUNKS);
@@ -1003,13 +1003,13 @@ int launch_step_masks(mgr_ctx *ctx, bool fp64)
     if (rm != ctx->root_major) ctx->graph_precision = -1;   // captured launches hold the old order
     ctx->root_major = rm;
     DeviceBuffer red, win, cnt, near_pw;
-    MGR_HIP(hipMalloc(&win.p, (size_t)N * STEP_MASK_CHUNKS * MAX_WIN * 2 * sizeof(double)));
-    MGR_HIP(hipMalloc(&cnt.p, (size_t)N * STEP_MASK_CHUNKS));
+    MGR_HIP(device_malloc(&win.p, (size_t)N * STEP_MASK_CHUNKS * MAX_WIN * 2 * sizeof(double)));
+    MGR_HIP(device_malloc(&cnt.p, (size_t)N * STEP_MASK_CHUNKS));
     // two bytes per chunk and step beside the trace's forty-odd; without memory
     // for them the bits (FP32) or nothing (FP64) is left out
     uint16_t *&span = fp64 ? ctx->span64 : ctx->span32;
     ctx->span_stride = (T + 3) / 4 * 4;
-    if (!span && block_malloc(ctx, (void **)&span, (size_t)nchunk * ctx->span_stride * sizeof(uint16_t)) != hipSuccess) {
+    if (!span && block_malloc(ctx->device, (void **)&span, (size_t)nchunk * ctx->span_stride * sizeof(uint16_t)) != hipSuccess) {
         (void)hipGetLastError();
         span = nullptr;
     }
@@ -1018,7 +1018,7 @@ int launch_step_masks(mgr_ctx *ctx, bool fp64)
         // the largest dz' bounds the row closings of out-of-window sub-points,
         // the largest populations what they can add
         std::vector<uint64_t> h(tb.L + 1, 0);
-        MGR_HIP(hipMalloc(&red.p, h.size() * sizeof(uint64_t)));
+        MGR_HIP(device_malloc(&red.p, h.size() * sizeof(uint64_t)));
         uint64_t *d = (uint64_t *)red.p;
         MGR_HIP(hipMemsetAsync(d, 0, h.size() * sizeof(uint64_t), ctx->stream));
         if (ctx->total_segments > 0)
@@ -1037,7 +1037,7 @@ int launch_step_masks(mgr_ctx *ctx, bool fp64)
         const double w2 = span && ctx->hdz32_max > 0.0f ? near_window2(ctx, ratio, p_min) : 0.0;
         near = w2 > 0.0;
         if (near) {
-            MGR_HIP(hipMalloc(&near_pw.p, (size_t)N * sizeof(double)));
+            MGR_HIP(device_malloc(&near_pw.p, (size_t)N * sizeof(double)));
             hipLaunchKernelGGL(k_near_widths, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, ctx->stream, N,
                                ctx->tables, ctx->pop_tot, ctx->IW64, ctx->pw_cmax, (const double *)d, w2,
                                (double *)near_pw.p);
@@ -1075,7 +1075,7 @@ extern "C" int mgr_window_skip_stats(mgr_ctx *ctx, int64_t *point_chunks, int64_
     const int64_t T = ctx->total_segments;
     const int nchunk = (int)std::min<int64_t>((ctx->F + mgr::WAVE - 1) / mgr::WAVE, mgr::STEP_MASK_CHUNKS);
     unsigned long long *d = nullptr, h[2] = {0, 0};
-    MGR_HIP(hipMalloc((void **)&d, sizeof(h)));
+    MGR_HIP(device_malloc((void **)&d, sizeof(h)));
     hipError_t e = hipMemsetAsync(d, 0, sizeof(h), ctx->stream);
     if (e == hipSuccess && T > 0) {
         hipLaunchKernelGGL(k_mask_stats, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, ctx->stream, T, nchunk,
@@ -1116,12 +1116,12 @@ int launch_trace_image(mgr_ctx *ctx, int64_t ray)
     const int mrc = launch_forward_masks(ctx);
     if (mrc) return mrc;
     if (!g.nseg) {
-        MGR_HIP(hipMalloc((void **)&g.nseg, NQ * sizeof(int32_t)));
-        MGR_HIP(hipMalloc((void **)&g.npts, NQ * sizeof(int32_t)));
-        MGR_HIP(hipMalloc((void **)&g.seg_off, (NQ + 1) * sizeof(int64_t)));
-        MGR_HIP(hipMalloc((void **)&g.far_cell, NQ * sizeof(int32_t)));
-        MGR_HIP(hipMalloc((void **)&g.far_shift, NQ * sizeof(double)));
-        MGR_HIP(hipMalloc((void **)&g.origin_shift, NQ * sizeof(double)));
+        MGR_HIP(device_malloc((void **)&g.nseg, NQ * sizeof(int32_t)));
+        MGR_HIP(device_malloc((void **)&g.npts, NQ * sizeof(int32_t)));
+        MGR_HIP(device_malloc((void **)&g.seg_off, (NQ + 1) * sizeof(int64_t)));
+        MGR_HIP(device_malloc((void **)&g.far_cell, NQ * sizeof(int32_t)));
+        MGR_HIP(device_malloc((void **)&g.far_shift, NQ * sizeof(double)));
+        MGR_HIP(device_malloc((void **)&g.origin_shift, NQ * sizeof(double)));
     }
     const unsigned grid = (unsigned)((NQ + 127) / 128);
     static const uint64_t one_bits[2] = {0x3FF0000000000000ull, 0x3FF0000000000000ull};   // 1.0, 1.0
@@ -1154,11 +1154,11 @@ int launch_trace_image(mgr_ctx *ctx, int64_t ray)
             if (p) (void)hipFree(p);
         g.seg_cell = nullptr; g.seg_shift = nullptr; g.seg_dZ = nullptr; g.seg_f32 = nullptr; g.seg_hdz32 = nullptr;
         const int64_t T = std::max<int64_t>(off[NQ], 1);
-        MGR_HIP(hipMalloc((void **)&g.seg_cell, T * sizeof(int32_t)));
-        MGR_HIP(hipMalloc((void **)&g.seg_shift, T * sizeof(double)));
-        MGR_HIP(hipMalloc((void **)&g.seg_dZ, T * sizeof(double)));
-        MGR_HIP(hipMalloc((void **)&g.seg_f32, T * sizeof(int4)));
-        MGR_HIP(hipMalloc((void **)&g.seg_hdz32, T * sizeof(float)));
+        MGR_HIP(device_malloc((void **)&g.seg_cell, T * sizeof(int32_t)));
+        MGR_HIP(device_malloc((void **)&g.seg_shift, T * sizeof(double)));
+        MGR_HIP(device_malloc((void **)&g.seg_dZ, T * sizeof(double)));
+        MGR_HIP(device_malloc((void **)&g.seg_f32, T * sizeof(int4)));
+        MGR_HIP(device_malloc((void **)&g.seg_hdz32, T * sizeof(float)));
         g.total_segments = T;
     }
     MGR_HIP(hipMemcpy(g.seg_off, off.data(), (NQ + 1) * sizeof(int64_t), hipMemcpyHostToDevice));
@@ -1217,10 +1217,10 @@ int mgr_get_ray(mgr_ctx *ctx, int64_t origin, int64_t ray, int64_t capacity, int
     const int64_t cap = std::max<int64_t>(capacity, 1);
     int64_t *dc = nullptr, *dn = nullptr;
     double *ds = nullptr, *dz = nullptr;
-    MGR_HIP(hipMalloc((void **)&dc, cap * sizeof(int64_t)));
-    MGR_HIP(hipMalloc((void **)&ds, cap * sizeof(double)));
-    MGR_HIP(hipMalloc((void **)&dz, cap * sizeof(double)));
-    MGR_HIP(hipMalloc((void **)&dn, sizeof(int64_t)));
+    MGR_HIP(device_malloc((void **)&dc, cap * sizeof(int64_t)));
+    MGR_HIP(device_malloc((void **)&ds, cap * sizeof(double)));
+    MGR_HIP(device_malloc((void **)&dz, cap * sizeof(double)));
+    MGR_HIP(device_malloc((void **)&dn, sizeof(int64_t)));
     hipLaunchKernelGGL(k_expand_ray, dim3(1), dim3(64), 0, ctx->stream, (int32_t)origin,
                        ctx->h_cell_qbase[origin] + ray, ctx->seg_off, ctx->nseg, ctx->seg_cell, ctx->seg_shift,
                        ctx->seg_dZ, ctx->dshift_max, capacity, dc, ds, dz, dn);
@@ -1250,8 +1250,8 @@ int mgr_get_npoints_on_rays_rest(mgr_ctx *ctx, int64_t *npoints)
     if (mrc) return mrc;
     const int64_t N = ctx->N, R = ctx->R, NQ = N * R;
     int32_t *d_ns = nullptr, *d_np = nullptr;
-    MGR_HIP(hipMalloc((void **)&d_ns, std::max<int64_t>(NQ, 1) * sizeof(int32_t)));
-    if (hipMalloc((void **)&d_np, std::max<int64_t>(NQ, 1) * sizeof(int32_t)) != hipSuccess) {
+    MGR_HIP(device_malloc((void **)&d_ns, std::max<int64_t>(NQ, 1) * sizeof(int32_t)));
+    if (device_malloc((void **)&d_np, std::max<int64_t>(NQ, 1) * sizeof(int32_t)) != hipSuccess) {
         (void)hipFree(d_ns);
         return ctx->fail(MGR_ERR_DEVICE, "out of device memory");
     }

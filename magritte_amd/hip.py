@@ -28,6 +28,7 @@ SIGNATURES = {
     "mgr_batch_info": ([_vp, _vp, _vp], _i),
     "mgr_batch_convergence": ([_vp, _vp, _vp], _i),
     "mgr_destroy": ([_vp], None),
+    "mgr_release_memory": ([], _i64),
     "mgr_last_error": ([_vp], C.c_char_p),
     "mgr_device_count": ([_vp], _i),
     "mgr_compute_spectral_discretisation": ([_vp], _i),
@@ -116,6 +117,13 @@ def device_count():
     n = C.c_int(0)
     load().mgr_device_count(C.byref(n))
     return n.value
+
+
+def release_memory():
+    """Give back the device memory that closed contexts left for the next one (2 GB
+    at most; the library takes it back by itself when an allocation of its own
+    fails).  Returns the bytes."""
+    return load().mgr_release_memory()
 
 
 def _p(a):
