@@ -390,7 +390,6 @@ int upload_models(mgr_ctx *ctx, const mgr_model_view *models, int64_t nmodels);
 int free_model(mgr_ctx *ctx);
 int launch_cell_tables(mgr_ctx *ctx);
 int launch_emissivity_opacity(mgr_ctx *ctx);
-int clear_near_bad(mgr_ctx *ctx);   // before the rows of newly set populations (outside graph capture)
 int launch_trace(mgr_ctx *ctx);
 int launch_forward_masks(mgr_ctx *ctx);   // candidate neighbours of every (cell, ray), once
 int launch_far_cache(mgr_ctx *ctx, int precision);   // outside graph capture

@@ -187,13 +187,15 @@ __global__ void k_boundary_intensities(int64_t NB, int F, const int32_t *__restr
 }
 
 // LineProducingSpecies::update_using_LTE (lineProducingSpecies.tpp:82-115).
+// near_bad: see k_emissivity_opacity, which sets it anew.
 __global__ void k_lte(int64_t N, int V, int nspecs, int num, const double *__restrict__ abundance,
                       const double *__restrict__ T, const double *__restrict__ weight,
                       const double *__restrict__ energy, double *__restrict__ pop,
-                      double *__restrict__ pop_tot)
+                      double *__restrict__ pop_tot, int32_t *__restrict__ near_bad)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= N) return;
+    if (p == 0) *near_bad = 0;
     const double ptot = abundance[p * nspecs + num];
     pop_tot[p] = ptot;
     double pf = 0.0;
@@ -204,6 +206,8 @@ __global__ void k_lte(int64_t N, int V, int nspecs, int num, const double *__res
     }
     for (int i = 0; i < V; i++) pop[p * V + i] *= ptot / pf;
 }
+
+__global__ void k_clear_word(int32_t *word) { *word = 0; }
 
 __global__ void k_pop_tot(int64_t N, int nspecs, int num, const double *__restrict__ abundance,
                           double *__restrict__ pop_tot)
@@ -277,12 +281,6 @@ int launch_emissivity_opacity(mgr_ctx *ctx)
                        ctx->jrad, ctx->pop, ctx->IW64, ctx->W11, ctx->emis, ctx->opac, ctx->row32,
                        ctx->row64, ctx->pop_tot, ctx->near_bad);
     MGR_LAUNCH_CHECK();
-    return MGR_OK;
-}
-
-int clear_near_bad(mgr_ctx *ctx)
-{
-    MGR_HIP(hipMemsetAsync(ctx->near_bad, 0, sizeof(int32_t), ctx->stream));
     return MGR_OK;
 }
 
@@ -1154,11 +1152,10 @@ int mgr_compute_LTE_level_populations(mgr_ctx *ctx)
         hipLaunchKernelGGL(k_lte, dim3(grid_for(ctx->N, 256)), dim3(256), 0, ctx->stream, ctx->N,
                            (int)ctx->sp_V[l], (int)ctx->nspecs, (int)ctx->sp_num[l], ctx->abundance,
                            ctx->temperature, ctx->lweight + ctx->sp_voff[l], ctx->energy + ctx->sp_voff[l],
-                           ctx->pop + ctx->N * ctx->sp_voff[l], ctx->pop_tot + ctx->N * l);
+                           ctx->pop + ctx->N * ctx->sp_voff[l], ctx->pop_tot + ctx->N * l, ctx->near_bad);
         MGR_LAUNCH_CHECK();
     }
-    int rc = clear_near_bad(ctx);
-    if (!rc) rc = launch_emissivity_opacity(ctx);
+    int rc = launch_emissivity_opacity(ctx);
     if (rc) return rc;
     MGR_HIP(hipStreamSynchronize(ctx->stream));
     ctx->pops_set = true;
@@ -1187,7 +1184,8 @@ int mgr_set_populations(mgr_ctx *ctx, const double *population)
     if (!ctx || !population) return MGR_ERR_ARGUMENT;
     int rc = copy_in(ctx, ctx->pop, population, ctx->N * ctx->V * sizeof(double));
     if (rc) return rc;
-    if ((rc = clear_near_bad(ctx))) return rc;
+    hipLaunchKernelGGL(k_clear_word, dim3(1), dim3(1), 0, ctx->stream, ctx->near_bad);
+    MGR_LAUNCH_CHECK();
     if ((rc = launch_emissivity_opacity(ctx))) return rc;
     MGR_HIP(hipStreamSynchronize(ctx->stream));
     ctx->pops_set = true;

@@ -625,14 +625,17 @@ __global__ __launch_bounds__(THREADS) void k_mlp_forward(const float *__restrict
 // The warm start's guard: a cell whose predicted populations are not all
 // finite and positive, or give one of its lines an opacity <= 0 (the sign of
 // n_j B_a - n_i B_s, as the emissivity/opacity kernel forms it), takes back
-// the populations it held before the prediction.
+// the populations it held before the prediction.  near_bad is cleared for that
+// kernel, which sets it anew.
 __global__ void k_warm_guard(int64_t N, int V, int L, const int32_t *__restrict__ irad,
                              const int32_t *__restrict__ jrad, const double *__restrict__ Ba,
                              const double *__restrict__ Bs, const double *__restrict__ prev,
-                             double *__restrict__ pop, unsigned long long *__restrict__ count)
+                             double *__restrict__ pop, unsigned long long *__restrict__ count,
+                             int32_t *__restrict__ near_bad)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= N) return;
+    if (p == 0) *near_bad = 0;
     double *x = pop + p * V;
     bool ok = true;
     for (int i = 0; i < V; i++) ok = ok && x[i] > 0.0 && __builtin_isfinite(x[i]);
@@ -1037,10 +1040,10 @@ extern "C" int mgr_warm_start(mgr_ctx *ctx, mgr_mlp *mlp)
         hipLaunchKernelGGL(k_mlp_forward, dim3(grid_for_rows(ctx->N, 1024)), dim3(THREADS), LDS_FORWARD, ctx->stream, dX,
                            ctx->N, mlp->wbf, mlp->P, mlp->norm, (float *)nullptr, ctx->pop_tot, ctx->pop);
         hipLaunchKernelGGL(k_warm_guard, dim3((unsigned)((ctx->N + 255) / 256)), dim3(256), 0, ctx->stream, ctx->N,
-                           (int)OUT, (int)ctx->L, ctx->irad, ctx->jrad, ctx->Ba, ctx->Bs, dPrev, ctx->pop, dCount);
+                           (int)OUT, (int)ctx->L, ctx->irad, ctx->jrad, ctx->Ba, ctx->Bs, dPrev, ctx->pop, dCount,
+                           ctx->near_bad);
         if (hipGetLastError() != hipSuccess) rc = ctx->fail(MGR_ERR_DEVICE, "warm-start launch failed");
     }
-    if (!rc) rc = clear_near_bad(ctx);
     if (!rc) rc = launch_emissivity_opacity(ctx);
     unsigned long long nfb = 0;
     if (!rc && (hipMemcpyAsync(&nfb, dCount, sizeof(nfb), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
