@@ -10,8 +10,8 @@
 //
 // With n_off_diag = 0 every rate-equation triplet couples levels of a single
 // cell, so the reference's global SparseLU<COLAMD> of size (N V)^2 is block
-// diagonal: here one thread solves one cell's V x V system with partial
-// pivoting in FP64 registers (V known at compile time for V <= 8).
+// diagonal: here eight lanes solve one cell's V x V system with partial
+// pivoting in FP64 registers for V <= 8, and one thread does above.
 #include <algorithm>
 #include <cmath>
 #include <mutex>
@@ -1090,7 +1090,7 @@ int launch_ng(mgr_ctx *ctx)
 }  // namespace mgr
 
 // The host's per-model activity flags to the device, unless every model was
-// active there already; and no error yet (outside graphs).
+// active there already (outside graphs).
 int mgr::set_active(mgr_ctx *ctx, bool all)
 {
     if (all)

@@ -58,7 +58,8 @@
 //   u = (p_A + p_B) / (y_A + y_B),  Lambda = (c_A + c_B) / (y_A + y_B).
 //
 // Line profiles.  FP64 variant: the window of get_eta_and_chi is decided in
-// FP64 exactly as the reference.  FP32 variant: each lane evaluates the lines
+// FP64 exactly as the reference, or, where each bin meets one line, on the
+// profile's argument (eta_chi_one).  FP32 variant: each lane evaluates the lines
 // whose +-11-width window can contain its bin at any point of the model (its
 // candidate lines; lines outside contribute exactly zero in FP64 too, and
 // inside the window but beyond ~10 widths exp(-x^2) underflows FP32), with the
@@ -1939,8 +1940,8 @@ __global__ void k_band_sum(int64_t N, int64_t SL, int nchunk, const double *__re
 }
 
 // Largest chunk of staged steps that fits the LDS budget with the cells'
-// line rows, at most CH_MAX.
-template <typename real, bool X64 = false>
+// line rows, at most CH_MAX: also the most points that a launch shape can ask for.
+template <typename real>
 int max_chunk(const mgr_ctx *ctx)
 {
     const size_t per_entry = sizeof(Step) + sizeof(typename Prec<real>::row_t) * ctx->L + 64;
@@ -1963,7 +1964,7 @@ void candidate_bounds(const mgr_ctx *ctx, double shift_min, double shift_max, do
 // rows, candidate-line bounds for shifts in [shift_min, shift_max], launch
 // shape (nwg waves of 64 bins per workgroup, chunks of ch staged steps) over
 // origins [o_begin, o_begin + o_count).  The trace pointers are the caller's.
-template <typename real, bool X64 = false>
+template <typename real>
 int make_args(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int ch, int64_t o_begin,
               int64_t o_count, double shift_min, double shift_max, RFArgs<real> &a)
 {
@@ -2007,7 +2008,7 @@ int make_args(mgr_ctx *ctx, const typename Prec<real>::row_t *rows, int nwg, int
     const int64_t groups = o_count * a.ngroups;
     if (groups > INT32_MAX - 8) return ctx->fail(MGR_ERR_UNSUPPORTED, "too many workgroups");
     a.grid_real = (int)groups;
-    if (ch < 2 || ch > max_chunk<real, X64>(ctx)) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
+    if (ch < 2 || ch > max_chunk<real>(ctx)) return ctx->fail(MGR_ERR_UNSUPPORTED, "line rows do not fit the LDS budget");
     a.ch = ch;
     a.row_offset = ((sizeof(Step) * (ch + 1) + 63) / 64) * 64;
     return MGR_OK;
@@ -2170,7 +2171,7 @@ int launch_image(mgr_ctx *ctx, const typename Prec<real>::row_t *rows)
     const int nchunk = (int)((ctx->F + WAVE - 1) / WAVE);
     const mgr_ctx::ImageTrace &g = ctx->img;
     RFArgs<real> a;
-    int rc = make_args<real, F32>(ctx, rows, F32 ? std::min(nchunk, MAX_WAVES) : 1, max_chunk<real, F32>(ctx), 0,
+    int rc = make_args<real>(ctx, rows, F32 ? std::min(nchunk, MAX_WAVES) : 1, max_chunk<real>(ctx), 0,
                                   ctx->N, g.shift_min, g.shift_max, a);
     if (rc) return rc;
     a.step_mask = nullptr;   // the masks index the co-moving cache, not the image's trace

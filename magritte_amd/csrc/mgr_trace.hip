@@ -146,15 +146,6 @@ __device__ __forceinline__ Walk trace_walk(int64_t N, const double *__restrict__
         }
         shift_nxt = REST ? rest_shift(vel, nxt, sx, sy, sz) : doppler_shift(vel, o, nxt, nx, ny, nz);
     }
-    // a co-moving walk owns its last block of four slots: those past its end are empty
-    if (FILL && !REST)
-        for (; w & 3; w++) {
-            seg_cell[w] = 0;
-            seg_shift[w] = 0.0;
-            seg_dZ[w] = 0.0;
-            seg_f32[w] = make_int4(0, 0, 0, 0);
-            seg_hdz32[w] = 0.0f;
-        }
     // the last, partly filled block of the record
     if (!FILL && rec && k.steps <= cap) rec[(k.steps - 1) >> 2] = acc;
     return k;
