@@ -15,6 +15,9 @@ per second over the timed steps.  The JSON line also carries:
                    (28 per point and bin) per second against MI355X's FP32
                    peak (157.3 TFLOP/s published; 78.6 without packed FP32,
                    which this build does not use, in "frac_non_packed").
+                   These count every point of every pair, also those that
+                   the kernel passes over as exact no-ops: what the vector
+                   ALUs did issue is "valu_issue_frac".
                    "traffic" and "hbm" give the measured HBM bytes per launch
                    and their rate against the 8 TB/s peak; "equivalent_bytes"
                    are the dtau/S/u/Lambda* bytes an HBM-staged solver would
@@ -76,7 +79,7 @@ PEAK_FP64_TFLOPS = 78.6
 # Kernel sources whose hash the counter summary under profiles/ records: the
 # counters describe the benched kernel only when the hashes agree.
 KERNEL_SOURCES = ("magritte_amd/csrc/mgr_radiation.hip", "magritte_amd/csrc/mgr_ray.hpp",
-                  "magritte_amd/csrc/mgr_common.hpp")
+                  "magritte_amd/csrc/mgr_common.hpp", "magritte_amd/csrc/mgr_lds.hpp")
 
 
 def log(msg):
@@ -266,6 +269,8 @@ def roofline_entry(sum_ndep, nfreqs, solves, k_ms, precision, kernel, counters_w
         "traffic": traffic,
         "kernel_ms": round(k_ms, 3),
         "flops_per_point_bin": FLOPS_PER_POINT_BIN,
+        "note": "achieved and its fractions count every point of every pair, also those passed over as exact "
+                "no-ops; valu_issue_frac is what the vector ALUs issued",
         "hbm": ({"achieved": round(traffic / (k_ms * 1e-3) / 1e9, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                  "frac": round(traffic / (k_ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 4)} if traffic else None),
         "valu_issue_frac": prof.get("valu_issue_frac") if same else None,
