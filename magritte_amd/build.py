@@ -32,6 +32,7 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}", "-Wall",
 
 UNITS = {
     "mgr_blocks.hip": [],
+    "mgr_copy.hip": [],
     "mgr_context.hip": ["-ffp-contract=off"],
     "mgr_trace.hip": ["-ffp-contract=off"],
     "mgr_radiation.hip": [],

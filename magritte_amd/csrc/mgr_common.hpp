@@ -12,6 +12,7 @@
 
 #include "../../include/magritte_hip.h"
 #include "mgr_blocks.hpp"
+#include "mgr_copy.hpp"
 
 namespace mgr {
 
@@ -138,10 +139,6 @@ __host__ __device__ inline int lane_bin(int i, int L, int F, bool root_major)
 // Device-resident model and state (SoA).  Indices follow the reference:
 // J(p,f) at f + p*F (radiation.tpp:11-15), populations at i + p*V
 // (lineProducingSpecies.tpp:24-30), emissivity/opacity at k + p*L (lines.tpp:19-34).
-namespace mgr {
-struct Bounce;
-}
-
 struct mgr_ctx {
     int         device = 0;
     hipStream_t stream = nullptr;
@@ -398,7 +395,7 @@ int tune_radiation_field(mgr_ctx *ctx, int precision);   // outside graph captur
 int launch_lambda(mgr_ctx *ctx);
 int launch_band(mgr_ctx *ctx);         // band elements of Lambda* (nband > 0)
 int launch_band_cells(mgr_ctx *ctx);   // band cells and their reverse map (at trace time)
-int copy_to_host(mgr_ctx *ctx, void *dst, const void *src, size_t bytes);
+int copy_to_host(mgr_ctx *ctx, void *dst, const void *src, size_t bytes);   // complete on return
 void free_trace(mgr_ctx *ctx);         // the trace's arrays and what is computed from them per step
 void free_far(mgr_ctx *ctx);           // the far-end intensity caches
 int launch_jeff(mgr_ctx *ctx, bool lambda);

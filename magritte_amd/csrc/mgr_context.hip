@@ -5,15 +5,11 @@
 // Compiled with -ffp-contract=off: these kernels restate FP64 expressions of
 // the reference and must round exactly as its scalar code does.
 #include <algorithm>
-#include <atomic>
 #include <cfloat>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <mutex>
 #include <numeric>
-#include <system_error>
-#include <thread>
 
 #include "mgr_common.hpp"
 
@@ -855,83 +851,11 @@ int free_model(mgr_ctx *ctx)
 
 // ---- C-ABI -------------------------------------------------------------------
 
-// Pinned staging memory of a context for large copies to the host, allocated by
-// the first one: a slot and an event for each worker.
-struct mgr::Bounce {
-    static constexpr size_t SLOT = 2 << 20;
-    static constexpr int    WORKERS = 8;
-    std::mutex busy;   // held by the copy that uses the slots
-    char      *slots = nullptr;
-    hipEvent_t event[WORKERS] = {};
-
-    bool allocate()
-    {
-        if (slots) return true;
-        for (auto &e : event)
-            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
-        return hipHostMalloc((void **)&slots, WORKERS * SLOT, hipHostMallocDefault) == hipSuccess;
-    }
-    ~Bounce()
-    {
-        for (auto e : event)
-            if (e) (void)hipEventDestroy(e);
-        if (slots) (void)hipHostFree(slots);
-    }
-};
-
-// Chunks of a copy to the host, each claimed by one worker: to its pinned slot
-// by the copy engine, and on to dst while other workers' chunks are on their way.
-static hipError_t copy_chunks(mgr_ctx *ctx, mgr::Bounce &b, int worker, std::atomic<size_t> &next, char *dst,
-                              const char *src, size_t bytes)
-{
-    hipError_t e = hipSetDevice(ctx->device);
-    char *slot = b.slots + worker * b.SLOT;
-    for (size_t off; e == hipSuccess && (off = next.fetch_add(b.SLOT)) < bytes;) {
-        const size_t n = std::min(b.SLOT, bytes - off);
-        e = hipMemcpyAsync(slot, src + off, n, hipMemcpyDeviceToHost, ctx->stream);
-        if (e == hipSuccess) e = hipEventRecord(b.event[worker], ctx->stream);
-        if (e == hipSuccess) e = hipEventSynchronize(b.event[worker]);
-        if (e == hipSuccess) std::memcpy(dst + off, slot, n);
-    }
-    return e;
-}
-
-// Device to host memory, complete on return; the context's stream is idle.
-// Into pageable memory a plain copy is bound by one thread that moves the data
-// and takes the page faults of a fresh array: 139 MB at 17 GB/s (4.5 fresh);
-// with up to 8 threads 38 GB/s (22 fresh).  Below 4 MB starting the threads
-// costs what they gain (4 MB: 0.24 ms plain, 0.19 so; 1 MB: 0.07 and 0.09).
 int mgr::copy_to_host(mgr_ctx *ctx, void *dst, const void *src, size_t bytes)
 {
-    if (bytes >= 2 * Bounce::SLOT) {
-        Bounce &b = *ctx->bounce;
-        std::unique_lock<std::mutex> mine(b.busy, std::try_to_lock);   // another thread's copy goes on by itself
-        if (mine && b.allocate()) {
-            std::atomic<size_t> next{0};
-            std::atomic<int> failed{0};
-            auto work = [&](int worker) {
-                const hipError_t e =
-                    copy_chunks(ctx, b, worker, next, static_cast<char *>(dst), static_cast<const char *>(src), bytes);
-                if (e != hipSuccess) failed = (int)e;
-            };
-            const int workers = (int)std::min<size_t>({(size_t)Bounce::WORKERS, (bytes + Bounce::SLOT - 1) / Bounce::SLOT,
-                                                       std::max<size_t>(1, std::thread::hardware_concurrency())});
-            std::thread th[Bounce::WORKERS];
-            try {
-                for (int w = 1; w < workers; w++) th[w] = std::thread(work, w);
-            } catch (const std::system_error &) {   // no more threads: those there are do it all
-            }
-            work(0);
-            for (auto &t : th)
-                if (t.joinable()) t.join();
-            if (!failed) return MGR_OK;
-            (void)hipStreamSynchronize(ctx->stream);   // no copy into the slots goes on
-            return ctx->fail(MGR_ERR_DEVICE, std::string("copy to the host: ") + hipGetErrorString((hipError_t)failed.load()));
-        }
-        if (mine) (void)hipGetLastError();   // no staging memory: the plain copy
-    }
-    MGR_HIP(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
-    return MGR_OK;
+    const hipError_t e = copy_out(*ctx->bounce, ctx->device, ctx->stream, dst, src, bytes);
+    return e == hipSuccess ? MGR_OK
+                           : ctx->fail(MGR_ERR_DEVICE, std::string("copy to the host: ") + hipGetErrorString(e));
 }
 
 extern "C" {

@@ -16,7 +16,9 @@
 // steps, the points that can lie in a line window (lane = step, then lane =
 // point; the spans of sub-points in the window are precomputed with the
 // trace), brings their line rows (1/width and the emissivity/opacity
-// prefactors per line) into LDS and walks them (sweep_pair).  J and the Lambda*
+// prefactors per line) into LDS and walks them (sweep_pair).  Some FP32 models
+// (many lines or bins, dark boundaries, very long steps) have the steps staged for
+// a workgroup of several chunks instead (sweep_staged, per_point).  J and the Lambda*
 // diagonal accumulate in FP64 registers over rays and are written once per
 // (cell, bin): no atomics.  Workgroups are mapped to XCDs in contiguous origin
 // ranges so that neighbouring origins share an L2.
@@ -27,7 +29,7 @@
 // and recurrences are 19.5 per point and wave, 65 % of all.  Decoding each
 // step in the elimination loop and stepping every point took 49 ms; on the
 // stress envelope (36^3, ~10 points per step) 44 against 19 ms.  FP64: 221
-// against 148 ms and 192 against 94 ms.
+// against 152 ms and 192 against 97 ms.
 //
 // The tridiagonal Feautrier system of a ray pair is solved two-sided: each ray
 // of the pair is eliminated from its boundary inwards in the Rybicki-Hummer
@@ -1794,7 +1796,7 @@ __device__ __forceinline__ double profile64(double width, double freq_diff)
 // (125 VGPRs, 8 KB of LDS).  A walk with per-step scalar loads and divisions in
 // every lane, three rcp per point, five arrays of 3 (nband + 1) points in LDS
 // and butterfly sums per element and transition took 9.5 ms at 20^3 cells, 84
-// bins and one band; this one takes 3.3 ms.
+// bins and one band; this one takes 3.4 ms.
 template <bool ONE>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_lambda_band(RFArgs<double> a)
 {
