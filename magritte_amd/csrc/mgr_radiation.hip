@@ -2456,7 +2456,8 @@ extern "C" int mgr_radiation_field_shape(mgr_ctx *ctx, int precision, int *waves
 {
     if (!ctx) return MGR_ERR_ARGUMENT;
     if (precision != MGR_FP32 && precision != MGR_FP64) return ctx->fail(MGR_ERR_ARGUMENT, "bad precision");
-    const int pi = shape_of(ctx, precision);
+    int pi = shape_of(ctx, precision);
+    if (pi == 2 && (!ctx->masks_valid || ctx->rf_nwg[2] == 0) && ctx->rf_nwg[0] > 0) pi = 0;   // not known yet: the last one
     if (waves_per_group) *waves_per_group = ctx->rf_nwg[pi];
     if (steps_per_chunk) *steps_per_chunk = ctx->rf_ch[pi];
     const int n = (int)ctx->tune_log.size();

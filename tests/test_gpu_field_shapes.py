@@ -62,3 +62,19 @@ def test_the_tuner_tries_the_window_that_fits(nlev, fit):
     assert {16, fit} <= tried
     assert ctx.radiation_field_shape("fp64")[0][1] in tried
     ctx.close()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+def test_the_shape_outlives_the_frequencies(precision):
+    """A tuned shape is reported, and used again, after the frequencies are set anew."""
+    from magritte_amd.hip import Context
+    ctx = Context(synthetic.envelope_model(n=7, seed=3, nside=1)).setup()
+    ctx.compute_radiation_field(precision)
+    tuned, J = ctx.radiation_field_shape(precision)[0], ctx.J()
+    assert tuned[0] > 0
+    ctx.compute_spectral_discretisation()
+    assert ctx.radiation_field_shape(precision)[0] == tuned
+    ctx.compute_boundary_intensities()
+    ctx.compute_radiation_field(precision)
+    assert ctx.radiation_field_shape(precision)[0] == tuned and np.array_equal(ctx.J(), J)
+    ctx.close()
