@@ -23,6 +23,14 @@ hipError_t block_malloc(int device, void **p, size_t bytes);
 // Given back when the stream, on which alone it was used, is idle.
 void       block_free(hipStream_t stream, void *p);
 
+// What only saves time is allocated where a quarter of the memory stays free for what
+// is needed: `bytes` more beside `taken` of it already there, `available` bytes being
+// free or kept.
+constexpr bool leaves_quarter(size_t bytes, size_t taken, size_t available)
+{
+    return bytes + taken <= (available + taken) / 4 * 3;
+}
+
 size_t blocks_kept(int device);   // bytes that device_malloc gives back before it fails
 size_t blocks_release();          // gives all of them back now; how many bytes they had
 

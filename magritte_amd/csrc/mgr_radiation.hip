@@ -2564,9 +2564,9 @@ namespace mgr {
 
 // Builds the far-end intensity cache of a precision when it is missing or
 // stale (once per trace, frequency grid and boundary intensities).  It is
-// skipped, and the kernel computes the intensities itself, when the cache
-// would take more than three quarters of the free device memory or an entry
-// has no boundary cell at its far end (the kernel then reports that error).
+// skipped, and the kernel computes the intensities itself, when the cache and
+// the spans would take more than three quarters of the device memory free
+// without them, or an entry has no boundary cell at its far end (the kernel then reports that error).
 int launch_far_cache(mgr_ctx *ctx, int precision)
 {
     const int pi = precision == MGR_FP64 ? 1 : 0;
@@ -2576,12 +2576,11 @@ int launch_far_cache(mgr_ctx *ctx, int precision)
     void **buf = pi ? (void **)&ctx->far_I64 : (void **)&ctx->far_I32;
     const size_t bytes = (size_t)ctx->NQ * (size_t)ctx->F * (pi ? sizeof(double) : sizeof(float));
     if (!*buf) {
-        // of the memory free without the spans, which are worth less, and kept blocks
         size_t fr = 0, tot = 0;
         const int64_t nspan = std::min<int64_t>((ctx->F + WAVE - 1) / WAVE, STEP_MASK_CHUNKS) *
                               ((ctx->span32 ? 1 : 0) + (ctx->span64 ? 1 : 0));
         const size_t spans = (size_t)(nspan * ctx->span_stride) * sizeof(uint16_t);
-        if (hipMemGetInfo(&fr, &tot) != hipSuccess || bytes > (fr + spans + blocks_kept(ctx->device)) / 4 * 3 ||
+        if (hipMemGetInfo(&fr, &tot) != hipSuccess || !leaves_quarter(bytes, spans, fr + blocks_kept(ctx->device)) ||
             block_malloc(ctx->device, buf, std::max<size_t>(bytes, 8)) != hipSuccess) {
             (void)hipGetLastError();
             *buf = nullptr;

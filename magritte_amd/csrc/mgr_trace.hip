@@ -997,12 +997,17 @@ int launch_step_masks(mgr_ctx *ctx, bool fp64)
     MGR_HIP(device_malloc(&win.p, (size_t)N * STEP_MASK_CHUNKS * MAX_WIN * 2 * sizeof(double)));
     MGR_HIP(device_malloc(&cnt.p, (size_t)N * STEP_MASK_CHUNKS));
     // two bytes per chunk and step beside the trace's forty-odd; without memory
-    // for them the bits (FP32) or nothing (FP64) is left out
+    // for them the steps are staged (FP32) or the bits are used (FP64)
     uint16_t *&span = fp64 ? ctx->span64 : ctx->span32;
     ctx->span_stride = (T + 3) / 4 * 4;
-    if (!span && block_malloc(ctx->device, (void **)&span, (size_t)nchunk * ctx->span_stride * sizeof(uint16_t)) != hipSuccess) {
-        (void)hipGetLastError();
-        span = nullptr;
+    if (!span) {
+        size_t fr = 0, tot = 0;
+        const size_t bytes = (size_t)nchunk * ctx->span_stride * sizeof(uint16_t);
+        if (hipMemGetInfo(&fr, &tot) != hipSuccess || !leaves_quarter(bytes, 0, fr + blocks_kept(ctx->device)) ||
+            block_malloc(ctx->device, (void **)&span, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            span = nullptr;
+        }
     }
     bool near = false;
     if (!fp64) {
